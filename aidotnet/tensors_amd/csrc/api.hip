@@ -340,6 +340,10 @@ int paged_common(void* ctx, void* stream, int kind, const void* q, const void* k
         if (need) { int st = acquire_ws(c, stream, need, &ws); if (st) return st; }
         return hip_status(c, aidn::attn_decode((hipStream_t)stream, kind, p, eff, ws), "paged attn_decode");
     }
+    // key-range partials where the query tiles alone leave most of the chip idle (as in attn_common)
+    const size_t need = aidn::attn_fwd_workspace_bytes(kind, p);
+    void* ws = nullptr;
+    if (need && acquire_ws(c, stream, need, &ws) == AIDN_OK) { p.workspace = ws; p.workspace_bytes = need; }
     return hip_status(c, aidn::attn_fwd((hipStream_t)stream, kind, p), "paged attn_fwd");
 }
 

@@ -217,16 +217,26 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     constexpr bool WIDE16 = EB == 2 && DP * EB > 128;
     auto k_swz = [](int key) -> int { return (EB == 4 || WIDE16) ? (key & 15) : ((key >> 1) & 7); };
     auto v_swz = [](int key) -> int { return EB == 4 ? (((key >> 2) & 1) << 3) : WIDE16 ? ((key & 3) << 2) : (((key >> 1) & 1) << 2); };
+    int rows = 0;                  // paged cache: pool rows of this wave's keys, one tile per lane
     auto issue_tile = [&](int tile, int stage) {
         constexpr int ROWB = DP * EB;                      // 256 / 128 bytes per key row
         constexpr int KPL = 1024 / ROWB;                   // keys per 1 KiB wave-load
         constexpr int LPW = BC / KPL / 4;                  // wave-loads per wave and tile (K and V each)
         constexpr int CPRW = ROWB / 16;                    // chunks per row
+        constexpr int NK = KPL * LPW;                      // keys per wave and tile
         const int ld_key = lane / CPRW, ld_pos = lane % CPRW;
+        // first row of the wave's keys and the last one to load, relative to it
+        int row0 = tile * BC + NK * wave_s, left = a.Sk - 1 - row0;
+        if (bt) {
+            const int last_group = (a.Sk - 1) / NK * NK;
+            if ((tile & 63) == 0) rows = paged_tile_rows(bt, a.bsz, a.dbsz, NK * wave_s, BC, tile, lane, last_group);
+            left = a.Sk - 1 - min(row0, last_group);
+            row0 = __builtin_amdgcn_readlane(rows, tile & 63);
+        }
 #pragma unroll
         for (int i = 0; i < LPW; i++) {
             const int key = KPL * (LPW * wave + i) + ld_key;               // key inside the tile
-            const long long gkey = min(tile * BC + key, a.Sk - 1);
+            const long long gkey = row0 + min(KPL * i + ld_key, left);
             attn_dma16(K + gkey * a.ks[2] + (ld_pos ^ k_swz(key)) * E, lds0 + stage * KBYTES + (LPW * wave_s + i) * 1024);
             attn_dma16(V + gkey * a.vs[2] + (ld_pos ^ v_swz(key)) * E,
                        lds0 + 2 * KBYTES + stage * VBYTES + (LPW * wave_s + i) * 1024);
@@ -478,7 +488,11 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 #define ATTN_HEAD_GROUP 4
 // Depth of the register ring that prefetches MFMA operand fragments from LDS inside a tile; must divide 8.
 #define AIDN_ATTN_RING 4
-template <typename T, typename OutT, int D = 128>
+// PAGED: K and V are pools behind a block table (block size a multiple of 16); a wave's 16 keys of a tile then lie in one block, and all
+// that changes is where the uniform base of its loads comes from (paged_tile_rows).  A 512-query chunk after 3584 keys (bf16, 32 / 8
+// heads) took 341 us on the general kernel, whose loads go through registers and which cannot split the keys of its 128 query tiles; here
+// 46 us and 16 us for the merge of its four key ranges.
+template <typename T, typename OutT, int D = 128, bool PAGED = false>
 __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(const AttnArgs a)
 {
     typedef uint16_t raw_t;
@@ -545,10 +559,13 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
     // keys this workgroup sees: all of them, or its split's range (which may be empty)
     int Sk = a.Sk;
     long long qoff = a.qoff;                 // causal: query i sees keys j <= i + qoff (j counted from the first key of the range)
+    int kbeg = 0;
     if (a.nsplit > 1) {
-        const int kbeg = split * a.chunk;
-        K += (long long)kbeg * a.ks[2];
-        V += (long long)kbeg * a.vs[2];
+        kbeg = split * a.chunk;
+        if constexpr (!PAGED) {
+            K += (long long)kbeg * a.ks[2];
+            V += (long long)kbeg * a.vs[2];
+        }
         Sk = max(0, min(a.chunk, a.Sk - kbeg));
         qoff -= kbeg;
     }
@@ -582,10 +599,24 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
     for (int i = 0; i < NL; i++) k_lane_off[i] = (uint32_t)(ld_key * k_row_bytes) + ((ld_pos ^ (KPL * i + ld_key)) << 4);
 #pragma unroll
     for (int i = 0; i < 2; i++) v_lane_off[i] = (uint32_t)(ld_key * v_row_bytes) + ((ld_pos ^ (((KPL * i + ld_key) & 3) << 2)) << 4);
+    // the row of the wave's first key of a tile, and for the last tile the rows that exist from there on
+    int rows = 0;
+    auto tile_row = [&](int tile) -> int {
+        if constexpr (!PAGED) return tile * BC + 16 * wave_s;
+        return __builtin_amdgcn_readlane(rows, tile & 63);
+    };
+    auto rows_left = [&](int tile) -> int {             // (a group of keys that lies past the end repeats the last group / the last row)
+        const int g = tile * BC + 16 * wave_s;
+        return Sk - 1 - (PAGED ? min(g, (Sk - 1) & ~15) : g);
+    };
+    auto next_rows = [&](int tile) {                     // ahead of the loads of a tile
+        if constexpr (PAGED)
+            if ((tile & 63) == 0) rows = paged_tile_rows(a.bt + b * a.bt_bs, a.bsz, a.dbsz, kbeg + 16 * wave_s, BC, tile, lane, (a.Sk - 1) & ~15);
+    };
     auto issue_k = [&](int tile) {
         const uint32_t dst = lds0 + (tile & 1) * KBYTES + wave_s * (16 * ROWB);
         if (tile * BC + BC <= Sk) {
-            const unsigned char* src = (const unsigned char*)K + (long long)(tile * BC + 16 * wave_s) * k_row_bytes;
+            const unsigned char* src = (const unsigned char*)K + (long long)tile_row(tile) * k_row_bytes;
             if (a.stream) {
 #pragma unroll
                 for (int i = 0; i < NL; i++) attn_dma16_base_stream(src + KPL * i * k_row_bytes, k_lane_off[i], dst + i * 1024);
@@ -594,18 +625,20 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
                 for (int i = 0; i < NL; i++) attn_dma16_base(src + KPL * i * k_row_bytes, k_lane_off[i], dst + i * 1024);
             }
         } else {
+            const long long row0 = tile_row(tile);
+            const int left = rows_left(tile);
 #pragma unroll
             for (int i = 0; i < NL; i++) {
                 int key = KPL * (wave * NL + i) + ld_key;          // key inside the tile
-                int gkey = min(tile * BC + key, Sk - 1);           // clamp: rows past the end are masked later
-                attn_dma16(K + (long long)gkey * a.ks[2] + (ld_pos ^ (key & 15)) * 8, dst + i * 1024);
+                const long long gkey = row0 + min(KPL * i + ld_key, left);      // clamp: rows past the end are masked later
+                attn_dma16(K + gkey * a.ks[2] + (ld_pos ^ (key & 15)) * 8, dst + i * 1024);
             }
         }
     };
     auto issue_v = [&](int tile) {
         const uint32_t dst = lds0 + 2 * KBYTES + (tile & 1) * VBYTES + wave_s * (16 * ROWB);
         if (tile * BC + BC <= Sk) {
-            const unsigned char* src = (const unsigned char*)V + (long long)(tile * BC + 16 * wave_s) * v_row_bytes;
+            const unsigned char* src = (const unsigned char*)V + (long long)tile_row(tile) * v_row_bytes;
             if (a.stream) {
 #pragma unroll
                 for (int i = 0; i < NL; i++) attn_dma16_base_stream(src + KPL * i * v_row_bytes, v_lane_off[i & 1], dst + i * 1024);
@@ -614,11 +647,13 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
                 for (int i = 0; i < NL; i++) attn_dma16_base(src + KPL * i * v_row_bytes, v_lane_off[i & 1], dst + i * 1024);
             }
         } else {
+            const long long row0 = tile_row(tile);
+            const int left = rows_left(tile);
 #pragma unroll
             for (int i = 0; i < NL; i++) {
                 int key = KPL * (wave * NL + i) + ld_key;
-                int gkey = min(tile * BC + key, Sk - 1);
-                attn_dma16(V + (long long)gkey * a.vs[2] + (ld_pos ^ ((key & 3) << 2)) * 8, dst + i * 1024);
+                const long long gkey = row0 + min(KPL * i + ld_key, left);
+                attn_dma16(V + gkey * a.vs[2] + (ld_pos ^ ((key & 3) << 2)) * 8, dst + i * 1024);
             }
         }
     };
@@ -659,7 +694,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
     const int klim = key_limit(qi) - 4 * h;
     const int wave_klim = __builtin_amdgcn_readfirstlane(key_limit(wq_min));
 
-    if (ntiles > 0) { issue_k(0); issue_v(0); }
+    if (ntiles > 0) { next_rows(0); issue_k(0); issue_v(0); }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
@@ -707,6 +742,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
         // issued one per MFMA inside the first phase below (a vector-memory instruction holds the wave's issue slot for
         // some tens of cycles; there it is covered by the running MFMA).  Otherwise all at once here.
         const bool spread = !a.stream && j < nact && j + 1 < ntiles && (j + 1) * BC + BC <= Sk;
+        if (j + 1 < ntiles) next_rows(j + 1);
         if (j + 1 < ntiles && !spread) { issue_k(j + 1); issue_v(j + 1); }
         if (j < nact) {
             const int kv0 = j * BC;
@@ -752,8 +788,8 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
             // takes them ahead of the other wave's instructions on the SIMD, whose exponentials fill the gaps (1-2 % measured)
             __builtin_amdgcn_s_setprio(2);
             if (spread) {
-                const unsigned char* ksrc = (const unsigned char*)K + (long long)((j + 1) * BC + 16 * wave_s) * k_row_bytes;
-                const unsigned char* vsrc = (const unsigned char*)V + (long long)((j + 1) * BC + 16 * wave_s) * v_row_bytes;
+                const unsigned char* ksrc = (const unsigned char*)K + (long long)tile_row(j + 1) * k_row_bytes;
+                const unsigned char* vsrc = (const unsigned char*)V + (long long)tile_row(j + 1) * v_row_bytes;
                 const uint32_t kdst = lds0 + (stage ^ 1) * KBYTES + wave_s * (16 * ROWB);
                 const uint32_t vdst = lds0 + 2 * KBYTES + (stage ^ 1) * VBYTES + wave_s * (16 * ROWB);
 #pragma unroll
@@ -966,10 +1002,10 @@ __global__ __launch_bounds__(128) void attn_split_merge_kernel(const AttnArgs a)
     if (t == 0 && a.lse) a.lse[row] = L > 0.0f ? (M + __builtin_amdgcn_logf(L)) * LN2 : -INFINITY;
 }
 
-template <typename T, typename OutT, int D = 128>
+template <typename T, typename OutT, int D = 128, bool PAGED = false>
 static hipError_t launch_attn_dl(AttnArgs a, hipStream_t stream)
 {
-    auto kern = attn_fwd_dl_kernel<T, OutT, D>;
+    auto kern = attn_fwd_dl_kernel<T, OutT, D, PAGED>;
     constexpr int smem = 2 * (64 * 2 * D + 64 * 2 * D);      // K and V tiles, two stages each (64 KB; 128 KB at head dimension 256)
     static unsigned long long attr_done = 0;
     if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done)) return e;
@@ -1269,10 +1305,12 @@ static bool attn_aligned16(const void* ptr, const long long* s, int bytes)
     return ((uintptr_t)ptr & 15u) == 0 && (s[0] * bytes) % 16 == 0 && (s[1] * bytes) % 16 == 0 && (s[2] * bytes) % 16 == 0;
 }
 
-// the fast kernel: 16-bit, head dimension 128, aligned contiguous rows, plain (optionally causal) attention
+// the fast kernel: 16-bit, head dimension 128, aligned rows, plain (optionally causal) attention
 static bool attn_dl_applies(int kind, const AttnParams& p)
 {
-    if (kind == 0 || p.D != 128 || !(p.scale > 0.0f) || p.block_table || !p.allow_fast_path) return false;
+    if (kind == 0 || p.D != 128 || !(p.scale > 0.0f) || !p.allow_fast_path) return false;
+    // (behind a block table: blocks of a multiple of 16 keys, fp32 output, which is what the paged entry points return)
+    if (p.block_table && (!paged_block_fits(p.block_table, p.block_size) || p.out16)) return false;
     if (p.bias != nullptr || (p.mask && p.mask_mode != 0) || p.softcap > 0.0f) return false;
     if (!(attn_aligned16(p.q, p.qs, 2) && attn_aligned16(p.k, p.ks, 2) && attn_aligned16(p.v, p.vs, 2))) return false;
     // the kernel addresses the K/V rows of a 4-key load group with unsigned 32-bit byte offsets
@@ -1326,6 +1364,7 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     for (int i = 0; i < 3; i++) { a.qs[i] = p.qs[i]; a.ks[i] = p.ks[i]; a.vs[i] = p.vs[i]; a.os[i] = p.os[i]; }
     a.qtiles = 0;
     a.bt = p.block_table; a.bsz = p.block_size; a.bt_bs = p.block_table_stride;
+    a.dbsz = make_fastdiv((uint32_t)(p.block_table ? p.block_size : 1));
     if (p.block_table && p.weights) return hipErrorInvalidValue;      // the weights output does not follow a block table
     const int eb = kind == 0 ? 4 : 2, e = 16 / eb;
     const int oeb = (kind == 0 || !p.out16) ? 4 : 2;
@@ -1335,12 +1374,14 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     a.vec_in = (p.D % e == 0) && al(p.q, p.qs, eb) && al(p.k, p.ks, eb) && al(p.v, p.vs, eb);
     a.vec_out = (p.D % 4 == 0) && al(p.o, p.os, oeb);
     const bool full = p.bias != nullptr || a.mask_mode != 0 || p.softcap > 0.0f;
+    // the direct-to-LDS instances: plain / causal, 16-byte aligned rows, contiguous or in blocks of a multiple of 16 keys
+    const bool dma = !full && a.vec_in && paged_block_fits(p.block_table, p.block_size) && g_attn_allow_dl;
     hipError_t err;
     // fast path: 16-bit, head dim 128, aligned rows, plain (optionally causal) attention
     // the fast kernel addresses K/V rows of a 4-key load group with unsigned 32-bit byte offsets
     const bool rows32 = p.ks[2] > 0 && p.ks[2] < (1LL << 28) && p.vs[2] > 0 && p.vs[2] < (1LL << 28);
-    const bool dl = kind != 0 && !full && a.vec_in && p.D == 128 && p.scale > 0.0f && rows32 && !p.block_table && g_attn_allow_dl;
-    if (dl && p.workspace && attn_dl_applies(kind, p)) {
+    const bool dl = attn_dl_applies(kind, p);
+    if (dl && p.workspace) {
         int chunk;
         const int ns = attn_dl_splits(p, &chunk);
         if (ns > 1 && p.workspace_bytes >= (size_t)p.B * p.H * p.Sq * ns * 130 * sizeof(float)) {
@@ -1357,30 +1398,32 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     }
     if (pipelined) err = launch_attn_prefill(kind, p.out16, a, stream);
     else
+    if (dl && p.block_table) err = kind == 1 ? launch_attn_dl<f16_t, float, 128, true>(a, stream) : launch_attn_dl<bf16_t, float, 128, true>(a, stream);
+    else
     if (dl) {
         if (kind == 1) err = p.out16 ? launch_attn_dl<f16_t, f16_t>(a, stream) : launch_attn_dl<f16_t, float>(a, stream);
         else err = p.out16 ? launch_attn_dl<bf16_t, bf16_t>(a, stream) : launch_attn_dl<bf16_t, float>(a, stream);
     } else
     if (kind == 0) {
         // fp32: 64-key tiles while two workgroups still fit the LDS of a CU (head dimension up to 64), else 32-key tiles
-        if (p.D == 64 && !full && a.vec_in && !p.block_table && g_attn_allow_dl) err = launch_attn<float, float, 64, 64, false, 2, true>(a, stream);
-        else if (p.D == 128 && !full && a.vec_in && !p.block_table && g_attn_allow_dl) err = launch_attn<float, float, 128, 32, false, 2, true>(a, stream);
+        if (p.D == 64 && dma) err = launch_attn<float, float, 64, 64, false, 2, true>(a, stream);
+        else if (p.D == 128 && dma) err = launch_attn<float, float, 128, 32, false, 2, true>(a, stream);
         else if (p.D <= 64) err = full ? (p.D <= 32 ? launch_attn<float, float, 32, 64, true, 2>(a, stream) : launch_attn<float, float, 64, 64, true, 2>(a, stream))
                                   : (p.D <= 32 ? launch_attn<float, float, 32, 64, false, 2>(a, stream) : launch_attn<float, float, 64, 64, false, 2>(a, stream));
         else err = dispatch_attn_d<float, float, 32>(a, full, stream);
     }
-    else if (p.D == 256 && !full && a.vec_in && !p.block_table && g_attn_allow_dl && rows32 && p.scale > 0.0f && p.allow_fast_path != 2) {
+    else if (p.D == 256 && dma && !p.block_table && rows32 && p.scale > 0.0f && p.allow_fast_path != 2) {
         // head dimension 256, plain / causal, aligned rows: the phase-structured kernel at that width (64-key tiles of 512-byte rows,
         // one workgroup per CU); allow_fast_path 2 (test hook) pins the older form below
         if (kind == 1) err = p.out16 ? launch_attn_dl<f16_t, f16_t, 256>(a, stream) : launch_attn_dl<f16_t, float, 256>(a, stream);
         else err = p.out16 ? launch_attn_dl<bf16_t, bf16_t, 256>(a, stream) : launch_attn_dl<bf16_t, float, 256>(a, stream);
     }
-    else if (p.D == 256 && !full && a.vec_in && !p.block_table && g_attn_allow_dl) {
+    else if (p.D == 256 && dma) {
         // head dimension 256, plain / causal, aligned contiguous K/V: the direct-to-LDS form on 32-key tiles (Q streamed)
         if (kind == 1) err = p.out16 ? launch_attn<f16_t, f16_t, 256, 32, false, 2, true>(a, stream) : launch_attn<f16_t, float, 256, 32, false, 2, true>(a, stream);
         else err = p.out16 ? launch_attn<bf16_t, bf16_t, 256, 32, false, 2, true>(a, stream) : launch_attn<bf16_t, float, 256, 32, false, 2, true>(a, stream);
     }
-    else if (p.D == 64 && !full && a.vec_in && !p.block_table && g_attn_allow_dl) {
+    else if (p.D == 64 && dma) {
         // head dimension 64, plain / causal, aligned contiguous K/V: the direct-to-LDS form of the general kernel
         if (kind == 1) err = p.out16 ? launch_attn<f16_t, f16_t, 64, 64, false, 2, true>(a, stream) : launch_attn<f16_t, float, 64, 64, false, 2, true>(a, stream);
         else err = p.out16 ? launch_attn<bf16_t, bf16_t, 64, 64, false, 2, true>(a, stream) : launch_attn<bf16_t, float, 64, 64, false, 2, true>(a, stream);

@@ -39,7 +39,22 @@ struct AttnArgs {
     int vec_in;    // q/k/v rows are 16-byte aligned and D is a multiple of the 16-byte element count
     int vec_out;
     const int* bt; int bsz; long long bt_bs;   // block table of a paged K/V cache (null = contiguous), block size, batch stride
+    FastDiv dbsz;  // direct-to-LDS kernels on a paged cache: the block size as a divisor
 };
+
+// Pool rows of a paged cache for the direct-to-LDS kernels.  A wave loads NK consecutive keys of every key tile (NK = 16 or 8), which
+// lie in one block when the block size is a multiple of 16, so one row number serves the wave and its loads keep the form of the
+// contiguous case (uniform base, fixed lane offsets).  Lane i of `rows` holds the row of the wave's first key in tile (tile0 + i), 64
+// tiles per table read: a tile costs one lane read instead of a table access in front of its loads.
+__device__ __forceinline__ int paged_tile_rows(const int* __restrict__ bt, int bsz, FastDiv dbsz, int first_key, int tile_keys, int tile0, int lane,
+                                               int last_group)
+{
+    const int key = min(first_key + (tile0 + lane) * tile_keys, last_group);      // (groups past the end repeat the last one)
+    const int blk = (int)fastdiv((uint32_t)key, dbsz);
+    return bt[blk] * bsz + (key - blk * bsz);
+}
+// block sizes the direct-to-LDS kernels take (the row numbers of a pool fit 31 bits at any size that fits the memory)
+inline bool paged_block_fits(const int* bt, int bsz) { return !bt || bsz % 16 == 0; }
 
 template <typename T> struct Raw2;
 template <> struct Raw2<float> { typedef uint32_t type; };
