@@ -147,6 +147,73 @@ template <> __device__ __forceinline__ uint32_t pack2_p<bf16_t>(float a, float b
     return __builtin_bit_cast(uint32_t, v);
 }
 
+// Merge of one query row's partials over key ranges: P = [n][2 + dpad] floats (m, l, unnormalised O), n <= 64, dpad even.  The row
+// is merged by WPR waves of the workgroup (1, or all 4), wave `part` of them taking the ranges part, part + WPR, ...; afterwards
+// lane i of wave part 0 holds the normalised elements 2 i, 2 i + 1 (and 128 + 2 i, + 1 with NV = 2) and the log-sum-exp.
+// Bound by memory latency: eight partial rows per wave are asked for together with the (m, l) pairs, so up to 8 WPR ranges cost one
+// round trip; up to eight ranges need no barrier and no LDS.  A range that saw no key weighs zero and adds nothing.
+typedef float f32x2p __attribute__((ext_vector_type(2)));
+template <int NV, int WPR>
+__device__ __forceinline__ float merge_partials(const float* __restrict__ P, int n, int dpad, int D, int part, int lane, f32x2p (&out)[NV])
+{
+    const long long stride = 2 + dpad;
+    const float* ml = P + min(lane, n - 1) * stride;
+    const float m = lane < n ? ml[0] : -INFINITY;
+    const float l = lane < n ? ml[1] : 0.0f;
+    f32x2p v[8][NV];
+    auto load8 = [&](int s0) {
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+#pragma unroll
+            for (int j = 0; j < NV; j++) {
+                v[u][j] = f32x2p{0.0f, 0.0f};
+                const int s = s0 + u * WPR;
+                if (s < n && 128 * j + 2 * lane < D) v[u][j] = *(const f32x2p*)(P + s * stride + 2 + 128 * j + 2 * lane);
+            }
+    };
+    load8(part);
+    float M = m;
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) M = fmaxf(M, shfl_xor_f(M, off));
+    M = max_with_partner32(max_with_partner16(M));
+    const float w = __builtin_amdgcn_exp2f(m - (M == -INFINITY ? 0.0f : M));
+    float L = l * w;
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) L += shfl_xor_f(L, off);
+    L = sum_with_partner32(sum_with_partner16(L));
+#pragma unroll
+    for (int j = 0; j < NV; j++) out[j] = f32x2p{0.0f, 0.0f};
+    for (int s0 = part; s0 < n; s0 += 8 * WPR) {
+        if (s0 != part) load8(s0);
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            // (past the last range the row read as zeros; the lane index is only kept inside the wave)
+            const float wu = as_f32((uint32_t)__builtin_amdgcn_readlane((int)as_u32(w), (s0 + u * WPR) & 63));
+#pragma unroll
+            for (int j = 0; j < NV; j++) { out[j][0] = fmaf(v[u][j][0], wu, out[j][0]); out[j][1] = fmaf(v[u][j][1], wu, out[j][1]); }
+        }
+    }
+    if constexpr (WPR > 1) {
+        __shared__ f32x2p sums[WPR - 1][NV][64];
+        if (part > 0) {
+#pragma unroll
+            for (int j = 0; j < NV; j++) sums[part - 1][j][lane] = out[j];
+        }
+        __syncthreads();
+        if (part == 0) {
+#pragma unroll
+            for (int q = 0; q < WPR - 1; q++)
+#pragma unroll
+                for (int j = 0; j < NV; j++) { out[j][0] += sums[q][j][lane][0]; out[j][1] += sums[q][j][lane][1]; }
+        }
+    }
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) { out[j][0] *= inv; out[j][1] *= inv; }
+    return L > 0.0f ? (M + __builtin_amdgcn_logf(L)) * LN2 : -INFINITY;
+}
+// waves per row of the merge passes: one (four rows to a workgroup) while a row's ranges fit one round of loads
+inline int merge_waves_per_row(int ranges) { return ranges <= 8 ? 1 : 4; }
 
 // 16-bit, head dimension 128, plain / causal attention in the software-pipelined form (attention_prefill.hip); kind: 1 fp16, 2 bf16
 bool attn_prefill_applies(const AttnArgs& a);

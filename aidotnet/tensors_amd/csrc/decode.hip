@@ -12,8 +12,7 @@
 // U * KPW keys (KPW = 64 / LPK keys per load, U loads in flight for K and U for V).  Every lane
 // keeps an online-softmax state (m, l, acc[E]) for its key slot and its 16-byte slice of the head
 // dim; slots and waves are merged through LDS, splits through a workspace and a second kernel.
-#include "common.hpp"
-#include "launch.hpp"
+#include "attention_common.hpp"
 
 namespace aidn {
 
@@ -240,52 +239,29 @@ __global__ __launch_bounds__(256) void decode_partial_kernel(const DecodeArgs a)
     }
 }
 
-// Merge the per-split (m, l, acc) triples: grid = B*H, one thread per head-dim element.  The split weights are formed once per
-// head (through LDS); the partial rows are then read eight splits at a time so that the loads of a thread overlap.
-template <typename OutT>
+// Merge the per-split (m, l, acc) triples, WPR waves per (batch, head) (merge_partials).
+template <typename OutT, int NV, int WPR>
 __global__ __launch_bounds__(256) void decode_reduce_kernel(const DecodeArgs a, int dpad)
 {
-    __shared__ float s_w[64], s_ml[2];
-    const int bh = blockIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int bh = blockIdx.x * (4 / WPR) + wave / WPR;
+    if (bh >= a.B * a.H) return;
     const int b = bh / a.H, hd = bh - b * a.H;
-    const long long stride = 2 + dpad;
-    const float* ws = a.ws + (long long)bh * a.splits * stride;
-    const int t = threadIdx.x;
-    // splits <= 64: lane s of the first wave holds split s
-    if (t < 64) {
-        const float m = t < a.splits ? ws[t * stride] : -INFINITY;
-        const float l = t < a.splits ? ws[t * stride + 1] : 0.0f;
-        float M = m;
+    f32x2p o[NV];
+    const float lse = merge_partials<NV, WPR>(a.ws + (long long)bh * a.splits * (2 + dpad), a.splits, dpad, a.D, wave % WPR, lane, o);
+    if (wave % WPR != 0) return;
+    typedef typename Raw3<OutT>::type out_t;
+    out_t* O = (out_t*)a.o + b * a.os[0] + hd * a.os[1];
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) M = fmaxf(M, shfl_xor_f(M, off));
-        const float Muse = (M == -INFINITY) ? 0.0f : M;
-        const float w = __builtin_amdgcn_exp2f(m - Muse);
-        float L = l * w;
+    for (int j = 0; j < NV; j++)
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) L += shfl_xor_f(L, off);
-        s_w[t] = w;
-        if (t == 0) { s_ml[0] = M; s_ml[1] = L; }
-    }
-    __syncthreads();
-    const float M = s_ml[0], L = s_ml[1];
-    for (int d = t; d < a.D; d += blockDim.x) {
-        float A = 0.0f;
-        int s0 = 0;
-        for (; s0 + 8 <= a.splits; s0 += 8) {
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = ws[(s0 + u) * stride + 2 + d];
-#pragma unroll
-            for (int u = 0; u < 8; u++) A += v[u] * s_w[s0 + u];
+        for (int e = 0; e < 2; e++) {
+            const int d = 128 * j + 2 * lane + e;
+            if (d >= a.D) continue;
+            if constexpr (Elem<OutT>::BYTES == 4) O[d] = as_u32(o[j][e]);
+            else O[d] = (out_t)Elem<OutT>::narrow(o[j][e]);
         }
-        for (; s0 < a.splits; s0++) A += ws[s0 * stride + 2 + d] * s_w[s0];
-        typedef typename Raw3<OutT>::type out_t;
-        out_t* O = (out_t*)a.o + b * a.os[0] + hd * a.os[1];
-        float r = L > 0.0f ? A / L : 0.0f;
-        if constexpr (Elem<OutT>::BYTES == 4) O[d] = as_u32(r);
-        else O[d] = (out_t)Elem<OutT>::narrow(r);
-        if (d == 0 && a.lse) a.lse[bh] = L > 0.0f ? (M + __builtin_amdgcn_logf(L)) * D_LN2 : -INFINITY;
-    }
+    if (lane == 0 && a.lse) a.lse[bh] = lse;
 }
 
 // ------------------------------------------------------------------ host side
@@ -338,6 +314,20 @@ size_t attn_decode_workspace_bytes(const AttnParams& p, int eff_splits)
     return (size_t)p.B * p.H * eff_splits * (2 + dpad) * sizeof(float);
 }
 
+template <typename OutT>
+static hipError_t launch_decode_reduce(const DecodeArgs& a, int dpad, hipStream_t stream)
+{
+    const unsigned rows = (unsigned)(a.B * a.H);
+    if (merge_waves_per_row(a.splits) == 1) {
+        if (a.D <= 128) hipLaunchKernelGGL((decode_reduce_kernel<OutT, 1, 1>), dim3((rows + 3) / 4), dim3(256), 0, stream, a, dpad);
+        else hipLaunchKernelGGL((decode_reduce_kernel<OutT, 2, 1>), dim3((rows + 3) / 4), dim3(256), 0, stream, a, dpad);
+    } else {
+        if (a.D <= 128) hipLaunchKernelGGL((decode_reduce_kernel<OutT, 1, 4>), dim3(rows), dim3(256), 0, stream, a, dpad);
+        else hipLaunchKernelGGL((decode_reduce_kernel<OutT, 2, 4>), dim3(rows), dim3(256), 0, stream, a, dpad);
+    }
+    return hipGetLastError();
+}
+
 template <typename T, typename OutT, int LPK, int U>
 static hipError_t launch_decode(DecodeArgs a, hipStream_t stream)
 {
@@ -353,12 +343,7 @@ static hipError_t launch_decode(DecodeArgs a, hipStream_t stream)
     else hipLaunchKernelGGL((decode_partial_kernel<T, OutT, LPK, U, 1>), grid, dim3(256), 0, stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (a.splits > 1) {
-        int threads = a.D <= 64 ? 64 : (a.D <= 128 ? 128 : 256);
-        hipLaunchKernelGGL((decode_reduce_kernel<OutT>), dim3((unsigned)(a.B * a.H)), dim3(threads), 0, stream, a, DPAD);
-        e = hipGetLastError();
-    }
-    return e;
+    return a.splits > 1 ? launch_decode_reduce<OutT>(a, DPAD, stream) : hipSuccess;
 }
 
 template <typename T, typename OutT>
@@ -389,11 +374,8 @@ hipError_t attn_decode(hipStream_t stream, int kind, const AttnParams& p, int ef
             r.qs[0] = p.qs[0]; r.qs[1] = p.qs[1]; r.os[0] = p.os[0]; r.os[1] = p.os[1];
             for (int i = 0; i < 3; i++) { r.ks[i] = p.ks[i]; r.vs[i] = p.vs[i]; }
             r.vec_in = 1; r.bt = nullptr; r.bsz = 0; r.bt_bs = 0;
-            const dim3 grid((unsigned)(p.B * p.H));
-            if (!p.out16) hipLaunchKernelGGL((decode_reduce_kernel<float>), grid, dim3(128), 0, stream, r, 128);
-            else if (kind == 1) hipLaunchKernelGGL((decode_reduce_kernel<f16_t>), grid, dim3(128), 0, stream, r, 128);
-            else hipLaunchKernelGGL((decode_reduce_kernel<bf16_t>), grid, dim3(128), 0, stream, r, 128);
-            return hipGetLastError();
+            if (!p.out16) return launch_decode_reduce<float>(r, 128, stream);
+            return kind == 1 ? launch_decode_reduce<f16_t>(r, 128, stream) : launch_decode_reduce<bf16_t>(r, 128, stream);
         }
         return hipSuccess;
     }
