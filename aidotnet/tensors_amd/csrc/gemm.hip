@@ -71,20 +71,60 @@ hipError_t ensure_dynamic_smem(const void* kernel, int bytes, unsigned long long
 }
 #endif
 
+// 1 / (1 + e^-x), the logistic function that GELU (tanh form: x times the logistic function of twice the inner polynomial), sigmoid and
+// swish are made of, on the vector pipe's exponential (base 2) and reciprocal.  The product x log2(e) is carried in two parts and the
+// reciprocal takes one Newton step, so the result is within about 2 units in the last place wherever it is above 1e-37 (the float64
+// check of the epilogue tests sees no more than the library functions gave); below, it is zero.  An epilogue holds nothing but these
+// values and nothing runs beside it on one tile per CU, so their length is time: with the library's tanhf / expf and an IEEE division,
+// chosen per element, the fp32 product 4096 x 3072 x 768 with GELU took 199 us, this way 149; bf16 1000 x 11008 x 4096 with swish
+// 129 and 106.
+__device__ __forceinline__ float logistic(float x)
+{
+    constexpr float L2E = 1.44269502f, L2E_LO = 1.92596299e-8f, LN2 = 0.693147181f;      // log2(e) = L2E + L2E_LO
+    const float y = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);                           // (keeps 1 + e^-y and its reciprocal normal)
+    const float t = y * -L2E;
+    const float lo = fmaf(y, -L2E_LO, fmaf(y, -L2E, -t));
+    float e = __builtin_amdgcn_exp2f(t);
+    e = fmaf(e, lo * LN2, e);
+    const float d = 1.0f + e;
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(r, fmaf(-d, r, 1.0f), r);
+    return x < -87.0f ? 0.0f : r;
+}
+
 // Pointwise activations of the fused projection epilogues, numbered like the reference's FusedActivationType
-// (src/AiDotNet.Tensors/Engines/FusedActivationType.cs:23-70) and computed like its HIP activation kernels
-// (src/AiDotNet.Tensors/Engines/DirectGpu/HIP/Kernels/HipActivationKernels.cs:19-70).
-__device__ __forceinline__ float apply_activation(float x, int act, float p)
+// (src/AiDotNet.Tensors/Engines/FusedActivationType.cs:23-70); the functions are those of its HIP activation kernels
+// (src/AiDotNet.Tensors/Engines/DirectGpu/HIP/Kernels/HipActivationKernels.cs:19-70).  NaN stays NaN in all of them.
+template <int ACT>
+__device__ __forceinline__ float activation(float x, float p)
+{
+    if constexpr (ACT == 1) return x < 0.0f ? 0.0f : x;                                   // ReLU, NaN-preserving form (CpuFusedOperations.cs:1271-1274)
+    else if constexpr (ACT == 2) return x * logistic(1.5957691216f * (x + 0.044715f * x * x * x));      // GELU, tanh form: (1 + tanh u) / 2 = logistic(2 u)
+    else if constexpr (ACT == 3) { const float r = logistic(x); return x == x ? r : x; }  // sigmoid
+    else if constexpr (ACT == 4) return tanhf(x);
+    else if constexpr (ACT == 5) return x > 0.0f ? x : p * x;                             // leaky ReLU, slope p
+    else if constexpr (ACT == 6) return x * logistic(x);                                  // swish
+    else return x;
+}
+// f(fn) with fn the activation `act`: the choice is made once around whatever f does with it, never per element (a tile of
+// accumulators with a test on each is thousands of branches)
+template <typename F>
+__device__ __forceinline__ void with_activation(int act, float p, F&& f)
 {
     switch (act) {
-    case 1: return x < 0.0f ? 0.0f : x;                                                      // ReLU, NaN-preserving form (CpuFusedOperations.cs:1271-1274)
-    case 2: return 0.5f * x * (1.0f + tanhf(0.7978845608f * (x + 0.044715f * x * x * x)));   // GELU, tanh form
-    case 3: return 1.0f / (1.0f + expf(-x));                                                 // sigmoid
-    case 4: return tanhf(x);
-    case 5: return x > 0.0f ? x : p * x;                                                     // leaky ReLU, slope p
-    case 6: return x / (1.0f + expf(-x));                                                    // swish
-    default: return x;
+    case 1: f([](float x) { return activation<1>(x, 0.0f); }); break;
+    case 2: f([](float x) { return activation<2>(x, 0.0f); }); break;
+    case 3: f([](float x) { return activation<3>(x, 0.0f); }); break;
+    case 4: f([](float x) { return activation<4>(x, 0.0f); }); break;
+    case 5: f([p](float x) { return activation<5>(x, p); }); break;
+    case 6: f([](float x) { return activation<6>(x, 0.0f); }); break;
+    default: f([](float x) { return x; }); break;
     }
+}
+__device__ __forceinline__ float apply_activation(float x, int act, float p)
+{
+    with_activation(act, p, [&](auto fn) { x = fn(x); });
+    return x;
 }
 
 // K extent of one tile of the general kernel in 16-byte chunks per row, and the LDS row pitch (one chunk of padding keeps the
@@ -471,21 +511,30 @@ __global__ __launch_bounds__(WM * WN * KS * 64) void gemm_kernel(const GemmArgs 
                 const int col = n0 + wn * WTN + j * 32 + l32;
                 float bias = 0.0f;
                 if constexpr (FUSED) bias = (g.bias && col < g.N) ? g.bias[col] : 0.0f;
+                f32x16 v = acc[i][j];
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int row = m0 + wm * WTM + i * 32 + acc_row(r, h);
+                    v[r] *= g.alpha;
+                    if (use_beta && row < g.M && col < g.N) {
+                        const out_t* p = C + (long long)row * g.ldc + col;
+                        if constexpr (Elem<OutT>::BYTES == 4) v[r] += g.beta * as_f32(*p);
+                        else v[r] += g.beta * Elem<OutT>::widen(*p);
+                    }
+                    v[r] += bias;
+                }
+                if constexpr (FUSED)
+                    with_activation(g.act, g.act_param, [&](auto fn) {
+#pragma unroll
+                        for (int r = 0; r < 16; r++) v[r] = fn(v[r]);
+                    });
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int row = m0 + wm * WTM + i * 32 + acc_row(r, h);
                     if (row < g.M && col < g.N) {
                         out_t* p = C + (long long)row * g.ldc + col;
-                        float v = g.alpha * acc[i][j][r];
-                        if constexpr (Elem<OutT>::BYTES == 4) {
-                            if (use_beta) v += g.beta * as_f32(*p);
-                            if constexpr (FUSED) v = apply_activation(v + bias, g.act, g.act_param);
-                            *p = as_u32(v);
-                        } else {
-                            if (use_beta) v += g.beta * Elem<OutT>::widen(*p);
-                            if constexpr (FUSED) v = apply_activation(v + bias, g.act, g.act_param);
-                            *p = (out_t)Elem<OutT>::narrow(v);
-                        }
+                        if constexpr (Elem<OutT>::BYTES == 4) *p = as_u32(v[r]);
+                        else *p = (out_t)Elem<OutT>::narrow(v[r]);
                     }
                 }
             }
@@ -843,7 +892,11 @@ __global__ __launch_bounds__((TILE == 256 ? 512 : 256) * KSW, TILE == 256 ? 1 : 
             if (fused) {                                  // bias and / or activation folded into the store
                 const float bias = (g.bias && col_ok) ? g.bias[col] : 0.0f;
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][j][r] = apply_activation(acc[i][j][r] + bias, g.act, g.act_param);
+                for (int r = 0; r < 16; r++) acc[i][j][r] += bias;
+                with_activation(g.act, g.act_param, [&](auto fn) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[i][j][r] = fn(acc[i][j][r]);
+                });
             }
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -1153,13 +1206,20 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
             constexpr int ip = decltype(ip_const)::value;
 #pragma unroll
             for (int ii = 0; ii < IPR; ii++) {
+                // (a row of blocks at a time: over the whole tile at once the choice outgrows the registers)
+                f32x4_acc w[TJ];
+#pragma unroll
+                for (int j = 0; j < TJ; j++) w[j] = acc[ip + ii][j];
+                if (fused)
+                    with_activation(g.act, g.act_param, [&](auto fn) {
+#pragma unroll
+                        for (int j = 0; j < TJ; j++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) w[j][e] = fn(w[j][e] + bias4[j][e]);
+                    });
 #pragma unroll
                 for (int j = 0; j < TJ; j++) {
-                    f32x4_acc v = acc[ip + ii][j];
-                    if (fused) {
-#pragma unroll
-                        for (int e = 0; e < 4; e++) v[e] = apply_activation(v[e] + bias4[j][e], g.act, g.act_param);
-                    }
+                    const f32x4_acc v = w[j];
                     const int row = ii * 16 + l16;
                     if constexpr (OB == 2) {
                         const uint32_t w0 = Elem<OutT>::narrow(v[0]) | (Elem<OutT>::narrow(v[1]) << 16);

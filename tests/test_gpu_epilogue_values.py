@@ -1,0 +1,73 @@
+"""Values of the fused activations over the whole range of their argument, through every kernel that applies them.  A is a shifted
+identity, so the product is exactly the chosen values and only the epilogue is looked at.
+
+Bound: relative error <= 4e-7 for the functions built on the logistic function where the result is above 1e-30 (argument rounding of
+the exponential is carried in a second part: two fp32 roundings of e^-x, one of 1 + e^-x, reciprocal within one unit after a Newton
+step, one product: 3.5 units of 2^-23); GELU's inner cubic adds 2 |2u| 2^-24 relative, below 3e-6 for |u| <= 22, beyond which the
+result is x or below 1e-19."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+VALUES = np.array([0.0, -0.0, 1e-30, -1e-30, 1e-4, -1e-4, 0.3, -0.3, 1.0, -1.0, 2.5, -2.5, 6.0, -6.0, 10.0, -10.0, 25.0, -25.0, 60.0, -60.0,
+                   86.9, -86.9, 88.0, -88.0, 120.0, -120.0, 1e4, -1e4, 1e20, -1e20], np.float32)
+
+
+def reference(x, act):
+    x = x.astype(np.float64)
+    with np.errstate(over="ignore"):
+        if act == 1: return np.maximum(x, 0)
+        if act == 2: return x / (1 + np.exp(-2 * 0.7978845608 * (x + 0.044715 * x ** 3)))
+        if act == 3: return 1 / (1 + np.exp(-x))
+        if act == 4: return np.tanh(x)
+        if act == 5: return np.where(x > 0, x, 0.125 * x)
+        if act == 6: return x / (1 + np.exp(-x))
+    return x
+
+
+# (M, N, K): few rows, the 64 / 128 / 256-wide direct-to-LDS tiles with and without edges, the general kernel (rows off the 16-byte grid)
+@pytest.mark.parametrize("M,N,K", [(4, 256, 64), (64, 64, 64), (130, 132, 32), (512, 4096, 32), (70, 33, 31), (24, 128, 64)])
+@pytest.mark.parametrize("act", range(7))
+def test_activation_values_fp32(M, N, K, act):
+    from aidotnet.tensors_amd import Mi355Engine
+    eng = Mi355Engine()
+    x = VALUES[(np.arange(K)[:, None] * 7 + np.arange(N)[None, :]) % len(VALUES)]
+    a = np.zeros((M, K), np.float32); a[np.arange(M), np.arange(M) % K] = 1.0
+    got = eng.FusedLinear(torch.from_numpy(a).cuda(), torch.from_numpy(x).cuda(), None, act, 0.125).cpu().numpy().astype(np.float64)
+    arg = x[np.arange(M) % K]
+    want = reference(arg, act)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    big = np.abs(want) > 1e-30
+    rel = np.abs(got - want)[big] / np.abs(want)[big]
+    u = np.abs(2 * 0.7978845608 * (arg.astype(np.float64) + 0.044715 * arg.astype(np.float64) ** 3))[big]
+    assert np.all(rel <= 4e-7 + (np.minimum(u, 100) * 2.0 ** -23 if act == 2 else 0.0))
+    assert np.all(np.abs(got[~big]) <= 2e-30)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 256, 64), (512, 1024, 64), (100, 200, 64)])
+@pytest.mark.parametrize("act", range(7))
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_activation_values_16bit(M, N, K, act, dtype):
+    """The 16-bit result is the fp32 epilogue rounded once: half a unit of the type (2^-11 fp16, 2^-8 bf16 ... relative) and, in fp16,
+    of the smallest subnormal."""
+    from aidotnet.tensors_amd import Mi355Engine
+    eng = Mi355Engine()
+    vals = VALUES[np.abs(VALUES) <= 1e4]
+    x = torch.from_numpy(vals[(np.arange(K)[:, None] * 7 + np.arange(N)[None, :]) % len(vals)]).cuda().to(dtype)
+    a = torch.zeros(M, K, dtype=dtype, device="cuda"); a[torch.arange(M), torch.arange(M) % K] = 1.0
+    got = eng.FusedLinear(a, x, None, act, 0.125).double().cpu().numpy()
+    want = reference(x.float().cpu().numpy()[np.arange(M) % K], act)
+    unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    assert np.all(np.abs(got - want) <= 1.01 * unit * np.abs(want) + 2.0 ** -25)
+
+
+def test_nan_stays_nan():
+    from aidotnet.tensors_amd import Mi355Engine
+    eng = Mi355Engine()
+    w = torch.full((64, 64), float("nan"), device="cuda")
+    for act in range(7):
+        assert bool(torch.isnan(eng.FusedLinear(torch.ones(64, 64, device="cuda"), w, None, act, 0.1)).all()), act
