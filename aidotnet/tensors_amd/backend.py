@@ -503,10 +503,11 @@ class Mi355Backend:
     # ------------------------------------------------------------------ multi-head attention forward
     def MultiHeadAttentionForward(self, kind: str, input: GpuBuffer, qWeight: GpuBuffer, kWeight: GpuBuffer, vWeight: GpuBuffer,
                                   outWeight: GpuBuffer, mask: Optional[GpuBuffer], output: GpuBuffer,
-                                  batch: int, seqLen: int, dModel: int, numHeads: int) -> None:
+                                  batch: int, seqLen: int, dModel: int, numHeads: int, keyMask: bool = False) -> None:
         """output[B,S,dModel] = MHA(input) with [dModel,dModel] weights and no biases, as three launches over a packed
         QKV activation (CpuEngine.MultiHeadAttention.cs:155-285 restated for the device; the reference has no GPU route).
-        kind "f32" / "f16" / "bf16"; mask: fp32 keep-mask of seqLen*seqLen (shared) or batch*numHeads*seqLen*seqLen elements."""
+        kind "f32" / "f16" / "bf16"; mask: fp32 keep-mask of seqLen*seqLen (shared) or batch*numHeads*seqLen*seqLen elements, or with
+        keyMask batch*seqLen bytes that hide a key from every head and query of its batch."""
         fn = {"f32": self._lib.aidn_mi355_mha_fwd_f32, "f16": self._lib.aidn_mi355_mha_fwd_f16,
               "bf16": self._lib.aidn_mi355_mha_fwd_bf16}.get(kind)
         if fn is None:
@@ -526,7 +527,10 @@ class Mi355Backend:
         for b, n in ((qWeight, "qWeight"), (kWeight, "kWeight"), (vWeight, "vWeight"), (outWeight, "outWeight")):
             self._capacity(b, dModel * dModel * es, n, op)
         mode = 0
-        if mask is not None:
+        if mask is not None and keyMask:
+            self._capacity(mask, batch * seqLen, "mask", op)
+            mode = 3
+        elif mask is not None:
             plane = seqLen * seqLen
             if mask.SizeInBytes == plane * 4:
                 mode = 1
@@ -679,10 +683,10 @@ class Mi355Backend:
     def ScaledDotProductAttention(self, query: GpuBuffer, key: GpuBuffer, value: GpuBuffer, output: GpuBuffer,
                                   attentionWeights: Optional[GpuBuffer], mask: Optional[GpuBuffer],
                                   batch: int, numHeads: int, seqQ: int, seqK: int, headDim: int, scale: float,
-                                  isCausal: bool, softcap: float = 0.0, numKVHeads: int = 0) -> None:
+                                  isCausal: bool, softcap: float = 0.0, numKVHeads: int = 0, keyMask: bool = False) -> None:
         """IDirectGpuBackend.cs:1395-1424 / HipBackend.cs:6118-6175: fp32, optional weights output,
         float mask (0 = masked; shared [seqQ*seqK] plane or full), bottom-right causal alignment,
-        grouped-query heads."""
+        grouped-query heads.  keyMask: the mask is batch*seqK bytes, each hiding a key from every head and query of its batch."""
         if batch <= 0 or numHeads <= 0 or seqQ <= 0 or seqK <= 0 or headDim <= 0:
             raise ArgumentOutOfRangeException("batch: Attention dimensions must be positive.")
         kvHeads = numKVHeads if numKVHeads > 0 else numHeads
@@ -699,11 +703,13 @@ class Mi355Backend:
             raise ArgumentException("Attention tensor buffers are smaller than the requested dimensions.")
         if attentionWeights is not None and attentionWeights.Size < wsz:
             raise ArgumentException("The attention-weights buffer is too small.")
-        if mask is not None and mask.Size < seqQ * seqK:
+        if mask is not None and keyMask:
+            self._capacity(mask, batch * seqK, "mask", "ScaledDotProductAttention")
+        elif mask is not None and mask.Size < seqQ * seqK:
             raise ArgumentException("The attention mask must contain at least seqQ * seqK elements.")
         d = AttnDesc(B=batch, H=numHeads, Hkv=kvHeads, Sq=seqQ, Sk=seqK, D=headDim, scale=scale,
                      causal=1 if isCausal else 0, causal_query_offset=seqK - seqQ, softcap=softcap,
-                     mask_mode=0 if mask is None else (2 if mask.Size >= wsz else 1))
+                     mask_mode=0 if mask is None else 3 if keyMask else (2 if mask.Size >= wsz else 1))
         self._attn("f32", query, key, value, output, None, None, mask, attentionWeights, d)
 
     def FlashAttentionV2(self, query: GpuBuffer, key: GpuBuffer, value: GpuBuffer, output: GpuBuffer,

@@ -112,7 +112,7 @@ int fill_params(Ctx* c, const aidn_attn_desc* d, aidn::AttnParams& p)
     if (hkv > d->H || d->H % hkv != 0)
         return fail(c, AIDN_ERR_INVALID_ARGUMENT, "attention: H must be an integer multiple of Hkv");
     if (d->D > 256) return fail(c, AIDN_ERR_UNSUPPORTED, "attention: head dimension above 256");
-    if (d->mask_mode < 0 || d->mask_mode > 2) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "attention: mask_mode must be 0, 1 or 2");
+    if (d->mask_mode < 0 || d->mask_mode > 3) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "attention: mask_mode must be 0, 1, 2 or 3");
     p.B = d->B; p.H = d->H; p.Hkv = hkv; p.Sq = d->Sq; p.Sk = d->Sk; p.D = d->D;
     p.scale = d->scale; p.causal = d->causal != 0; p.qoff = d->causal_query_offset; p.softcap = d->softcap;
     p.mask_mode = d->mask_mode; p.out16 = d->out_is_16bit != 0; p.bias_bs = d->bias_batch_stride;
@@ -260,7 +260,7 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
     if (dModel % heads != 0) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "mha: dModel must be divisible by the number of heads");
     const int dHead = dModel / heads;
     if (dHead > 256) return fail(c, AIDN_ERR_UNSUPPORTED, "mha: head dimension above 256");
-    if (mask_mode < 0 || mask_mode > 2) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "mha: mask_mode must be 0, 1 or 2");
+    if (mask_mode < 0 || mask_mode > 3) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "mha: mask_mode must be 0, 1, 2 or 3");
     if (mask_mode != 0 && !mask) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "mha: mask_mode set but mask is null");
     const long long rows = (long long)B * S;
     if (rows > 0x7FFFFFFFLL || 3LL * dModel > 0x7FFFFFFFLL) return fail(c, AIDN_ERR_UNSUPPORTED, "mha: B*S or 3*dModel exceeds 2^31");

@@ -26,9 +26,13 @@ namespace aidn {
 // XOR-swizzled 16-byte chunks (K: c ^ (key & 15) for the b128 fragment reads; V: c ^ (((key >> 2) & 1) << 3), read as the
 // A operand of O^T += V^T P^T with 32-bit LDS reads, the two lane halves -- keys 4 apart -- in different bank halves).  This
 // removes the register -> LDS store path (and the V transpose in registers) of the general form.
-template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false>
+// KM (DMA form): a keep-mask of the keys shared by the heads and queries of a batch (mask_mode 3).  A tile's mask is one ballot, tested
+// per element by a constant bit and only where the tile is mixed; a tile without a visible key is not computed.  A padded batch (bf16 B8
+// H12 S512 d64, lengths 256 .. 512) took 85.6 us with the mask as a [B,H,S,S] tensor on the general form, 23.0 this way.
+template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
 __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 {
+    static_assert(!KM || DMA, "the key mask of a tile is formed beside direct-to-LDS loads");
     static_assert(!DMA || (!FULL && ((DP == 64 && BC == 64) || (Elem<T>::BYTES == 4 && DP == 128 && BC == 32) ||
                                      (Elem<T>::BYTES == 2 && DP == 256 && BC == 32))),
                   "DMA form: head dimension 64 with 64-key tiles (or fp32 128 / 16-bit 256 with 32-key tiles), plain / causal");
@@ -242,8 +246,15 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                        lds0 + 2 * KBYTES + stage * VBYTES + (LPW * wave_s + i) * 1024);
         }
     };
+    // KM: visible keys of the current tile (keys past the end are not), the same in every wave
+    const unsigned char* __restrict__ kmask = KM ? (const unsigned char*)a.mask + (long long)b * a.Sk : nullptr;
+    auto tile_keys = [&](int kv0, unsigned keep) -> uint64_t {
+        return __builtin_amdgcn_ballot_w64(lane < BC && kv0 + lane < a.Sk && keep != 0);
+    };
+    uint64_t kbits = ~0ull;
     if constexpr (DMA) {
         if (ntiles > 0) issue_tile(0, 0);
+        if constexpr (KM) kbits = tile_keys(0, kmask[min(lane, a.Sk - 1)]);
         __builtin_amdgcn_s_waitcnt(0);
     } else {
         if (ntiles > 0) {
@@ -256,11 +267,13 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     for (int j = 0; j < ntiles; j++) {
         const int stage = j & 1;
         const int kv0 = j * BC;
+        unsigned next_keep = 0;        // (read with the next tile's loads, looked at when they have landed)
+        if constexpr (KM) next_keep = kmask[min(kv0 + BC + lane, a.Sk - 1)];
         if constexpr (DMA) { if (j + 1 < ntiles) issue_tile(j + 1, stage ^ 1); }
         else if (j + 1 < ntiles) load_tile(kv0 + BC);
 
         // a wave whose 32 rows are all above the causal diagonal of this tile only helps with the copies
-        const bool active = !(a.causal && (long long)kv0 > (long long)wq_max + a.qoff);
+        const bool active = !(a.causal && (long long)kv0 > (long long)wq_max + a.qoff) && (!KM || kbits != 0);
         if (active) {
             const unsigned char* ks = Ks + stage * KBYTES + l32 * KPITCH + h * 16;
             const unsigned char* vs = Vs + stage * VBYTES + l32 * VPITCH + h * 16;
@@ -299,9 +312,11 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 
             // ---- logits in the log2 domain, masks
             const bool need_mask = (kv0 + BC > a.Sk) || (a.causal && (long long)kv0 + BC - 1 > (long long)wq_min + a.qoff);
+            const bool mixed = KM && (BC == 64 ? kbits != ~0ull : (uint32_t)kbits != ~0u);
             float mloc = -INFINITY;
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) {
+                const uint32_t kept = (uint32_t)(kbits >> (32 * kt)) >> (4 * h);       // bit acc_row(r, 0): the key of element r
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     float x;
@@ -311,7 +326,9 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                         if (a.softcap > 0.0f) x = a.softcap * tanhf(x / a.softcap);
                         const bool inb = qi < a.Sq && key < a.Sk;
                         if (a.bias && inb) x += a.bias[b * a.bias_bs + ((long long)hd * a.Sq + qi) * a.Sk + key];
-                        if (a.mask_mode != 0 && inb) {
+                        if (a.mask_mode == 3 && inb) {
+                            if (((const unsigned char*)a.mask)[(long long)b * a.Sk + key] == 0) x = -INFINITY;
+                        } else if (a.mask_mode != 0 && inb) {
                             long long mi = (a.mask_mode == 2 ? ((long long)bh * a.Sq + qi) : (long long)qi) * a.Sk + key;
                             if (a.mask[mi] == 0.0f) x = -INFINITY;
                         }
@@ -322,6 +339,8 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                     if (need_mask) {
                         if (key >= a.Sk || (a.causal && (long long)key > (long long)qi + a.qoff)) x = -INFINITY;
                     }
+                    if constexpr (KM)
+                        if (mixed && !(kept >> acc_row(r, 0) & 1u)) x = -INFINITY;
                     st[kt][r] = x;
                     mloc = fmaxf(mloc, x);
                 }
@@ -398,6 +417,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
         }
         if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0);      // this wave's loads of tile j + 1 have landed
         else if (j + 1 < ntiles) store_tile(stage ^ 1);
+        if constexpr (KM) kbits = tile_keys(kv0 + BC, next_keep);
         __syncthreads();
     }
 
@@ -492,7 +512,8 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 // that changes is where the uniform base of its loads comes from (paged_tile_rows).  A 512-query chunk after 3584 keys (bf16, 32 / 8
 // heads) took 341 us on the general kernel, whose loads go through registers and which cannot split the keys of its 128 query tiles; here
 // 46 us and 16 us for the merge of its four key ranges.
-template <typename T, typename OutT, int D = 128, bool PAGED = false>
+// KM: a keep-mask of the keys shared by the heads and queries of a batch (mask_mode 3), one ballot per tile as in the kernel above.
+template <typename T, typename OutT, int D = 128, bool PAGED = false, bool KM = false>
 __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(const AttnArgs a)
 {
     typedef uint16_t raw_t;
@@ -694,7 +715,12 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
     const int klim = key_limit(qi) - 4 * h;
     const int wave_klim = __builtin_amdgcn_readfirstlane(key_limit(wq_min));
 
+    // KM: visible keys of the current tile, the same in every wave
+    const unsigned char* __restrict__ kmask = KM ? (const unsigned char*)a.mask + (long long)b * a.Sk + kbeg : nullptr;
+    auto tile_keys = [&](int kv0, unsigned keep) -> uint64_t { return __builtin_amdgcn_ballot_w64(kv0 + lane < Sk && keep != 0); };
+    uint64_t kbits = ~0ull;
     if (ntiles > 0) { next_rows(0); issue_k(0); issue_v(0); }
+    if constexpr (KM) { if (ntiles > 0) kbits = tile_keys(0, kmask[min(lane, Sk - 1)]); }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
@@ -741,17 +767,26 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
         // Loads of the next tile: when this wave computes and the next tile lies fully inside the sequence they are
         // issued one per MFMA inside the first phase below (a vector-memory instruction holds the wave's issue slot for
         // some tens of cycles; there it is covered by the running MFMA).  Otherwise all at once here.
-        const bool spread = !a.stream && j < nact && j + 1 < ntiles && (j + 1) * BC + BC <= Sk;
+        const bool computes = j < nact && (!KM || kbits != 0);
+        const bool spread = !a.stream && computes && j + 1 < ntiles && (j + 1) * BC + BC <= Sk;
+        unsigned next_keep = 0;
+        if constexpr (KM) next_keep = kmask[min(j * BC + BC + lane, Sk - 1)];
         if (j + 1 < ntiles) next_rows(j + 1);
         if (j + 1 < ntiles && !spread) { issue_k(j + 1); issue_v(j + 1); }
-        if (j < nact) {
+        if (computes) {
             const int kv0 = j * BC;
-            const bool need_mask = kv0 + BC - 1 > wave_klim;
+            const bool need_mask = kv0 + BC - 1 > wave_klim || (KM && kbits != ~0ull);
             const int rel_lim = klim - kv0;                   // keys of this tile with index > rel_lim are masked
             auto mask_sub = [&](int kt, f32x16& st) {
 #pragma unroll
                 for (int r = 0; r < 16; r++)
                     if (kt * 32 + 8 * (r >> 2) + (r & 3) > rel_lim) st[r] = -INFINITY;
+                if constexpr (KM) {
+                    const uint32_t kept = (uint32_t)(kbits >> (32 * kt)) >> (4 * h);
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        if (!(kept >> (8 * (r >> 2) + (r & 3)) & 1u)) st[r] = -INFINITY;
+                }
             };
             auto sub_max = [&](const f32x16& st) -> float {
                 float m = -INFINITY;
@@ -873,6 +908,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
             __builtin_amdgcn_s_setprio(0);
         }
         __builtin_amdgcn_s_waitcnt(0);      // this wave's DMA of tile j+1 has landed ...
+        if constexpr (KM) kbits = tile_keys(j * BC + BC, next_keep);
         __syncthreads();                    // ... everyone's has, and everyone is done with tile j
     };
     for (int j = 0; j < ntiles; j += 2) {
@@ -984,10 +1020,10 @@ __global__ __launch_bounds__(256) void attn_split_merge_kernel(const AttnArgs a,
     if (lane == 0 && a.lse) a.lse[row] = lse;
 }
 
-template <typename T, typename OutT, int D = 128, bool PAGED = false>
+template <typename T, typename OutT, int D = 128, bool PAGED = false, bool KM = false>
 static hipError_t launch_attn_dl(AttnArgs a, hipStream_t stream)
 {
-    auto kern = attn_fwd_dl_kernel<T, OutT, D, PAGED>;
+    auto kern = attn_fwd_dl_kernel<T, OutT, D, PAGED, KM>;
     constexpr int smem = 2 * (64 * 2 * D + 64 * 2 * D);      // K and V tiles, two stages each (64 KB; 128 KB at head dimension 256)
     static unsigned long long attr_done = 0;
     if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done)) return e;
@@ -1191,7 +1227,15 @@ __global__ __launch_bounds__(256) void attn_weights_kernel(const AttnArgs a, flo
 #pragma unroll
                 for (int r = 0; r < 16; r++) s[j][r] += Bi[(long long)min(qw + acc_row(r, h), a.Sq - 1) * a.Sk + min(keys[j], a.Sk - 1)];
         }
-        if (a.mask_mode != 0) {
+        if (a.mask_mode == 3) {
+            const unsigned char* __restrict__ Mk = (const unsigned char*)a.mask + (long long)b * a.Sk;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const bool hidden = Mk[min(keys[j], a.Sk - 1)] == 0;
+#pragma unroll
+                for (int r = 0; r < 16; r++) s[j][r] = hidden ? -INFINITY : s[j][r];
+            }
+        } else if (a.mask_mode != 0) {
             const float* __restrict__ Mk = a.mask + (a.mask_mode == 2 ? (long long)bh * a.Sq * a.Sk : 0LL);
 #pragma unroll
             for (int j = 0; j < 2; j++)
@@ -1233,10 +1277,10 @@ __global__ __launch_bounds__(256) void attn_weights_kernel(const AttnArgs a, flo
 }
 
 // ------------------------------------------------------------------ host side
-template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false>
+template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
 static hipError_t launch_attn(AttnArgs a, hipStream_t stream)
 {
-    auto kern = attn_fwd_kernel<T, OutT, DP, BC, FULL, MINB, DMA>;
+    auto kern = attn_fwd_kernel<T, OutT, DP, BC, FULL, MINB, DMA, KM>;
     constexpr int EB = Elem<T>::BYTES;
     constexpr int smem = DMA ? 4 * BC * DP * EB : 2 * (BC * (DP * EB + 16) + DP * (BC * EB + 16));
     static unsigned long long attr_done = 0;
@@ -1294,7 +1338,7 @@ static bool attn_dl_applies(int kind, const AttnParams& p)
     if (kind == 0 || p.D != 128 || !(p.scale > 0.0f) || !p.allow_fast_path) return false;
     // (behind a block table: blocks of a multiple of 16 keys, fp32 output, which is what the paged entry points return)
     if (p.block_table && (!paged_block_fits(p.block_table, p.block_size) || p.out16)) return false;
-    if (p.bias != nullptr || (p.mask && p.mask_mode != 0) || p.softcap > 0.0f) return false;
+    if (p.bias != nullptr || (p.mask && p.mask_mode != 0 && (p.mask_mode != 3 || p.block_table)) || p.softcap > 0.0f) return false;
     if (!(attn_aligned16(p.q, p.qs, 2) && attn_aligned16(p.k, p.ks, 2) && attn_aligned16(p.v, p.vs, 2))) return false;
     // the kernel addresses the K/V rows of a 4-key load group with unsigned 32-bit byte offsets
     return p.ks[2] > 0 && p.ks[2] < (1LL << 28) && p.vs[2] > 0 && p.vs[2] < (1LL << 28);
@@ -1357,8 +1401,10 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     a.vec_in = (p.D % e == 0) && al(p.q, p.qs, eb) && al(p.k, p.ks, eb) && al(p.v, p.vs, eb);
     a.vec_out = (p.D % 4 == 0) && al(p.o, p.os, oeb);
     const bool full = p.bias != nullptr || a.mask_mode != 0 || p.softcap > 0.0f;
+    // a mask of the keys alone is followed by the direct-to-LDS instances at head dimensions 64 and 128 as well
+    const bool km = a.mask_mode == 3 && !p.block_table && (p.D == 64 || p.D == 128);
     // the direct-to-LDS instances: plain / causal, 16-byte aligned rows, contiguous or in blocks of a multiple of 16 keys
-    const bool dma = !full && a.vec_in && paged_block_fits(p.block_table, p.block_size) && g_attn_allow_dl;
+    const bool dma = p.bias == nullptr && !(p.softcap > 0.0f) && (a.mask_mode == 0 || km) && a.vec_in && paged_block_fits(p.block_table, p.block_size) && g_attn_allow_dl;
     hipError_t err;
     // fast path: 16-bit, head dim 128, aligned rows, plain (optionally causal) attention
     // the fast kernel addresses K/V rows of a 4-key load group with unsigned 32-bit byte offsets
@@ -1376,20 +1422,26 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     // are short: the partial tile is then a larger share of a pass, and the pipelined kernel walks it in plain steps (509 against
     // 530 at S 1100).  allow_fast_path 2 / 3 (test hooks) pin the choice.
     bool pipelined = false;
-    if (dl && a.nsplit == 1 && attn_prefill_applies(a)) {      // (dense arrays: its tile loads count on rows 256 bytes apart)
+    if (dl && a.nsplit == 1 && a.mask_mode == 0 && attn_prefill_applies(a)) {      // (dense arrays: its tile loads count on rows 256 bytes apart)
         pipelined = p.allow_fast_path == 3 || (p.allow_fast_path == 1 && (p.Sk % 64 == 0 || p.Sk >= 2048));
     }
     if (pipelined) err = launch_attn_prefill(kind, p.out16, a, stream);
     else
     if (dl && p.block_table) err = kind == 1 ? launch_attn_dl<f16_t, float, 128, true>(a, stream) : launch_attn_dl<bf16_t, float, 128, true>(a, stream);
     else
+    if (dl && km) {
+        if (kind == 1) err = p.out16 ? launch_attn_dl<f16_t, f16_t, 128, false, true>(a, stream) : launch_attn_dl<f16_t, float, 128, false, true>(a, stream);
+        else err = p.out16 ? launch_attn_dl<bf16_t, bf16_t, 128, false, true>(a, stream) : launch_attn_dl<bf16_t, float, 128, false, true>(a, stream);
+    } else
     if (dl) {
         if (kind == 1) err = p.out16 ? launch_attn_dl<f16_t, f16_t>(a, stream) : launch_attn_dl<f16_t, float>(a, stream);
         else err = p.out16 ? launch_attn_dl<bf16_t, bf16_t>(a, stream) : launch_attn_dl<bf16_t, float>(a, stream);
     } else
     if (kind == 0) {
         // fp32: 64-key tiles while two workgroups still fit the LDS of a CU (head dimension up to 64), else 32-key tiles
-        if (p.D == 64 && dma) err = launch_attn<float, float, 64, 64, false, 2, true>(a, stream);
+        if (p.D == 64 && dma && km) err = launch_attn<float, float, 64, 64, false, 2, true, true>(a, stream);
+        else if (p.D == 128 && dma && km) err = launch_attn<float, float, 128, 32, false, 2, true, true>(a, stream);
+        else if (p.D == 64 && dma) err = launch_attn<float, float, 64, 64, false, 2, true>(a, stream);
         else if (p.D == 128 && dma) err = launch_attn<float, float, 128, 32, false, 2, true>(a, stream);
         else if (p.D <= 64) err = full ? (p.D <= 32 ? launch_attn<float, float, 32, 64, true, 2>(a, stream) : launch_attn<float, float, 64, 64, true, 2>(a, stream))
                                   : (p.D <= 32 ? launch_attn<float, float, 32, 64, false, 2>(a, stream) : launch_attn<float, float, 64, 64, false, 2>(a, stream));
@@ -1405,6 +1457,10 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
         // head dimension 256, plain / causal, aligned contiguous K/V: the direct-to-LDS form on 32-key tiles (Q streamed)
         if (kind == 1) err = p.out16 ? launch_attn<f16_t, f16_t, 256, 32, false, 2, true>(a, stream) : launch_attn<f16_t, float, 256, 32, false, 2, true>(a, stream);
         else err = p.out16 ? launch_attn<bf16_t, bf16_t, 256, 32, false, 2, true>(a, stream) : launch_attn<bf16_t, float, 256, 32, false, 2, true>(a, stream);
+    }
+    else if (p.D == 64 && dma && km) {
+        if (kind == 1) err = p.out16 ? launch_attn<f16_t, f16_t, 64, 64, false, 2, true, true>(a, stream) : launch_attn<f16_t, float, 64, 64, false, 2, true, true>(a, stream);
+        else err = p.out16 ? launch_attn<bf16_t, bf16_t, 64, 64, false, 2, true, true>(a, stream) : launch_attn<bf16_t, float, 64, 64, false, 2, true, true>(a, stream);
     }
     else if (p.D == 64 && dma) {
         // head dimension 64, plain / causal, aligned contiguous K/V: the direct-to-LDS form of the general kernel

@@ -205,7 +205,8 @@ AIDN_API int aidn_mi355_convert_bf16_to_f32(void* ctx, void* stream, const uint1
  *            (bias_batch_stride = 0), added after the scale, or NULL (IDirectGpuBackend.cs:1465-1466).
  *   mask     fp32, 0.0f = masked, anything else = keep (HipAttentionKernels.cs:78); mask_mode 0 none,
  *            1 one [Sq,Sk] plane shared by all (batch, head), 2 full [B,H,Sq,Sk]
- *            (HipBackend.cs:6150-6151).
+ *            (HipBackend.cs:6150-6151), 3 one row of BYTES [B,Sk] per batch, 0 = key masked for every
+ *            head and query (padding; the pointer is then that of the bytes).
  *   softcap  > 0: logit = softcap * tanh(scale * qk / softcap) before bias / masks
  *            (CpuEngine.cs:27806-27807); 0 disables.
  *   weights  fp32 [B,H,Sq,Sk] normalised probabilities or NULL (the optional attentionWeights of
@@ -320,7 +321,8 @@ AIDN_API int aidn_mi355_rope_interleaved_bf16(void* ctx, void* stream, const uin
  * fp32 path :155-285, fused SDPA over the packed activation :358-522), which has no GPU route in the reference.
  * Three launches and no permutes: one GEMM writes the packed [B*S, 3 dModel] activation, the attention kernel reads it through
  * strides and writes [B,S,H,d], one GEMM projects.  mask (may be null): fp32, non-zero = keep; mask_mode 1 = one [S,S] plane
- * shared by all (b,h), 2 = full [B,H,S,S] (what a broadcast of the reference's Tensor<bool> mask materialises to).
+ * shared by all (b,h), 2 = full [B,H,S,S] (what a broadcast of the reference's Tensor<bool> mask materialises to), 3 = one row of
+ * bytes [B,S] per batch, 0 = key masked for every head and query (padding; the pointer is then that of the bytes).
  * The 16-bit forms keep every intermediate in the input type and accumulate in fp32.  Intermediates live in the context's workspace. */
 AIDN_API int aidn_mi355_mha_fwd_f32(void* ctx, void* stream, const float* input, const float* wq, const float* wk, const float* wv,
                            const float* wo, const float* mask, int mask_mode, float* output, int B, int S, int dModel, int heads);
