@@ -29,22 +29,26 @@ namespace aidn {
 // KM (DMA form): a keep-mask of the keys shared by the heads and queries of a batch (mask_mode 3).  A tile's mask is one ballot, tested
 // per element by a constant bit and only where the tile is mixed; a tile without a visible key is not computed.  A padded batch (bf16 B8
 // H12 S512 d64, lengths 256 .. 512) took 85.6 us with the mask as a [B,H,S,S] tensor on the general form, 23.0 this way.
-template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
+// KG: how many waves share a query row's keys (launch_attn): a workgroup holds 128 / KG rows, a wave takes BC / KG keys of every tile for
+// its 32 rows, and the KG unnormalised results of a row are merged through LDS behind the last tile.
+template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false, int KG = 1>
 __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 {
     static_assert(!KM || DMA, "the key mask of a tile is formed beside direct-to-LDS loads");
-    static_assert(!DMA || (!FULL && ((DP == 64 && BC == 64) || (Elem<T>::BYTES == 4 && DP == 128 && BC == 32) ||
-                                     (Elem<T>::BYTES == 2 && DP == 256 && BC == 32))),
-                  "DMA form: head dimension 64 with 64-key tiles (or fp32 128 / 16-bit 256 with 32-key tiles), plain / causal");
+    static_assert(!DMA || (!FULL && (DP == 64 || (Elem<T>::BYTES == 4 && DP == 128) || (Elem<T>::BYTES == 2 && DP == 256))),
+                  "DMA form: head dimension 64 (or fp32 128 / 16-bit 256), plain / causal");
+    static_assert(!KM || BC <= 64, "a tile's key mask is one ballot");
     typedef typename Raw2<T>::type raw_t;
     constexpr int E = Elem<T>::PER16, EB = Elem<T>::BYTES;
-    constexpr int NT = 256, BR = 128;
+    constexpr int WQ = 4 / KG;                 // waves over the query rows; the KG waves of a row group share the keys of a tile
+    constexpr int NT = 256, BR = 32 * WQ;
     constexpr int KS = Mma32<T>::KS;
     constexpr int DSTEPS = DP / KS;            // fragment steps over the head dim (QK^T)
     constexpr int KPITCH = DP * EB + 16;       // K tile [key][d] row pitch, bytes
     constexpr int VPITCH = BC * EB + 16;       // V^T tile [d][key] row pitch, bytes
     constexpr int KBYTES = DMA ? BC * DP * EB : BC * KPITCH, VBYTES = DMA ? BC * DP * EB : DP * VPITCH;
-    constexpr int KT = BC / 32;                // 32-key sub-tiles per tile
+    constexpr int KT = BC / 32 / KG;           // 32-key sub-tiles per tile and wave
+    static_assert(KT >= 1, "every key group has a sub-tile of its own");
     constexpr int DT = DP / 32;                // 32-row tiles of O^T
     constexpr int PSTEPS = 32 / KS;            // PV fragment steps per key sub-tile
     constexpr int CPR = DP / E;                // 16-byte chunks per K row
@@ -100,7 +104,8 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     const int b = bh / a.H, hd = bh - b * a.H;
     const int kvh = hd / (a.H / a.Hkv);
     const int q0 = qt * BR;
-    const int qi = q0 + wave * 32 + l32;       // this lane's query row
+    const int wq = wave % WQ, kg = wave / WQ;  // this wave's row group and key group
+    const int qi = q0 + wq * 32 + l32;         // this lane's query row
     const bool vec = a.vec_in != 0;
 
     const raw_t* __restrict__ Q = (const raw_t*)a.q + b * a.qs[0] + hd * a.qs[1];
@@ -207,7 +212,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     float m_run = -INFINITY;     // running max of the log2-domain logits of query qi (same in lanes l and l^32)
     float l_run = 0.0f;          // this lane's share of the running sum
 
-    const int wq_min = q0 + wave * 32, wq_max = wq_min + 31;
+    const int wq_min = q0 + wq * 32, wq_max = wq_min + 31;
     const float sl2 = a.scale * LOG2E;
 
     // DMA form: this wave's loads of a tile are K and V wave-loads 4 wave .. 4 wave + 3 (4 keys x 256 bytes each); rows past
@@ -267,16 +272,18 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     for (int j = 0; j < ntiles; j++) {
         const int stage = j & 1;
         const int kv0 = j * BC;
+        const int kw0 = kv0 + kg * KT * 32;      // first key of this wave's sub-tiles
         unsigned next_keep = 0;        // (read with the next tile's loads, looked at when they have landed)
         if constexpr (KM) next_keep = kmask[min(kv0 + BC + lane, a.Sk - 1)];
         if constexpr (DMA) { if (j + 1 < ntiles) issue_tile(j + 1, stage ^ 1); }
         else if (j + 1 < ntiles) load_tile(kv0 + BC);
 
-        // a wave whose 32 rows are all above the causal diagonal of this tile only helps with the copies
-        const bool active = !(a.causal && (long long)kv0 > (long long)wq_max + a.qoff) && (!KM || kbits != 0);
+        // a wave whose 32 rows are all above the causal diagonal of its keys, or past the last row or key, only helps with the copies
+        const bool active = wq_min < a.Sq && kw0 < a.Sk && !(a.causal && (long long)kw0 > (long long)wq_max + a.qoff) && (!KM || kbits != 0);
         if (active) {
-            const unsigned char* ks = Ks + stage * KBYTES + l32 * KPITCH + h * 16;
-            const unsigned char* vs = Vs + stage * VBYTES + l32 * VPITCH + h * 16;
+            const int kr0 = kg * KT * 32;        // this wave's first key inside the tile
+            const unsigned char* ks = Ks + stage * KBYTES + (kr0 + l32) * KPITCH + h * 16;
+            const unsigned char* vs = Vs + stage * VBYTES + l32 * VPITCH + kr0 * EB + h * 16;
 
             f32x16 st[KT];
 #pragma unroll
@@ -303,7 +310,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 #pragma unroll
                 for (int kt = 0; kt < KT; kt++) {
                     u32x4 kf;
-                    if constexpr (DMA) kf = *(const u32x4*)(Ks + stage * KBYTES + (kt * 32 + l32) * (DP * EB) + (((2 * s + h) ^ k_swz(l32)) << 4));
+                    if constexpr (DMA) kf = *(const u32x4*)(Ks + stage * KBYTES + (kr0 + kt * 32 + l32) * (DP * EB) + (((2 * s + h) ^ k_swz(l32)) << 4));
                     else kf = *(const u32x4*)(ks + kt * 32 * KPITCH + s * 32);
                     Mma32<T>::run(st[kt], kf, qs);
                 }
@@ -311,16 +318,16 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
             if constexpr (EB == 4) __builtin_amdgcn_s_setprio(0);
 
             // ---- logits in the log2 domain, masks
-            const bool need_mask = (kv0 + BC > a.Sk) || (a.causal && (long long)kv0 + BC - 1 > (long long)wq_min + a.qoff);
+            const bool need_mask = (kw0 + KT * 32 > a.Sk) || (a.causal && (long long)kw0 + KT * 32 - 1 > (long long)wq_min + a.qoff);
             const bool mixed = KM && (BC == 64 ? kbits != ~0ull : (uint32_t)kbits != ~0u);
             float mloc = -INFINITY;
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) {
-                const uint32_t kept = (uint32_t)(kbits >> (32 * kt)) >> (4 * h);       // bit acc_row(r, 0): the key of element r
+                const uint32_t kept = (uint32_t)(kbits >> (kr0 + 32 * kt)) >> (4 * h);       // bit acc_row(r, 0): the key of element r
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     float x;
-                    const int key = kv0 + kt * 32 + acc_row(r, h);
+                    const int key = kw0 + kt * 32 + acc_row(r, h);
                     if constexpr (FULL) {
                         x = st[kt][r] * a.scale;
                         if (a.softcap > 0.0f) x = a.softcap * tanhf(x / a.softcap);
@@ -389,7 +396,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                         if constexpr (DMA && EB == 4) {
                             // V[key = 32 kt + 8 ps + 4 h + q][d = 32 i + l32]; (key >> 2) & 1 == h
                             const int d = i * 32 + l32;
-                            const unsigned char* vp = Vs + stage * VBYTES + (kt * 32 + 8 * ps + 4 * h) * (DP * 4) + ((((d >> 2) ^ (h << 3)) << 4) + (d & 3) * 4);
+                            const unsigned char* vp = Vs + stage * VBYTES + (kr0 + kt * 32 + 8 * ps + 4 * h) * (DP * 4) + ((((d >> 2) ^ (h << 3)) << 4) + (d & 3) * 4);
 #pragma unroll
                             for (int q = 0; q < 4; q++) vf[q] = *(const uint32_t*)(vp + q * (DP * 4));
                         } else if constexpr (DMA) {
@@ -400,7 +407,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                             const int chunk = (i * 32 + 16 * ((lane >> 4) & 1) + 4 * (jl & 3)) >> 3;
 #pragma unroll
                             for (int q = 0; q < 2; q++) {
-                                const int row = kt * 32 + 16 * ps + 8 * q + 4 * h + (jl >> 2);
+                                const int row = kr0 + kt * 32 + 16 * ps + 8 * q + 4 * h + (jl >> 2);
                                 u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                                     (__attribute__((address_space(3))) s16x4a*)(Vs + stage * VBYTES + row * (DP * 2) + ((chunk ^ v_swz(row)) << 4) + (jl & 1) * 8)));
                                 vf[2 * q] = w[0];
@@ -421,6 +428,46 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
         __syncthreads();
     }
 
+    // ---- key groups: the waves of groups 1 .. KG - 1 leave (O, m, l) in the idle tile memory and group 0 merges them.  The areas of
+    // row group wq are the ones its own output staging below overwrites.
+    if constexpr (KG > 1) {
+        constexpr int AREA = DT * 16 * 64;                          // floats of one wave's O
+        static_assert((KG - 1) * WQ * (AREA + 128) * 4 <= 2 * (KBYTES + VBYTES), "the partial results fit the tile memory");
+        static_assert(KG == 2 || WQ == 1, "a row group's partial results lie where that row group stages its output");
+        float* O1 = (float*)smem + wq * (KG - 1) * AREA;
+        float* ML = (float*)smem + (KG - 1) * WQ * AREA + wq * (KG - 1) * 128;
+        if (kg > 0) {
+            f32x4* dst = (f32x4*)(O1 + (kg - 1) * AREA);
+#pragma unroll
+            for (int i = 0; i < DT; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    dst[(i * 4 + g) * 64 + lane] = f32x4{oacc[i][4 * g], oacc[i][4 * g + 1], oacc[i][4 * g + 2], oacc[i][4 * g + 3]};
+            ML[(kg - 1) * 128 + lane] = m_run;
+            ML[(kg - 1) * 128 + 64 + lane] = l_run;
+        }
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int u = 0; u < KG - 1; u++) {
+            const float m1 = ML[u * 128 + lane], l1 = ML[u * 128 + 64 + lane];
+            const float m_new = fmaxf(m_run, m1);
+            const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
+            const float w0 = __builtin_amdgcn_exp2f(m_run - m_use), w1 = __builtin_amdgcn_exp2f(m1 - m_use);
+            m_run = m_new;
+            l_run = l_run * w0 + l1 * w1;
+            const f32x4* src = (const f32x4*)(O1 + u * AREA);
+#pragma unroll
+            for (int i = 0; i < DT; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const f32x4 v = src[(i * 4 + g) * 64 + lane];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) oacc[i][4 * g + e] = oacc[i][4 * g + e] * w0 + v[e] * w1;
+                }
+        }
+    }
+
     // ---- normalise and store: lane holds query qi, head-dim elements i*32 + 8 g + 4 h + (0..3)
     const float l_tot = l_run + shfl_xor_f(l_run, 32);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
@@ -431,7 +478,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
             // of one row, 64 partial lines per instruction.  Every wave left the last tile at the barrier that ends the loop.
             constexpr int CH = DP / 4;                   // 16-byte chunks of a row
             constexpr int RPI = 64 / CH;                 // rows per store instruction
-            unsigned char* stg = smem + wave * (32 * DP * 4);
+            unsigned char* stg = smem + wq * (32 * DP * 4);
 #pragma unroll
             for (int i = 0; i < DT; i++)
 #pragma unroll
@@ -444,7 +491,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 #pragma unroll
             for (int q = 0; q < 32 / RPI; q++) {
                 const int r = RPI * q + lane / CH;
-                const int row = q0 + wave * 32 + r;
+                const int row = q0 + wq * 32 + r;
                 const f32x4 v = *(const f32x4*)(stg + r * (DP * 4) + ((c ^ (r & (CH - 1))) << 4));
                 f32x4* dst = (f32x4*)((float*)a.o + b * a.os[0] + hd * a.os[1] + (long long)row * a.os[2] + c * 4);
                 if (row < a.Sq) __builtin_nontemporal_store(v, dst);
@@ -1277,15 +1324,16 @@ __global__ __launch_bounds__(256) void attn_weights_kernel(const AttnArgs a, flo
 }
 
 // ------------------------------------------------------------------ host side
-template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
-static hipError_t launch_attn(AttnArgs a, hipStream_t stream)
+template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false, int KG = 1>
+static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
 {
-    auto kern = attn_fwd_kernel<T, OutT, DP, BC, FULL, MINB, DMA, KM>;
+    constexpr int BR = 128 / KG;
+    auto kern = attn_fwd_kernel<T, OutT, DP, BC, FULL, MINB, DMA, KM, KG>;
     constexpr int EB = Elem<T>::BYTES;
     constexpr int smem = DMA ? 4 * BC * DP * EB : 2 * (BC * (DP * EB + 16) + DP * (BC * EB + 16));
     static unsigned long long attr_done = 0;
     if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done)) return e;
-    a.qtiles = (a.Sq + 127) / 128;
+    a.qtiles = (a.Sq + BR - 1) / BR;
     long long nblk = (long long)a.qtiles * a.B * a.H;
     if (nblk > 0x7FFFFFFFLL) return hipErrorInvalidValue;
     // causal order: up to 768 workgroups the balanced placement of a grid that is (nearly) resident at once (measured equal or
@@ -1293,6 +1341,37 @@ static hipError_t launch_attn(AttnArgs a, hipStream_t stream)
     a.hgroup = !a.causal ? 0 : nblk <= 768 ? -1 : (a.qtiles >= 8 ? 16 : (128 + a.qtiles - 1) / a.qtiles);
     hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(256), smem, stream, a);
     return hipGetLastError();
+}
+
+// How many waves share the keys of a query row's tiles (KG).  With one (128 query rows per workgroup, 32 per wave) a grid that does not
+// fill the chip takes as long as its longest wave: fp32 B4 H12 S512 d64 causal is 192 workgroups whose last ones run eight tiles of 64
+// MFMAs of 64 cycles with nothing else on their SIMDs, 44 us -- as long as twice the batch.  Two waves per 32 rows (64-row workgroups,
+// each wave half of every tile, merged through LDS at the end): 27 us; B1 H12 S1024 81 -> 48, and 32 with four.  Once the chip is full
+// the same matrix work only pays for more tile loads and merges (B16 H12 S512 83 -> 89 us).  The lines, as workgroups of the finer
+// grid, from a sweep over 58 shapes (time with one / two key groups in us at the last size on either side):
+//   64-key tiles, two workgroups per CU, head dimension up to 64: 768 (fp32 S512 causal 46 / 44, plain 74 / 67; 960: 54 / 54, S900 89 / 118);
+//     16-bit causal 1024 (S500 19.3 / 14.8, S1900 46 / 35; plain 20.4 / 21.1; 1536: 21 / 28)
+//   up to 128: 512, all resident at once (16-bit d80 plain 28.1 / 26.5; 768: 32.8 / 46.4)
+//   fp32 above 64: 64-key tiles need 128 KiB, one workgroup per CU: 256 (plain d128 151 / 88; 384: 66 / 83), causal 384 (64 / 42)
+//   four groups on 128-key tiles (head dimension 64, dense K and V, no mask): 256, causal 384, from 192 keys on (two / four groups: plain
+//     B4 H8 S256 16.0 / 12.2, causal B1 H32 S300 18.8 / 16.3; plain at 304 32 / 40, 64 keys 7.9 / 8.8)
+// The lines do not depend on how the tiles are loaded, so the direct-to-LDS and the register-staged forms add up the same way.
+template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
+static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
+{
+    constexpr bool WIDE32 = Elem<T>::BYTES == 4 && BC == 32 && DP == 128;
+    if constexpr ((BC == 64 && MINB == 2) || WIDE32) {
+        auto grid = [&](int rows) { return (long long)((a.Sq + rows - 1) / rows) * a.B * a.H; };
+        if constexpr (!FULL && !KM && DP == 64) {
+            if (!a.bt && a.Sk >= 192 && grid(32) <= (a.causal ? 384 : 256)) return launch_attn_kg<T, OutT, DP, 128, FULL, 1, DMA, KM, 4>(a, stream);
+        }
+        long long line;
+        if constexpr (WIDE32) line = a.causal ? 384 : 256;
+        else if constexpr (DP > 64) line = 512;
+        else line = !FULL && Elem<T>::BYTES == 2 && a.causal ? 1024 : 768;
+        if (grid(64) <= line) return launch_attn_kg<T, OutT, DP, 64, FULL, WIDE32 ? 1 : 2, DMA, KM, 2>(a, stream);
+    }
+    return launch_attn_kg<T, OutT, DP, BC, FULL, MINB, DMA, KM>(a, stream);
 }
 
 template <typename T>
