@@ -231,24 +231,36 @@ int gemm16_rope_common(void* ctx, void* stream, int kind, const uint16_t* A, con
     return hip_status(c, aidn::gemm_16_rope((hipStream_t)stream, kind, A, B, C, M, N, K, c->force_tile, ws, ws ? need : 0, rope), "gemm_16_rope");
 }
 
-// [Wq|Wk|Wv] side by side in one [dModel, 3 dModel] matrix (three strided device copies), the weight operand of the fused
-// QKV projection.
+// [Wq|Wk|Wv] side by side in one [dModel, 3 dModel] matrix, the weight operand of the fused QKV projection.  One launch of E-wide copies,
+// `width` of them to a row of each source (three strided device copies took 3 us and a gap each for 768 x 768 in 16-bit).
+template <typename E>
+__global__ __launch_bounds__(256) void gather_qkv_kernel(const E* __restrict__ wq, const E* __restrict__ wk, const E* __restrict__ wv, E* __restrict__ packed,
+                                                         int rows, int width)
+{
+    const int col = blockIdx.x * 256 + threadIdx.x;
+    if (col >= 3 * width) return;
+    const int which = col / width;
+    const E* src = (which == 0 ? wq : which == 1 ? wk : wv) + (col - which * width);
+    for (int r = blockIdx.y; r < rows; r += gridDim.y) packed[(long long)r * 3 * width + col] = src[(long long)r * width];
+}
+
 hipError_t gather_qkv(hipStream_t sm, const void* wq, const void* wk, const void* wv, void* packed, int dModel, size_t es)
 {
-    const void* w3[3] = {wq, wk, wv};
-    for (int j = 0; j < 3; j++) {
-        hipError_t e = hipMemcpy2DAsync((unsigned char*)packed + (size_t)j * dModel * es, (size_t)3 * dModel * es, w3[j], (size_t)dModel * es,
-                                        (size_t)dModel * es, (size_t)dModel, hipMemcpyDeviceToDevice, sm);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    auto go = [&](auto e, int width) {
+        typedef decltype(e) E;
+        hipLaunchKernelGGL(gather_qkv_kernel<E>, dim3((unsigned)((3LL * width + 255) / 256), (unsigned)std::min(dModel, 65535)), dim3(256), 0, sm, (const E*)wq, (const E*)wk,
+                           (const E*)wv, (E*)packed, dModel, width);
+        return hipGetLastError();
+    };
+    const bool vec = (((uintptr_t)wq | (uintptr_t)wk | (uintptr_t)wv | (uintptr_t)packed) & 15u) == 0 && (size_t)dModel * es % 16 == 0;
+    if (vec) return go(uint4{}, (int)((size_t)dModel * es / 16));
+    return es == 4 ? go((uint32_t)0, dModel) : go((uint16_t)0, dModel);
 }
 
 // Multi-head attention forward as three launches and no permutes: fused [Wq|Wk|Wv] projection into a packed
 // [B*S, 3*dModel] activation, attention reading it through strides and writing [B, S, H, d], output projection.
 // kind: 0 fp32, 1 fp16, 2 bf16 (16-bit: every intermediate stays in the input type, accumulation in fp32).
-// wqkv non-null: the caller's pre-packed [dModel, 3 dModel] weight (nothing is gathered); else wq, wk, wv are gathered into the
-// workspace on every call.
+// wqkv non-null: the caller's pre-packed [dModel, 3 dModel] weight; else wq, wk, wv, read in place or gathered into the workspace.
 int mha_common(void* ctx, void* stream, int kind, const void* input, const void* wq, const void* wk, const void* wv, const void* wqkv,
                const void* wo, const float* mask, int mask_mode, void* output, int B, int S, int dModel, int heads)
 {
@@ -266,7 +278,12 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
     if (rows > 0x7FFFFFFFLL || 3LL * dModel > 0x7FFFFFFFLL) return fail(c, AIDN_ERR_UNSUPPORTED, "mha: B*S or 3*dModel exceeds 2^31");
     const size_t es = kind == 0 ? 4 : 2;
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t wf_bytes = wqkv ? 0 : up((size_t)dModel * 3 * dModel * es), qkv_bytes = up((size_t)rows * 3 * dModel * es);
+    // the three weights are multiplied where they are, in one launch, unless their column tiles load the chip worse than those of the
+    // gathered matrix (bf16, 4096 rows x 768: 62 us a layer with the gather, 54 without; 2048 x 512 31 / 25)
+    // (weights off the 16-byte grid are gathered: the copy is what aligns them)
+    const uintptr_t at = wqkv ? (uintptr_t)wqkv : (uintptr_t)wq | (uintptr_t)wk | (uintptr_t)wv;
+    const bool x3 = c->force_tile == 0 && (at & 15u) == 0 && aidn::gemm_x3_suits(kind, (int)rows, dModel, dModel);
+    const size_t wf_bytes = wqkv || x3 ? 0 : up((size_t)dModel * 3 * dModel * es), qkv_bytes = up((size_t)rows * 3 * dModel * es);
     const size_t cc_bytes = up((size_t)rows * dModel * es);
     void* ws = nullptr;
     int st = acquire_ws(c, stream, wf_bytes + qkv_bytes + cc_bytes, &ws);
@@ -276,14 +293,26 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
     unsigned char* cc = qkv + qkv_bytes;
     hipStream_t sm = (hipStream_t)stream;
     hipError_t e;
-    if (!wqkv) {
+    if (!wqkv && !x3) {
         e = gather_qkv(sm, wq, wk, wv, wf, dModel, es);
         if (e != hipSuccess) return hip_status(c, e, "mha: weight gather");
     }
     const void* w3 = wqkv ? wqkv : (const void*)wf;
     const int M = (int)rows, N3 = 3 * dModel;
     const int tile32 = c->force_tile;
-    if (kind == 0) e = aidn::gemm_f32(sm, (const float*)input, (const float*)w3, (float*)qkv, M, N3, dModel, 1.0f, 0.0f, 0, 1, 0, 0, 0, tile32);
+    if (x3) {
+        const void* b[3] = {wq, wk, wv};
+        if (wqkv) for (int j = 0; j < 3; j++) b[j] = (const unsigned char*)wqkv + (size_t)j * dModel * es;
+        const int ldb = wqkv ? N3 : dModel;
+        if (kind == 0) {
+            const float* const b32[3] = {(const float*)b[0], (const float*)b[1], (const float*)b[2]};
+            e = aidn::gemm_f32_x3(sm, (const float*)input, b32, (float*)qkv, M, dModel, dModel, ldb, 0);
+        } else {
+            const uint16_t* const b16[3] = {(const uint16_t*)b[0], (const uint16_t*)b[1], (const uint16_t*)b[2]};
+            e = aidn::gemm_16_x3(sm, kind - 1, (const uint16_t*)input, b16, (uint16_t*)qkv, M, dModel, dModel, ldb, 0);
+        }
+    }
+    else if (kind == 0) e = aidn::gemm_f32(sm, (const float*)input, (const float*)w3, (float*)qkv, M, N3, dModel, 1.0f, 0.0f, 0, 1, 0, 0, 0, tile32);
     else e = aidn::gemm_16(sm, kind - 1, (const uint16_t*)input, (const uint16_t*)w3, qkv, 0, M, N3, dModel, c->force_tile, nullptr, 0);
     if (e != hipSuccess) return hip_status(c, e, "mha: QKV projection");
 

@@ -79,9 +79,10 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
             // dispatch: hand the query tiles out heaviest first across ALL heads, so the workgroups that end up sharing a
             // CU are a heavy one and, later in the id order, a light one.
             // (the first 256 ids, one per CU, in ascending weight, so that the ids after them -- which land on the same
-            // CUs in the same order -- pair the lightest of the first round with the heaviest of the second)
+            // CUs in the same order -- pair the lightest of the first round with the heaviest of the second; reversed by eights, so that
+            // where 8 divides the number of heads all query tiles of a head stay on one XCD, 1-4 % against reversing one by one)
             const int nbh = nblk / a.qtiles;
-            const int rank = (nblk > 256 && pid < 256) ? 255 - pid : pid;
+            const int rank = (nblk > 256 && pid < 256) ? 255 - (pid | 7) + (pid & 7) : pid;
             qt = a.qtiles - 1 - rank / nbh;
             bh = rank - (rank / nbh) * nbh;
         } else if (a.causal && a.hgroup > 0) {
@@ -1349,7 +1350,8 @@ static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
 // each wave half of every tile, merged through LDS at the end): 27 us; B1 H12 S1024 81 -> 48, and 32 with four.  Once the chip is full
 // the same matrix work only pays for more tile loads and merges (B16 H12 S512 83 -> 89 us).  The lines, as workgroups of the finer
 // grid, from a sweep over 58 shapes (time with one / two key groups in us at the last size on either side):
-//   64-key tiles, two workgroups per CU, head dimension up to 64: 768 (fp32 S512 causal 46 / 44, plain 74 / 67; 960: 54 / 54, S900 89 / 118);
+//   64-key tiles, two workgroups per CU, head dimension up to 64: 768 (fp32 plain S512 74 / 67, causal S4096 308 / 253; 960: 54 / 54, S900
+//     89 / 118); short causal fp32 sequences 640, beyond which the halved workgroups' starts and merges cost what they balance (S512 44.0 / 44.2);
 //     16-bit causal 1024 (S500 19.3 / 14.8, S1900 46 / 35; plain 20.4 / 21.1; 1536: 21 / 28)
 //   up to 128: 512, all resident at once (16-bit d80 plain 28.1 / 26.5; 768: 32.8 / 46.4)
 //   fp32 above 64: 64-key tiles need 128 KiB, one workgroup per CU: 256 (plain d128 151 / 88; 384: 66 / 83), causal 384 (64 / 42)
@@ -1368,7 +1370,8 @@ static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
         long long line;
         if constexpr (WIDE32) line = a.causal ? 384 : 256;
         else if constexpr (DP > 64) line = 512;
-        else line = !FULL && Elem<T>::BYTES == 2 && a.causal ? 1024 : 768;
+        else if constexpr (Elem<T>::BYTES == 2) line = !FULL && a.causal ? 1024 : 768;
+        else line = a.causal && a.Sk < 1024 ? 640 : 768;
         if (grid(64) <= line) return launch_attn_kg<T, OutT, DP, 64, FULL, WIDE32 ? 1 : 2, DMA, KM, 2>(a, stream);
     }
     return launch_attn_kg<T, OutT, DP, BC, FULL, MINB, DMA, KM>(a, stream);

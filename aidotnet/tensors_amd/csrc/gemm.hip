@@ -54,9 +54,21 @@ struct GemmArgs {
     // many columns (fewer than N, the columns past them are padding of B that is computed and dropped) and ldc is any element
     // count, so a row of C may start off a 16-byte boundary
     int c_cols = 0;
+    // three products with one A in one launch (three batches): the B of batches 1 and 2; null: batch b reads B + b * sB
+    const void* B1 = nullptr;
+    const void* B2 = nullptr;
 };
 
+// B of batch bz, in units of B's elements of EB bytes
+template <int EB>
+__device__ __forceinline__ const unsigned char* batch_b(const GemmArgs& g, long long bz)
+{
+    if (g.B1) return (const unsigned char*)(bz == 0 ? g.B : bz == 1 ? g.B1 : g.B2);
+    return (const unsigned char*)g.B + bz * g.sB * EB;
+}
+
 [[maybe_unused]] static bool aligned16(const void* p) { return (((uintptr_t)p) & 15u) == 0; }
+[[maybe_unused]] static bool b_aligned16(const GemmArgs& g) { return aligned16(g.B) && aligned16(g.B1) && aligned16(g.B2); }
 
 #if AIDN_GEMM_PART == 0
 hipError_t ensure_dynamic_smem(const void* kernel, int bytes, unsigned long long* done_mask)
@@ -236,7 +248,7 @@ __global__ __launch_bounds__(WM * WN * KS * 64) void gemm_kernel(const GemmArgs 
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const long long bz = blockIdx.z;
     const raw_t* __restrict__ A = (const raw_t*)g.A + bz * g.sA;
-    const raw_t* __restrict__ B = (const raw_t*)g.B + bz * g.sB;
+    const raw_t* __restrict__ B = (const raw_t*)batch_b<sizeof(raw_t)>(g, bz);
 
     // Global loads run two tiles ahead where the registers allow it (tile t travels in register set t & 1 and has two
     // iterations to arrive from memory: what a small problem with one workgroup per CU needs), otherwise one tile ahead.
@@ -632,7 +644,7 @@ __global__ __launch_bounds__((TILE == 256 ? 512 : 256) * KSW, TILE == 256 ? 1 : 
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const long long bz = blockIdx.z;                                         // batch index (strides in elements)
     const unsigned char* __restrict__ A = (const unsigned char*)g.A + bz * g.sA * EB;
-    const unsigned char* __restrict__ B = (const unsigned char*)g.B + bz * g.sB * EB;
+    const unsigned char* __restrict__ B = batch_b<EB>(g, bz);
 
     // Chunk swizzle of the B tile (which 16-byte chunk position of its LDS row a chunk of k-row `row` occupies):
     //   16-bit: c ^ ((row & 3) << 2)  -- the four rows one transposing read touches go to different bank groups (rows of 256
@@ -989,7 +1001,7 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const long long bz = blockIdx.z;
     const unsigned char* __restrict__ A = (const unsigned char*)g.A + bz * g.sA * EB;
-    const unsigned char* __restrict__ B = (const unsigned char*)g.B + bz * g.sB * EB;
+    const unsigned char* __restrict__ B = batch_b<EB>(g, bz);
 
     // Chunk swizzle of a B k-row (position of 16-byte chunk c in its 512-byte LDS row: c ^ b_swz(row)): the four rows one
     // transposing read touches go to different bank groups, and rows 8 apart -- the two 16-lane groups that share a cycle of
@@ -1289,7 +1301,7 @@ static hipError_t launch_gemm_dl16(GemmArgs g, int batch, hipStream_t stream)
     // tiles that later workgroups re-read (alternated in one process: fp16 8192^3 1336 -> 1408 TFLOP/s, bf16 1397 -> 1464,
     // 16384 x 8192 x 1024 989 -> 1166, 8192 x 50304 x 768 764 -> 873); a problem that fits the cache is better left to its
     // write-back path (4096 x 3072 x 768 881 -> 770, 8192 x 8192 x 2048 1283 -> 1248 with such stores).
-    const long long footprint = ((long long)g.M * g.K + (long long)g.K * g.N) * 2 * batch + (long long)g.M * g.N * batch * Elem<OutT>::BYTES;
+    const long long footprint = ((long long)g.M * g.K * (g.sA == 0 ? 1 : batch) + (long long)g.K * g.N * batch) * 2 + (long long)g.M * g.N * batch * Elem<OutT>::BYTES;
     const bool nts = footprint > (240LL << 20);
     if constexpr (!HALF) {
         if (nts) {
@@ -2242,7 +2254,7 @@ template <typename OutT>
 static bool dl16_applies(const GemmArgs& g)
 {
     const int OB = Elem<OutT>::BYTES;
-    return aligned16(g.A) && aligned16(g.B) && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.sA % 8 == 0 && g.sB % 8 == 0 &&
+    return aligned16(g.A) && b_aligned16(g) && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.sA % 8 == 0 && g.sB % 8 == 0 &&
            g.lda < (1 << 21) && g.ldb < (1 << 21) &&
            aligned16(g.C) && ((long long)g.ldc * OB) % 16 == 0 && (g.sC * OB) % 16 == 0 && (g.bias == nullptr || aligned16(g.bias)) &&
            g.alpha == 1.0f && g.beta == 0.0f;
@@ -2301,7 +2313,7 @@ template <typename T, typename OutT, bool TRANSB>
 static hipError_t dispatch_gemm(const GemmArgs& g, int batch, hipStream_t stream, int force_tile)
 {
     constexpr int E = Elem<T>::PER16;
-    const bool vec = aligned16(g.A) && aligned16(g.B) && g.lda % E == 0 && g.ldb % E == 0 && g.K % E == 0 &&
+    const bool vec = aligned16(g.A) && b_aligned16(g) && g.lda % E == 0 && g.ldb % E == 0 && g.K % E == 0 &&
                      (TRANSB || g.N % E == 0) && g.sA % E == 0 && g.sB % E == 0;
     auto tiles = [&](int bm, int bn) { return (long long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * batch; };
     int tile = force_tile;
@@ -2413,6 +2425,37 @@ static hipError_t dispatch_gemm(const GemmArgs& g, int batch, hipStream_t stream
         return launch_gemm<T, OutT, 64, 64, 2, 2, TRANSB, false, true>(g, batch, stream);
     }
     return hipErrorInvalidValue;
+}
+
+// C [M, 3 n] = A [M, K] x [B0 | B1 | B2], the three [K, n] blocks wherever they are (row stride ldb): one launch of three batches that
+// share A.  gemm_x3_suits: the tiles of an n-wide product load the chip as well as those of the 3 n-wide one would (n a multiple of 64,
+// so that no tile is cut that was not cut before; estimates within 3 %) -- then B need not be copied side by side for it.
+#if AIDN_GEMM_PART == 0
+bool gemm_x3_suits(int kind, int M, int n, int K)
+{
+    if (n % 64 != 0) return false;
+    if (kind == 0) {
+        const int t1 = f32_tile(M, 3 * n, K, 1, true), t3 = f32_tile(M, n, K, 3, true);
+        return f32_time_us(M, n, K, 3, t3, 1) <= 1.03 * f32_time_us(M, 3 * n, K, 1, t1, 1);
+    }
+    double s1, s3;
+    dl16_width(M, 3 * n, K, 1, &s1);
+    dl16_width(M, n, K, 3, &s3);
+    return s3 >= 0.97 * s1;
+}
+hipError_t gemm_f32_x3(hipStream_t stream, const float* A, const float* const (&B)[3], float* C, int M, int n, int K, int ldb, int force_tile)
+{
+    GemmArgs g{A, B[0], C, M, n, K, K, ldb, 3 * n, 0, 0, n, 1.0f, 0.0f, 0, 0, nullptr, 0, 0.0f};
+    g.B1 = B[1]; g.B2 = B[2];
+    return dispatch_gemm<float, float, false>(g, 3, stream, force_tile);
+}
+#endif
+template <typename T>
+static hipError_t gemm_16_x3_typed(hipStream_t stream, const uint16_t* A, const uint16_t* const (&B)[3], uint16_t* C, int M, int n, int K, int ldb, int force_tile)
+{
+    GemmArgs g{A, B[0], C, M, n, K, K, ldb, 3 * n, 0, 0, n, 1.0f, 0.0f, 0, 0, nullptr, 0, 0.0f};
+    g.B1 = B[1]; g.B2 = B[2];
+    return dispatch_gemm<T, T, false>(g, 3, stream, force_tile);
 }
 
 #if AIDN_GEMM_PART == 0
@@ -2599,6 +2642,8 @@ hipError_t gemm_16_f16(hipStream_t stream, const uint16_t* A, const uint16_t* B,
                        int M, int N, int K, int force_tile, void* workspace, size_t workspace_bytes, const float* bias, int act, float act_param, const uint16_t* Bpre);
 hipError_t gemm_16_bf16(hipStream_t stream, const uint16_t* A, const uint16_t* B, void* C, int out32,
                         int M, int N, int K, int force_tile, void* workspace, size_t workspace_bytes, const float* bias, int act, float act_param, const uint16_t* Bpre);
+hipError_t gemm_16_x3_f16(hipStream_t stream, const uint16_t* A, const uint16_t* const (&B)[3], uint16_t* C, int M, int n, int K, int ldb, int force_tile);
+hipError_t gemm_16_x3_bf16(hipStream_t stream, const uint16_t* A, const uint16_t* const (&B)[3], uint16_t* C, int M, int n, int K, int ldb, int force_tile);
 hipError_t gemm_16_rope_f16(hipStream_t stream, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int force_tile,
                             void* workspace, size_t workspace_bytes, const RopeEpilogue& rope);
 hipError_t gemm_16_rope_bf16(hipStream_t stream, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int force_tile,
@@ -2623,6 +2668,8 @@ static hipError_t gemm_16_rope_typed(hipStream_t stream, const uint16_t* A, cons
 hipError_t gemm_16_f16(hipStream_t stream, const uint16_t* A, const uint16_t* B, void* C, int out32,
                        int M, int N, int K, int force_tile, void* workspace, size_t workspace_bytes, const float* bias, int act, float act_param, const uint16_t* Bpre)
 { return gemm_16_typed<f16_t>(stream, A, B, C, out32, M, N, K, force_tile, workspace, workspace_bytes, bias, act, act_param, Bpre); }
+hipError_t gemm_16_x3_f16(hipStream_t stream, const uint16_t* A, const uint16_t* const (&B)[3], uint16_t* C, int M, int n, int K, int ldb, int force_tile)
+{ return gemm_16_x3_typed<f16_t>(stream, A, B, C, M, n, K, ldb, force_tile); }
 hipError_t gemm_16_rope_f16(hipStream_t stream, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int force_tile,
                             void* workspace, size_t workspace_bytes, const RopeEpilogue& rope)
 { return gemm_16_rope_typed<f16_t>(stream, A, B, C, M, N, K, force_tile, workspace, workspace_bytes, rope); }
@@ -2630,6 +2677,8 @@ hipError_t gemm_16_rope_f16(hipStream_t stream, const uint16_t* A, const uint16_
 hipError_t gemm_16_bf16(hipStream_t stream, const uint16_t* A, const uint16_t* B, void* C, int out32,
                         int M, int N, int K, int force_tile, void* workspace, size_t workspace_bytes, const float* bias, int act, float act_param, const uint16_t* Bpre)
 { return gemm_16_typed<bf16_t>(stream, A, B, C, out32, M, N, K, force_tile, workspace, workspace_bytes, bias, act, act_param, Bpre); }
+hipError_t gemm_16_x3_bf16(hipStream_t stream, const uint16_t* A, const uint16_t* const (&B)[3], uint16_t* C, int M, int n, int K, int ldb, int force_tile)
+{ return gemm_16_x3_typed<bf16_t>(stream, A, B, C, M, n, K, ldb, force_tile); }
 hipError_t gemm_16_rope_bf16(hipStream_t stream, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int force_tile,
                              void* workspace, size_t workspace_bytes, const RopeEpilogue& rope)
 { return gemm_16_rope_typed<bf16_t>(stream, A, B, C, M, N, K, force_tile, workspace, workspace_bytes, rope); }
@@ -2640,6 +2689,10 @@ hipError_t gemm_16(hipStream_t stream, int kind, const uint16_t* A, const uint16
 {
     if (kind == 0) return gemm_16_f16(stream, A, B, C, out32, M, N, K, force_tile, workspace, workspace_bytes, bias, act, act_param, Bpre);
     return gemm_16_bf16(stream, A, B, C, out32, M, N, K, force_tile, workspace, workspace_bytes, bias, act, act_param, Bpre);
+}
+hipError_t gemm_16_x3(hipStream_t stream, int kind, const uint16_t* A, const uint16_t* const (&B)[3], uint16_t* C, int M, int n, int K, int ldb, int force_tile)
+{
+    return kind == 0 ? gemm_16_x3_f16(stream, A, B, C, M, n, K, ldb, force_tile) : gemm_16_x3_bf16(stream, A, B, C, M, n, K, ldb, force_tile);
 }
 hipError_t gemm_16_rope(hipStream_t stream, int kind, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int force_tile,
                         void* workspace, size_t workspace_bytes, const RopeEpilogue& rope)

@@ -32,6 +32,12 @@ size_t gemm_16_workspace_bytes(int M, int N, int K);
 hipError_t gemm_16(hipStream_t stream, int kind, const uint16_t* A, const uint16_t* B, void* C, int out32,
                    int M, int N, int K, int force_tile, void* workspace, size_t workspace_bytes, const float* bias = nullptr, int act = 0,
                    float act_param = 0.0f, const uint16_t* Bpre = nullptr);
+// C [M, 3 n] = A [M, K] x [B[0] | B[1] | B[2]] with the three [K, n] blocks in place (row stride ldb); gemm_x3_suits (kind 0 fp32, 1 / 2
+// 16-bit): whether that is as fast as the product with the blocks side by side in one matrix
+bool gemm_x3_suits(int kind, int M, int n, int K);
+hipError_t gemm_f32_x3(hipStream_t stream, const float* A, const float* const (&B)[3], float* C, int M, int n, int K, int ldb, int force_tile);
+hipError_t gemm_16_x3(hipStream_t stream, int kind, const uint16_t* A, const uint16_t* const (&B)[3], uint16_t* C, int M, int n, int K, int ldb,
+                      int force_tile);
 // C = A B followed by interleaved RoPE over the first rope.cols columns of C (heads of rope.head_dim elements side by side; row m at
 // position rope.start_position + m % rope.seq_len); C has the inputs' type.  Where the product has a summing pass of its own (few
 // rows: K ranges side by side) the rotation rides on that pass, otherwise it is a second launch over C.

@@ -330,8 +330,9 @@ AIDN_API int aidn_mi355_mha_fwd_f16(void* ctx, void* stream, const uint16_t* inp
                            const uint16_t* wo, const float* mask, int mask_mode, uint16_t* output, int B, int S, int dModel, int heads);
 AIDN_API int aidn_mi355_mha_fwd_bf16(void* ctx, void* stream, const uint16_t* input, const uint16_t* wq, const uint16_t* wk, const uint16_t* wv,
                             const uint16_t* wo, const float* mask, int mask_mode, uint16_t* output, int B, int S, int dModel, int heads);
-/* The forms above gather [Wq|Wk|Wv] into the workspace on every call (3 dModel^2 elements read and written).  For constant
- * weights, pack once into a caller-owned [dModel, 3 dModel] buffer (elem_bytes 4 for fp32, 2 for fp16 / bf16) and call the
+/* The forms above multiply the three weights in place where dModel is a multiple of 64 whose column tiles load the chip well and the
+ * weights are 16-byte aligned; otherwise they gather [Wq|Wk|Wv] into the workspace on every call (3 dModel^2 elements read and
+ * written).  For constant weights of that kind, pack once into a caller-owned [dModel, 3 dModel] buffer (elem_bytes 4 for fp32, 2 for fp16 / bf16) and call the
  * *_packed forms, which read it in place: the concatenated weight of SimdGemm.SgemmConcatenatedProjections
  * (Engines/Simd/SimdGemm.NParallelSmallM.cs:95-109) and of the fused QKV GEMM in CpuEngine.MultiHeadAttention.cs:358-420. */
 AIDN_API int aidn_mi355_mha_pack_qkv(void* ctx, void* stream, const void* wq, const void* wk, const void* wv, void* packed,
