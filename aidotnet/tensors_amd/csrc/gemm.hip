@@ -1320,6 +1320,217 @@ static hipError_t launch_gemm_dl16(GemmArgs g, int batch, hipStream_t stream)
 }
 
 // ---------------------------------------------------------------------------------------------
+// 16-bit, rows at any element offset (N or K not a multiple of 8, or an operand off the 16-byte grid), B stored [K,N]: BM x 128 tile, 8
+// waves (2 x 4, wave tile BM/2 x 32 of 16 x 16 x 32 blocks), K-tiles of 64.  The direct-to-LDS loads want whole 16-byte chunks, so the
+// tiles travel through registers: every load is 16 bytes at element alignment and consecutive lanes take consecutive chunks of a row
+// (128 bytes of A, 256 of B), two K-tiles ahead, and is written to the LDS layout of gemm_dl16_kernel, from which the fragments are read
+// as there (transposing reads for B).  What bounds it is the stream of B for few rows and the load / LDS-write work beyond.
+// The general kernel's loads of B are 16 rows of 64 bytes to an instruction, each cache line asked for twice: 64 x 50257 x 768
+// took 44 us there and takes 17.5 here (84 MB), 212 x 36669 x 704 103 / 28, 512 x 30001 x 4096 232 through padded copies / 156.
+// kper > 0: workgroups z take K ranges of kper (a multiple of 64) each and C is their fp32 partials, sum_stride elements apart.
+// Bounds: the last K-tile of the matrix is loaded under guards (zeros past K; whole chunks where they fit their row); in the others a
+// chunk of B that crosses column N reads on into the next row, which exists, and is only multiplied into columns that are not stored.
+// Rows of A past M and chunks of B past N are clamped likewise.  N >= 8.
+template <typename T, typename OutT, int BM>
+__global__ __launch_bounds__(512, 4) void gemm_any16_kernel(const GemmArgs g, int kper, long long sum_stride)
+{
+    typedef typename Raw<T>::type raw_t;
+    typedef u32x4 u32x4_elem __attribute__((aligned(2)));
+    constexpr int BN = 128, BK = 64, TI = BM / 32, TJ = 2;
+    constexpr int AROW = 128, BROW = 2 * BN;
+    constexpr int ABYTES = BM * AROW, STAGE = ABYTES + BK * BROW;
+    constexpr int LA = BM / 64, LB = 2;                      // chunks of A and B per thread and tile
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int l16 = lane & 15, g4 = lane >> 4;
+    const int wm = wave >> 2, wn = wave & 3;
+    int tile_m, tile_n;
+    tile_of_block(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tile_m, tile_n);
+    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int kbeg = kper > 0 ? (int)blockIdx.z * kper : 0;
+    const int K = kper > 0 ? min(kper, g.K - kbeg) : g.K;
+    const int KT = (K + BK - 1) / BK;
+
+    auto b_swz = [](int row) -> int { return ((row & 3) << 2) | (((row >> 3) & 1) << 1); };
+    // this thread's chunks: A rows t / 8 + 64 i, chunk t % 8; B k-rows t / 16 + 32 i, chunk t % 16
+    const int ach = t & 7, bch = t & 15;
+    // (element offsets from wave-uniform bases that advance with the tile: lda, ldb < 2^21)
+    const raw_t* a_base = (const raw_t*)g.A + (long long)m0 * g.lda + kbeg;
+    const raw_t* b_base = (const raw_t*)g.B + (long long)kbeg * g.ldb;
+    uint32_t pa[LA];
+    int a_lds[LA], b_lds[LB];
+#pragma unroll
+    for (int i = 0; i < LA; i++) {
+        const int row = (t >> 3) + 64 * i;
+        pa[i] = (uint32_t)((min(m0 + row, g.M - 1) - m0) * g.lda + ach * 8);
+        a_lds[i] = row * AROW + ((ach ^ ((row >> 1) & 7)) << 4);
+    }
+    const int bcol = min(n0 + bch * 8, g.N - 1);
+    const uint32_t pb = (uint32_t)((t >> 4) * g.ldb + bcol);
+#pragma unroll
+    for (int i = 0; i < LB; i++) {
+        const int row = (t >> 4) + 32 * i;
+        b_lds[i] = ABYTES + row * BROW + ((bch ^ b_swz(row)) << 4);
+    }
+    u32x4 ra[2][LA], rb[2][LB];
+    auto load_plain = [&](int kt, auto set) {
+        constexpr int S = decltype(set)::value;
+#pragma unroll
+        for (int i = 0; i < LA; i++) ra[S][i] = *(const u32x4_elem*)(a_base + kt * BK + pa[i]);
+#pragma unroll
+        for (int i = 0; i < LB; i++) rb[S][i] = *(const u32x4_elem*)(b_base + (long long)(kt * BK + 32 * i) * g.ldb + pb);
+    };
+    auto load_any = [&](int kt, auto set) {
+        constexpr int S = decltype(set)::value;
+        if (kt < KT - 1) { load_plain(kt, set); return; }
+        if (kt >= KT) return;
+#pragma unroll
+        for (int i = 0; i < LA; i++) {
+            const int valid = K - (kt * BK + ach * 8);
+            ra[S][i] = u32x4{0u, 0u, 0u, 0u};
+            if (valid > 0) ra[S][i] = load16_guarded<T>(a_base + kt * BK + pa[i], valid);
+        }
+#pragma unroll
+        for (int i = 0; i < LB; i++) {
+            const int k = kt * BK + 32 * i + (t >> 4);
+            rb[S][i] = u32x4{0u, 0u, 0u, 0u};
+            if (k < K) rb[S][i] = load16_guarded<T>(b_base + (long long)(kt * BK + 32 * i) * g.ldb + pb, g.N - bcol);
+        }
+    };
+    auto store_tile = [&](int stage, auto set) {
+        constexpr int S = decltype(set)::value;
+        unsigned char* st = smem + stage * STAGE;
+#pragma unroll
+        for (int i = 0; i < LA; i++) *(u32x4*)(st + a_lds[i]) = ra[S][i];
+#pragma unroll
+        for (int i = 0; i < LB; i++) *(u32x4*)(st + b_lds[i]) = rb[S][i];
+    };
+
+    // fragments: as in gemm_dl16_kernel
+    const int a_row0 = (wm * (BM / 2) + l16) * AROW, a_sw = (l16 >> 1) & 7;
+    const int b_rowl = 8 * g4 + (l16 >> 2), b_half = (l16 & 1) * 8, b_chunk0 = wn * (2 * TJ) + ((l16 & 3) >> 1);
+    f32x4_acc acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++) acc[i][j] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
+    auto multiply = [&](int stage) {
+        const unsigned char* as = smem + stage * STAGE;
+        const unsigned char* bs = as + ABYTES;
+#pragma unroll
+        for (int s2 = 0; s2 < 2; s2++) {
+            u32x4 fa[TI], fb[TJ];
+#pragma unroll
+            for (int i = 0; i < TI; i++) fa[i] = *(const u32x4*)(as + a_row0 + i * (16 * AROW) + (((4 * s2 + g4) ^ a_sw) << 4));
+#pragma unroll
+            for (int j = 0; j < TJ; j++)
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const int row = 32 * s2 + 4 * q + b_rowl;
+                    const u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) s16x4*)(bs + row * BROW + (((b_chunk0 + 2 * j) ^ b_swz(row)) << 4) + b_half)));
+                    fb[j][2 * q] = w[0];
+                    fb[j][2 * q + 1] = w[1];
+                }
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int j = 0; j < TJ; j++) Mma16<T>::run(acc[i][j], fb[j], fa[i]);
+        }
+    };
+    // iteration kt: tile kt is in stage kt & 1; tile kt + 2 goes into the register set whose tile was stored an iteration ago, tile
+    // kt + 1 from the other set into the other stage, which everyone left at the barrier that ended iteration kt - 1
+    typedef std::integral_constant<int, 0> Set0;
+    typedef std::integral_constant<int, 1> Set1;
+    load_any(0, Set0{});
+    load_any(1, Set1{});
+    store_tile(0, Set0{});
+    __syncthreads();
+    auto step = [&](int kt, auto plain, auto mine, auto other) {
+        constexpr int P = decltype(mine)::value;
+        if constexpr (decltype(plain)::value) load_plain(kt + 2, mine);
+        else load_any(kt + 2, mine);
+        multiply(P);
+        if (decltype(plain)::value || kt + 1 < KT) store_tile(P ^ 1, other);
+        __syncthreads();
+    };
+    int kt = 0;
+    // (the loop proper loads whole tiles that are not the last one: no branch stands between its loads and their use)
+    for (; kt + 4 < KT; kt += 2) {
+        step(kt, std::true_type{}, Set0{}, Set1{});
+        step(kt + 1, std::true_type{}, Set1{}, Set0{});
+    }
+    for (; kt < KT; kt += 2) {
+        step(kt, std::false_type{}, Set0{}, Set1{});
+        if (kt + 1 < KT) step(kt + 1, std::false_type{}, Set1{}, Set0{});
+    }
+
+    // epilogue: acc[i][j] holds C[row 16 i + l16][columns 16 j + 4 g4 .. + 3] of the wave tile; staged through the dead stages (16-byte
+    // chunk c of row r at position c ^ (r & 15)) so that rows leave in 16-byte stores at element alignment
+    constexpr int OB = Elem<OutT>::BYTES, PITCH = BN * OB, CPR = PITCH / 16, PER = 16 / OB;
+    static_assert(BM * PITCH <= 2 * STAGE, "C staging must stay inside the tile memory");
+    const bool fused = g.bias != nullptr || g.act != 0;
+    f32x4_acc bias[TJ];
+    if (fused) {
+#pragma unroll
+        for (int j = 0; j < TJ; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int col = n0 + wn * 32 + 16 * j + 4 * g4 + e;
+                bias[j][e] = g.bias && col < g.N ? g.bias[col] : 0.0f;
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < TI; i++) {
+        const int row = wm * (BM / 2) + 16 * i + l16;
+        f32x4_acc w[TJ];
+#pragma unroll
+        for (int j = 0; j < TJ; j++) w[j] = acc[i][j];
+        if (fused)
+            with_activation(g.act, g.act_param, [&](auto fn) {
+#pragma unroll
+                for (int j = 0; j < TJ; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) w[j][e] = fn(w[j][e] + bias[j][e]);
+            });
+#pragma unroll
+        for (int j = 0; j < TJ; j++) {
+            const int col = wn * 32 + 16 * j + 4 * g4;
+            unsigned char* dst = smem + row * PITCH + ((((col * OB) >> 4) ^ (row & 15)) << 4);
+            if constexpr (OB == 2) *(u32x2*)(dst + (g4 & 1) * 8) = u32x2{Elem<OutT>::narrow(w[j][0]) | (Elem<OutT>::narrow(w[j][1]) << 16),
+                                                                        Elem<OutT>::narrow(w[j][2]) | (Elem<OutT>::narrow(w[j][3]) << 16)};
+            else *(u32x4*)dst = u32x4{as_u32(w[j][0]), as_u32(w[j][1]), as_u32(w[j][2]), as_u32(w[j][3])};
+        }
+    }
+    __syncthreads();
+    typedef typename Raw<OutT>::type out_t;
+    out_t* C = (out_t*)g.C + (kper > 0 ? (long long)blockIdx.z * sum_stride : 0);
+#pragma unroll 4
+    for (int u = t; u < BM * CPR; u += 512) {
+        const int row = u / CPR, c = u % CPR, col = n0 + c * PER;
+        if (m0 + row >= g.M || col >= g.N) continue;
+        const u32x4 v = *(const u32x4*)(smem + row * PITCH + ((c ^ (row & 15)) << 4));
+        out_t* dst = C + (long long)(m0 + row) * g.ldc + col;
+        if (col + PER <= g.N) *(u32x4_elem*)dst = v;
+        else
+            for (int e = 0; e < g.N - col; e++) dst[e] = (out_t)(OB == 2 ? v[e >> 1] >> ((e & 1) * 16) : v[e]);
+    }
+}
+
+template <typename T, typename OutT, int BM>
+static hipError_t launch_any16(GemmArgs g, hipStream_t stream, int ks = 1, int kper = 0)
+{
+    constexpr int smem = 2 * (BM * 128 + 64 * 256);
+    auto kern = gemm_any16_kernel<T, OutT, BM>;
+    static unsigned long long attr_done = 0;
+    if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done)) return e;
+    g.tiles_m = (g.M + BM - 1) / BM;
+    g.tiles_n = (g.N + 127) / 128;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(g.tiles_m * g.tiles_n), 1, (unsigned)ks), dim3(512), smem, stream, g, ks > 1 ? kper : 0, (long long)g.M * g.N);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------
 // Skinny-M path (decode projections): M <= 32, 16-bit, B stored [K,N], N % 128 == 0, K % 64 == 0.
 // HBM-bound: B (K x N) is read exactly once.  grid = (N / 128, KS), about one workgroup per CU: each workgroup streams a
 // 128-column slab of B over its K range with the direct global->LDS load through a ring of NS 20 KB stages, filled NS - 1
@@ -1623,11 +1834,32 @@ static bool pad16_layout(int M, int N, int K, PadPlan* pl)
 static bool pad16_plan(int M, int N, int K, PadPlan* pl)
 {
     if (N % 8 == 0 && K % 8 == 0) return false;
-    if (N < 16 || (double)M * N * K < (double)(1 << 21)) return false;        // launch-bound either way
-    // few rows over a short K: the copy of B would cost more than the product; the general kernel reads such rows in place with
-    // element-aligned 16-byte loads (64 x 50257 x 768: 42 us against 51 us through the copies)
-    if (M <= 512 && K <= 1024) return false;
+    // gemm_any16_kernel reads such rows in place at about 0.8 PFLOP/s, the kernels for aligned rows reach about 1.25 and the copies
+    // (read and write of B, of A where K is padded) run at about 4 TB/s with 8 us of launches: many rows repay them.  In place /
+    // copied, us: 700 x 9001 x 8000 134 / 195, 4000 x 3001 x 1000 40 / 44, 4096 x 4095 x 4096 154 / 117, 8000 x 5001 x 3001 319 / 240.
+    const double gain_us = 0.9e-9 * M * N * K, copy_us = 1e-6 * ((double)K * N + (K % 64 ? (double)M * K : 0.0)) + 8.0;
+    if (gain_us <= copy_us) return false;
     return pad16_layout(M, N, K, pl);
+}
+
+// gemm_any16_kernel: tile height and K ranges (kper, a multiple of 64; 0 = none).  128 rows where such tiles fill the chip (212 x 36669 x
+// 704 28 us against 31 with 64 rows, 2000 x 2001 x 2000 27 / 33), else 64 (1049 x 1216 x 398 7.1 / 9.0) and, with few tiles, K ranges summed by a
+// pass of their own.  The estimate (us): 0.6 a K-tile with up to two workgroups per CU, 2 for the start, 3 for the second launch and the
+// partials at 3 TB/s; 30 x 300 x 9001 80 -> 12 in 16 ranges, 100 x 1003 x 5000 36 -> 13, 16 x 5910 x 1600 18 -> 12 in four.
+static int any16_plan(int M, int N, int K, int* kper, int* ranges)
+{
+    const long long tn = (N + 127) / 128, t128 = (M + 127) / 128 * tn, t64 = (M + 63) / 64 * tn;
+    *kper = 0; *ranges = 1;
+    if (M > 64 && t128 >= 256) return 128;
+    const int kt = (K + 63) / 64;
+    double best = 0.0;
+    for (int ks = 1; ks <= 32 && ks <= kt; ks++) {
+        const int per = (kt + ks - 1) / ks, n = (kt + per - 1) / per;
+        const double load = (double)(t64 * n) / 512.0;
+        const double us = 0.6 * per * (load > 1.0 ? load : 1.0) + (n > 1 ? 3.0 + 0.08 * n + (double)n * M * N * 8.0 / 3e6 : 0.0);
+        if (ks == 1 || us < best) { best = us; *ranges = n; *kper = n > 1 ? 64 * per : 0; }
+    }
+    return 64;
 }
 
 // dst [rows_dst, cols_dst] (16-byte aligned rows) <- src [rows_src, cols_src] (dense, any alignment), zeros elsewhere; E = element.
@@ -1792,8 +2024,14 @@ size_t gemm_16_workspace_bytes(int M, int N, int K)
 {
     PadPlan pl;
     const size_t inner = gemm_16_inner_workspace_bytes(M, N, K);
-    if (pad16_plan(M, N, K, &pl) && pl.total > inner) return pl.total;
-    return inner;
+    size_t need = inner;
+    if (pad16_plan(M, N, K, &pl) && pl.total > need) need = pl.total;
+    if (N % 8 != 0 || K % 8 != 0) {
+        int kper, ks;
+        any16_plan(M, N, K, &kper, &ks);
+        if (ks > 1) need = std::max(need, (size_t)ks * M * N * sizeof(float));
+    }
+    return need;
 }
 // Pre-packed B (the caller keeps it): B [K,N] zero-padded to [Kp, Np] -- the copy that an unaligned product otherwise makes on every
 // call, made once.  An aligned weight is packed the same way (its K and N padded to whole tiles).
@@ -2603,6 +2841,21 @@ static hipError_t gemm_16_typed(hipStream_t stream, const uint16_t* A, const uin
         return padC ? unpad_rows(stream, Cp, C, M, N, pl.Np, out32 ? 4 : 2) : hipSuccess;
     }
     GemmArgs g{A, B, C, M, N, K, K, N, N, 0, 0, 0, 1.0f, 0.0f, 0, 0, bias, act, act_param};
+    if (force_tile == 0 && !(N % 8 == 0 && K % 8 == 0 && aligned16(A) && aligned16(B)) && N >= 16 && N < (1 << 21) && K < (1 << 21)) {
+        int kper, ks;
+        const int bm = any16_plan(M, N, K, &kper, &ks);
+        if (ks > 1 && (size_t)ks * M * N * sizeof(float) <= workspace_bytes) {
+            GemmArgs gp = g;
+            gp.C = workspace; gp.bias = nullptr; gp.act = 0;
+            if (hipError_t e = launch_any16<T, float, 64>(gp, stream, ks, kper)) return e;
+            const unsigned grid = (unsigned)(((long long)M * N + 255) / 256);
+            if (out32) hipLaunchKernelGGL((skinny_reduce_kernel<float>), dim3(grid), dim3(256), 0, stream, (const float*)workspace, C, M, N, ks, bias, act, act_param, 1.0f, 0.0f);
+            else hipLaunchKernelGGL((skinny_reduce_kernel<T>), dim3(grid), dim3(256), 0, stream, (const float*)workspace, C, M, N, ks, bias, act, act_param, 1.0f, 0.0f);
+            return hipGetLastError();
+        }
+        if (bm == 64) return out32 ? launch_any16<T, float, 64>(g, stream) : launch_any16<T, T, 64>(g, stream);
+        return out32 ? launch_any16<T, float, 128>(g, stream) : launch_any16<T, T, 128>(g, stream);
+    }
     if (force_tile == 0 && workspace && skinny_applies(M, N, K) && aligned16(A) && aligned16(B) &&
         (size_t)skinny_ksplit(N, K) * M * N * sizeof(float) <= workspace_bytes) {
         float* ws = (float*)workspace;
