@@ -2120,6 +2120,11 @@ __global__ __launch_bounds__(256) void gemm_smallm_kernel(const GemmArgs g, floa
                 u32x2 w = __builtin_nontemporal_load((const u32x2*)p);
                 r[0] = f16_bits_to_float(w[0] & 0xFFFFu); r[1] = f16_bits_to_float(w[0] >> 16);
                 r[2] = f16_bits_to_float(w[1] & 0xFFFFu); r[3] = f16_bits_to_float(w[1] >> 16);
+            } else if (nvalid >= 4) {
+                typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+                const u32x2 w = *(const u32x2_a2*)p;
+                r[0] = f16_bits_to_float(w[0] & 0xFFFFu); r[1] = f16_bits_to_float(w[0] >> 16);
+                r[2] = f16_bits_to_float(w[1] & 0xFFFFu); r[3] = f16_bits_to_float(w[1] >> 16);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; e++) if (e < nvalid) r[e] = f16_bits_to_float(p[e]);
@@ -2127,7 +2132,11 @@ __global__ __launch_bounds__(256) void gemm_smallm_kernel(const GemmArgs g, floa
         } else {
             const float* p = (const float*)g.B + (long long)k * g.ldb + n;
             if (VEC) r = __builtin_nontemporal_load((const f32x4*)p);      // B is read once per launch
-            else {
+            else if (nvalid >= 4) {
+                // (rows off the 16-byte grid: one load at element alignment instead of four: 1 x 40109 x 1088 45 -> 35 us)
+                typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+                r = __builtin_nontemporal_load((const f32x4_a4*)p);
+            } else {
 #pragma unroll
                 for (int e = 0; e < 4; e++) if (e < nvalid) r[e] = p[e];
             }
@@ -2192,6 +2201,97 @@ __global__ __launch_bounds__(256) void gemm_smallm_kernel(const GemmArgs g, floa
             }
         }
     }
+}
+
+// The same product in one launch for weights of a few megabytes, where the second launch and the partials cost more than the stream: a
+// workgroup of 16 waves owns 64 columns and all of K.  A wave-load is four k-rows of 256 bytes; wave w takes the rows 4 w .. 4 w + 3 of
+// every 64, SMALLM1_DEPTH of them in flight, against the rows of A in LDS ([k][MR], read as whole rows); the four k-rows of a wave are
+// summed by lane exchanges, the waves through LDS, and the epilogue is applied there.  What bounds it is the memory round trip:
+// 8 x 768 x 768 10.4 us in two launches, 7.2 in one, 1 x 768 x 768 6.5 / 4.2, 8 x 1024 x 1024 10.5 / 8.5, 1 x 16384 x 256 9.8 / 3.4; fp16
+// weights 8 x 768 x 768 13.2 / 8.2, 1 x 4096 x 1024 18.1 / 6.2.  Beyond a K of 1024 a workgroup's own stream is the longer (8 x 2048 x 2048
+// 11.7 / 13.8, 1 x 768 x 3072 6.2 / 9.1), and wide weights keep every CU busy either way (1 x 40109 x 1088 35 / 36).
+#define SMALLM1_DEPTH 6
+static bool smallm1_suits(int N, int K) { return K <= 1024 && (long long)N * K <= (1LL << 22); }
+template <int MR, bool B16>
+__global__ __launch_bounds__(1024) void gemm_smallm1_kernel(const GemmArgs g)
+{
+    extern __shared__ __attribute__((aligned(16))) float sm1[];
+    float* As = sm1;                                          // [K][MR]
+    float* red = sm1 + (long long)g.K * MR;                   // [16 waves][MR][64]
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int n0 = blockIdx.x * 64, n = n0 + 4 * (lane & 15);
+    const int kr = 4 * wave + (lane >> 4);
+    const int nvalid = g.N - n;
+    auto load_b = [&](int k) -> f32x4 {
+        f32x4 r = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (nvalid <= 0 || k >= g.K) return r;
+        if constexpr (B16) {
+            const uint16_t* p = (const uint16_t*)g.B + (long long)k * g.ldb + n;
+            typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+            if (nvalid >= 4) {
+                const u32x2 w = *(const u32x2_a2*)p;
+                r[0] = f16_bits_to_float(w[0] & 0xFFFFu); r[1] = f16_bits_to_float(w[0] >> 16);
+                r[2] = f16_bits_to_float(w[1] & 0xFFFFu); r[3] = f16_bits_to_float(w[1] >> 16);
+            } else
+                for (int e = 0; e < 3; e++) if (e < nvalid) r[e] = f16_bits_to_float(p[e]);
+        } else {
+            const float* p = (const float*)g.B + (long long)k * g.ldb + n;
+            typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+            if (nvalid >= 4) r = *(const f32x4_a4*)p;
+            else
+                for (int e = 0; e < 3; e++) if (e < nvalid) r[e] = p[e];
+        }
+        return r;
+    };
+    f32x4 b[SMALLM1_DEPTH];
+#pragma unroll
+    for (int u = 0; u < SMALLM1_DEPTH; u++) b[u] = load_b(kr + 64 * u);
+    for (int k = t; k < g.K; k += 1024) {
+        float a[MR];
+#pragma unroll
+        for (int m = 0; m < MR; m++) a[m] = ((const float*)g.A)[(long long)min(m, g.M - 1) * g.lda + k];
+#pragma unroll
+        for (int m = 0; m < MR; m++) As[k * MR + m] = a[m];
+    }
+    __syncthreads();
+    f32x4 acc[MR];
+#pragma unroll
+    for (int m = 0; m < MR; m++) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k0 = kr; k0 < g.K; k0 += 64 * SMALLM1_DEPTH) {
+        if (k0 != kr) {
+#pragma unroll
+            for (int u = 0; u < SMALLM1_DEPTH; u++) b[u] = load_b(k0 + 64 * u);
+        }
+#pragma unroll
+        for (int u = 0; u < SMALLM1_DEPTH; u++) {
+            const int k = k0 + 64 * u;
+            if (k >= g.K) break;
+#pragma unroll
+            for (int m = 0; m < MR; m++) {
+                const float av = As[k * MR + m];
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[m][e] = fmaf(av, b[u][e], acc[m][e]);
+            }
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < MR; m++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[m][e] = sum_with_partner32(sum_with_partner16(acc[m][e]));
+        if (lane < 16) *(f32x4*)(red + (wave * MR + m) * 64 + 4 * lane) = acc[m];
+    }
+    __syncthreads();
+    if (t >= MR * 64) return;
+    const int m = t >> 6, col = n0 + lane;
+    if (m >= g.M || col >= g.N) return;
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 16; w++) v += red[(w * MR + m) * 64 + lane];
+    v *= g.alpha;
+    float* c = (float*)g.C + (long long)m * g.ldc + col;
+    if (g.beta != 0.0f) v += g.beta * *c;
+    if (g.bias) v += g.bias[col];
+    *c = apply_activation(v, g.act, g.act_param);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2438,12 +2538,21 @@ size_t gemm_f32_workspace_bytes(int M, int N, int K, int transB)
 template <bool B16>
 static hipError_t launch_smallm(const GemmArgs& g, hipStream_t stream, float* ws)
 {
+    const int mr = g.M <= 1 ? 1 : g.M <= 2 ? 2 : g.M <= 4 ? 4 : 8;
+    if (smallm1_suits(g.N, g.K)) {
+        const int bytes = (g.K + 16 * 64) * mr * 4;                       // A and the waves' sums: 64 KiB at most
+        const dim3 one((unsigned)((g.N + 63) / 64));
+        if (mr == 1) hipLaunchKernelGGL((gemm_smallm1_kernel<1, B16>), one, dim3(1024), bytes, stream, g);
+        else if (mr == 2) hipLaunchKernelGGL((gemm_smallm1_kernel<2, B16>), one, dim3(1024), bytes, stream, g);
+        else if (mr == 4) hipLaunchKernelGGL((gemm_smallm1_kernel<4, B16>), one, dim3(1024), bytes, stream, g);
+        else hipLaunchKernelGGL((gemm_smallm1_kernel<8, B16>), one, dim3(1024), bytes, stream, g);
+        return hipGetLastError();
+    }
     const int kper = smallm_kper(g.N, g.K);
     const int ks = (g.K + kper - 1) / kper;
     // whole 16-byte loads of B: rows in 16-byte steps that hold every chunk a lane may touch (N a multiple of 4, or rows padded to one)
     const bool vec = (g.N % 4 == 0 || g.ldb >= (g.N + 3) / 4 * 4) && g.ldb % 4 == 0 && (((uintptr_t)g.B) & (B16 ? 7u : 15u)) == 0;
     const dim3 grid((unsigned)((g.N + 255) / 256), (unsigned)ks);
-    const int mr = g.M <= 1 ? 1 : g.M <= 2 ? 2 : g.M <= 4 ? 4 : 8;
 #define AIDN_SMALLM(MR_)                                                                                               \
     do {                                                                                                               \
         if (vec) hipLaunchKernelGGL((gemm_smallm_kernel<MR_, B16, true>), grid, dim3(256), 0, stream, g, ws, kper);     \
