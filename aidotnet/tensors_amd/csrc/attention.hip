@@ -105,7 +105,8 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     const int b = bh / a.H, hd = bh - b * a.H;
     const int kvh = hd / (a.H / a.Hkv);
     const int q0 = qt * BR;
-    const int wq = wave % WQ, kg = wave / WQ;  // this wave's row group and key group
+    // this wave's row group and key group (a constant with one group: the compiler does not know that wave < 4)
+    const int wq = KG == 1 ? wave : wave % WQ, kg = KG == 1 ? 0 : wave / WQ;
     const int qi = q0 + wq * 32 + l32;         // this lane's query row
     const bool vec = a.vec_in != 0;
 
