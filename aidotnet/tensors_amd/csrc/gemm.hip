@@ -2216,8 +2216,8 @@ template <int MR, bool B16>
 __global__ __launch_bounds__(1024) void gemm_smallm1_kernel(const GemmArgs g)
 {
     extern __shared__ __attribute__((aligned(16))) float sm1[];
-    float* As = sm1;                                          // [K][MR]
-    float* red = sm1 + (long long)g.K * MR;                   // [16 waves][MR][64]
+    float* red = sm1;                                         // [16 waves][MR][64]; first, so that its 16-byte stores are aligned at any K
+    float* As = sm1 + 16 * MR * 64;                           // [K][MR]
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int n0 = blockIdx.x * 64, n = n0 + 4 * (lane & 15);
     const int kr = 4 * wave + (lane >> 4);
