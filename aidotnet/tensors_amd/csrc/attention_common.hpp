@@ -53,7 +53,8 @@ __device__ __forceinline__ int paged_tile_rows(const int* __restrict__ bt, int b
     const int blk = (int)fastdiv((uint32_t)key, dbsz);
     return bt[blk] * bsz + (key - blk * bsz);
 }
-// block sizes the direct-to-LDS kernels take (the row numbers of a pool fit 31 bits at any size that fits the memory)
+// block sizes the direct-to-LDS kernels take (their rows are at least 128 bytes long: the row numbers of a K and a V pool that fit the
+// memory together fit 31 bits)
 inline bool paged_block_fits(const int* bt, int bsz) { return !bt || bsz % 16 == 0; }
 
 template <typename T> struct Raw2;

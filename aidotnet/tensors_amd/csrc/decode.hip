@@ -152,20 +152,25 @@ __global__ __launch_bounds__(256) void decode_partial_kernel(const DecodeArgs a)
 
     // Keys of load u of this wave's iteration `it`: KPW consecutive ones from first_key(it, u) on, lane group sk the sk-th.  Their row is
     // uniform: the key itself, or on a paged cache a pool row that one lane of `rows` looked up for the wave (16 iterations per table
-    // read, so that no load waits for a table access).
+    // read, so that no load waits for a table access).  64 bits: one K/V head of 8 elements makes rows of 16 bytes, of which a pool that fits
+    // the memory holds more than 2^31.
     const int wave_s = __builtin_amdgcn_readfirstlane(wave);
     const int first = kbeg + wave_s * (U * KPW);
     constexpr int STEP = NWV * U * KPW;
     auto first_key = [&](int it, int u) { return first + it * STEP + u * KPW; };
     const long long k_lane = sk * a.ks[2] + d0, v_lane = sk * a.vs[2] + d0;
     const bool in_row = d0 < a.D;                       // (lanes past the head dimension load nothing)
-    int rows = 0;
+    long long rows = 0;
+    auto pool_row = [&](int i) -> long long {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)rows, i), hi = (uint32_t)__builtin_amdgcn_readlane((int)(rows >> 32), i);
+        return (long long)(((uint64_t)hi << 32) | lo);
+    };
     auto load = [&](int it, u32x4 (&kx)[U], u32x4 (&vx)[U]) {
         if constexpr (ROWS) {
             if (bt && it % (64 / U) == 0) {
                 const int key = min(first_key(it + lane / U, lane % U), (a.Sk - 1) / KPW * KPW);
                 const int blk = (int)fastdiv((uint32_t)key, a.dbsz);
-                rows = bt[blk] * a.bsz + (key - blk * a.bsz);
+                rows = (long long)bt[blk] * a.bsz + (key - blk * a.bsz);
             }
         }
 #pragma unroll
@@ -174,7 +179,7 @@ __global__ __launch_bounds__(256) void decode_partial_kernel(const DecodeArgs a)
             const bool ok = in_row && key < kend;
             kx[u] = vx[u] = u32x4{0u, 0u, 0u, 0u};
             if constexpr (ROWS) {
-                const long long row = bt ? __builtin_amdgcn_readlane(rows, (it * U + u) & 63) : first_key(it, u);
+                const long long row = bt ? pool_row((it * U + u) & 63) : first_key(it, u);
                 const raw_t* kp = K + row * a.ks[2];
                 const raw_t* vp = V + row * a.vs[2];
                 if (ok) {
