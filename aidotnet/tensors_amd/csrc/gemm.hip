@@ -2470,7 +2470,7 @@ static int smallm_kper(int N, int K)
 #if AIDN_GEMM_PART == 0
 size_t gemm_smallm_workspace_bytes(int M, int N, int K)
 {
-    if (!smallm_applies(M, N, K)) return 0;
+    if (!smallm_applies(M, N, K) || smallm1_suits(N, K)) return 0;      // (the one-launch form keeps its sums in LDS)
     const int kper = smallm_kper(N, K);
     return (size_t)((K + kper - 1) / kper) * M * N * sizeof(float);
 }
@@ -2525,6 +2525,7 @@ size_t gemm_f32_workspace_bytes(int M, int N, int K, int transB)
 {
     size_t need = 0;
     auto upto = [&](size_t n) { if (n > need) need = n; };
+    if (!transB && smallm_applies(M, N, K) && smallm1_suits(N, K)) return 0;      // taken at any alignment
     Pad32Plan pl;
     if (pad32_plan(M, N, K, transB, &pl)) upto(pl.total);
     if (!transB && smallm_applies(M, N, K)) upto(gemm_smallm_workspace_bytes(M, N, K));
@@ -2815,7 +2816,7 @@ hipError_t gemm_f32(hipStream_t stream, const float* A, const float* B, float* C
     if (!workspace) workspace_bytes = 0;
     // every plan below that writes to the workspace first holds its own need against the bytes handed in, and is passed over
     // (down to the tiled kernels, which need none) when they do not suffice
-    const bool smallm_fits = workspace && smallm_applies(M, N, K) && gemm_smallm_workspace_bytes(M, N, K) <= workspace_bytes;
+    const bool smallm_fits = smallm_applies(M, N, K) && gemm_smallm_workspace_bytes(M, N, K) <= workspace_bytes;
     if (!Bpre && force_tile == 0 && smallm_fits && !transB && batch == 1)
         return launch_smallm<false>(g, stream, (float*)workspace);
     // Bpre: B already packed by gemm_f32_pack_b (B itself is then not read); such a call always takes the padded shapes
@@ -2885,7 +2886,8 @@ hipError_t gemm_f32_f16weight(hipStream_t stream, const float* A, const uint16_t
                               int force_tile, const float* bias, int act, float act_param, void* workspace, size_t workspace_bytes)
 {
     GemmArgs g{A, B, C, M, N, K, K, N, N, 0, 0, 0, 1.0f, 0.0f, 0, 0, bias, act, act_param};
-    if (force_tile == 0 && workspace && smallm_applies(M, N, K) && gemm_smallm_workspace_bytes(M, N, K) <= workspace_bytes)
+    if (!workspace) workspace_bytes = 0;
+    if (force_tile == 0 && smallm_applies(M, N, K) && gemm_smallm_workspace_bytes(M, N, K) <= workspace_bytes)
         return launch_smallm<true>(g, stream, (float*)workspace);
     // rows of A in 16-byte steps, rows of the fp16 B in 8-byte steps
     const bool vec = aligned16(A) && K % 4 == 0 && (((uintptr_t)B) & 7u) == 0 && N % 4 == 0;
