@@ -2206,12 +2206,15 @@ __global__ __launch_bounds__(256) void gemm_smallm_kernel(const GemmArgs g, floa
 // The same product in one launch for weights of a few megabytes, where the second launch and the partials cost more than the stream: a
 // workgroup of 16 waves owns 64 columns and all of K.  A wave-load is four k-rows of 256 bytes; wave w takes the rows 4 w .. 4 w + 3 of
 // every 64, SMALLM1_DEPTH of them in flight, against the rows of A in LDS ([k][MR], read as whole rows); the four k-rows of a wave are
-// summed by lane exchanges, the waves through LDS, and the epilogue is applied there.  What bounds it is the memory round trip:
-// 8 x 768 x 768 10.4 us in two launches, 7.2 in one, 1 x 768 x 768 6.5 / 4.2, 8 x 1024 x 1024 10.5 / 8.5, 1 x 16384 x 256 9.8 / 3.4; fp16
-// weights 8 x 768 x 768 13.2 / 8.2, 1 x 4096 x 1024 18.1 / 6.2.  Beyond a K of 1024 a workgroup's own stream is the longer (8 x 2048 x 2048
-// 11.7 / 13.8, 1 x 768 x 3072 6.2 / 9.1), and wide weights keep every CU busy either way (1 x 40109 x 1088 35 / 36).
+// summed by lane exchanges, the waves through LDS, and the epilogue is applied there.  What bounds it is the memory round trip (times in
+// one graph, two launches / one): 8 x 768 x 512 11.2 / 6.3 us, 1 x 768 x 512 7.0 / 3.8, 8 x 1024 x 1024 11.2 / 8.4, 1 x 16384 x 256 9.7 / 3.4; fp16
+// weights 8 x 4096 x 512 12.4 / 7.0.
+// Beyond a K of 1024 a workgroup's own stream is the longer (8 x 2048 x 2048 11.7 / 13.8, 1 x 768 x 3072 6.2 / 9.1), and wide weights keep
+// every CU busy either way (1 x 40109 x 1088 35 / 36).  Up to one workgroup per CU (16384 columns) the form wins at any K (8 x 16384 x 1 4.9 /
+// 4.6, x 16 6.2 / 4.9); with more of them a CU pays for starting and summing 16 waves several times over, which only the rows of a K of
+// 128 or more repay (8 x 32768 x 128 11.3 / 8.7, but x 64 7.3 / 7.9; 8 x 65536 x 32 7.2 / 13.9; 8 x 262144 x 16 13.3 / 48).
 #define SMALLM1_DEPTH 6
-static bool smallm1_suits(int N, int K) { return K <= 1024 && (long long)N * K <= (1LL << 22); }
+static bool smallm1_suits(int N, int K) { return K <= 1024 && (long long)N * K <= (1LL << 22) && (N <= 16384 || K >= 128); }
 template <int MR, bool B16>
 __global__ __launch_bounds__(1024) void gemm_smallm1_kernel(const GemmArgs g)
 {
