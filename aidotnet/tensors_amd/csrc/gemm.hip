@@ -1823,7 +1823,7 @@ static bool pad16_layout(int M, int N, int K, PadPlan* pl)
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     size_t off = 0;
     pl->Np = Np; pl->Kp = Kp;
-    pl->a_off = off; off += up((size_t)M * Kp * 2);
+    pl->a_off = off; if (Kp != K) off += up((size_t)M * Kp * 2);      // (an A in whole K-tiles is read where it is)
     pl->b_off = off; off += up((size_t)Kp * Np * 2);
     pl->c_off = off; off += up((size_t)M * Np * 4);
     pl->bias_off = off; off += up((size_t)Np * 4);
