@@ -1831,17 +1831,6 @@ static bool pad16_layout(int M, int N, int K, PadPlan* pl)
     pl->total = off;
     return off <= ((size_t)4 << 30);
 }
-static bool pad16_plan(int M, int N, int K, PadPlan* pl)
-{
-    if (N % 8 == 0 && K % 8 == 0) return false;
-    // gemm_any16_kernel reads such rows in place at about 0.8 PFLOP/s, the kernels for aligned rows reach about 1.25 and the copies
-    // (read and write of B, of A where K is padded) run at about 4 TB/s with 8 us of launches: many rows repay them.  In place /
-    // copied, us: 700 x 9001 x 8000 134 / 195, 4000 x 3001 x 1000 40 / 44, 4096 x 4095 x 4096 154 / 117, 8000 x 5001 x 3001 319 / 240.
-    const double gain_us = 0.9e-9 * M * N * K, copy_us = 1e-6 * ((double)K * N + (K % 64 ? (double)M * K : 0.0)) + 8.0;
-    if (gain_us <= copy_us) return false;
-    return pad16_layout(M, N, K, pl);
-}
-
 // gemm_any16_kernel: tile height and K ranges (kper, a multiple of 64; 0 = none).  128 rows where such tiles fill the chip (212 x 36669 x
 // 704 28 us against 31 with 64 rows, 2000 x 2001 x 2000 27 / 33), else 64 (1049 x 1216 x 398 7.1 / 9.0) and, with few tiles, K ranges summed by a
 // pass of their own.  The estimate (us): 0.6 a K-tile with up to two workgroups per CU, 2 for the start, 3 for the second launch and the
@@ -1860,6 +1849,40 @@ static int any16_plan(int M, int N, int K, int* kper, int* ranges)
         if (ks == 1 || us < best) { best = us; *ranges = n; *kper = n > 1 ? 64 * per : 0; }
     }
     return 64;
+}
+
+// Whether the copies repay themselves.  Both ways are estimated in us (fitted on 420 shapes of 100 - 9000 rows, 64 - 66000 columns, K 64 -
+// 9000, to 9 and 13 %) and the copies, which served all these shapes before the kernel above, taken up to an estimate 8 % higher: of the
+// 420 shapes 8 are then more than 3 % slower than through copies (the worst 6074 x 560 x 3833, 60 -> 70 us), 285 more than 3 % faster.  In
+// place: a K-tile takes 0.48 us (64 rows) / 0.75 (128) with one workgroup on a CU and 0.83 / 1.35 with two,
+// 15 % less where the rows of A are aligned.  Copied: the passes over the copies at 5.5 TB/s and the aligned kernel at 1.57 PFLOP/s times
+// the score of its tiles.  In place / copied, us: 700 x 9001 x 8000 134 / 195, 1677 x 3683 x 3455 79 / 68, 3722 x 1021 x 7711 116 / 95,
+// 4096 x 4095 x 4096 154 / 117, 8000 x 5001 x 3001 319 / 240, 2020 x 49751 x 179 118 / 97; three and more K ranges always win in place (372 x
+// 2901 x 4904 35 / 64).
+static bool pad16_plan(int M, int N, int K, PadPlan* pl)
+{
+    if (N % 8 == 0 && K % 8 == 0) return false;
+    const double mn = (double)M * N, mk = (double)M * K, kn = (double)K * N;
+    if (N < 16) {
+        // in place these run on the general kernel: an A of whole K-tiles, which is not copied, from 10^10 multiply-adds on (65536 x 12 x
+        // 16384 1161 / 388, 200000 x 15 x 8192 3478 / 685)
+        return K % 64 == 0 && 0.9e-9 * mn * K > 1e-6 * kn + 8.0 && pad16_layout(M, N, K, pl);
+    }
+    if (mn * K < 2e9) return false;                   // the launches of the copies alone take as long
+    int kper, ranges;
+    const bool tall = any16_plan(M, N, K, &kper, &ranges) == 128;
+    if (ranges > 2 || !pad16_layout(M, N, K, pl)) return false;
+    const long long wgs = (long long)((M + (tall ? 127 : 63)) / (tall ? 128 : 64)) * ((N + 127) / 128) * ranges;
+    const double one = tall ? 0.75 : 0.48, two = tall ? 1.35 : 0.83;
+    const int last = (int)(wgs % 512);                // (beyond four rounds of 512 the workgroups no longer run in step)
+    const double rounds = wgs >= 2048 ? two * wgs / 512.0 : two * (double)(wgs / 512) + (last == 0 ? 0.0 : last <= 256 ? one : two);
+    const double tiles = kper > 0 ? kper / 64 : (K + 63) / 64;
+    const double in_place = 5.5 + rounds * tiles * (K % 8 == 0 ? 0.85 : 1.0) + mn / 1.7e6 + (ranges > 1 ? 3.2 + mn * 16.0 / 3e6 : 0.0);
+    double score = 0.0;
+    dl16_width(M, pl->Np, pl->Kp, 1, &score);
+    const double copied = 13.0 + 4.0 * (kn + (pl->Kp != K ? mk : 0.0) + (pl->Np % 128 ? mn : 0.0)) / 5.5e6 +
+                          2.0 * M * (double)pl->Np * pl->Kp / (1.57e9 * score) + mn / 1.55e6;
+    return score > 0.0 && copied * (ranges == 1 ? 0.92 : 1.0) < in_place;
 }
 
 // dst [rows_dst, cols_dst] (16-byte aligned rows) <- src [rows_src, cols_src] (dense, any alignment), zeros elsewhere; E = element.
