@@ -54,21 +54,19 @@ struct GemmArgs {
     // many columns (fewer than N, the columns past them are padding of B that is computed and dropped) and ldc is any element
     // count, so a row of C may start off a 16-byte boundary
     int c_cols = 0;
-    // three products with one A in one launch (three batches): the B of batches 1 and 2; null: batch b reads B + b * sB
-    const void* B1 = nullptr;
-    const void* B2 = nullptr;
+    // three products with one A in one launch (three batches): their Bs lie anywhere, B at B, B + sB and B + 2 sB + sB2.  (A stride and not
+    // two pointers: choosing one by branches in front of the first load cost every kernel 0.1 - 0.3 us, 9 % of a 1 x 256 x 101 product)
+    long long sB2 = 0;
 };
 
 // B of batch bz, in units of B's elements of EB bytes
 template <int EB>
 __device__ __forceinline__ const unsigned char* batch_b(const GemmArgs& g, long long bz)
 {
-    if (g.B1) return (const unsigned char*)(bz == 0 ? g.B : bz == 1 ? g.B1 : g.B2);
-    return (const unsigned char*)g.B + bz * g.sB * EB;
+    return (const unsigned char*)g.B + (bz * g.sB + (bz == 2 ? g.sB2 : 0LL)) * EB;
 }
 
 [[maybe_unused]] static bool aligned16(const void* p) { return (((uintptr_t)p) & 15u) == 0; }
-[[maybe_unused]] static bool b_aligned16(const GemmArgs& g) { return aligned16(g.B) && aligned16(g.B1) && aligned16(g.B2); }
 
 #if AIDN_GEMM_PART == 0
 hipError_t ensure_dynamic_smem(const void* kernel, int bytes, unsigned long long* done_mask)
@@ -2628,7 +2626,7 @@ template <typename OutT>
 static bool dl16_applies(const GemmArgs& g)
 {
     const int OB = Elem<OutT>::BYTES;
-    return aligned16(g.A) && b_aligned16(g) && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.sA % 8 == 0 && g.sB % 8 == 0 &&
+    return aligned16(g.A) && aligned16(g.B) && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.sA % 8 == 0 && g.sB % 8 == 0 && g.sB2 % 8 == 0 &&
            g.lda < (1 << 21) && g.ldb < (1 << 21) &&
            aligned16(g.C) && ((long long)g.ldc * OB) % 16 == 0 && (g.sC * OB) % 16 == 0 && (g.bias == nullptr || aligned16(g.bias)) &&
            g.alpha == 1.0f && g.beta == 0.0f;
@@ -2687,8 +2685,8 @@ template <typename T, typename OutT, bool TRANSB>
 static hipError_t dispatch_gemm(const GemmArgs& g, int batch, hipStream_t stream, int force_tile)
 {
     constexpr int E = Elem<T>::PER16;
-    const bool vec = aligned16(g.A) && b_aligned16(g) && g.lda % E == 0 && g.ldb % E == 0 && g.K % E == 0 &&
-                     (TRANSB || g.N % E == 0) && g.sA % E == 0 && g.sB % E == 0;
+    const bool vec = aligned16(g.A) && aligned16(g.B) && g.lda % E == 0 && g.ldb % E == 0 && g.K % E == 0 &&
+                     (TRANSB || g.N % E == 0) && g.sA % E == 0 && g.sB % E == 0 && g.sB2 % E == 0;
     auto tiles = [&](int bm, int bn) { return (long long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * batch; };
     int tile = force_tile;
     if (tile == 0) {
@@ -2801,6 +2799,14 @@ static hipError_t dispatch_gemm(const GemmArgs& g, int batch, hipStream_t stream
     return hipErrorInvalidValue;
 }
 
+template <typename E>
+[[maybe_unused]] static void set_b3(GemmArgs& g, const E* const (&B)[3])
+{
+    auto at = [&](int i) { return (long long)((intptr_t)B[i] - (intptr_t)B[0]) / (long long)sizeof(E); };      // (whole elements: the blocks are aligned)
+    g.sB = at(1);
+    g.sB2 = at(2) - 2 * at(1);
+}
+
 // C [M, 3 n] = A [M, K] x [B0 | B1 | B2], the three [K, n] blocks wherever they are (row stride ldb): one launch of three batches that
 // share A.  gemm_x3_suits: the tiles of an n-wide product load the chip as well as those of the 3 n-wide one would (n a multiple of 64,
 // so that no tile is cut that was not cut before; estimates within 3 %) -- then B need not be copied side by side for it.
@@ -2820,7 +2826,7 @@ bool gemm_x3_suits(int kind, int M, int n, int K)
 hipError_t gemm_f32_x3(hipStream_t stream, const float* A, const float* const (&B)[3], float* C, int M, int n, int K, int ldb, int force_tile)
 {
     GemmArgs g{A, B[0], C, M, n, K, K, ldb, 3 * n, 0, 0, n, 1.0f, 0.0f, 0, 0, nullptr, 0, 0.0f};
-    g.B1 = B[1]; g.B2 = B[2];
+    set_b3(g, B);
     return dispatch_gemm<float, float, false>(g, 3, stream, force_tile);
 }
 #endif
@@ -2828,7 +2834,7 @@ template <typename T>
 static hipError_t gemm_16_x3_typed(hipStream_t stream, const uint16_t* A, const uint16_t* const (&B)[3], uint16_t* C, int M, int n, int K, int ldb, int force_tile)
 {
     GemmArgs g{A, B[0], C, M, n, K, K, ldb, 3 * n, 0, 0, n, 1.0f, 0.0f, 0, 0, nullptr, 0, 0.0f};
-    g.B1 = B[1]; g.B2 = B[2];
+    set_b3(g, B);
     return dispatch_gemm<T, T, false>(g, 3, stream, force_tile);
 }
 
