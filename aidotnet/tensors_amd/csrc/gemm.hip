@@ -523,15 +523,19 @@ __global__ __launch_bounds__(WM * WN * KS * 64) void gemm_kernel(const GemmArgs 
                 if constexpr (FUSED) bias = (g.bias && col < g.N) ? g.bias[col] : 0.0f;
                 f32x16 v = acc[i][j];
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int row = m0 + wm * WTM + i * 32 + acc_row(r, h);
-                    v[r] *= g.alpha;
-                    if (use_beta && row < g.M && col < g.N) {
-                        const out_t* p = C + (long long)row * g.ldc + col;
+                for (int r = 0; r < 16; r++) v[r] *= g.alpha;
+                if (use_beta) {                  // (clamped addresses: a guard per element would make every load wait for the one before)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const int row = min(m0 + wm * WTM + i * 32 + acc_row(r, h), g.M - 1);
+                        const out_t* p = C + (long long)row * g.ldc + min(col, g.N - 1);
                         if constexpr (Elem<OutT>::BYTES == 4) v[r] += g.beta * as_f32(*p);
                         else v[r] += g.beta * Elem<OutT>::widen(*p);
                     }
-                    v[r] += bias;
+                }
+                if constexpr (FUSED) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) v[r] += bias;
                 }
                 if constexpr (FUSED)
                     with_activation(g.act, g.act_param, [&](auto fn) {
