@@ -1853,6 +1853,11 @@ static int any16_plan(int M, int N, int K, int* kper, int* ranges)
     return 64;
 }
 
+// Up to 16 rows on at most 256 k-rows of at most 16384 columns, with the rows of B aligned and those of A not: the general kernel, which
+// reads such a B in whole chunks and starts half as many threads, is as fast or faster (4 x 15424: K 101 4.8 us / 5.3 in place above, 255 6.1 /
+// 6.8, 150 6.0 / 5.6; 16 x 15424 x 209 5.9 / 6.3; beyond: 4 x 15424 x 260 7.1 / 6.1, 4 x 32768 x 129 6.1 / 5.4, 32 x 15424 x 209 6.3 and more / 5.5).
+static bool general_few_rows(int M, int N, int K) { return M <= 16 && N <= 16384 && K <= 256; }
+
 // Whether the copies repay themselves.  Both ways are estimated in us (fitted on 420 shapes of 100 - 9000 rows, 64 - 66000 columns, K 64 -
 // 9000, to 9 and 13 %) and the copies, which served all these shapes before the kernel above, taken up to an estimate 8 % higher: of the
 // 420 shapes 8 are then more than 3 % slower than through copies (the worst 6074 x 560 x 3833, 60 -> 70 us), 285 more than 3 % faster.  In
@@ -2988,7 +2993,8 @@ static hipError_t gemm_16_typed(hipStream_t stream, const uint16_t* A, const uin
         return padC ? unpad_rows(stream, Cp, C, M, N, pl.Np, out32 ? 4 : 2) : hipSuccess;
     }
     GemmArgs g{A, B, C, M, N, K, K, N, N, 0, 0, 0, 1.0f, 0.0f, 0, 0, bias, act, act_param};
-    if (force_tile == 0 && !(N % 8 == 0 && K % 8 == 0 && aligned16(A) && aligned16(B)) && N >= 16 && N < (1 << 21) && K < (1 << 21)) {
+    const bool b_rows = N % 8 == 0 && aligned16(B);                       // rows of B in whole 16-byte chunks
+    if (force_tile == 0 && !(b_rows && K % 8 == 0 && aligned16(A)) && !(b_rows && general_few_rows(M, N, K)) && N >= 16 && N < (1 << 21) && K < (1 << 21)) {
         int kper, ks;
         const int bm = any16_plan(M, N, K, &kper, &ks);
         if (ks > 1 && (size_t)ks * M * N * sizeof(float) <= workspace_bytes) {
