@@ -208,9 +208,11 @@ __device__ __forceinline__ float merge_partials(const float* __restrict__ P, int
                 for (int j = 0; j < NV; j++) { out[j][0] += sums[q][j][lane][0]; out[j][1] += sums[q][j][lane][1]; }
         }
     }
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    // (divided, as a single range is: a reciprocal would round twice, and a sum that is no number has to give zeros here as there)
 #pragma unroll
-    for (int j = 0; j < NV; j++) { out[j][0] *= inv; out[j][1] *= inv; }
+    for (int j = 0; j < NV; j++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) out[j][e] = L > 0.0f ? out[j][e] / L : 0.0f;
     return L > 0.0f ? (M + __builtin_amdgcn_logf(L)) * LN2 : -INFINITY;
 }
 // waves per row of the merge passes: one (four rows to a workgroup) while a row's ranges fit one round of loads
