@@ -81,53 +81,56 @@ hipError_t ensure_dynamic_smem(const void* kernel, int bytes, unsigned long long
 }
 #endif
 
-// 1 / (1 + e^-x), the logistic function that GELU (tanh form: x times the logistic function of twice the inner polynomial), sigmoid and
-// swish are made of, on the vector pipe's exponential (base 2) and reciprocal.  The product x log2(e) is carried in two parts and the
-// reciprocal takes one Newton step, so the result is within about 2 units in the last place wherever it is above 1e-37 (the float64
-// check of the epilogue tests sees no more than the library functions gave); below, it is zero.  An epilogue holds nothing but these
-// values and nothing runs beside it on one tile per CU, so their length is time: with the library's tanhf / expf and an IEEE division,
-// chosen per element, the fp32 product 4096 x 3072 x 768 with GELU took 199 us, this way 149; bf16 1000 x 11008 x 4096 with swish
-// 129 and 106.
-__device__ __forceinline__ float logistic(float x)
+// num / (1 + e^-v): GELU (tanh form: (1 + tanh u) / 2 is the logistic function of 2 u), sigmoid and swish, on the vector pipe's exponential
+// (base 2) and reciprocal.  The exponent is split into its nearest whole number, added to the exponent field, and a remainder formed from
+// v log2(e) in two parts (LONG: with one rounding, for arguments of any size; GELU's matter near zero, where two do as well).  The quotient is
+// corrected by its remainder against 1 + e^-v and what that sum lost, so that the error is that of e^-v and one rounding of the result.
+// Numerator and denominator are scaled by 2^-4, which keeps the reciprocal normal down to the v where e^-v overflows; below it is zero.
+// Largest errors against float64 in units in the last place, with the library's expf or tanhf and an IEEE division / this way: sigmoid
+// 2.6 / 2.6 at -20 to -10, 2.2 / 1.7 to 0, 1.5 / 0.8 above; swish 2.7 / 2.7, 2.1 / 1.7, 1.5 / 0.9; GELU above -0.1 1.8 / 1.2, at -2 to -1 15 / 5.5.
+// An epilogue holds nothing but these values and nothing runs beside it on one tile per CU, so their length is time: the fp32 product
+// 4096 x 3072 x 768 with GELU took 199 us with the library functions chosen per element and takes 149, bf16 1000 x 11008 x 4096 with swish
+// 130 and 112 (107 with an exponential rounded twice and the product with the reciprocal: errors up to 3.5 units, zero below -87).
+template <bool LONG>
+__device__ __forceinline__ float over_one_plus_exp(float num, float v)
 {
-    constexpr float L2E = 1.44269502f, L2E_LO = 1.92596299e-8f, LN2 = 0.693147181f;      // log2(e) = L2E + L2E_LO
-    const float y = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);                           // (keeps 1 + e^-y and its reciprocal normal)
-    const float t = y * -L2E;
-    const float lo = fmaf(y, -L2E_LO, fmaf(y, -L2E, -t));
-    float e = __builtin_amdgcn_exp2f(t);
-    e = fmaf(e, lo * LN2, e);
-    const float d = 1.0f + e;
-    float r = __builtin_amdgcn_rcpf(d);
-    r = fmaf(r, fmaf(-d, r, 1.0f), r);
-    return x < -87.0f ? 0.0f : r;
+#pragma clang fp contract(off)
+    constexpr float L2E = 1.44269502f, L2E_LO = 1.92596299e-8f;                          // log2(e) = L2E + L2E_LO
+    constexpr float WHOLE = 12582912.0f, ONE = 0x1p-4f;                                  // 1.5 2^23: a sum with it is rounded to a whole number
+    float whole, rest;
+    if constexpr (LONG) {
+        const float t = v * -L2E;
+        whole = t + WHOLE;
+        rest = fmaf(v, -L2E_LO, fmaf(v, -L2E, -t)) + (t - (whole - WHOLE));
+    } else {
+        whole = fmaf(v, -L2E, WHOLE);
+        rest = fmaf(v, -L2E_LO, fmaf(v, -L2E, WHOLE - whole));
+    }
+    const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(rest), __builtin_bit_cast(int, whole) - (__builtin_bit_cast(int, WHOLE) + 4));
+    const float d = e + ONE, lost = e - (d - ONE);
+    const float n = num * ONE, r = __builtin_amdgcn_rcpf(d);
+    float q = n * r;
+    q = fmaf(-fmaf(lost, q, fmaf(d, q, -n)), r, q);                                      // (in this order a zero keeps its sign)
+    q = v < -88.72f ? num * 0.0f : q;
+    return v > 88.0f ? num : q;
 }
 
 // Pointwise activations of the fused projection epilogues, numbered like the reference's FusedActivationType
 // (src/AiDotNet.Tensors/Engines/FusedActivationType.cs:23-70); the functions are those of its HIP activation kernels
 // (src/AiDotNet.Tensors/Engines/DirectGpu/HIP/Kernels/HipActivationKernels.cs:19-70).  NaN stays NaN in all of them.
-template <int ACT>
-__device__ __forceinline__ float activation(float x, float p)
-{
-    if constexpr (ACT == 1) return x < 0.0f ? 0.0f : x;                                   // ReLU, NaN-preserving form (CpuFusedOperations.cs:1271-1274)
-    else if constexpr (ACT == 2) return x * logistic(1.5957691216f * (x + 0.044715f * x * x * x));      // GELU, tanh form: (1 + tanh u) / 2 = logistic(2 u)
-    else if constexpr (ACT == 3) { const float r = logistic(x); return x == x ? r : x; }  // sigmoid
-    else if constexpr (ACT == 4) return tanhf(x);
-    else if constexpr (ACT == 5) return x > 0.0f ? x : p * x;                             // leaky ReLU, slope p
-    else if constexpr (ACT == 6) return x * logistic(x);                                  // swish
-    else return x;
-}
 // f(fn) with fn the activation `act`: the choice is made once around whatever f does with it, never per element (a tile of
-// accumulators with a test on each is thousands of branches)
+// accumulators with a test on each is thousands of branches).  Sigmoid and swish share a body: with one each the 256 x 256 fp32 tile's
+// epilogue outgrows what the compiler unrolls, and its accumulators go to scratch memory.
 template <typename F>
 __device__ __forceinline__ void with_activation(int act, float p, F&& f)
 {
     switch (act) {
-    case 1: f([](float x) { return activation<1>(x, 0.0f); }); break;
-    case 2: f([](float x) { return activation<2>(x, 0.0f); }); break;
-    case 3: f([](float x) { return activation<3>(x, 0.0f); }); break;
-    case 4: f([](float x) { return activation<4>(x, 0.0f); }); break;
-    case 5: f([p](float x) { return activation<5>(x, p); }); break;
-    case 6: f([](float x) { return activation<6>(x, 0.0f); }); break;
+    case 1: f([](float x) { return x < 0.0f ? 0.0f : x; }); break;                       // ReLU, NaN-preserving form (CpuFusedOperations.cs:1271-1274)
+    case 2: f([](float x) { return over_one_plus_exp<false>(x, x * fmaf(0.0713548163f, x * x, 1.5957691216f)); }); break;      // GELU, tanh form: 2 u = 2 0.7978845608 (x + 0.044715 x^3)
+    case 3:                                                                               // sigmoid
+    case 6: f([act](float x) { return over_one_plus_exp<true>(act == 3 ? 1.0f : x, x); }); break;      // swish
+    case 4: f([](float x) { return tanhf(x); }); break;
+    case 5: f([p](float x) { return x > 0.0f ? x : p * x; }); break;                      // leaky ReLU, slope p
     default: f([](float x) { return x; }); break;
     }
 }

@@ -71,3 +71,25 @@ def test_nan_stays_nan():
     w = torch.full((64, 64), float("nan"), device="cuda")
     for act in range(7):
         assert bool(torch.isnan(eng.FusedLinear(torch.ones(64, 64, device="cuda"), w, None, act, 0.1)).all()), act
+
+
+def test_errors_of_the_logistic_functions():
+    """Over the whole range of their argument.  In units of 2^-23: the hardware exponential 1, its argument's rounding ln 2 / 4, the sum with
+    1 compensated up to 2^24 and at most 1 where it begins to be (e^-x itself beyond), the quotient 1/2: 2.75.  Subnormal results (sigmoid
+    below -87.3) within the smallest subnormal beside that.  GELU where the rounding of its argument 2 u (three halves, times 2 u and the
+    logistic function of -2 u) does not lead."""
+    from aidotnet.tensors_amd import Mi355Engine
+    eng = Mi355Engine()
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    one = torch.ones(1, 1, device="cuda")
+    for act in (3, 6, 2):
+        for lo, hi in ((-88.7, -87.3), (-87.3, -20.0), (-20.0, -2.0), (-2.0, 0.1), (-0.1, 2.0), (2.0, 20.0), (20.0, 120.0)):
+            if act == 2 and lo < -2.0:
+                continue
+            x = lo + (hi - lo) * torch.rand(1, 1 << 16, device="cuda", generator=gen)
+            got = eng.FusedLinear(one, x, None, act).double()
+            z = x.double()
+            u2 = 2 * 0.7978845608 * (z + 0.044715 * z ** 3) if act == 2 else z
+            want = (1.0 if act == 3 else z) / (1 + torch.exp(-u2))
+            bound = 2.75 * 2.0 ** -23 + (1.5 * 2.0 ** -23 * u2.abs() * torch.sigmoid(-u2) if act == 2 else 0.0)
+            assert bool(((got - want).abs() <= bound * want.abs() + 2.0 ** -149).all()), (act, lo)
