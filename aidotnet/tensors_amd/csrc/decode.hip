@@ -97,7 +97,9 @@ constexpr float D_LN2 = 0.6931471805599453f;
 // grouped-query cache are then fetched once per GH query heads instead of once per head.
 // ROWS: rows of whole 16-byte chunks whose number is uniform over a load (contiguous cache, or blocks of a multiple of KPW keys); other
 // operands take guarded loads and a row per key.
-template <typename T, typename OutT, int LPK, int U, int GH, bool ROWS>
+// AHEAD: two register sets of loads in turn.  At four query heads these are 174 registers, two workgroups on a CU where the plain loop has
+// four: a grid of up to two per CU gains (launch_decode).
+template <typename T, typename OutT, int LPK, int U, int GH, bool ROWS, bool AHEAD>
 __global__ __launch_bounds__(256) void decode_partial_kernel(const DecodeArgs a)
 {
     typedef typename Raw3<T>::type raw_t;
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(256) void decode_partial_kernel(const DecodeArgs a)
         }
     };
     const int nit = first < kend ? (kend - first + STEP - 1) / STEP : 0;
-    if constexpr (ROWS) {
+    if constexpr (AHEAD) {
         // the loads of the next iteration are in flight while this one is used (register sets in turn)
         u32x4 kx[2][U], vx[2][U];
         if (nit > 0) load(0, kx[0], vx[0]);
@@ -399,10 +401,13 @@ static hipError_t launch_decode(DecodeArgs a, hipStream_t stream)
     if (nwg > 0x7FFFFFFFLL) return hipErrorInvalidValue;
     dim3 grid((unsigned)nwg);
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, a); };
-    if (!a.rows_uniform) gh == 4 ? go(decode_partial_kernel<T, OutT, LPK, U, 4, false>) : gh == 2 ? go(decode_partial_kernel<T, OutT, LPK, U, 2, false>) : go(decode_partial_kernel<T, OutT, LPK, U, 1, false>);
-    else if (gh == 4) go(decode_partial_kernel<T, OutT, LPK, U, 4, true>);
-    else if (gh == 2) go(decode_partial_kernel<T, OutT, LPK, U, 2, true>);
-    else go(decode_partial_kernel<T, OutT, LPK, U, 1, true>);
+    // four query heads in more than two workgroups per CU (256 CUs): one set of loads and four workgroups (bf16 B5 16 / 2 heads d32 KV6530, 520
+    // workgroups: 16.8 us, 22.1 with the loads an iteration ahead; B45 16 / 4 d32 KV2898, 1080: 29.1 / 36.4; up to 512 3 to 23 % the other way)
+    if (!a.rows_uniform) gh == 4 ? go(decode_partial_kernel<T, OutT, LPK, U, 4, false, false>) : gh == 2 ? go(decode_partial_kernel<T, OutT, LPK, U, 2, false, false>) : go(decode_partial_kernel<T, OutT, LPK, U, 1, false, false>);
+    else if (gh == 4 && nwg > 512) go(decode_partial_kernel<T, OutT, LPK, U, 4, true, false>);
+    else if (gh == 4) go(decode_partial_kernel<T, OutT, LPK, U, 4, true, true>);
+    else if (gh == 2) go(decode_partial_kernel<T, OutT, LPK, U, 2, true, true>);
+    else go(decode_partial_kernel<T, OutT, LPK, U, 1, true, true>);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return a.splits > 1 ? launch_decode_reduce<OutT>(a, DPAD, stream) : hipSuccess;
