@@ -1366,6 +1366,13 @@ static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
 //   fp32 above 64: 64-key tiles need 128 KiB, one workgroup per CU: 256 (plain d128 151 / 88; 384: 66 / 83), causal 384 (64 / 42)
 //   four groups on 128-key tiles (head dimension 64, dense K and V, no mask): 256, causal 384, from 192 keys on (two / four groups: plain
 //     B4 H8 S256 16.0 / 12.2, causal B1 H32 S300 18.8 / 16.3; plain at 304 32 / 40, 64 keys 7.9 / 8.8)
+// Short sequences do not repay the merge by balance, only where the finer grid saves a round of workgroups (240 shapes of 12 - 300 keys):
+//   one 64-key tile: up to 256, and up to 512 where the 128-row grid needs a second workgroup per CU (fp32 Sq 130 n 480 14.7 / 11.1, bf16 Sq 131
+//     n 429 7.1 / 6.9; but fp32 Sq 69 n 286 9.7 / 10.8, n 618 13.8 / 16.5, bf16 Sq 105 n 848 7.2 / 8.9); up to 256 keys the same of fp32 plain
+//     at n 257 - 512 (S 115 n 360 14.7 / 15.5)
+//   16-bit causal beyond 768: a 128-row grid of more than 512, or long rows (S 300 n 1000 14.0 / 11.9; but S 232 n 944 10.5 / 11.5)
+//   fp32 above 64: up to 32 keys the second group has none (Sk 12 10.6 / 12.8); causal 384 only where the row tiles differ in length
+//     (Sq 204 n 288 44 / 35; but Sq 62, Sk 12 n 352 16 / 26)
 // The lines do not depend on how the tiles are loaded, so the direct-to-LDS and the register-staged forms add up the same way.
 template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
 static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
@@ -1377,9 +1384,10 @@ static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
             if (!a.bt && a.Sk >= 192 && grid(32) <= (a.causal ? 384 : 256)) return launch_attn_kg<T, OutT, DP, 128, FULL, 1, DMA, KM, 4>(a, stream);
         }
         long long line;
-        if constexpr (WIDE32) line = a.causal ? 384 : 256;
+        if constexpr (WIDE32) line = a.Sk <= 32 ? 0 : a.causal && a.Sq > 64 && a.Sk > 128 ? 384 : 256;
+        else if (a.Sk <= 64 || (Elem<T>::BYTES == 4 && !FULL && !a.causal && a.Sk <= 256 && grid(128) <= 256)) line = grid(128) > 256 ? 512 : 256;
         else if constexpr (DP > 64) line = 512;
-        else if constexpr (Elem<T>::BYTES == 2) line = !FULL && a.causal ? 1024 : 768;
+        else if constexpr (Elem<T>::BYTES == 2) line = !FULL && a.causal && (a.Sk >= 448 || grid(128) > 512) ? 1024 : 768;
         else line = a.causal && a.Sk < 1024 ? 640 : 768;
         if (grid(64) <= line) return launch_attn_kg<T, OutT, DP, 64, FULL, WIDE32 ? 1 : 2, DMA, KM, 2>(a, stream);
     }
