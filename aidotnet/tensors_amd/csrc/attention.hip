@@ -289,6 +289,11 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
             const unsigned char* ks = Ks + stage * KBYTES + (kr0 + l32) * KPITCH + h * 16;
             const unsigned char* vs = Vs + stage * VBYTES + l32 * VPITCH + kr0 * EB + h * 16;
 
+            // general form: a mask of the keys alone as one ballot per tile too (a third kind of mask in the test of every element cost the
+            // calls with planes and biases up to 5 %)
+            unsigned keep = 1;
+            if constexpr (FULL) { if (a.mask_mode == 3) keep = ((const unsigned char*)a.mask)[(long long)b * a.Sk + min(kv0 + lane, a.Sk - 1)]; }
+
             f32x16 st[KT];
 #pragma unroll
             for (int kt = 0; kt < KT; kt++)
@@ -323,7 +328,52 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 
             // ---- logits in the log2 domain, masks
             const bool need_mask = (kw0 + KT * 32 > a.Sk) || (a.causal && (long long)kw0 + KT * 32 - 1 > (long long)wq_min + a.qoff);
-            const bool mixed = KM && (BC == 64 ? kbits != ~0ull : (uint32_t)kbits != ~0u);
+            if constexpr (FULL) kbits = __builtin_amdgcn_ballot_w64(keep != 0);      // (keys past the end are masked below)
+            const bool mixed = (KM || FULL) && (BC == 64 ? kbits != ~0ull : (uint32_t)kbits != ~0u);
+            if constexpr (FULL) {
+                // one pass over the tile per option, out-of-range elements on clamped addresses: with the options tested per element every
+                // load waited for itself (fp32 B4 H4 235 x 1436 d64 causal with a mask plane 237 us, 123 this way; B6 H16 309 x 552 d64 with a bias
+                // 176 / 96; B12 H32 398 x 293 d64, a full chip, 284 / 274)
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) st[kt][r] *= a.scale;
+                if (a.softcap > 0.0f) {
+#pragma unroll
+                    for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) {
+                            st[kt][r] = a.softcap * tanhf(st[kt][r] / a.softcap);
+                            if (DP == 256) __builtin_amdgcn_sched_barrier(0);
+                        }
+                }
+                // (rows and keys are formed anew, the keys for each pass, and few loads are asked for at a time where registers are short)
+                int qr = min(qi, a.Sq - 1), key0 = kw0 + 4 * h;
+                asm volatile("" : "+v"(qr));
+                const int last = a.Sk - 1;
+                constexpr int FEW = DP == 256 ? 2 : DP == 128 ? 4 : 16;
+                auto groups = [&](auto f) {
+#pragma unroll
+                    for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                        for (int r0 = 0; r0 < 16; r0 += FEW) {
+                            if (kw0 + kt * 32 + acc_row(r0, 0) >= a.Sk) continue;              // (past the end for every lane: masked below)
+#pragma unroll
+                            for (int r = r0; r < r0 + FEW; r++) f(kt, r, min(key0 + kt * 32 + acc_row(r, 0), last));
+                            if (FEW < 16) __builtin_amdgcn_sched_barrier(0);
+                        }
+                };
+                if (a.bias) {
+                    asm volatile("" : "+v"(key0));
+                    const float* __restrict__ row = a.bias + b * a.bias_bs + ((long long)hd * a.Sq + qr) * a.Sk;
+                    groups([&](int kt, int r, int key) { st[kt][r] += row[key]; });
+                }
+                if (a.mask_mode == 1 || a.mask_mode == 2) {
+                    asm volatile("" : "+v"(key0));
+                    const float* __restrict__ row = a.mask + ((a.mask_mode == 2 ? (long long)bh * a.Sq : 0LL) + qr) * a.Sk;
+                    groups([&](int kt, int r, int key) { if (row[key] == 0.0f) st[kt][r] = -INFINITY; });
+                }
+            }
             float mloc = -INFINITY;
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) {
@@ -332,25 +382,12 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                 for (int r = 0; r < 16; r++) {
                     float x;
                     const int key = kw0 + kt * 32 + acc_row(r, h);
-                    if constexpr (FULL) {
-                        x = st[kt][r] * a.scale;
-                        if (a.softcap > 0.0f) x = a.softcap * tanhf(x / a.softcap);
-                        const bool inb = qi < a.Sq && key < a.Sk;
-                        if (a.bias && inb) x += a.bias[b * a.bias_bs + ((long long)hd * a.Sq + qi) * a.Sk + key];
-                        if (a.mask_mode == 3 && inb) {
-                            if (((const unsigned char*)a.mask)[(long long)b * a.Sk + key] == 0) x = -INFINITY;
-                        } else if (a.mask_mode != 0 && inb) {
-                            long long mi = (a.mask_mode == 2 ? ((long long)bh * a.Sq + qi) : (long long)qi) * a.Sk + key;
-                            if (a.mask[mi] == 0.0f) x = -INFINITY;
-                        }
-                        x *= LOG2E;
-                    } else {
-                        x = st[kt][r] * sl2;
-                    }
+                    if constexpr (FULL) x = st[kt][r] * LOG2E;
+                    else x = st[kt][r] * sl2;
                     if (need_mask) {
                         if (key >= a.Sk || (a.causal && (long long)key > (long long)qi + a.qoff)) x = -INFINITY;
                     }
-                    if constexpr (KM)
+                    if constexpr (KM || FULL)
                         if (mixed && !(kept >> acc_row(r, 0) & 1u)) x = -INFINITY;
                     st[kt][r] = x;
                     mloc = fmaxf(mloc, x);
