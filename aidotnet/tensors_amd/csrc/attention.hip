@@ -79,12 +79,10 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
             // dispatch: hand the query tiles out heaviest first across ALL heads, so the workgroups that end up sharing a
             // CU are a heavy one and, later in the id order, a light one.
             // (the first 256 ids, one per CU, in ascending weight, so that the ids after them -- which land on the same
-            // CUs in the same order -- pair the lightest of the first round with the heaviest of the second; reversed by eights, where 8
-            // divides the number of heads, so that all query tiles of a head stay on one XCD, 1-4 % against reversing one by one; with other
-            // numbers that does not hold and one by one is better: bf16 218 heads, 219 x 239, d64 11.6 us against 12.3)
+            // CUs in the same order -- pair the lightest of the first round with the heaviest of the second; reversed by eights, so that
+            // where 8 divides the number of heads all query tiles of a head stay on one XCD, 1-4 % against reversing one by one)
             const int nbh = nblk / a.qtiles;
-            const int flip = (nbh & 7) == 0 ? 7 : 0;
-            const int rank = (nblk > 256 && pid < 256) ? 255 - (pid | flip) + (pid & flip) : pid;
+            const int rank = (nblk > 256 && pid < 256) ? 255 - (pid | 7) + (pid & 7) : pid;
             qt = a.qtiles - 1 - rank / nbh;
             bh = rank - (rank / nbh) * nbh;
         } else if (a.causal && a.hgroup > 0) {
