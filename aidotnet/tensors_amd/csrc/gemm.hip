@@ -1333,7 +1333,9 @@ static hipError_t launch_gemm_dl16(GemmArgs g, int batch, hipStream_t stream)
 // The general kernel's loads of B are 16 rows of 64 bytes to an instruction, each cache line asked for twice: 64 x 50257 x 768
 // took 44 us there and takes 17.5 here (84 MB), 212 x 36669 x 704 103 / 28, 512 x 30001 x 4096 232 through padded copies / 156.
 // kper > 0: workgroups z take K ranges of kper (a multiple of 64) each and C is their fp32 partials, sum_stride elements apart.
-// Bounds: the last K-tile of the matrix is loaded under guards (zeros past K; whole chunks where they fit their row); in the others a
+// Bounds: the last K-tile of the matrix is loaded under guards (zeros past K; whole chunks where they fit their row), which costs about 1 us;
+// where all rows are whole chunks (operands off the 16-byte grid) from clamped addresses instead (20 x 272 x 248 6.8 -> 5.8 us, 3 x 7224 x 512
+// 8.9 -> 6.9).  In the others a
 // chunk of B that crosses column N reads on into the next row, which exists, and is only multiplied into columns that are not stored.
 // Rows of A past M and chunks of B past N are clamped likewise.  N >= 8.
 template <typename T, typename OutT, int BM>
@@ -1370,7 +1372,9 @@ __global__ __launch_bounds__(512, 4) void gemm_any16_kernel(const GemmArgs g, in
         pa[i] = (uint32_t)((min(m0 + row, g.M - 1) - m0) * g.lda + ach * 8);
         a_lds[i] = row * AROW + ((ach ^ ((row >> 1) & 7)) << 4);
     }
-    const int bcol = min(n0 + bch * 8, g.N - 1);
+    // whole: no chunk crosses the end of a row, and the last K-tile is loaded like the others, from clamped addresses (64 rows, where it counts)
+    const bool whole = BM == 64 && ((g.K | g.N) & 7) == 0;
+    const int bcol = min(n0 + bch * 8, whole ? g.N - 8 : g.N - 1);
     const uint32_t pb = (uint32_t)((t >> 4) * g.ldb + bcol);
 #pragma unroll
     for (int i = 0; i < LB; i++) {
@@ -1389,6 +1393,19 @@ __global__ __launch_bounds__(512, 4) void gemm_any16_kernel(const GemmArgs g, in
         constexpr int S = decltype(set)::value;
         if (kt < KT - 1) { load_plain(kt, set); return; }
         if (kt >= KT) return;
+        if (whole) {
+            const int ak = kt * BK + ach * 8, bk = kt * BK + (t >> 4);
+#pragma unroll
+            for (int i = 0; i < LA; i++) ra[S][i] = *(const u32x4_elem*)(a_base + ((int)pa[i] - ach * 8 + min(ak, K - 8)));
+#pragma unroll
+            for (int i = 0; i < LB; i++)
+                if (i == 0 || kt * BK + 32 * i < K) rb[S][i] = *(const u32x4_elem*)(b_base + (long long)(min(bk + 32 * i, K - 1) - (t >> 4)) * g.ldb + pb);
+#pragma unroll
+            for (int i = 0; i < LA; i++) ra[S][i] = ak < K ? ra[S][i] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int i = 0; i < LB; i++) rb[S][i] = bk + 32 * i < K ? rb[S][i] : u32x4{0u, 0u, 0u, 0u};
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int valid = K - (kt * BK + ach * 8);
@@ -1837,9 +1854,15 @@ static bool pad16_layout(int M, int N, int K, PadPlan* pl)
     return off <= ((size_t)4 << 30);
 }
 // gemm_any16_kernel: tile height and K ranges (kper, a multiple of 64; 0 = none).  128 rows where such tiles fill the chip (212 x 36669 x
-// 704 28 us against 31 with 64 rows, 2000 x 2001 x 2000 27 / 33), else 64 (1049 x 1216 x 398 7.1 / 9.0) and, with few tiles, K ranges summed by a
-// pass of their own.  The estimate (us): 0.6 a K-tile with up to two workgroups per CU, 2 for the start, 3 for the second launch and the
-// partials at 3 TB/s; 30 x 300 x 9001 80 -> 12 in 16 ranges, 100 x 1003 x 5000 36 -> 13, 16 x 5910 x 1600 18 -> 12 in four.
+// 704 28 us against 31 with 64 rows, 2000 x 2001 x 2000 27 / 33), else 64 (1049 x 1216 x 398 7.4 / 9.0) and, with few tiles, K ranges summed by a
+// pass of their own.  The estimate (us): a K-tile of 64 rows 0.6 with one workgroup on a CU and 0.95 with two; with ranges 3 for the second
+// launch, 0.08 a range and the partials, written and read, at 3 TB/s.  30 x 300 x 9001 87 us in one range, 11 in 29; 100 x 1003 x 5000 57, 13 in
+// ten; 16 x 5910 x 1600 21, 11 in five; but 273 x 5224 x 3936 stays whole, 33 us against 37 in two.
+static double any16_rounds(long long wgs, double one, double two)
+{
+    const int last = (int)(wgs % 512);                // (beyond four rounds of 512 the workgroups no longer run in step)
+    return wgs >= 2048 ? two * wgs / 512.0 : two * (double)(wgs / 512) + (last == 0 ? 0.0 : last <= 256 ? one : two);
+}
 static int any16_plan(int M, int N, int K, int* kper, int* ranges)
 {
     const long long tn = (N + 127) / 128, t128 = (M + 127) / 128 * tn, t64 = (M + 63) / 64 * tn;
