@@ -198,7 +198,7 @@ int gemm16_common(void* ctx, void* stream, int kind, const uint16_t* A, const ui
     if (!A || !B || !C) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "gemm: A, B and C must not be null");
     if (M <= 0 || N <= 0 || K <= 0) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "gemm: dimensions must be positive");
     void* ws = nullptr;
-    size_t need = c->force_tile == 0 ? aidn::gemm_16_workspace_bytes(M, N, K) : 0;
+    size_t need = c->force_tile == 0 ? aidn::gemm_16_workspace_bytes(M, N, K, (((uintptr_t)A | (uintptr_t)B) & 15u) != 0) : 0;
     if (need) {
         int st = acquire_ws(c, stream, need, &ws);
         if (st == AIDN_ERR_WORKSPACE) ws = nullptr;      // under capture and not reserved: the tiled kernel needs no workspace
@@ -221,7 +221,7 @@ int gemm16_rope_common(void* ctx, void* stream, int kind, const uint16_t* A, con
         return fail(c, AIDN_ERR_INVALID_ARGUMENT, "gemm_rope: rope_cols must be a multiple of head_dim within N, and N even");
     if (start_position < 0) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "gemm_rope: start position must not be negative");
     void* ws = nullptr;
-    size_t need = c->force_tile == 0 ? aidn::gemm_16_workspace_bytes(M, N, K) : 0;
+    size_t need = c->force_tile == 0 ? aidn::gemm_16_workspace_bytes(M, N, K, (((uintptr_t)A | (uintptr_t)B) & 15u) != 0) : 0;
     if (need) {
         int st = acquire_ws(c, stream, need, &ws);
         if (st == AIDN_ERR_WORKSPACE) ws = nullptr;      // under capture and not reserved: the tiled kernel and a second launch for the rotation

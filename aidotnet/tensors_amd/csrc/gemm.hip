@@ -1872,8 +1872,7 @@ static int any16_plan(int M, int N, int K, int* kper, int* ranges)
     double best = 0.0;
     for (int ks = 1; ks <= 32 && ks <= kt; ks++) {
         const int per = (kt + ks - 1) / ks, n = (kt + per - 1) / per;
-        const double load = (double)(t64 * n) / 512.0;
-        const double us = 0.6 * per * (load > 1.0 ? load : 1.0) + (n > 1 ? 3.0 + 0.08 * n + (double)n * M * N * 8.0 / 3e6 : 0.0);
+        const double us = per * any16_rounds(t64 * n, 0.6, 0.95) + (n > 1 ? 3.0 + 0.08 * n + (double)n * M * N * 8.0 / 3e6 : 0.0);
         if (ks == 1 || us < best) { best = us; *ranges = n; *kper = n > 1 ? 64 * per : 0; }
     }
     return 64;
@@ -1906,9 +1905,7 @@ static bool pad16_plan(int M, int N, int K, PadPlan* pl)
     const bool tall = any16_plan(M, N, K, &kper, &ranges) == 128;
     if (ranges > 2 || !pad16_layout(M, N, K, pl)) return false;
     const long long wgs = (long long)((M + (tall ? 127 : 63)) / (tall ? 128 : 64)) * ((N + 127) / 128) * ranges;
-    const double one = tall ? 0.75 : 0.48, two = tall ? 1.35 : 0.83;
-    const int last = (int)(wgs % 512);                // (beyond four rounds of 512 the workgroups no longer run in step)
-    const double rounds = wgs >= 2048 ? two * wgs / 512.0 : two * (double)(wgs / 512) + (last == 0 ? 0.0 : last <= 256 ? one : two);
+    const double rounds = tall ? any16_rounds(wgs, 0.75, 1.35) : any16_rounds(wgs, 0.48, 0.83);
     const double tiles = kper > 0 ? kper / 64 : (K + 63) / 64;
     const double in_place = 5.5 + rounds * tiles * (K % 8 == 0 ? 0.85 : 1.0) + mn / 1.7e6 + (ranges > 1 ? 3.2 + mn * 16.0 / 3e6 : 0.0);
     double score = 0.0;
@@ -2076,13 +2073,13 @@ hipError_t unpad_rows(hipStream_t stream, const void* src, void* dst, long long 
 
 // The largest need over the plans gemm_16 may take for these dimensions (the choice also depends on operand alignment; every
 // plan checks its own need against the bytes it is handed).
-size_t gemm_16_workspace_bytes(int M, int N, int K)
+size_t gemm_16_workspace_bytes(int M, int N, int K, bool off_grid)
 {
     PadPlan pl;
     const size_t inner = gemm_16_inner_workspace_bytes(M, N, K);
     size_t need = inner;
     if (pad16_plan(M, N, K, &pl) && pl.total > need) need = pl.total;
-    if (N % 8 != 0 || K % 8 != 0) {
+    if (off_grid || N % 8 != 0 || K % 8 != 0) {
         int kper, ks;
         any16_plan(M, N, K, &kper, &ks);
         if (ks > 1) need = std::max(need, (size_t)ks * M * N * sizeof(float));

@@ -25,8 +25,9 @@ size_t gemm_smallm_workspace_bytes(int M, int N, int K);
 hipError_t gemm_f32_f16weight(hipStream_t stream, const float* A, const uint16_t* B, float* C, int M, int N, int K,
                               int force_tile, const float* bias = nullptr, int act = 0, float act_param = 0.0f,
                               void* workspace = nullptr, size_t workspace_bytes = 0);
-// workspace: gemm_16_workspace_bytes(M, N, K) bytes (0 = none needed); without it the skinny-M path is not taken
-size_t gemm_16_workspace_bytes(int M, int N, int K);
+// workspace: gemm_16_workspace_bytes bytes (0 = none needed; off_grid: A or B is not 16-byte aligned); without it neither the skinny-M path
+// nor K ranges are taken
+size_t gemm_16_workspace_bytes(int M, int N, int K, bool off_grid);
 // Bpre: B packed once by gemm_16_pack_b into gemm_16_packed_b_bytes(N, K) bytes (B itself is then ignored); the workspace must then
 // hold gemm_16_packed_workspace_bytes(M, N, K) bytes
 hipError_t gemm_16(hipStream_t stream, int kind, const uint16_t* A, const uint16_t* B, void* C, int out32,
