@@ -1393,7 +1393,7 @@ static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
 // MFMAs of 64 cycles with nothing else on their SIMDs, 44 us -- as long as twice the batch.  Two waves per 32 rows (64-row workgroups,
 // each wave half of every tile, merged through LDS at the end): 27 us; B1 H12 S1024 81 -> 48, and 32 with four.  Once the chip is full
 // the same matrix work only pays for more tile loads and merges (B16 H12 S512 83 -> 89 us).  The lines, as workgroups of the finer
-// grid, from a sweep over 58 shapes (time with one / two key groups in us at the last size on either side):
+// grid on 256 CUs, from a sweep over 58 shapes (time with one / two key groups in us at the last size on either side):
 //   64-key tiles, two workgroups per CU, head dimension up to 64: 768 (fp32 plain S512 74 / 67, causal S4096 308 / 253; 960: 54 / 54, S900
 //     89 / 118); short causal fp32 sequences 640, beyond which the halved workgroups' starts and merges cost what they balance (S512 44.0 / 44.2);
 //     16-bit causal 1024 (S500 19.3 / 14.8, S1900 46 / 35; plain 20.4 / 21.1; 1536: 21 / 28)
@@ -1401,10 +1401,13 @@ static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
 //   fp32 above 64: 64-key tiles need 128 KiB, one workgroup per CU: 256 (plain d128 151 / 88; 384: 66 / 83), causal 384 (64 / 42)
 //   four groups on 128-key tiles (head dimension 64, dense K and V, no mask): 256, causal 384, from 192 keys on (two / four groups: plain
 //     B4 H8 S256 16.0 / 12.2, causal B1 H32 S300 18.8 / 16.3; plain at 304 32 / 40, 64 keys 7.9 / 8.8)
-// Short sequences do not repay the merge by balance, only where the finer grid saves a round of workgroups (240 shapes of 12 - 300 keys):
-//   one 64-key tile: up to 256, and up to 512 where the 128-row grid needs a second workgroup per CU (fp32 Sq 130 n 480 14.7 / 11.1, bf16 Sq 131
-//     n 429 7.1 / 6.9; but fp32 Sq 69 n 286 9.7 / 10.8, n 618 13.8 / 16.5, bf16 Sq 105 n 848 7.2 / 8.9); up to 256 keys the same of fp32 plain
-//     at n 257 - 512 (S 115 n 360 14.7 / 15.5)
+// Beyond 64 queries, where the finer grid has more workgroups, short sequences do not repay the merge by balance but only by a round of
+// workgroups saved (240 shapes of 12 - 300 keys; up to 64 queries the second group takes waves that would idle, and the lines above hold):
+//   one 64-key tile, plain or causal: up to 256, and up to 512 (head dimension 32, of whose workgroups a CU holds more: 768) where the 128-row
+//     grid needs a second workgroup per CU (fp32 Sq 130 n 480 14.7 / 11.1, bf16 Sq 131 n 429 7.1 / 6.9, d32 Sq 256 n 628 10.7 / 10.1; but fp32
+//     Sq 69 n 286 9.7 / 10.8, n 618 13.8 / 16.5, bf16 Sq 105 n 848 7.2 / 8.9); masks and biases up to 512 (Sq 310 n 400 12.3 / 10.7), at
+//     head dimension 32 as above
+//   up to 256 keys, fp32 plain: not at n 257 - 512 on a 128-row grid of up to 256 (S 115 n 360 14.7 / 15.5)
 //   16-bit causal beyond 768: a 128-row grid of more than 512, or long rows (S 300 n 1000 14.0 / 11.9; but S 232 n 944 10.5 / 11.5)
 //   fp32 above 64: up to 32 keys the second group has none (Sk 12 10.6 / 12.8); causal 384 only where the row tiles differ in length
 //     (Sq 204 n 288 44 / 35; but Sq 62, Sk 12 n 352 16 / 26)
@@ -1420,7 +1423,8 @@ static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
         }
         long long line;
         if constexpr (WIDE32) line = a.Sk <= 32 ? 0 : a.causal && a.Sq > 64 && a.Sk > 128 ? 384 : 256;
-        else if (a.Sk <= 64 || (Elem<T>::BYTES == 4 && !FULL && !a.causal && a.Sk <= 256 && grid(128) <= 256)) line = grid(128) > 256 ? 512 : 256;
+        else if (grid(64) > grid(128) && a.Sk <= 64 && !(FULL && DP == 32)) line = FULL ? 512 : grid(128) <= 256 ? 256 : DP == 32 ? 768 : 512;
+        else if (Elem<T>::BYTES == 4 && !FULL && !a.causal && a.Sk <= 256 && grid(64) > grid(128) && grid(128) <= 256) line = 256;
         else if constexpr (DP > 64) line = 512;
         else if constexpr (Elem<T>::BYTES == 2) line = !FULL && a.causal && (a.Sk >= 448 || grid(128) > 512) ? 1024 : 768;
         else line = a.causal && a.Sk < 1024 ? 640 : 768;

@@ -1,4 +1,5 @@
-"""Paged prefill on the direct-to-LDS kernels: key tiles of 64 (fp32 at head dimension 128: 32) fetched block by block, pool rows looked
+"""Paged prefill on the direct-to-LDS kernels: key tiles of 64 (fp32 at head dimension 128 on larger grids 32, and head dimension 256:
+test_gpu_attention_large_grids.py) fetched block by block, pool rows looked
 up 64 tiles at a time, the keys of a few query tiles cut into ranges.  Sizes on both sides of each of those edges, block sizes that are
 multiples of 16 (powers of two or not) and one that is not, against a float64 softmax over the gathered cache.
 
