@@ -1331,14 +1331,16 @@ static hipError_t launch_gemm_dl16(GemmArgs g, int batch, hipStream_t stream)
 // (128 bytes of A, 256 of B), two K-tiles ahead, and is written to the LDS layout of gemm_dl16_kernel, from which the fragments are read
 // as there (transposing reads for B).  What bounds it is the stream of B for few rows and the load / LDS-write work beyond.
 // The general kernel's loads of B are 16 rows of 64 bytes to an instruction, each cache line asked for twice: 64 x 50257 x 768
-// took 44 us there and takes 17.5 here (84 MB), 212 x 36669 x 704 103 / 28, 512 x 30001 x 4096 232 through padded copies / 156.
+// takes 43 us there and 17.5 here (84 MB), 212 x 36669 x 704 101 / 27, 512 x 30001 x 4096 232 through padded copies / 157 (ten calls in a
+// graph).
 // kper > 0: workgroups z take K ranges of kper (a multiple of 64) each and C is their fp32 partials, sum_stride elements apart.
 // Bounds: the last K-tile of the matrix is loaded under guards (zeros past K; whole chunks where they fit their row), which costs about 1 us;
-// where all rows are whole chunks (operands off the 16-byte grid) from clamped addresses instead (20 x 272 x 248 6.8 -> 5.8 us, 3 x 7224 x 512
-// 8.9 -> 6.9).  In the others a
+// where all rows are whole chunks (operands off the 16-byte grid) tiles of 64 rows take it from clamped addresses instead (20 x 272 x 248 6.8 ->
+// 5.8 us, 3 x 7224 x 512 8.9 -> 6.9).  In the others a
 // chunk of B that crosses column N reads on into the next row, which exists, and is only multiplied into columns that are not stored.
 // Rows of A past M and chunks of B past N are clamped likewise.  N >= 8.
-template <typename T, typename OutT, int BM>
+// WHOLE: no chunk crosses the end of a row (N and K multiples of 8).
+template <typename T, typename OutT, int BM, bool WHOLE>
 __global__ __launch_bounds__(512, 4) void gemm_any16_kernel(const GemmArgs g, int kper, long long sum_stride)
 {
     typedef typename Raw<T>::type raw_t;
@@ -1372,9 +1374,7 @@ __global__ __launch_bounds__(512, 4) void gemm_any16_kernel(const GemmArgs g, in
         pa[i] = (uint32_t)((min(m0 + row, g.M - 1) - m0) * g.lda + ach * 8);
         a_lds[i] = row * AROW + ((ach ^ ((row >> 1) & 7)) << 4);
     }
-    // whole: no chunk crosses the end of a row, and the last K-tile is loaded like the others, from clamped addresses (64 rows, where it counts)
-    const bool whole = BM == 64 && ((g.K | g.N) & 7) == 0;
-    const int bcol = min(n0 + bch * 8, whole ? g.N - 8 : g.N - 1);
+    const int bcol = min(n0 + bch * 8, WHOLE ? g.N - 8 : g.N - 1);
     const uint32_t pb = (uint32_t)((t >> 4) * g.ldb + bcol);
 #pragma unroll
     for (int i = 0; i < LB; i++) {
@@ -1393,7 +1393,7 @@ __global__ __launch_bounds__(512, 4) void gemm_any16_kernel(const GemmArgs g, in
         constexpr int S = decltype(set)::value;
         if (kt < KT - 1) { load_plain(kt, set); return; }
         if (kt >= KT) return;
-        if (whole) {
+        if constexpr (WHOLE) {
             const int ak = kt * BK + ach * 8, bk = kt * BK + (t >> 4);
 #pragma unroll
             for (int i = 0; i < LA; i++) ra[S][i] = *(const u32x4_elem*)(a_base + ((int)pa[i] - ach * 8 + min(ak, K - 8)));
@@ -1539,17 +1539,25 @@ __global__ __launch_bounds__(512, 4) void gemm_any16_kernel(const GemmArgs g, in
     }
 }
 
-template <typename T, typename OutT, int BM>
-static hipError_t launch_any16(GemmArgs g, hipStream_t stream, int ks = 1, int kper = 0)
+template <typename T, typename OutT, int BM, bool WHOLE>
+static hipError_t launch_any16_as(GemmArgs g, hipStream_t stream, int ks, int kper)
 {
     constexpr int smem = 2 * (BM * 128 + 64 * 256);
-    auto kern = gemm_any16_kernel<T, OutT, BM>;
+    auto kern = gemm_any16_kernel<T, OutT, BM, WHOLE>;
     static unsigned long long attr_done = 0;
     if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done)) return e;
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + 127) / 128;
     hipLaunchKernelGGL(kern, dim3((unsigned)(g.tiles_m * g.tiles_n), 1, (unsigned)ks), dim3(512), smem, stream, g, ks > 1 ? kper : 0, (long long)g.M * g.N);
     return hipGetLastError();
+}
+template <typename T, typename OutT, int BM>
+static hipError_t launch_any16(const GemmArgs& g, hipStream_t stream, int ks = 1, int kper = 0)
+{
+    if constexpr (BM == 64) {
+        if (((g.K | g.N) & 7) == 0) return launch_any16_as<T, OutT, BM, true>(g, stream, ks, kper);
+    }
+    return launch_any16_as<T, OutT, BM, false>(g, stream, ks, kper);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -1,10 +1,9 @@
 """Values of the fused activations over the whole range of their argument, through every kernel that applies them.  A is a shifted
 identity, so the product is exactly the chosen values and only the epilogue is looked at.
 
-Bound: relative error <= 4e-7 for the functions built on the logistic function where the result is above 1e-30 (argument rounding of
-the exponential is carried in a second part: two fp32 roundings of e^-x, one of 1 + e^-x, reciprocal within one unit after a Newton
-step, one product: 3.5 units of 2^-23); GELU's inner cubic adds 2 |2u| 2^-24 relative, below 3e-6 for |u| <= 22, beyond which the
-result is x or below 1e-19."""
+Bound: relative error <= 4e-7 for the functions built on the logistic function where the result is above 1e-30 (the hardware exponential
+and its argument's rounding, the sum with 1 and the quotient: at most 2.75 units of 2^-23, 3.3e-7, see the last test); GELU's inner
+cubic adds 2 |2u| 2^-24 relative, below 3e-6 for |u| <= 22, beyond which the result is x or below 1e-19."""
 import math
 
 import numpy as np
