@@ -16,7 +16,8 @@ LIB_NAME = "libaidotnet_mi355.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 # (source, object name, extra flags): gemm.hip is compiled in three parts so that its template instances build in parallel
 SOURCES = [("gemm.hip", "gemm.o", ["-DAIDN_GEMM_PART=0"]), ("gemm.hip", "gemm_f16.o", ["-DAIDN_GEMM_PART=1"]),
-           ("gemm.hip", "gemm_bf16.o", ["-DAIDN_GEMM_PART=2"]), ("attention.hip", "attention.o", []), ("attention_prefill.hip", "attention_prefill.o", []),
+           ("gemm.hip", "gemm_bf16.o", ["-DAIDN_GEMM_PART=2"]), ("gemm_split.hip", "gemm_split.o", []),
+           ("attention.hip", "attention.o", []), ("attention_prefill.hip", "attention_prefill.o", []),
            ("decode.hip", "decode.o", []),
            ("convert.hip", "convert.o", []), ("api.hip", "api.o", [])]
 # -packed-fp32-ops off: packed fp32 VALU forms are kept out of all device code.

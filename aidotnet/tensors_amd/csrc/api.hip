@@ -482,13 +482,13 @@ AIDN_API int aidn_mi355_set_attention_fast_path(void* ctx, int enabled)
     return AIDN_OK;
 }
 
-// workspace of the fp32 paths that need one: small M (M <= 8, B [K,N]) and split-K partials; mode 0 B [K,N], 1 B [N,K], 2 fp16
-// weights (small M only).  *ws stays null when no such path applies or a tile size is forced
+// workspace of the fp32 paths that need one: small M (M <= 8, B [K,N]) and K ranges; mode 0 B [K,N], 1 B [N,K], 2 fp16
+// weights.  *ws stays null when no such path applies or a tile size is forced
 static int smallm_ws(Ctx* c, void* stream, int M, int N, int K, int transB, void** ws, size_t* ws_bytes)
 {
     *ws = nullptr; *ws_bytes = 0;
     if (c->force_tile != 0) return 0;
-    size_t need = transB == 2 ? aidn::gemm_smallm_workspace_bytes(M, N, K) : aidn::gemm_f32_workspace_bytes(M, N, K, transB);
+    size_t need = transB == 2 ? aidn::gemm_f32_f16weight_workspace_bytes(M, N, K) : aidn::gemm_f32_workspace_bytes(M, N, K, transB);
     if (!need) return 0;
     const int st = acquire_ws(c, stream, need, ws);
     // a stream under capture whose workspace would have to grow: the tiled kernel needs none

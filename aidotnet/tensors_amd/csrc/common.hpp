@@ -140,6 +140,29 @@ __device__ __forceinline__ long long paged_row(const int* __restrict__ bt, int b
     return (long long)bt[blk] * bsz + (key - blk * bsz);
 }
 
+// ---------------------------------------------------------------- fp32 values as three bf16 values
+// x = h + m + l with h = bf16(x), m = bf16(x - h), l = x - h - m: exact for |x| >= 2^-110, cut at 2^-134 below; infinities and values
+// that round to one do not survive it (NaN).
+typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+// two values to NP words of bf16 pairs.  (Opaque words: the compiler otherwise converts the low half a second time by itself.)
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b)
+{
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 v = {(__bf16)a, (__bf16)b};
+    uint32_t u = __builtin_bit_cast(uint32_t, v);
+    asm("" : "+v"(u));
+    return u;
+}
+template <int NP>
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&p)[NP])
+{
+#pragma unroll
+    for (int s = 0; s < NP; s++) {
+        p[s] = bf16_pair(a, b);
+        if (s + 1 < NP) { a -= as_f32(p[s] << 16); b -= as_f32(p[s] & 0xFFFF0000u); }
+    }
+}
+
 // ---------------------------------------------------------------- wave helpers
 __device__ __forceinline__ float shfl_xor_f(float v, int mask) { return __shfl_xor(v, mask, WAVE); }
 

@@ -16,9 +16,7 @@
 //   stored to the other stage before its last k-step; one barrier per K-tile.
 // The 16-bit 256 x 256 kernel further down loads global -> LDS directly; the skinny (M <= 32, 16-bit) and
 // small-M (M <= 8, fp32) kernels are bandwidth-bound split-K streams of B.
-#include "common.hpp"
-#include "launch.hpp"
-#include <type_traits>
+#include "gemm_common.hpp"
 
 // This file is compiled three times (the build passes -DAIDN_GEMM_PART=0/1/2) so that its template instances build in
 // parallel: part 0 holds the fp32 entry points and everything that exists once, part 1 the fp16 and part 2 the bf16 instances.
@@ -27,46 +25,6 @@
 #endif
 
 namespace aidn {
-
-// f(std::integral_constant<int, I>) for I = BEGIN, BEGIN + STEP, ... < END: a loop the compiler cannot leave rolled (register
-// arrays indexed by the loop variable need constant indices)
-template <int BEGIN, int END, int STEP, typename F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    if constexpr (BEGIN < END) {
-        f(std::integral_constant<int, BEGIN>{});
-        static_for<BEGIN + STEP, END, STEP>(f);
-    }
-}
-
-struct GemmArgs {
-    const void* A; const void* B; void* C;
-    int M, N, K;
-    int lda, ldb, ldc;
-    long long sA, sB, sC;   // batch strides in elements
-    float alpha, beta;
-    int tiles_m, tiles_n;
-    // fused epilogue: C = act(alpha * A B + beta * C + bias[col]); bias may be null, act 0 = none
-    const float* bias;
-    int act;
-    float act_param;
-    // direct-to-LDS kernels only (the 16 x 16 x 32 one and the instances of the 32 x 32 one with edge handling).  > 0: C has this
-    // many columns (fewer than N, the columns past them are padding of B that is computed and dropped) and ldc is any element
-    // count, so a row of C may start off a 16-byte boundary
-    int c_cols = 0;
-    // three products with one A in one launch (three batches): their Bs lie anywhere, B at B, B + sB and B + 2 sB + sB2.  (A stride and not
-    // two pointers: choosing one by branches in front of the first load cost every kernel 0.1 - 0.3 us, 9 % of a 1 x 256 x 101 product)
-    long long sB2 = 0;
-};
-
-// B of batch bz, in units of B's elements of EB bytes
-template <int EB>
-__device__ __forceinline__ const unsigned char* batch_b(const GemmArgs& g, long long bz)
-{
-    return (const unsigned char*)g.B + (bz * g.sB + (bz == 2 ? g.sB2 : 0LL)) * EB;
-}
-
-[[maybe_unused]] static bool aligned16(const void* p) { return (((uintptr_t)p) & 15u) == 0; }
 
 #if AIDN_GEMM_PART == 0
 hipError_t ensure_dynamic_smem(const void* kernel, int bytes, unsigned long long* done_mask)
@@ -81,89 +39,11 @@ hipError_t ensure_dynamic_smem(const void* kernel, int bytes, unsigned long long
 }
 #endif
 
-// num / (1 + e^-v): GELU (tanh form: (1 + tanh u) / 2 is the logistic function of 2 u), sigmoid and swish, on the vector pipe's exponential
-// (base 2) and reciprocal.  The exponent is split into its nearest whole number, added to the exponent field, and a remainder formed from
-// v log2(e) in two parts (LONG: with one rounding, for arguments of any size; GELU's matter near zero, where two do as well).  The quotient is
-// corrected by its remainder against 1 + e^-v and what that sum lost, so that the error is that of e^-v and one rounding of the result.
-// Numerator and denominator are scaled by 2^-4, which keeps the reciprocal normal down to the v where e^-v overflows; below it is zero.
-// Largest errors against float64 in units in the last place, with the library's expf or tanhf and an IEEE division / this way: sigmoid
-// 2.6 / 2.6 at -20 to -10, 2.2 / 1.7 to 0, 1.5 / 0.8 above; swish 2.7 / 2.7, 2.1 / 1.7, 1.5 / 0.9; GELU above -0.1 1.8 / 1.2, at -2 to -1 15 / 5.5.
-// An epilogue holds nothing but these values and nothing runs beside it on one tile per CU, so their length is time: the fp32 product
-// 4096 x 3072 x 768 with GELU took 199 us with the library functions chosen per element and takes 149, bf16 1000 x 11008 x 4096 with swish
-// 130 and 112 (107 with an exponential rounded twice and the product with the reciprocal: errors up to 3.5 units, zero below -87).
-template <bool LONG>
-__device__ __forceinline__ float over_one_plus_exp(float num, float v)
-{
-#pragma clang fp contract(off)
-    constexpr float L2E = 1.44269502f, L2E_LO = 1.92596299e-8f;                          // log2(e) = L2E + L2E_LO
-    constexpr float WHOLE = 12582912.0f, ONE = 0x1p-4f;                                  // 1.5 2^23: a sum with it is rounded to a whole number
-    float whole, rest;
-    if constexpr (LONG) {
-        const float t = v * -L2E;
-        whole = t + WHOLE;
-        rest = fmaf(v, -L2E_LO, fmaf(v, -L2E, -t)) + (t - (whole - WHOLE));
-    } else {
-        whole = fmaf(v, -L2E, WHOLE);
-        rest = fmaf(v, -L2E_LO, fmaf(v, -L2E, WHOLE - whole));
-    }
-    const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(rest), __builtin_bit_cast(int, whole) - (__builtin_bit_cast(int, WHOLE) + 4));
-    const float d = e + ONE, lost = e - (d - ONE);
-    const float n = num * ONE, r = __builtin_amdgcn_rcpf(d);
-    float q = n * r;
-    q = fmaf(-fmaf(lost, q, fmaf(d, q, -n)), r, q);                                      // (in this order a zero keeps its sign)
-    q = v < -88.72f ? num * 0.0f : q;
-    return v > 88.0f ? num : q;
-}
-
-// Pointwise activations of the fused projection epilogues, numbered like the reference's FusedActivationType
-// (src/AiDotNet.Tensors/Engines/FusedActivationType.cs:23-70); the functions are those of its HIP activation kernels
-// (src/AiDotNet.Tensors/Engines/DirectGpu/HIP/Kernels/HipActivationKernels.cs:19-70).  NaN stays NaN in all of them.
-// f(fn) with fn the activation `act`: the choice is made once around whatever f does with it, never per element (a tile of
-// accumulators with a test on each is thousands of branches).  Sigmoid and swish share a body: with one each the 256 x 256 fp32 tile's
-// epilogue outgrows what the compiler unrolls, and its accumulators go to scratch memory.
-template <typename F>
-__device__ __forceinline__ void with_activation(int act, float p, F&& f)
-{
-    switch (act) {
-    case 1: f([](float x) { return x < 0.0f ? 0.0f : x; }); break;                       // ReLU, NaN-preserving form (CpuFusedOperations.cs:1271-1274)
-    case 2: f([](float x) { return over_one_plus_exp<false>(x, x * fmaf(0.0713548163f, x * x, 1.5957691216f)); }); break;      // GELU, tanh form: 2 u = 2 0.7978845608 (x + 0.044715 x^3)
-    case 3:                                                                               // sigmoid
-    case 6: f([act](float x) { return over_one_plus_exp<true>(act == 3 ? 1.0f : x, x); }); break;      // swish
-    case 4: f([](float x) { return tanhf(x); }); break;
-    case 5: f([p](float x) { return x > 0.0f ? x : p * x; }); break;                      // leaky ReLU, slope p
-    default: f([](float x) { return x; }); break;
-    }
-}
-__device__ __forceinline__ float apply_activation(float x, int act, float p)
-{
-    with_activation(act, p, [&](auto fn) { x = fn(x); });
-    return x;
-}
-
 // K extent of one tile of the general kernel in 16-byte chunks per row, and the LDS row pitch (one chunk of padding keeps the
 // b128 fragment reads conflict-free).  The 64 x 64 tile takes twice the K per barrier: its waves have too little MFMA work
 // per tile to hide one barrier every 128 bytes of K.
 constexpr int gemm_k_chunks(int bm, int bn) { return bm * bn <= 64 * 64 ? 16 : 8; }
 constexpr int gemm_row_pitch(int bm, int bn) { return gemm_k_chunks(bm, bn) * 16 + 16; }
-constexpr int GROUP_M = 8;   // tile rows walked together so one XCD's L2 sees a compact footprint
-
-// Workgroup id -> (tile row, tile col).  Hardware hands consecutive workgroup ids to the 8
-// XCDs round-robin; remap so each XCD owns a contiguous run of logical ids, then walk
-// that run in GROUP_M-tall column-major groups.
-__device__ __forceinline__ void tile_of_block(int pid, int nblk, int tiles_m, int tiles_n, int& tm, int& tn)
-{
-    int per = nblk >> 3, rem = nblk & 7;
-    int xcd = pid & 7, idx = pid >> 3;
-    int logical = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + idx;
-    int width = GROUP_M * tiles_n;
-    int group = logical / width;
-    int first = group * GROUP_M;
-    int gsz = min(tiles_m - first, GROUP_M);
-    int in = logical - group * width;
-    tm = first + in % gsz;
-    tn = in / gsz;
-}
-
 template <typename T> struct Raw;
 template <> struct Raw<float> { typedef uint32_t type; };
 template <> struct Raw<f16_t> { typedef uint16_t type; };
@@ -2515,6 +2395,89 @@ __global__ __launch_bounds__(256, NS <= 3 ? 2 : 1) void gemm_skinny32_kernel(con
     return best_ks;
 }
 
+#if AIDN_GEMM_PART == 0
+// ---- fp32 products on the bf16 matrix pipe (gemm_split.hip): tile and K ranges by an estimate of the run time in microseconds.
+// A WG advances by one K-tile of 32 in us[n - 1] with n of them on a CU and needs `once` for its first loads and its epilogue; the operands
+// come at 6 TB/s at best; ranges add the summing pass, 8 bytes a partial element at 5 TB/s.  Fitted on 963 (fp32) and 325 (fp16
+// weights) timings of 140 shapes, M 9 - 8192, N 64 - 60000, K 64 - 16384, to 9 and 11 %; the plan it picks is 1 and 2 % behind the best one in the mean.
+struct SplitTile { int id, rows, cols, resident; double us[2][3], once[2]; };
+static const SplitTile kSplitTiles[3] = {{64, 64, 128, 3, {{1.25, 1.77, 2.30}, {0.97, 1.34, 1.72}}, {0.0, 0.0}},
+                                         {128, 128, 128, 2, {{1.89, 2.57, 0.0}, {1.66, 2.10, 0.0}}, {1.7, 0.9}},
+                                         {192, 128, 192, 2, {{3.00, 4.17, 0.0}, {2.74, 4.43, 0.0}}, {3.6, 6.7}}};
+struct SplitPlan { int tile = 0, ks = 1, kper = 0; double us = 1e30; };
+static SplitPlan split_plan(int M, int N, int K, int batch, bool b16, size_t partial_bytes)
+{
+    SplitPlan best;
+    if (N < 2 || N >= (1 << 21) || K >= (1 << 21)) return best;
+    const int kt = (K + 31) / 32;
+    // (a B beyond the last-level cache, 54 x 42236 x 1216: 76 us from memory, 64 from the cache)
+    const double b_bytes = (b16 ? 2.0 : 4.0) * K * N * batch;
+    const double bytes_us = (4.0 * M * K * batch + b_bytes) / (b_bytes > 1.5e8 ? 2.9e6 : b16 ? 4.5e6 : 6.4e6);
+    static const int ranges[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+    for (const SplitTile& s : kSplitTiles) {
+        if (s.id == 192 && (M % 128 != 0 || N % 192 != 0 || K % 32 != 0)) continue;
+        const long long tiles = (long long)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols) * batch;
+        for (int want : ranges) {
+            if (want > 1 && (batch > 1 || kt / want < 2 || tiles * want > 1600)) break;
+            const int per = (kt + want - 1) / want, ks = (kt + per - 1) / per;
+            if (ks > 1 && (size_t)ks * M * N * sizeof(float) > partial_bytes) break;
+            const long long wgs = tiles * ks, slots = 256LL * s.resident;
+            double rounds, tile_us;                       // rounds of resident workgroups, and the time of one K-tile in all of them
+            if (wgs >= 4 * slots) { rounds = (double)wgs / slots; tile_us = rounds * s.us[b16][s.resident - 1]; }
+            else {
+                const long long full = wgs / slots, last = (wgs - full * slots + 255) / 256;
+                rounds = (double)full + (last ? 1.0 : 0.0);
+                tile_us = full * s.us[b16][s.resident - 1] + (last ? s.us[b16][last - 1] : 0.0);
+            }
+            double us = tile_us * per + rounds * s.once[b16];
+            if (us < bytes_us) us = bytes_us;
+            us += (b16 ? 5.6 : 5.4) + (ks > 1 ? 3.0 + 8.0 * ks * M * N / 5.0e6 : 0.0);
+            if (us < best.us) best = SplitPlan{s.id, ks, ks > 1 ? per * 32 : 0, us};
+        }
+    }
+    return best;
+}
+// What the kernels on the fp32 pipe need for the same product: the estimate above for rows in whole 16-byte chunks; else (and for fp16
+// weights) the general kernel's 64 x 64 tiles at the measured time of 64 k.  They stay ahead on small products, whose few K-tiles they
+// walk with twice the K to a barrier (288 x 512 x 192 7.0 us against 10.1, 41 x 2304 x 1536 12.9 / 16.9).
+static double fp32_pipe_us(int M, int N, int K, int batch, bool b16, bool* two_launches)
+{
+    *two_launches = false;
+    const bool chunks = K % 4 == 0 && N % 4 == 0;
+    if (!b16 && chunks) {
+        double us = f32_time_us(M, N, K, batch, f32_tile(M, N, K, batch, true), 1);
+        const int ks = batch == 1 ? splitk32_ranges(M, N, K) : 1;
+        if (ks > 1) { us = std::min(f32_time_us(M, N, K, 1, 128, ks), f32_time_us(M, N, K, 1, 64, ks)); *two_launches = true; }
+        return us + 2.5;
+    }
+    const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
+    // (244 x 853 x 1024 0.66 a step, 2317 x 90 x 512 and 605 x 1338 x 12992 1.6 - 1.7; beyond one tile per CU the tiles share it)
+    const double step = (b16 ? (chunks ? 2.0 : 3.2) : K % 4 != 0 ? 1.3 : M <= 512 && K <= 1024 ? 0.72 : 1.6) * (tiles > 256 ? 2.0 : 1.0);
+    return 5.0 + step * ((K + 63) / 64) * ((tiles + 255) / 256);
+}
+static SplitPlan split_choice(int M, int N, int K, int batch, bool b16, size_t partial_bytes)
+{
+    const SplitPlan p = split_plan(M, N, K, batch, b16, partial_bytes);
+    bool two;
+    const double other = fp32_pipe_us(M, N, K, batch, b16, &two);
+    // a call costs its caller about 12 us, one of two launches 15.5, whatever its kernels take (10 x 320 x 640: one launch of 14.5, two of 11)
+    auto call = [](double us, bool two_launches) { return std::max(us, two_launches ? 15.5 : 12.0) + 0.05 * us; };
+    return 1.08 * call(p.us, p.ks > 1) < call(other, two) ? p : SplitPlan{};
+}
+static hipError_t run_split(const GemmArgs& g, const SplitPlan& p, int batch, hipStream_t stream, void* workspace, bool b16)
+{
+    if (p.ks == 1) return launch_gemm_split(g, batch, stream, p.tile, b16);
+    GemmArgs gp = g;                                      // the K ranges as batches into fp32 partials, summed in their order
+    gp.C = workspace; gp.K = p.kper; gp.k_total = g.K; gp.ldc = g.N; gp.alpha = 1.0f; gp.beta = 0.0f;
+    gp.sA = p.kper; gp.sB = (long long)p.kper * g.ldb; gp.sB2 = 0; gp.sC = (long long)g.M * g.N;
+    gp.bias = nullptr; gp.act = 0;
+    if (hipError_t e = launch_gemm_split(gp, p.ks, stream, p.tile, b16)) return e;
+    hipLaunchKernelGGL((skinny_reduce_kernel<float>), dim3((unsigned)(((long long)g.M * g.N + 255) / 256)), dim3(256), 0, stream, (const float*)workspace,
+                       g.C, g.M, g.N, p.ks, g.bias, g.act, g.act_param, g.alpha, g.beta);
+    return hipGetLastError();
+}
+#endif
+
 static bool smallm_applies(int M, int N, int K) { return M >= 1 && M <= 8 && (long long)N * K >= 4096; }
 
 // K range of one workgroup: about 1024 workgroups, at least 128 k-rows each (32 per wave), a multiple of 32
@@ -2538,9 +2501,9 @@ size_t gemm_smallm_workspace_bytes(int M, int N, int K)
     const int kper = smallm_kper(N, K);
     return (size_t)((K + kper - 1) / kper) * M * N * sizeof(float);
 }
-// fp32 problems whose rows are not whole 16-byte chunks (K, or N with B [K,N], not a multiple of 4): zero-padded copies of A and B
-// in the workspace (K up to a multiple of 32, N up to a multiple of 4) feed the direct-to-LDS kernel, whose element stores put the N
-// real columns straight into the caller's C.  Same sums as the plain product: the padding contributes exact zeros.
+// fp32 problems with B [N,K] whose rows are not whole 16-byte chunks (K not a multiple of 4): zero-padded copies of A and B in the
+// workspace (K up to a multiple of 32) feed the direct-to-LDS kernel.  Same sums as the plain product: the padding contributes exact
+// zeros.  The layout (with N up to a multiple of 4 for B [K,N]) is also that of a packed B.
 struct Pad32Plan { int Np, Kp; size_t a_off, b_off, total; };
 static bool pad32_layout(int M, int N, int K, int transB, Pad32Plan* pl)
 {
@@ -2553,12 +2516,11 @@ static bool pad32_layout(int M, int N, int K, int transB, Pad32Plan* pl)
     pl->total = pl->b_off + up((size_t)(transB ? N : pl->Kp) * (transB ? pl->Kp : pl->Np) * 4);
     return pl->total <= ((size_t)4 << 30);
 }
-static bool pad32_plan(int M, int N, int K, int transB, Pad32Plan* pl)
+static bool pad32_plan(int M, int N, int K, Pad32Plan* pl)       // B [N,K]
 {
-    if (K % 4 == 0 && (transB || N % 4 == 0)) return false;
-    if (N < 16 || (double)M * N * K < (double)(1 << 21)) return false;
+    if (K % 4 == 0 || N < 16 || (double)M * N * K < (double)(1 << 21)) return false;
     if (M <= 512 && K <= 1024) return false;          // as for 16-bit: the general kernel reads the rows in place
-    return pad32_layout(M, N, K, transB, pl);
+    return pad32_layout(M, N, K, 1, pl);
 }
 
 // Pre-packed fp32 B (the caller keeps it): [K,N] zero-padded to [Kp, Np], or [N,K] to [N, Kp] -- the GPU form of the reference's
@@ -2579,8 +2541,20 @@ size_t gemm_f32_packed_workspace_bytes(int M, int N, int K, int transB)
 {
     Pad32Plan pl;
     if (!pad32_layout(M, N, K, transB, &pl)) return 0;
-    const size_t small = !transB && smallm_applies(M, N, K) ? gemm_smallm_workspace_bytes(M, N, K) : 0;
-    return pl.b_off > small ? pl.b_off : small;                       // the padded copy of A, or the small-M partials
+    size_t need = pl.b_off;                                           // the padded copy of A, or partials
+    if (!transB) {
+        if (smallm_applies(M, N, K)) need = std::max(need, gemm_smallm_workspace_bytes(M, N, K));
+        const SplitPlan sp = split_choice(M, N, K, 1, false, SIZE_MAX);
+        if (sp.ks > 1) need = std::max(need, (size_t)sp.ks * M * N * sizeof(float));
+    }
+    return need;
+}
+
+size_t gemm_f32_f16weight_workspace_bytes(int M, int N, int K)
+{
+    if (smallm_applies(M, N, K)) return gemm_smallm_workspace_bytes(M, N, K);
+    const SplitPlan sp = split_choice(M, N, K, 1, true, SIZE_MAX);
+    return sp.ks > 1 ? (size_t)sp.ks * M * N * sizeof(float) : 0;
 }
 
 // The largest need over every plan gemm_f32 may take for these dimensions: which one it takes also depends on the alignment of
@@ -2591,7 +2565,11 @@ size_t gemm_f32_workspace_bytes(int M, int N, int K, int transB)
     auto upto = [&](size_t n) { if (n > need) need = n; };
     if (!transB && smallm_applies(M, N, K) && smallm1_suits(N, K)) return 0;      // taken at any alignment
     Pad32Plan pl;
-    if (pad32_plan(M, N, K, transB, &pl)) upto(pl.total);
+    if (transB && pad32_plan(M, N, K, &pl)) upto(pl.total);
+    if (!transB && !smallm_applies(M, N, K) && !skinny32_applies(M, N, K)) {
+        const SplitPlan sp = split_choice(M, N, K, 1, false, SIZE_MAX);
+        if (sp.ks > 1) upto((size_t)sp.ks * M * N * sizeof(float));
+    }
     if (!transB && smallm_applies(M, N, K)) upto(gemm_smallm_workspace_bytes(M, N, K));
     if (!transB && skinny32_applies(M, N, K)) upto((size_t)skinny32_ksplit(N, K) * M * N * sizeof(float));
     const int ks = splitk32_ranges(M, N, K);
@@ -2855,6 +2833,8 @@ bool gemm_x3_suits(int kind, int M, int n, int K)
 {
     if (n % 64 != 0) return false;
     if (kind == 0) {
+        const SplitPlan s1 = split_choice(M, 3 * n, K, 1, false, 0), s3 = split_choice(M, n, K, 3, false, 0);
+        if (s1.tile || s3.tile) return s3.tile && (!s1.tile || s3.us <= 1.03 * s1.us);
         const int t1 = f32_tile(M, 3 * n, K, 1, true), t3 = f32_tile(M, n, K, 3, true);
         return f32_time_us(M, n, K, 3, t3, 1) <= 1.03 * f32_time_us(M, 3 * n, K, 1, t1, 1);
     }
@@ -2867,6 +2847,8 @@ hipError_t gemm_f32_x3(hipStream_t stream, const float* A, const float* const (&
 {
     GemmArgs g{A, B[0], C, M, n, K, K, ldb, 3 * n, 0, 0, n, 1.0f, 0.0f, 0, 0, nullptr, 0, 0.0f};
     set_b3(g, B);
+    const SplitPlan sp = force_tile == 0 ? split_choice(M, n, K, 3, false, 0) : SplitPlan{};
+    if (sp.tile) return run_split(g, sp, 3, stream, nullptr, false);
     return dispatch_gemm<float, float, false>(g, 3, stream, force_tile);
 }
 #endif
@@ -2891,18 +2873,26 @@ hipError_t gemm_f32(hipStream_t stream, const float* A, const float* B, float* C
     const bool smallm_fits = smallm_applies(M, N, K) && gemm_smallm_workspace_bytes(M, N, K) <= workspace_bytes;
     if (!Bpre && force_tile == 0 && smallm_fits && !transB && batch == 1)
         return launch_smallm<false>(g, stream, (float*)workspace);
-    // Bpre: B already packed by gemm_f32_pack_b (B itself is then not read); such a call always takes the padded shapes
+    // Bpre: B already packed by gemm_f32_pack_b (B itself is then not read)
     Pad32Plan pl;
-    if (Bpre && !transB && batch == 1 && smallm_fits && aligned16(Bpre) && pad32_layout(M, N, K, 0, &pl)) {
+    if (Bpre && !(batch == 1 && aligned16(Bpre) && pad32_layout(M, N, K, transB, &pl))) return hipErrorInvalidValue;
+    if (Bpre && !transB) {
         GemmArgs gs = g;
         gs.B = Bpre; gs.ldb = pl.Np;                 // the padded rows; only the first K of them are read
-        return launch_smallm<false>(gs, stream, (float*)workspace);
+        if (smallm_fits) return launch_smallm<false>(gs, stream, (float*)workspace);
+        const SplitPlan sp = split_choice(M, N, K, 1, false, workspace_bytes);
+        if (sp.tile) return run_split(gs, sp, 1, stream, workspace, false);
     }
-    if (Bpre && !(batch == 1 && aligned16(Bpre) && pad32_layout(M, N, K, transB, &pl) &&
-                  (pl.Kp == K ? aligned16(A) : (workspace && aligned16(workspace) && pl.b_off <= workspace_bytes))))
-        return hipErrorInvalidValue;
-    if (Bpre || (force_tile == 0 && workspace && batch == 1 && aligned16(workspace) && pad32_plan(M, N, K, transB, &pl) && pl.total <= workspace_bytes &&
-                 (pl.Kp != K || aligned16(A)))) {
+    if (Bpre && !(pl.Kp == K ? aligned16(A) : (workspace && aligned16(workspace) && pl.b_off <= workspace_bytes))) return hipErrorInvalidValue;
+    if (!Bpre && force_tile == 0 && !transB) {
+        // (M <= 32 on whole slabs: bound by the stream of B, which the skinny kernel below keeps fuller)
+        int ks;
+        const bool skinny = batch == 1 && workspace && skinny32_applies(M, N, K) && aligned16(A) && aligned16(B) && skinny32_plan(N, K, &ks) > 0 &&
+                            (size_t)ks * M * N * sizeof(float) <= workspace_bytes;
+        const SplitPlan sp = skinny ? SplitPlan{} : split_choice(M, N, K, batch, false, workspace_bytes);
+        if (sp.tile) return run_split(g, sp, batch, stream, workspace, false);
+    }
+    if (Bpre || (transB && force_tile == 0 && workspace && batch == 1 && aligned16(workspace) && pad32_plan(M, N, K, &pl) && pl.total <= workspace_bytes)) {
         unsigned char* w = (unsigned char*)workspace;
         const float* Ap = A;
         if (pl.Kp != K) {
@@ -2911,7 +2901,7 @@ hipError_t gemm_f32(hipStream_t stream, const float* A, const float* B, float* C
         }
         const void* Bp = Bpre;
         if (!Bpre) {
-            if (hipError_t e = transB ? pad_rows(stream, B, w + pl.b_off, N, K, N, pl.Kp, 4) : pad_rows(stream, B, w + pl.b_off, K, N, pl.Kp, pl.Np, 4)) return e;
+            if (hipError_t e = pad_rows(stream, B, w + pl.b_off, N, K, N, pl.Kp, 4)) return e;
             Bp = w + pl.b_off;
         }
         GemmArgs gp{Ap, Bp, C, M, pl.Np, pl.Kp, pl.Kp, transB ? pl.Kp : pl.Np, N, 0, 0, 0, alpha, beta, 0, 0, bias, act, act_param};
@@ -2961,6 +2951,10 @@ hipError_t gemm_f32_f16weight(hipStream_t stream, const float* A, const uint16_t
     if (!workspace) workspace_bytes = 0;
     if (force_tile == 0 && smallm_applies(M, N, K) && gemm_smallm_workspace_bytes(M, N, K) <= workspace_bytes)
         return launch_smallm<true>(g, stream, (float*)workspace);
+    if (force_tile == 0) {
+        const SplitPlan sp = split_choice(M, N, K, 1, true, workspace_bytes);
+        if (sp.tile) return run_split(g, sp, 1, stream, workspace, true);
+    }
     // rows of A in 16-byte steps, rows of the fp16 B in 8-byte steps
     const bool vec = aligned16(A) && K % 4 == 0 && (((uintptr_t)B) & 7u) == 0 && N % 4 == 0;
     auto tiles = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
