@@ -32,12 +32,15 @@ struct GemmArgs {
     // many columns (fewer than N, the columns past them are padding of B that is computed and dropped) and ldc is any element
     // count, so a row of C may start off a 16-byte boundary
     int c_cols = 0;
+    // gemm_split_kernel only.  > 0: the batches are ranges of one K this long; all but the last hold K elements
+    // (here it fills the block to eight bytes: one more word moves the grid's size, which every kernel reads first, to a third cache line of
+    // the kernel arguments, 0.2 us a launch)
+    int k_total = 0;
     // three products with one A in one launch (three batches): their Bs lie anywhere, B at B, B + sB and B + 2 sB + sB2.  (A stride and not
     // two pointers: choosing one by branches in front of the first load cost every kernel 0.1 - 0.3 us, 9 % of a 1 x 256 x 101 product)
     long long sB2 = 0;
-    // gemm_split_kernel only.  > 0: the batches are ranges of one K this long; all but the last hold K elements
-    int k_total = 0;
 };
+static_assert(sizeof(GemmArgs) == 0x78, "the hidden arguments follow in the second cache line");
 
 // B of batch bz, in units of B's elements of EB bytes
 template <int EB>
