@@ -822,8 +822,8 @@ static hipError_t launch_gemm_dl(GemmArgs g, int batch, hipStream_t stream)
 
 // ---------------------------------------------------------------------------------------------
 // 256 x 256 x 64 direct-to-LDS kernel for 16-bit inputs on v_mfma_f32_16x16x32 (the form the large exact-fit problems take:
-// N a multiple of the tile width, K % 64 == 0, B stored [K,N]; M may be ragged: the rows of A past M are clamped loads of row
-// M - 1 whose products are never stored).  Same tile, loads and LDS layout as gemm_dl_kernel<.., 256>; what
+// K % 64 == 0, B stored [K,N]; M and N may be ragged, N in whole 16-byte chunks: the rows of A past M and the chunks of B past N are
+// clamped loads of the last ones, whose products are never stored).  Same tile, loads and LDS layout as gemm_dl_kernel<.., 256>; what
 // differs is the matrix instruction.  Under load this part runs at the clock its power limit allows, and per multiply-add the
 // 16 x 16 x 32 instruction moves 20 % fewer register bytes than 32 x 32 x 16 (half the accumulator traffic, twice the
 // operand traffic): with random fp16 operands and nothing else running it sustains 1.71 PFLOP/s against 1.52, and this kernel
@@ -859,7 +859,9 @@ template <> struct Mma16<bf16_t> {
 #define DL16_HALF_STAGES 4
 // NTS: C is written with non-temporal stores (a compile-time switch: as a run-time branch the two stores are merged by the compiler
 // and the hint is lost).
-template <typename T, typename OutT, int TJ = 4, bool HALF = false, bool NTS = false, int HS = DL16_HALF_STAGES>
+// CUT: N is not a multiple of the tile width (an instance of its own: with the clamps and tests in all of them whole tiles took longer,
+// 8192 x 768 x 768 17.2 -> 17.5 us).
+template <typename T, typename OutT, int TJ = 4, bool HALF = false, bool NTS = false, int HS = DL16_HALF_STAGES, bool CUT = false>
 __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
 {
     static_assert(!HALF || TJ == 2, "the 128-row tile is built for 128 columns");
@@ -894,7 +896,8 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
     auto b_swz = [](int row) -> int { return ((row & 3) << 2) | (((row >> 3) & 1) << 1); };
     const int wave_s = __builtin_amdgcn_readfirstlane(wave);
     const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)smem);
-    // A rows past M (the last tile row of a ragged M) are clamped to row M - 1: valid loads whose products are never stored
+    // A rows past M (the last tile row of a ragged M) are clamped to row M - 1 and B chunks past N to the last one: valid loads whose
+    // products are never stored
     uint32_t a_lane_off[LA], b_lane_off[LB];
 #pragma unroll
     for (int i = 0; i < LA; i++) {
@@ -907,6 +910,7 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
         const int rb = lane / LPR, pos_b = lane % LPR;
         int chunk = pos_b ^ b_swz(RPL * (LB * wave + i) + rb);
         if (chunk >= BCH) chunk -= LPR - BCH >= BCH ? BCH : LPR - BCH;    // a valid chunk again (its LDS position is never read)
+        if constexpr (CUT) chunk = min(chunk, (g.N - n0) / E - 1);
         b_lane_off[i] = (uint32_t)(rb * g.ldb + chunk * E) * (uint32_t)EB;
     }
     const unsigned char* a_base = A + (long long)m0 * g.lda * EB;
@@ -1095,10 +1099,10 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
 #pragma unroll
         for (int j = 0; j < TJ; j++) {
             bias4[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (g.bias) bias4[j] = *(const f32x4*)(g.bias + n0 + wn * WTN + 16 * j + 4 * g4);
+            if (g.bias) bias4[j] = *(const f32x4*)(g.bias + (CUT ? min(n0 + wn * WTN + 16 * j + 4 * g4, g.N - 4) : n0 + wn * WTN + 16 * j + 4 * g4));
         }
         unsigned char* Cw = (unsigned char*)g.C + (bz * g.sC + (long long)(m0 + wm * WTM) * g.ldc + n0 + wn * WTN) * OB;
-        const bool whole_tile = __builtin_amdgcn_readfirstlane(m0 + (HALF ? 128 : 256) <= g.M && g.c_cols == 0);
+        const bool whole_tile = __builtin_amdgcn_readfirstlane(m0 + BM <= g.M && (!CUT || n0 + BN <= g.N) && g.c_cols == 0);
         static_for<0, TI, IPR>([&](auto ip_const) {
             constexpr int ip = decltype(ip_const)::value;
 #pragma unroll
@@ -1129,8 +1133,8 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
                     }
                 }
             }
-            // a workgroup whose tile lies inside the matrix (every one but the last tile row of a ragged M) stores without a
-            // test per row: with the test the compiler serialises LDS read and store of every chunk, which costs the short-K
+            // a workgroup whose tile lies inside the matrix (every one but the last tile row or column of a ragged M or N) stores without a
+            // test per chunk: with the test the compiler serialises LDS read and store of every chunk, which costs the short-K
             // shapes 3-5 %
             if (whole_tile) {
 #pragma unroll
@@ -1168,19 +1172,19 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
                                     else ((out_t*)dst)[e] = v[e];
                                 }
                         }
-                    } else *dst = v;
+                    } else if (!CUT || n0 + wn * WTN + c * (16 / OB) < g.N) *dst = v;
                 }
             }
         });
     }
 }
 
-template <typename T, typename OutT, int TJ = 4, bool HALF = false, int HS = DL16_HALF_STAGES>
-static hipError_t launch_gemm_dl16(GemmArgs g, int batch, hipStream_t stream)
+template <typename T, typename OutT, int TJ, bool HALF, int HS, bool CUT>
+static hipError_t launch_dl16_as(GemmArgs g, int batch, hipStream_t stream)
 {
     constexpr int smem = HALF ? HS * (128 * 128 + 64 * 256) : 2 * (256 * 128 + 128 * 256);
-    g.tiles_m = (g.M + (HALF ? 127 : 255)) / (HALF ? 128 : 256);      // the last tile row may be partial
-    g.tiles_n = g.N / (64 * TJ);
+    g.tiles_m = (g.M + (HALF ? 127 : 255)) / (HALF ? 128 : 256);      // the last tile row and column may be partial
+    g.tiles_n = (g.N + 64 * TJ - 1) / (64 * TJ);
     const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), 1, (unsigned)batch);
     // Non-temporal stores of C when A, B and C together exceed the 256 MB last-level cache: C then no longer displaces the operand
     // tiles that later workgroups re-read (alternated in one process: fp16 8192^3 1336 -> 1408 TFLOP/s, bf16 1397 -> 1464,
@@ -1190,18 +1194,23 @@ static hipError_t launch_gemm_dl16(GemmArgs g, int batch, hipStream_t stream)
     const bool nts = footprint > (240LL << 20);
     if constexpr (!HALF) {
         if (nts) {
-            auto kern = gemm_dl16_kernel<T, OutT, TJ, false, true>;
+            auto kern = gemm_dl16_kernel<T, OutT, TJ, false, true, HS, CUT>;
             static unsigned long long attr_done_nt = 0;
             if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done_nt)) return e;
             hipLaunchKernelGGL(kern, grid, dim3(512), smem, stream, g);
             return hipGetLastError();
         }
     }
-    auto kern = gemm_dl16_kernel<T, OutT, TJ, HALF, false, HS>;
+    auto kern = gemm_dl16_kernel<T, OutT, TJ, HALF, false, HS, CUT>;
     static unsigned long long attr_done = 0;
     if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done)) return e;
     hipLaunchKernelGGL(kern, grid, dim3(512), smem, stream, g);
     return hipGetLastError();
+}
+template <typename T, typename OutT, int TJ = 4, bool HALF = false, int HS = DL16_HALF_STAGES>
+static hipError_t launch_gemm_dl16(const GemmArgs& g, int batch, hipStream_t stream)
+{
+    return g.N % (64 * TJ) == 0 ? launch_dl16_as<T, OutT, TJ, HALF, HS, false>(g, batch, stream) : launch_dl16_as<T, OutT, TJ, HALF, HS, true>(g, batch, stream);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2644,41 +2653,49 @@ template <typename OutT>
 static bool dl16_applies(const GemmArgs& g)
 {
     const int OB = Elem<OutT>::BYTES;
-    return aligned16(g.A) && aligned16(g.B) && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.sA % 8 == 0 && g.sB % 8 == 0 && g.sB2 % 8 == 0 &&
+    return g.N % 8 == 0 && aligned16(g.A) && aligned16(g.B) && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.sA % 8 == 0 && g.sB % 8 == 0 && g.sB2 % 8 == 0 &&
            g.lda < (1 << 21) && g.ldb < (1 << 21) &&
            aligned16(g.C) && ((long long)g.ldc * OB) % 16 == 0 && (g.sC * OB) % 16 == 0 && (g.bias == nullptr || aligned16(g.bias)) &&
            g.alpha == 1.0f && g.beta == 0.0f;
 }
 
-// Tile width (in 64-column units: 4, 3 or 2) of the 16 x 16 x 32 kernel for a 16-bit problem with K % 64 == 0 (any M), or 0
-// when none of the widths divides N or the 128 x 128 / 64 x 64 tiles of the 32 x 32 x 16 kernel are expected to finish earlier.
+// Tile width (in 64-column units: 4, 3 or 2) of the 16 x 16 x 32 kernel for a 16-bit problem with K % 64 == 0 (any M and N), or 0
+// when the 128 x 128 / 64 x 64 tiles of the 32 x 32 x 16 kernel are expected to finish earlier.
 // Every candidate is scored as (how evenly its tiles load the 256 CUs) x (its rate per flop relative to the 256 x 256 tile): a
 // narrower tile moves more A bytes per flop (and the 256 x 128 one wastes half of its B loads); the 128 x 128 tile runs at about
 // 0.55 and the 64 x 64 tile at about 0.45 of the 256 x 256 rate (2048^3: 128 tiles of 256 x 128 take 36 us, 256 tiles of 128 x 128 29 us).
+// A last tile column that N does not fill costs only its padding: before, such an N went to the next width that divides it or to the
+// 32 x 32 x 16 kernel with its checks on every K-tile (bf16, us before / now: 1000 x 11008 x 4096 94 / 86, 917 x 15416 x 4416 156 / 113,
+// 1158 x 3008 x 1088 20.2 / 13.9, 5236 x 6464 x 6400 469 / 397; 44 drawn sizes 1.07x in the geometric mean).
 #define DL16_HALF_EFF 0.7
-#define DL16_HALF2_EFF 0.82
+// The 128 x 128 tile on the two-stage ring runs two workgroups per CU, so that one's first loads and stores run under the other's products:
+// the shorter K, the more that counts (rate against the 256 x 256 tile's, us before / with the entry for that K: 7002 x 8112 x 64 44.8 / 33.0,
+// 8192 x 14592 x 128 83 / 75, 7002 x 3072 x 256 24.7 / 22.6, 4096 x 10112 x 576, on 256 x 256 tiles, 58.7 / 56.2; at 0.95 8192 x 14592 x 576
+// goes 182 -> 203)
+static double dl16_half2_eff(int K) { return K <= 128 ? 1.2 : K <= 384 ? 0.95 : K <= 640 ? 0.9 : 0.82; }
 static int dl16_width(int M, int N, int K, int batch, double* score_out)
 {
     if (score_out) *score_out = 0.0;
     if (K % 64 != 0) return 0;
-    // M may be ragged (the last tile row is partial: clamped loads, guarded stores); the rows a tile height pads count as waste
+    // M and N may be ragged (partial last tiles: clamped loads, guarded stores); the rows and columns a tile pads count as waste
     const long long tm256 = (M + 255) / 256, tm128 = (M + 127) / 128, tm64 = (M + 63) / 64;
-    const double use256 = (double)M / (double)(tm256 * 256), use128 = (double)M / (double)(tm128 * 128), use64 = (double)M / (double)(tm64 * 64);
+    const double use256 = (double)M / (double)(tm256 * 256), rows128 = (double)M / (double)(tm128 * 128), rows64 = (double)M / (double)(tm64 * 64);
+    const long long tn128 = (N + 127) / 128, tn64 = (N + 63) / 64;
+    const double use128 = rows128 * (double)N / (double)(tn128 * 128), use64 = rows64 * (double)N / (double)(tn64 * 64);
     const int widths[3] = {4, 3, 2};
     const double eff[3] = {1.0, 0.94, 0.8};
     int best = 0;
     double best_score = 0.0;
     for (int i = 0; i < 3; i++) {
         const int bn = 64 * widths[i];
-        if (N % bn != 0) continue;
-        const long long t = tm256 * (N / bn) * batch;
-        const double score = cu_fill(t) * eff[i] * use256;
+        const long long tn = (N + bn - 1) / bn, t = tm256 * tn * batch;
+        const double score = cu_fill(t) * eff[i] * use256 * ((double)N / (double)(tn * bn));
         if (score > best_score) { best_score = score; best = widths[i]; }
     }
-    const long long t128 = tm128 * ((N + 127) / 128) * batch;
-    const long long t64 = tm64 * ((N + 63) / 64) * batch;
-    // the 128 x 128 tile of this kernel (code 1): whole column tiles only
-    if (N % 128 == 0 && DL16_HALF_EFF * cu_fill(t128) * use128 > best_score) { best_score = DL16_HALF_EFF * cu_fill(t128) * use128; best = 1; }
+    const long long t128 = tm128 * tn128 * batch;
+    const long long t64 = tm64 * tn64 * batch;
+    // the 128 x 128 tile of this kernel (code 1)
+    if (DL16_HALF_EFF * cu_fill(t128) * use128 > best_score) { best_score = DL16_HALF_EFF * cu_fill(t128) * use128; best = 1; }
     // the same tile on a two-stage ring, two workgroups per CU (code 5): with more tiles than CUs and a K of at most 6144 one
     // workgroup's first loads, barrier waits and store phase run under the other's MFMAs (8192 x 768 x 3072 50.4 -> 41.8 us,
     // 512 x 12288 x 4096 64.8 -> 54.4 us, 384 x 13824 x 5120 79.8 -> 65.8 us); one tile per CU (2048^3 20.7 -> 27.6 us) and long K
@@ -2686,12 +2703,12 @@ static int dl16_width(int M, int N, int K, int batch, double* score_out)
     // (beyond one round of 512 resident workgroups only when the last round is nearly full: a workgroup alone on its CU has nothing
     // to hide the two-stage ring's waits behind -- 3000 x 4096 x 4096, 768 tiles: 83 -> 106 us)
     const double fill2 = (double)t128 / (double)(((t128 + 511) / 512) * 512);
-    if (N % 128 == 0 && t128 > 256 && K <= 6144 && (t128 <= 512 || fill2 >= 0.85)) {
-        const double s2 = DL16_HALF2_EFF * (t128 <= 512 ? cu_fill(t128) : fill2) * use128;
+    if (t128 > 256 && K <= 6144 && (t128 <= 512 || fill2 >= 0.85)) {
+        const double s2 = dl16_half2_eff(K) * (t128 <= 512 ? cu_fill(t128) : fill2) * use128;
         if (s2 > best_score) { best_score = s2; best = 5; }
     }
     const double s128 = 0.55 * cu_fill(t128) * use128, s64 = 0.45 * cu_fill(t64) * use64;
-    if (score_out) *score_out = best_score > s128 ? (best_score > s64 ? best_score : s64) : (s128 > s64 ? s128 : s64);
+    if (score_out) *score_out = best_score > s128 ? (best_score > s64 ? std::min(best_score, 1.0) : s64) : (s128 > s64 ? s128 : s64);
     if (s128 > best_score || s64 > best_score) return 0;
     return best;
 }
