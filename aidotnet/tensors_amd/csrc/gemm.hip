@@ -1450,8 +1450,8 @@ static hipError_t launch_any16(const GemmArgs& g, hipStream_t stream, int ks = 1
 }
 
 // ---------------------------------------------------------------------------------------------
-// Skinny-M path (decode projections): M <= 32, 16-bit, B stored [K,N], N % 128 == 0, K % 64 == 0.
-// HBM-bound: B (K x N) is read exactly once.  grid = (N / 128, KS), about one workgroup per CU: each workgroup streams a
+// Skinny-M path (decode projections): M <= 32, 16-bit, B stored [K,N], N % 8 == 0, K % 64 == 0.
+// HBM-bound: B (K x N) is read exactly once.  grid = (ceil(N / 128), KS), about one workgroup per CU: each workgroup streams a
 // 128-column slab of B over its K range with the direct global->LDS load through a ring of NS 20 KB stages, filled NS - 1
 // K-tiles ahead -- seven stages and one workgroup per CU (120 KB in flight per CU: one memory round trip covers a whole K range of
 // up to six tiles, where a two-stage ring paid one round trip per tile), or three stages and two workgroups per CU for wide
@@ -1483,7 +1483,7 @@ __global__ __launch_bounds__(256, NS <= 3 ? 2 : 1) void gemm_skinny_kernel(const
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         int row = 4 * (wave * 4 + i) + (lane >> 4), pos = lane & 15;
-        pb[i] = B + (long long)(kbeg + row) * g.ldb + n0 + (pos ^ ((row & 3) << 2)) * 8;
+        pb[i] = B + (long long)(kbeg + row) * g.ldb + min(n0 + (pos ^ ((row & 3) << 2)) * 8, g.N - 8);      // (past N: the last chunk, never stored)
     }
     const raw_t* pa;
     {
@@ -1548,7 +1548,7 @@ __global__ __launch_bounds__(256, NS <= 3 ? 2 : 1) void gemm_skinny_kernel(const
 #pragma unroll
     for (int r = 0; r < 16; r++) {
         const int row = acc_row(r, h);
-        if (row < g.M) ws[((long long)ks * g.M + row) * g.N + col] = acc[r];
+        if (row < g.M && col < g.N) ws[((long long)ks * g.M + row) * g.N + col] = acc[r];
     }
 }
 
@@ -1609,7 +1609,19 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_kernel(const float* __
     }
 }
 
-static bool skinny_applies(int M, int N, int K) { return M <= 32 && N % 128 == 0 && K % 64 == 0 && N >= 128; }
+// The stream and its summing pass are two launches: from K = 1024 on (768 for up to eight rows) they are faster than the one launch of the
+// tiled kernels (us, tiled / here: 8 x 512 x 384 5.0 / 6.7, 8 x 512 x 768 6.8 / 6.6, 32 x 4096 x 768 7.0 / 7.9, 32 x 4096 x 1024 8.2 / 8.3, 8 x 1024 x
+// 1536 10.3 / 8.0).  With a ragged last slab (clamped loads) they are taken where the tiled kernels take longer than the 15 us that two
+// launches cost their caller anyway (3 x 192 x 6400 32.2 / 6.9, 5 x 5680 x 6272 52 / 20, 17 x 6592 x 2240 21.2 / 11.2, 2 x 4104 x 1536 15.1 / 8.9); the rows of
+// such a B share cache lines between slabs, which a streaming load fetches twice, so that more than 256 tiles of 64 columns win over it
+// (32 x 12296 x 1536 16.6 / 18.5, 32 x 40008 x 1024 20.7 / 33.0).
+static bool skinny_applies(int M, int N, int K)
+{
+    if (M > 32 || N % 8 != 0 || K % 64 != 0 || N < 128) return false;
+    if (N % 128 == 0) return K >= (M <= 8 ? 768 : 1024);
+    return K >= (N <= 4096 ? 2560 : M <= 8 || N <= 8192 ? 1536 : 2048) && N <= 16384;
+}
+static int skinny_slabs(int N) { return (N + 127) / 128; }
 
 // How evenly `tiles` workgroups load the 256 CUs: a CU works through its tiles at about the same rate whether it holds one or
 // several at a time, so what counts is the largest number of tiles any CU gets.
@@ -1638,7 +1650,7 @@ static int skinny_plan(int slabs, int tiles, int* ks_out, int per_cu = 1, double
     if (score_out) *score_out = best;
     return best_kper;
 }
-static int skinny_ksplit(int N, int K) { int ks; skinny_plan(N / 128, K / 64, &ks, N / 128 > 64 && K <= 4096 ? 2 : 1); return ks; }
+static int skinny_ksplit(int N, int K) { int ks; skinny_plan(skinny_slabs(N), K / 64, &ks, skinny_slabs(N) > 64 && K <= 4096 ? 2 : 1); return ks; }
 
 // Split-K for 16-bit problems whose 128 x 128 tiles fill less than half the chip over a long K (M <= 512 against a 4096-wide
 // weight): K ranges run as the batch dimension of the 128 x 128 kernel into fp32 partials, summed in range order by
@@ -2011,18 +2023,19 @@ static hipError_t launch_skinny(const GemmArgs& g, hipStream_t stream, float* ws
     // more than 64 column slabs over a K of at most 4096 (16 x 28672 x 8192 went 77 -> 88 us): the three-stage form, two workgroups per CU (a workgroup's first memory round trip and its last
     // tiles run under the other's stream: 32 x 11008 x 4096 24.5 -> 22.9 us, 32 x 128256 x 4096 193 -> 187 us); with fewer slabs the
     // K ranges of that plan get too short (32 x 4096 x 4096 12.3 -> 14.1 us) and the seven-stage form, one per CU, stays
-    const bool three = g.N / 128 > 64 && g.K <= 4096;
-    const int kper = 64 * skinny_plan(g.N / 128, g.K / 64, &ks, three ? 2 : 1);
+    const int slabs = skinny_slabs(g.N);
+    const bool three = slabs > 64 && g.K <= 4096;
+    const int kper = 64 * skinny_plan(slabs, g.K / 64, &ks, three ? 2 : 1);
     if (three) {
         constexpr int smem = 3 * (32 * 128 + 64 * 256);
         static unsigned long long attr_done3 = 0;
         if (hipError_t e0 = ensure_dynamic_smem((const void*)gemm_skinny_kernel<T, 3>, smem, &attr_done3)) return e0;
-            hipLaunchKernelGGL((gemm_skinny_kernel<T, 3>), dim3((unsigned)(g.N / 128), (unsigned)ks), dim3(256), smem, stream, g, ws, ks, kper);
+            hipLaunchKernelGGL((gemm_skinny_kernel<T, 3>), dim3((unsigned)slabs, (unsigned)ks), dim3(256), smem, stream, g, ws, ks, kper);
     } else {
         constexpr int smem = SKINNY_STAGES * (32 * 128 + 64 * 256);
         static unsigned long long attr_done = 0;
         if (hipError_t e0 = ensure_dynamic_smem((const void*)gemm_skinny_kernel<T, SKINNY_STAGES>, smem, &attr_done)) return e0;
-        hipLaunchKernelGGL((gemm_skinny_kernel<T, SKINNY_STAGES>), dim3((unsigned)(g.N / 128), (unsigned)ks), dim3(256), smem, stream, g, ws, ks, kper);
+        hipLaunchKernelGGL((gemm_skinny_kernel<T, SKINNY_STAGES>), dim3((unsigned)slabs, (unsigned)ks), dim3(256), smem, stream, g, ws, ks, kper);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
