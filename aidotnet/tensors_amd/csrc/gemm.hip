@@ -916,7 +916,8 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
     const unsigned char* a_base = A + (long long)m0 * g.lda * EB;
     const unsigned char* b_base = B + ((long long)(RPL * LB * wave_s) * g.ldb + n0) * EB;
     const long long b_step = (long long)RPL * g.ldb * EB;
-    const int KT = g.K / BK;
+    // (the instances that take K ranges: fp32 partials)
+    const int KT = (OB == 4 && (HALF || TJ == 4) && g.k_total ? min(g.K, g.k_total - (int)bz * g.K) : g.K) / BK;
     auto issue_loads = [&](int kt, int stage) {
         const uint32_t as = lds0 + stage * STAGE + wave_s * (LA * 1024);
         const uint32_t bs = lds0 + stage * STAGE + ABYTES + wave_s * (LB * 1024);
@@ -1654,29 +1655,45 @@ static int skinny_ksplit(int N, int K) { int ks; skinny_plan(skinny_slabs(N), K 
 
 // Split-K for 16-bit problems whose 128 x 128 tiles fill less than half the chip over a long K (M <= 512 against a 4096-wide
 // weight): K ranges run as the batch dimension of the 128 x 128 kernel into fp32 partials, summed in range order by
-// skinny_reduce_kernel (deterministic; bias and activation there).  Returns the number of ranges, 0 = not worth it.
+// skinny_reduce_kernel (deterministic; bias and activation there).  Returns the number of ranges, 0 = not worth it.  Ranges are whole
+// K-tiles and the last may be shorter, so that any K takes as many as suit the tiles (with equal ranges K = 193 x 64 had none: 233 x 528 x
+// 12352 100 us / 18, 332 x 2936 x 13888 114 / 48, 129 x 256 x 3904 21 / 12, 2838 x 512 x 4416 39 / 27; 40 drawn sizes of 33 - 512 rows 1.5x).
 static int dl16_width(int M, int N, int K, int batch, double* score_out = nullptr);
 // Share of a split-K product's time that is the product: the fp32 partials are written and read once per range, 8 bytes per output
 // element and range at about 4 TB/s, against 2 K flops per element at about 1.4 PFLOP/s (512 x 8192 x 8192 in four ranges: 49 us of
 // product, 33 us of partials)
 static double splitk16_partials_factor(int K, int ks) { return 1.0 / (1.0 + 1000.0 * ks / K); }
-static int splitk16_ranges(int M, int N, int K, int* big_tile = nullptr)
+static int splitk16_ranges(int M, int N, int K, int* kper, int* big_tile = nullptr)
 {
     if (big_tile) *big_tile = 0;
-    if (N % 128 != 0 || K % 64 != 0) return 0;
+    *kper = K;
+    if (N % 8 != 0 || N < 128 || K % 64 != 0) return 0;
+    const int kt = K / 64;
+    // (the last range may be shorter by up to a K-tile per range)
     auto ranges = [&](long long t, int min_k) {
         int ks = (int)(256 / t);
         if (ks > 16) ks = 16;
-        while (ks > 1 && (K % (ks * 64) != 0 || K / ks < min_k)) ks--;
-        return ks;
+        while (ks > 1 && K / ks < min_k) ks--;
+        const int per = (kt + ks - 1) / ks;
+        *kper = 64 * per;
+        return (kt + per - 1) / per;
     };
-    // (a ragged M: the last tile row is partial)
-    const long long t = (long long)((M + 127) / 128) * (N / 128);
+    // (a ragged M or N: the last tile row or column is partial)
+    const long long t = (long long)((M + 127) / 128) * ((N + 127) / 128);
     if (t <= 128) {                           // up to half a chip of 128 x 128 tiles
-        const int ks = ranges(t, 512);
-        // the partials cost 8 bytes of traffic per output element and range; the product must be worth it
-        // (a ragged M only from K = 2048 on: below, the second launch costs what the ranges save -- 1000 x 1024 x 1024 8 -> 15 us)
-        return ks >= 2 && (long long)K >= (M % 128 == 0 ? 1024 : 2048) ? ks : 0;
+        // (below K = 2048 the second launch costs what the ranges save: 1000 x 1024 x 1024 8 -> 15 us, 512 x 1024 x 1344 8.9 -> 14.0, 768 x 1024 x
+        // 1856 17.4 -> 17.1; 128 x 136 x 2112, whose one launch is shorter than what two cost the caller)
+        if (K < (N % 128 == 0 ? 2048 : 2560)) return 0;
+        // estimates in us: 0.5 a K-tile and 3 a launch, 0.5 more for the sums, the partials written and read at 3.5 TB/s (2048 x 1024 x 2112 20.2
+        // in one, 23.3 in two; 1340 x 256 x 6144 16.6 in eight, 17.9 in eleven; 1024 x 1024 x 2112 17.4 in three, 18.4 in four)
+        int best = 1;
+        double best_us = 0.5 * kt + 3.0;
+        for (int ks = 2; ks <= 16 && ks * t <= 256 && K / ks >= 512; ks++) {
+            const int per = (kt + ks - 1) / ks, n = (kt + per - 1) / per;
+            const double us = 0.5 * per + 6.5 + (double)n * M * N * 8.0 / 3.5e6;
+            if (us < best_us) { best_us = us; best = n; *kper = 64 * per; }
+        }
+        return best >= 2 ? best : 0;
     }
     // Larger problems whose 256 x 256 tiles still fill at most half the chip over a long K (M about 1000 against an 8192-wide
     // weight with K = 28672): narrower tiles would fill the chip but move twice the operand bytes per flop through the L2, which
@@ -1709,8 +1726,8 @@ static int msplit16_rows(int M, int N, int K)
     auto score = [&](int m) {
         double single = 0.0;
         dl16_width(m, N, K, 1, &single);
-        int big = 0;
-        const int ks = splitk16_ranges(m, N, K, &big);
+        int big = 0, kper;
+        const int ks = splitk16_ranges(m, N, K, &kper, &big);
         if (ks && big) {
             const long long t256 = (long long)((m + 255) / 256) * (N / 256);
             const double split = cu_fill(t256 * ks) * ((double)m / (double)(((m + 255) / 256) * 256)) * splitk16_partials_factor(K, ks);
@@ -1741,8 +1758,8 @@ static size_t gemm_16_inner_workspace_bytes(int M, int N, int K)
         if (a > need) need = a;
         if (b > need) need = b;
     }
-    int big;
-    const int ks = splitk16_ranges(M, N, K, &big);
+    int big, kper;
+    const int ks = splitk16_ranges(M, N, K, &kper, &big);
     const size_t split = ks ? (size_t)ks * M * N * sizeof(float) : 0;
     return split > need ? split : need;
 }
@@ -3078,12 +3095,12 @@ static hipError_t gemm_16_typed(hipStream_t stream, const uint16_t* A, const uin
         }
     }
     if (force_tile == 0 && workspace) {
-        int big = 0;
-        const int ks = splitk16_ranges(M, N, K, &big);
+        int big = 0, kper;
+        const int ks = splitk16_ranges(M, N, K, &kper, &big);
         if (ks && (size_t)ks * M * N * sizeof(float) <= workspace_bytes) {
             GemmArgs gp = g;
-            gp.C = workspace; gp.K = K / ks; gp.ldc = N;
-            gp.sA = K / ks; gp.sB = (long long)(K / ks) * N; gp.sC = (long long)M * N;
+            gp.C = workspace; gp.K = kper; gp.k_total = K; gp.ldc = N;
+            gp.sA = kper; gp.sB = (long long)kper * N; gp.sC = (long long)M * N;
             gp.bias = nullptr; gp.act = 0;
             if (dl16_applies<float>(gp)) {
                 if (hipError_t e = big ? launch_gemm_dl16<T, float, 4>(gp, ks, stream) : launch_gemm_dl16<T, float, 2, true>(gp, ks, stream)) return e;

@@ -32,7 +32,7 @@ struct GemmArgs {
     // many columns (fewer than N, the columns past them are padding of B that is computed and dropped) and ldc is any element
     // count, so a row of C may start off a 16-byte boundary
     int c_cols = 0;
-    // gemm_split_kernel only.  > 0: the batches are ranges of one K this long; all but the last hold K elements
+    // gemm_split_kernel and the 16-bit K ranges.  > 0: the batches are ranges of one K this long; all but the last hold K elements
     // (here it fills the block to eight bytes: one more word moves the grid's size, which every kernel reads first, to a third cache line of
     // the kernel arguments, 0.2 us a launch)
     int k_total = 0;
