@@ -498,8 +498,10 @@ __device__ __forceinline__ void dma16_addr(const void* gptr, uint32_t lds_dst)
 // KSW = 2 (fp32, 64 x 64 tile, whole tiles): eight waves, two groups of four that take half of the k-steps of every K-tile each and are
 // summed through LDS at the end (group 0 + group 1, a fixed order).  With about one such tile per CU the four-wave form runs one wave
 // per SIMD, which has nothing to switch to while it issues loads or waits at the tile barrier (matrix pipe 69 % busy at 1024^3).
-template <typename T, typename OutT, bool EDGE = false, int TILE = 256, bool TRANSB = false, int KSW = 1>
-__global__ __launch_bounds__((TILE == 256 ? 512 : 256) * KSW, TILE == 256 ? 1 : 2) void gemm_dl_kernel(const GemmArgs g)
+// Args = GemmRopeArgs (16-bit output): the leading columns of C are rotated as they are stored (launch.hpp's RopeEpilogue).
+struct GemmRopeArgs : GemmArgs { RopeEpilogue rope; };
+template <typename T, typename OutT, bool EDGE = false, int TILE = 256, bool TRANSB = false, int KSW = 1, typename Args = GemmArgs>
+__global__ __launch_bounds__((TILE == 256 ? 512 : 256) * KSW, TILE == 256 ? 1 : 2) void gemm_dl_kernel(const Args g)
 {
     constexpr int E = Elem<T>::PER16, EB = Elem<T>::BYTES;
     static_assert(TILE == 256 || TILE == 128 || TILE == 64, "tile edge");
@@ -687,8 +689,32 @@ __global__ __launch_bounds__((TILE == 256 ? 512 : 256) * KSW, TILE == 256 ? 1 : 
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
     issue_loads(0, 0);
+    constexpr bool ROPE = std::is_same<Args, GemmRopeArgs>::value;
+    static_assert(!ROPE || (TM == 1 && TN == 1), "one block of C to a wave");
+    float turn_cos[ROPE ? 16 : 1], turn_sin[ROPE ? 16 : 1];      // (loaded here, they arrive with the first tile)
+    if constexpr (ROPE) {
+        const RopeEpilogue& rope = g.rope;
+        const int col = n0 + wn * WTN + l32, half = rope.head_dim >> 1;
+        const int pair = col < rope.cols ? (col % rope.head_dim) >> 1 : 0;
+        const long long first = (long long)rope.start_position * half + pair;
+        if (rope.seq_len == 1) {                                 // every row at one position, as in a decode step: without sixteen divisions, 0.7 us a launch
+            const float c = rope.cosc[first], s = rope.sinc[first];
+#pragma unroll
+            for (int r = 0; r < 16; r++) { turn_cos[r] = c; turn_sin[r] = s; }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {                       // (rows past the end repeat the last one)
+                const long long at = first + (long long)(min(m0 + wm * WTM + acc_row(r, h), g.M - 1) % rope.seq_len) * half;
+                turn_cos[r] = rope.cosc[at]; turn_sin[r] = rope.sinc[at];
+            }
+        }
+    }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
+    if constexpr (ROPE) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) asm volatile("" : "+v"(turn_cos[r]), "+v"(turn_sin[r]));
+    }
 
     // Software pipeline: the fragments of k-step s+1 are read from LDS before the MFMAs of step s are issued, so the
     // LDS latency runs under 8 MFMAs; the barrier that publishes tile kt+1 sits before the MFMAs of the last step, and the
@@ -786,6 +812,19 @@ __global__ __launch_bounds__((TILE == 256 ? 512 : 256) * KSW, TILE == 256 ? 1 : 
         for (int j = 0; j < TN; j++) {
             const int col = n0 + wn * WTN + j * 32 + l32;
             const bool col_ok = !EDGE || col < (g.c_cols > 0 ? g.c_cols : g.N);
+            if constexpr (ROPE) {
+                // the pair is rounded to the output type before it is rotated, as a product followed by the rotation kernel does it; its other
+                // half is in the neighbouring lane
+                const bool turn = col < g.rope.cols, odd = col & 1;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const float mine = Elem<OutT>::widen(Elem<OutT>::narrow(acc[i][j][r]));
+                    const float other = as_f32((uint32_t)__builtin_amdgcn_update_dpp(0, (int)as_u32(mine), 0xB1, 0xF, 0xF, true));      // quad_perm 1, 0, 3, 2
+                    float even_out, odd_out;
+                    rope_rotate(odd ? other : mine, odd ? mine : other, turn_cos[r], turn_sin[r], even_out, odd_out);
+                    acc[i][j][r] = turn ? (odd ? odd_out : even_out) : mine;
+                }
+            }
             if (fused) {                                  // bias and / or activation folded into the store
                 const float bias = (g.bias && col_ok) ? g.bias[col] : 0.0f;
 #pragma unroll
@@ -807,10 +846,10 @@ __global__ __launch_bounds__((TILE == 256 ? 512 : 256) * KSW, TILE == 256 ? 1 : 
         }
 }
 
-template <typename T, typename OutT, bool EDGE = false, int TILE = 256, bool TRANSB = false, int KSW = 1>
-static hipError_t launch_gemm_dl(GemmArgs g, int batch, hipStream_t stream)
+template <typename T, typename OutT, bool EDGE = false, int TILE = 256, bool TRANSB = false, int KSW = 1, typename Args = GemmArgs>
+static hipError_t launch_gemm_dl(Args g, int batch, hipStream_t stream)
 {
-    auto kern = gemm_dl_kernel<T, OutT, EDGE, TILE, TRANSB, KSW>;
+    auto kern = gemm_dl_kernel<T, OutT, EDGE, TILE, TRANSB, KSW, Args>;
     constexpr int smem = 2 * (TILE * 128 + 128 * TILE);         // A tile + B tile (128 bytes of K each), two stages
     static unsigned long long attr_done = 0;
     if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done)) return e;
@@ -3129,18 +3168,28 @@ hipError_t gemm_16_rope_f16(hipStream_t stream, const uint16_t* A, const uint16_
                             void* workspace, size_t workspace_bytes, const RopeEpilogue& rope);
 hipError_t gemm_16_rope_bf16(hipStream_t stream, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int force_tile,
                              void* workspace, size_t workspace_bytes, const RopeEpilogue& rope);
+// Few rows over a K too short for skinny_applies: gemm_16_typed goes to the 64 x 64 direct-to-LDS tile with edge handling (M <= 32 leaves half
+// of its rows empty, three quarters of every larger tile's; N up to 16384 is at most one such tile per CU, so no larger one loads the
+// chip better), and the rotation rides on its stores: same sums, one launch (us, product and rotation in two launches / here / on the stream's
+// summing pass: 1 x 4096 x 512 7.5 / 6.6 / 6.8, 32 x 512 x 384 7.2 / 6.1 / 7.2, 32 x 12288 x 768 12.6 / 11.0 / 11.7; only towards the
+// upper end of that K the stream would be ahead: 1 x 2048 x 704 8.4 / 7.4 / 6.9, 32 x 1024 x 960 9.8 / 8.6 / 7.7, where the plain product is not).
+static bool rope_on_tile(const GemmArgs& g)
+{
+    return g.M <= 32 && g.N % 128 == 0 && g.N <= 16384 && g.K % 64 == 0 && !skinny_applies(g.M, g.N, g.K) && aligned16(g.A) && aligned16(g.B);
+}
 // C = A B, then interleaved RoPE over the leading columns of C (launch.hpp)
 template <typename T>
 static hipError_t gemm_16_rope_typed(hipStream_t stream, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int force_tile,
                                      void* workspace, size_t workspace_bytes, const RopeEpilogue& rope)
 {
     if (!workspace) workspace_bytes = 0;
+    GemmArgs g{A, B, C, M, N, K, K, N, N, 0, 0, 0, 1.0f, 0.0f, 0, 0, nullptr, 0, 0.0f};
     // the plan of gemm_16_typed that sums K ranges in a pass of its own takes the rotation into that pass
     if (force_tile == 0 && workspace && skinny_applies(M, N, K) && aligned16(A) && aligned16(B) &&
         (size_t)skinny_ksplit(N, K) * M * N * sizeof(float) <= workspace_bytes) {
-        GemmArgs g{A, B, C, M, N, K, K, N, N, 0, 0, 0, 1.0f, 0.0f, 0, 0, nullptr, 0, 0.0f};
         return launch_skinny<T, T>(g, stream, (float*)workspace, &rope);
     }
+    if (force_tile == 0 && rope.cols > 0 && rope_on_tile(g)) return launch_gemm_dl<T, T, true, 64, false, 1, GemmRopeArgs>(GemmRopeArgs{g, rope}, 1, stream);
     if (hipError_t e = gemm_16_typed<T>(stream, A, B, C, 0, M, N, K, force_tile, workspace, workspace_bytes, nullptr, 0, 0.0f)) return e;
     return rope_cols16(stream, std::is_same<T, f16_t>::value ? 1 : 2, C, rope.cosc, rope.sinc, M, N, rope.cols, rope.head_dim, rope.seq_len, rope.start_position);
 }

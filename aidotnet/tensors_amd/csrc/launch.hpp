@@ -42,7 +42,8 @@ hipError_t gemm_16_x3(hipStream_t stream, int kind, const uint16_t* A, const uin
                       int force_tile);
 // C = A B followed by interleaved RoPE over the first rope.cols columns of C (heads of rope.head_dim elements side by side; row m at
 // position rope.start_position + m % rope.seq_len); C has the inputs' type.  Where the product has a summing pass of its own (few
-// rows: K ranges side by side) the rotation rides on that pass, otherwise it is a second launch over C.
+// rows: K ranges side by side) the rotation rides on that pass, on a shorter K of few rows on the tile's stores, otherwise it is a
+// second launch over C.
 struct RopeEpilogue { const float* cosc; const float* sinc; int head_dim, cols, seq_len, start_position; };
 hipError_t gemm_16_rope(hipStream_t stream, int kind, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K, int force_tile,
                         void* workspace, size_t workspace_bytes, const RopeEpilogue& rope);

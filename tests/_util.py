@@ -46,3 +46,18 @@ def round_to(x: np.ndarray, kind: str):
 
 
 TORCH16 = {"f16": torch.float16, "bf16": torch.bfloat16}
+
+
+def kernels_of(call):
+    """Names of the library's kernels that `call` launches, in order (template arguments included): which plan a call takes."""
+    import warnings
+
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        with profile(activities=[ProfilerActivity.CUDA]) as prof:
+            call()
+            torch.cuda.synchronize()
+        ours = [e for e in prof.events() if "aidn::" in e.name]
+    return [e.name.split("aidn::", 1)[1].split("(", 1)[0].replace("aidn::", "") for e in sorted(ours, key=lambda e: e.time_range.start)]
