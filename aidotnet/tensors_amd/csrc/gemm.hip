@@ -1723,16 +1723,17 @@ static int splitk16_ranges(int M, int N, int K, int* kper, int* big_tile = nullp
     // (a ragged M or N: the last tile row or column is partial)
     const long long t = (long long)((M + 127) / 128) * ((N + 127) / 128);
     if (t <= 128) {                           // up to half a chip of 128 x 128 tiles
-        // (below K = 2048 the second launch costs what the ranges save: 1000 x 1024 x 1024 8 -> 15 us, 512 x 1024 x 1344 8.9 -> 14.0, 768 x 1024 x
-        // 1856 17.4 -> 17.1; 128 x 136 x 2112, whose one launch is shorter than what two cost the caller)
-        if (K < (N % 128 == 0 ? 2048 : 2560)) return 0;
-        // estimates in us: 0.5 a K-tile and 3 a launch, 0.5 more for the sums, the partials written and read at 3.5 TB/s (2048 x 1024 x 2112 20.2
-        // in one, 23.3 in two; 1340 x 256 x 6144 16.6 in eight, 17.9 in eleven; 1024 x 1024 x 2112 17.4 in three, 18.4 in four)
+        // (below, the second launch costs what the ranges save: 1000 x 1024 x 1024 8 -> 15 us, 512 x 1024 x 1344 8.9 -> 14.0, 64 x 512 x 1536 9.4 -> 9.8;
+        // 128 x 136 x 2112, whose one launch is shorter than what two cost the caller)
+        if (K < (N % 128 == 0 ? 1792 : 2560)) return 0;
+        // estimates in us: in one launch 0.5 a K-tile and 3; in ranges 0.425 a K-tile, 6.9 for both launches and the sums, and the partials
+        // written and read at 3.55 TB/s (fitted on 310 timings of 60 shapes to 5 %; one / two / three / four: 2048 x 512 x 2048 19.3 / 18.5 / 17.8 /
+        // 18.0, 1000 x 1024 x 2048 20.0 / 17.8 / 17.5 / 18.2, 512 x 1024 x 1792 16.5 / 15.6 / 15.3 / 15.2; 2048 x 1024 x 2112 19.9 in one, 23.1 in two)
         int best = 1;
         double best_us = 0.5 * kt + 3.0;
         for (int ks = 2; ks <= 16 && ks * t <= 256 && K / ks >= 512; ks++) {
             const int per = (kt + ks - 1) / ks, n = (kt + per - 1) / per;
-            const double us = 0.5 * per + 6.5 + (double)n * M * N * 8.0 / 3.5e6;
+            const double us = 0.425 * per + 6.9 + (double)n * M * N * 8.0 / 3.55e6;
             if (us < best_us) { best_us = us; best = n; *kper = 64 * per; }
         }
         return best >= 2 ? best : 0;
