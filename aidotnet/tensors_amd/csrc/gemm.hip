@@ -2780,7 +2780,13 @@ static int dl16_width(int M, int N, int K, int batch, double* score_out)
         const double s2 = dl16_half2_eff(K) * (t128 <= 512 ? cu_fill(t128) : fill2) * use128;
         if (s2 > best_score) { best_score = s2; best = 5; }
     }
-    const double s128 = 0.55 * cu_fill(t128) * use128, s64 = 0.45 * cu_fill(t64) * use64;
+    // M and N multiples of 64 and N not of 128: the 64 x 64 tile runs without edge handling and wastes nothing where every wider one is cut.
+    // Against one round of 128 x 128 tiles it then counts for more, and at K = 128 against two workgroups per CU too (us, cut 128 x 128 / 64 x 64:
+    // 512 x 4672 x 512 9.2 / 8.4, 384 x 6976 x 768 11.6 / 11.0, 640 x 3648 x 832 11.2 / 10.7, 1152 x 4032 x 128 7.8 / 7.3; from K = 192 on
+    // two workgroups win, 1024 x 6464 x 384 11.7 / 13.0)
+    const bool fits64 = M % 64 == 0 && N % 64 == 0 && N % 128 != 0;
+    const double eff64 = fits64 && K <= 128 ? 0.76 : fits64 && best == 1 ? 0.53 : 0.45;
+    const double s128 = 0.55 * cu_fill(t128) * use128, s64 = eff64 * cu_fill(t64) * use64;
     if (score_out) *score_out = best_score > s128 ? (best_score > s64 ? std::min(best_score, 1.0) : s64) : (s128 > s64 ? s128 : s64);
     if (s128 > best_score || s64 > best_score) return 0;
     return best;

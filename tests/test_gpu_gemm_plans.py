@@ -7,7 +7,9 @@ from _util import kernels_of
 pytestmark = pytest.mark.gpu
 
 RANGES = ["gemm_dl16_kernel<bf16_t, float, 2, true", "skinny_reduce_kernel"]       # K ranges of 128 x 128 tiles and their sum
-CASES = [(2048, 512, 2048, RANGES), (1000, 1024, 2048, RANGES), (512, 1024, 1792, RANGES), (1024, 1024, 2048, RANGES)]
+TILE64 = ["gemm_dl_kernel<bf16_t, bf16_t, false, 64"]                              # 64 x 64 tiles without edge handling
+CASES = [(2048, 512, 2048, RANGES), (1000, 1024, 2048, RANGES), (512, 1024, 1792, RANGES), (1024, 1024, 2048, RANGES),
+         (512, 4672, 512, TILE64), (384, 6976, 768, TILE64), (640, 3648, 832, TILE64), (1152, 4032, 128, TILE64)]
 
 
 @pytest.mark.parametrize("M,N,K,want", CASES)
