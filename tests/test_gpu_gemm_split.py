@@ -110,3 +110,12 @@ def test_extreme_magnitudes(M, N, K, scale_a, scale_b):
     # (results below 2^-126 are whole multiples of 2^-149, and so is every partial sum)
     bound = (K + 10) * (2.0 ** -24 * (a.double().abs() @ b.double().abs()) + 2.0 ** -149)
     assert bool(((c.double() - want).abs() <= bound).all())
+
+
+# one to three terms: exact products and a rounding per term, |error| <= K 2^-24 sum |a| |b|
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("K", [1, 2, 3])
+def test_shortest_sums(K, half):
+    a, b = operands(2047, 2049, K, half, 20 + K)
+    c = call(a, b).double()
+    assert bool(((c - a.double() @ b.double()).abs() <= K * 2.0 ** -24 * (a.double().abs() @ b.double().abs())).all())
