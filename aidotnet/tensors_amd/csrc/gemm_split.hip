@@ -1,7 +1,8 @@
 // fp32 products on the bf16 matrix pipe.  Every operand value is split into three bf16 values, x = h + m + l (h = bf16(x), m = bf16(x - h),
 // l = x - h - m, exact for |x| >= 2^-110), and the six products whose weight is at least 2^-18 of the largest are formed: h h, h m, m h,
-// m m, h l, l h.  What is left out is below 2^-26 of the product; the fp32 pipe rounds its sum after every second product, this one after
-// every sixth of 32.
+// m m, h l, l h.  What is left out (m l, l m, l l) is at most 2^-24 of a product; the fp32 pipe, whose products are exact, rounds its sum
+// after every second of them, this one after every sixth of 32.  From four terms on the error is the smaller one; a sum that one term rules
+// (a row with a single value in it, no power of two) keeps the error of its product, up to 2.6 x 2^-24 where that pipe rounds once.
 #include "gemm_common.hpp"
 
 namespace aidn {
@@ -23,9 +24,13 @@ namespace aidn {
 // 2048 x 12288 x 1024 416 / 260, 2368 x 64 x 16181 998 / 70; fp16 weights (five products) 1991 x 2849 x 4800 1149 / 307, 50 x 192 x 5888
 // 246 / 16.  Error against float64, |error| / |result| over 140 shapes: 0.21 - 0.45 of the fp32 pipe's (4096 x 3072 x 768 5.0e-7 / 1.05e-7).
 //
-// Where the split is not exact enough the tile is computed again on the fp32 pipe: a result that is not finite (infinities and values
-// that round to one do not survive a split), or an operand value below 2^-110, which a split cuts at 2^-134, beside one above 2^30 or a
-// result below 2^-60 (otherwise what is cut is less than 2^-40 of the smallest result).
+// Where the split is not exact enough a result is computed again on the fp32 pipe: one that is not finite (infinities and values that round
+// to one do not survive a split), and one whose row or column holds a value below 2^-110 (which a split cuts at 2^-134) where the largest
+// possible sum of what is cut, K 2^-134 times the other operand's largest magnitude, exceeds 2^-30 of it.  A result's own row and column
+// decide that and nothing beside them, and zeros decide nothing.  us, 4096 x 3072 x 768 / 2048 x 2048 x 4096: normal values 109 / 200, every
+// seventh row zero 110 / 206, one NaN 186 / 268, A of probabilities down to 0 (every tile's operands looked at again) 125 / 360; the fp32 pipe
+// 157 / 258 for all of them; with whole tiles computed again, by one load at a time, and the second look taken for zeros too 109 / 202, 134 / 257,
+// 1690 / 2950, 102 / 2980.
 // EDGES: 0 whole tiles, 1 ragged M or N, 2 a remainder of K too.
 template <int BM, int CPT, int PB, int EDGES>
 __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_split_kernel(const GemmArgs g)
@@ -38,7 +43,7 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_split_kernel(const
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* As = smem;
     unsigned char* Bs = smem + 3 * APL;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, l16 = lane & 15, gq = lane >> 4;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l16 = lane & 15, gq = lane >> 4;
     const int wm = wave >> 1, wn = wave & 1;
     int tm, tn;
     tile_of_block(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
@@ -61,12 +66,12 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_split_kernel(const
         aoff[i] = 4u * (uint32_t)(min(u >> 2, g.M - 1 - m0) * g.lda + 8 * (u & 3));
     }
     const int bcol = n0 + lane * CPT, past = EDGE ? max(bcol - (g.N - CPT), 0) : 0;      // columns past the end repeat the last one (never stored)
-    const int bwave = __builtin_amdgcn_readfirstlane(8 * wave);
+    const int bwave = 8 * wave;
     const unsigned char* bbase = (const unsigned char*)(B + (long long)bwave * g.ldb);
     const uint32_t boff = (uint32_t)sizeof(b_t) * (uint32_t)(bcol - past);
     auto b_at = [&](const unsigned char* row, int c) { return *(const b_t*)(row + boff + c * sizeof(b_t)); };
-    u32x4 ra[NSET][UA][2];
-    b_t rb[NSET][8][CPT];
+    u32x4 ra[2][UA][2];                                           // (the second look uses both everywhere)
+    b_t rb[2][8][CPT];
     int loaded = 0;
     auto load = [&](auto set) {
         constexpr int S = decltype(set)::value;
@@ -103,9 +108,36 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_split_kernel(const
             for (int c = 0; c < CPT; c++) { const b_t x = b_at(row, c); rb[0][r][c] = k < K ? x : (b_t)0; }
         }
     };
-    float big = 0.0f;                                             // the largest magnitude this thread staged
+    // the smallest magnitude but zero that this thread staged, if below 2^-110: bits doubled (no sign) less one (zero wraps to the largest).
+    // What a tile holds is first compared as it is, zeros included, half an instruction a value; the exact form follows where that was small
+    uint32_t tiny = 0xFFFFFFFFu;
+    auto nonzero = [](float x) { return 2u * as_u32(x) - 1u; };
     auto stage = [&](auto set) {
         constexpr int S = decltype(set)::value;
+        float least = INFINITY;
+#pragma unroll
+        for (int i = 0; i < UA; i++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) least = fminf(least, fabsf(as_f32(ra[S][i][e >> 2][e & 3])));
+        if (least < 0x1p-110f) {
+#pragma unroll
+            for (int i = 0; i < UA; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) tiny = min(tiny, nonzero(as_f32(ra[S][i][e >> 2][e & 3])));
+        }
+        if constexpr (!B16) {
+            least = INFINITY;
+#pragma unroll
+            for (int r = 0; r < 8; r++)
+#pragma unroll
+                for (int c = 0; c < CPT; c++) least = fminf(least, fabsf(rb[S][r][c]));
+            if (least < 0x1p-110f) {
+#pragma unroll
+                for (int r = 0; r < 8; r++)
+#pragma unroll
+                    for (int c = 0; c < CPT; c++) tiny = min(tiny, nonzero(rb[S][r][c]));
+            }
+        }
 #pragma unroll
         for (int i = 0; i < UA; i++) {
             const int u = t + 256 * i, row = u >> 2, kg = u & 3;
@@ -113,7 +145,6 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_split_kernel(const
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const float x = as_f32(ra[S][i][e >> 1][2 * (e & 1)]), y = as_f32(ra[S][i][e >> 1][2 * (e & 1) + 1]);
-                big = fmaxf(fmaxf(big, fabsf(x)), fabsf(y));
                 uint32_t p[3];
                 split_pair(x, y, p);
 #pragma unroll
@@ -135,7 +166,7 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_split_kernel(const
                 };
                 const b_t bx = pick(2 * e), by = pick(2 * e + 1);
                 if constexpr (B16) { x = f16_bits_to_float(bx); y = f16_bits_to_float(by); }
-                else { x = bx; y = by; big = fmaxf(fmaxf(big, fabsf(x)), fabsf(y)); }
+                else { x = bx; y = by; }
                 uint32_t p[PB];
                 split_pair(x, y, p);
 #pragma unroll
@@ -144,7 +175,6 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_split_kernel(const
 #pragma unroll
             for (int s = 0; s < PB; s++) *(u32x4*)(Bs + s * BPL + wave * (BN * 16) + ((c * 64 + lane) ^ (2 * wave)) * 16) = w[s];
         }
-        asm volatile("" : "+v"(big));                             // (formed here: moved behind the loads it keeps the old values alive)
     };
 
     f32x4 acc[TI][TJ];                                            // block (i, j): rows 16 i, columns j / 2 + CPT (16 (j & 1) + lane % 16)
@@ -222,76 +252,189 @@ __global__ __launch_bounds__(256, BM == 64 ? 3 : 2) void gemm_split_kernel(const
     }
 
     // ---- is the split exact enough here?
-    float poison = 0.0f, least = INFINITY;
+    constexpr uint32_t CUT_BELOW = 2u * (17u << 23) - 1u;         // 2^-110
+    float poison = 0.0f;
 #pragma unroll
     for (int i = 0; i < TI; i++)
 #pragma unroll
         for (int j = 0; j < TJ; j++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                poison = fmaf(acc[i][j][r], 0.0f, poison);        // NaN once a value is infinite or NaN
-                least = fminf(least, fabsf(acc[i][j][r]));
-            }
-    int redo = poison != poison;
-    if (__syncthreads_or(redo | (big > 0x1p30f) | (least < 0x1p-60f))) {
-        if (!__syncthreads_or(redo)) {                            // (no infinity:) does an operand value lose bits?
-            float tiny = 1.0f;
-            auto look = [&](float x) { tiny = x != 0.0f ? fminf(tiny, fabsf(x)) : tiny; };
-            auto look_all = [&]() {
+            for (int r = 0; r < 4; r++) poison = fmaf(acc[i][j][r], 0.0f, poison);        // NaN once a value is infinite or NaN
+    const bool lossy = tiny < CUT_BELOW;
+    int ln = __lane_id();
+    asm volatile("" : "+v"(ln));                                  // (what follows is addressed from here: nothing of it is kept through the loop above)
+    if (__syncthreads_or(lossy | (poison != poison))) {
+        const int th = 64 * wave + ln, row16 = ln & 15, quad = ln >> 4;
+        // of the tile's rows, then columns: 1 if it holds a value below 2^-110, and its largest magnitude times K 2^-104
+        float* low = (float*)smem;
+        float* high = low + BM + BN;
+        const bool look = __syncthreads_or(lossy);
+        for (int q = th; q < BM + BN; q += 256) { low[q] = 0.0f; high[q] = 0.0f; }
+        __syncthreads();
+        if (look) {
+            uint32_t lo_a[UA], lo_b[CPT];
+            float hi_a[UA], hi_b[CPT];
+#pragma unroll
+            for (int i = 0; i < UA; i++) { lo_a[i] = 0xFFFFFFFFu; hi_a[i] = 0.0f; }
+#pragma unroll
+            for (int c = 0; c < CPT; c++) { lo_b[c] = 0xFFFFFFFFu; hi_b[c] = 0.0f; }
+            auto look_at = [&](auto set) {
+                constexpr int S = decltype(set)::value;
 #pragma unroll
                 for (int i = 0; i < UA; i++)
 #pragma unroll
-                    for (int e = 0; e < 8; e++) look(as_f32(ra[0][i][e >> 2][e & 3]));
-                if constexpr (!B16) {
+                    for (int e = 0; e < 8; e++) {
+                        const float x = as_f32(ra[S][i][e >> 2][e & 3]);
+                        lo_a[i] = min(lo_a[i], nonzero(x)); hi_a[i] = fmaxf(hi_a[i], fabsf(x));
+                    }
 #pragma unroll
-                    for (int r = 0; r < 8; r++)
+                for (int r = 0; r < 8; r++)
 #pragma unroll
-                        for (int c = 0; c < CPT; c++) look(rb[0][r][c]);
-                }
+                    for (int c = 0; c < CPT; c++) {
+                        if constexpr (B16) hi_b[c] = fmaxf(hi_b[c], fabsf(f16_bits_to_float(rb[S][r][c])));
+                        else { lo_b[c] = min(lo_b[c], nonzero(rb[S][r][c])); hi_b[c] = fmaxf(hi_b[c], fabsf(rb[S][r][c])); }
+                    }
             };
             const int back = tiles > 0 ? 32 * (tiles - 1) : 0;    // where the loads have left the pointers
             abase -= 4 * back;
             bbase -= (long long)back * g.ldb * sizeof(b_t);
             if constexpr (REST) {
-                if (K % 32 != 0) { load_remainder(); look_all(); }
+                if (K % 32 != 0) { load_remainder(); look_at(first); }
             }
-            loaded = 0;
+            if (tiles > 0) {
+                loaded = 0;
+                load(first);
 #pragma unroll 1
-            for (int it = 0; it < tiles; it++) { load(first); look_all(); }
-            redo = tiny < 0x1p-110f;
+                for (int it = 0; it < tiles; it += 2) {           // (past the last tile it is looked at again)
+                    load(std::integral_constant<int, 1>{});
+                    __builtin_amdgcn_sched_barrier(0);
+                    look_at(first);
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(first);
+                    __builtin_amdgcn_sched_barrier(0);
+                    look_at(std::integral_constant<int, 1>{});
+                }
+            }
+            const float scale = (float)K * 0x1p-104f;
+            auto mark = [&](int q, uint32_t lo, float hi) {
+                if (q < 0) return;                                // (a column of the tile before)
+                if (lo < CUT_BELOW) low[q] = 1.0f;
+                atomicMax((uint32_t*)&high[q], as_u32(hi * scale));          // (not negative: ordered like its bits)
+            };
+#pragma unroll
+            for (int i = 0; i < UA; i++) mark((th + 256 * i) >> 2, lo_a[i], hi_a[i]);
+#pragma unroll
+            for (int c = 0; c < CPT; c++) {
+                const int q = ln * CPT - past + c;
+                mark(q < 0 ? -1 : BM + q, lo_b[c], hi_b[c]);
+            }
+            __syncthreads();
         }
-        if (__syncthreads_or(redo)) {
-            static_for<0, TI, 1>([&](auto ic) {
-                static_for<0, TJ, 1>([&](auto jc) {
-                    constexpr int i = decltype(ic)::value, j = decltype(jc)::value;
-                    const float* x = A + (long long)min(m0 + wm * (BM / 2) + 16 * i + l16, g.M - 1) * g.lda;
-                    const b_t* y = B + min(n0 + (wn * 32 + 16 * (j & 1) + l16) * CPT + (j >> 1), g.N - 1);
-                    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+        // which results the split does not hold: a bit per column block and row of the block, a word per row block; and the blocks of this wave
+        uint32_t want[TI], blocks = 0;
+        float column_low[TJ], column_high[TJ];
+#pragma unroll
+        for (int j = 0; j < TJ; j++) {
+            const int q = BM + (wn * 32 + 16 * (j & 1) + row16) * CPT + (j >> 1);
+            column_low[j] = low[q]; column_high[j] = high[q];
+        }
+        static_for<0, TI, 1>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            uint32_t w = 0;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int q = wm * (BM / 2) + 16 * i + 4 * quad + r;
+                const float row_low = low[q], row_high = high[q];
+#pragma unroll
+                for (int j = 0; j < TJ; j++) {
+                    const float v = fabsf(acc[i][j][r]);
+                    w |= !(v < INFINITY) | (v < fmaf(row_low, column_high[j], column_low[j] * row_high)) ? 1u << (4 * j + r) : 0u;
+                }
+            }
+            asm volatile("" : "+v"(w));                           // (formed here, row block by row block: the tests of all of them do not fit the registers)
+            want[i] = w;
+#pragma unroll
+            for (int j = 0; j < TJ; j++) blocks |= __ballot(w >> (4 * j) & 15u) ? 1u << (TJ * i + j) : 0u;
+        });
+        // those blocks again on the fp32 pipe, one after the other, RK k at a time, the next RK in flight: lane (quad, row16) holds k = 4 quad .. 4 quad + 3
+        // of every 16, of its row and of its column, one of them to an instruction
+        constexpr int RK = CPT == 3 ? 32 : 64;                    // (what the registers hold beside the accumulators)
+        static_for<0, TI, 1>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;                // (a loop of its own for each: one over all blocks copies every accumulator, which do not fit twice)
 #pragma unroll 1
-                    for (int k = gq; k - gq < K; k += 4) {
-                        float va = 0.0f, vb = 0.0f;
-                        if (k < K) {
-                            va = x[k];
-                            if constexpr (B16) vb = f16_bits_to_float(y[(long long)k * g.ldb]);
-                            else vb = y[(long long)k * g.ldb];
-                        }
-                        s = __builtin_amdgcn_mfma_f32_16x16x4f32(va, vb, s, 0, 0, 0);
+            for (int bj = 0; bj < TJ; bj++) {
+                if (!(blocks >> (TJ * i + bj) & 1)) continue;
+                int at = ln;
+                asm volatile("" : "+v"(at));
+                const int row16 = at & 15, quad = at >> 4;
+                const float* x = A + (long long)min(m0 + wm * (BM / 2) + 16 * i + row16, g.M - 1) * g.lda + 4 * quad;
+                const int column = min(n0 + (wn * 32 + 16 * (bj & 1) + row16) * CPT + (bj >> 1), g.N - 1);
+                const b_t* y = B + (long long)(4 * quad) * g.ldb + column;
+                f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f}, va[2][RK / 16];
+                b_t vb[2][RK / 16][4];
+                auto fetch = [&](int s, int k) {
+#pragma unroll
+                    for (int q = 0; q < RK / 16; q++) {
+                        va[s][q] = __builtin_bit_cast(f32x4, *(const u32x4_a4*)(x + (k + 16 * q)));
+#pragma unroll
+                        for (int e = 0; e < 4; e++) vb[s][q][e] = y[(long long)(k + 16 * q + e) * g.ldb];
                     }
-                    acc[i][j] = s;
+                };
+                auto multiply16 = [&](const f32x4& a, const b_t (&b)[4]) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        float v;
+                        if constexpr (B16) v = f16_bits_to_float(b[e]);
+                        else v = b[e];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], v, sum, 0, 0, 0);
+                    }
+                };
+                auto multiply_all = [&](int s) {
+#pragma unroll
+                    for (int q = 0; q < RK / 16; q++) multiply16(va[s][q], vb[s][q]);
+                };
+                const int whole = K / RK * RK;
+                if (whole > 0) fetch(0, 0);
+#pragma unroll 1
+                for (int k = 0; k < whole; k += 2 * RK) {
+                    fetch(1, min(k + RK, whole - RK));
+                    multiply_all(0);
+                    if (k + RK >= whole) break;
+                    fetch(0, min(k + 2 * RK, whole - RK));
+                    multiply_all(1);
+                }
+#pragma unroll 1
+                for (int k0 = whole; (REST || RK > 32) && k0 < K; k0 += 16) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int k = k0 + e, last = K - 1 - 4 * quad;      // (x and y start at k = 4 quad, which may be past the end)
+                        const float v = x[min(k, last)];
+                        const b_t w = y[(long long)min(k, last) * g.ldb];
+                        va[0][0][e] = k <= last ? v : 0.0f; vb[0][0][e] = k <= last ? w : (b_t)0;
+                    }
+                    multiply16(va[0][0], vb[0][0]);
+                }
+                asm volatile("" : "+v"(want[i]));
+                static_for<0, TJ, 1>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value;
+                    uint32_t here = bj == j ? 15u << (4 * j) : 0u;
+                    asm volatile("" : "+s"(here));                    // (selected and not branched to)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[i][j][r] = want[i] & here & 1u << (4 * j + r) ? sum[r] : acc[i][j][r];
                 });
-            });
-        }
+            }
+        });
     }
 
-    // ---- epilogue: rows 4 gq + r of a block, CPT consecutive columns to a lane
+    // ---- epilogue: rows 4 (lane / 16) + r of a block, CPT consecutive columns to a lane
     float* __restrict__ C = (float*)g.C + bz * g.sC;
     const bool rows_cut = EDGE && m0 + BM > g.M, cut = EDGE && n0 + BN > g.N;
     static_for<0, TI, 1>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        const int row0 = m0 + wm * (BM / 2) + 16 * i + 4 * gq;
+        const int row0 = m0 + wm * (BM / 2) + 16 * i + 4 * (ln >> 4);
         static_for<0, 2, 1>([&](auto hc) {
             constexpr int h = decltype(hc)::value;
-            const int col = n0 + (wn * 32 + 16 * h + l16) * CPT;
+            const int col = n0 + (wn * 32 + 16 * h + (ln & 15)) * CPT;
             float v[4][CPT];
 #pragma unroll
             for (int r = 0; r < 4; r++)
