@@ -2480,12 +2480,13 @@ __global__ __launch_bounds__(256, NS <= 3 ? 2 : 1) void gemm_skinny32_kernel(con
 #if AIDN_GEMM_PART == 0
 // ---- fp32 products on the bf16 matrix pipe (gemm_split.hip): tile and K ranges by an estimate of the run time in microseconds.
 // A WG advances by one K-tile of 32 in us[n - 1] with n of them on a CU and needs `once` for its first loads and its epilogue; the operands
-// come at 6 TB/s at best; ranges add the summing pass, 8 bytes a partial element at 5 TB/s.  Fitted on 963 (fp32) and 325 (fp16
+// come at 6.4 TB/s (fp16 weights 4.5), or 2.9 where B lies beyond the last-level cache; ranges add the summing pass, 8 bytes a partial
+// element at 5 TB/s.  Fitted on 963 (fp32) and 325 (fp16
 // weights) timings of 140 shapes, M 9 - 8192, N 64 - 60000, K 64 - 16384, to 9 and 11 %; the plan it picks is 1 and 2 % behind the best one in the mean.
 struct SplitTile { int id, rows, cols, resident; double us[2][3], once[2]; };
 static const SplitTile kSplitTiles[3] = {{64, 64, 128, 3, {{1.25, 1.77, 2.30}, {0.97, 1.34, 1.72}}, {0.0, 0.0}},
                                          {128, 128, 128, 2, {{1.89, 2.57, 0.0}, {1.66, 2.10, 0.0}}, {1.7, 0.9}},
-                                         {192, 128, 192, 2, {{3.00, 4.17, 0.0}, {2.74, 4.43, 0.0}}, {3.6, 6.7}}};
+                                         {192, 128, 192, 2, {{3.00, 4.17, 0.0}, {0.0, 0.0, 0.0}}, {3.6, 0.0}}};      // (fp32 only)
 struct SplitPlan { int tile = 0, ks = 1, kper = 0; double us = 1e30; };
 static SplitPlan split_plan(int M, int N, int K, int batch, bool b16, size_t partial_bytes)
 {
@@ -2499,7 +2500,7 @@ static SplitPlan split_plan(int M, int N, int K, int batch, bool b16, size_t par
     const double bytes_us = (4.0 * M * K * batch + b_bytes) / (b_bytes > 1.5e8 ? 2.9e6 : b16 ? 4.5e6 : 6.4e6);
     static const int ranges[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
     for (const SplitTile& s : kSplitTiles) {
-        if (s.id == 192 && (M % 128 != 0 || N % 192 != 0 || K % 32 != 0)) continue;
+        if (s.id == 192 && (b16 || M % 128 != 0 || N % 192 != 0 || K % 32 != 0)) continue;
         const long long tiles = (long long)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols) * batch;
         for (int want : ranges) {
             if (want > 1 && (batch > 1 || kt / want < 2 || tiles * want > 1600)) break;

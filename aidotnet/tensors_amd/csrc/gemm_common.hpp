@@ -130,8 +130,8 @@ __device__ __forceinline__ void tile_of_block(int pid, int nblk, int tiles_m, in
 }
 
 // fp32 products on the bf16 matrix pipe (gemm_split.hip): C = act(alpha A B + beta C + bias), B [K,N] of fp32 or (b16) fp16, N >= 2,
-// lda and ldb below 2^21, operands at any element.  tile: 64 or 128 rows by 128 columns; 192, whole 128 x 192 tiles over whole K-tiles
-// of 32 only.
+// lda and ldb below 2^21, operands at any element.  tile: 64 or 128 rows by 128 columns; 192, fp32 and whole 128 x 192
+// tiles over whole K-tiles of 32 only.
 hipError_t launch_gemm_split(const GemmArgs& g, int batch, hipStream_t stream, int tile, bool b16);
 
 }  // namespace aidn

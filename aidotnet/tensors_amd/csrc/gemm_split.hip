@@ -501,7 +501,7 @@ static hipError_t launch_split_tile(const GemmArgs& g, int batch, hipStream_t st
 }
 hipError_t launch_gemm_split(const GemmArgs& g, int batch, hipStream_t stream, int tile, bool b16)
 {
-    if (tile == 192) return b16 ? launch_split_tile<128, 3, 2>(g, batch, stream) : launch_split_tile<128, 3, 3>(g, batch, stream);
+    if (tile == 192) return b16 ? hipErrorInvalidValue : launch_split_tile<128, 3, 3>(g, batch, stream);
     if (tile == 128) return b16 ? launch_split_tile<128, 2, 2>(g, batch, stream) : launch_split_tile<128, 2, 3>(g, batch, stream);
     if (tile == 64) return b16 ? launch_split_tile<64, 2, 2>(g, batch, stream) : launch_split_tile<64, 2, 3>(g, batch, stream);
     return hipErrorInvalidValue;
