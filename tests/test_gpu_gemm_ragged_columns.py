@@ -8,10 +8,13 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# 256 x 192 / 256 x 256 / 256 x 128 tiles; 128 x 128 on both rings; K ranges; 256 x 256 in K ranges; few rows (one, two slabs, two workgroups per CU)
+# 256 x 192 / 256 x 128 / 128 x 128 on both rings with a partial last column; K ranges of 128 x 128 tiles; few rows (one, two slabs, two workgroups
+# per CU); 256 x 256 in two K ranges of uneven length; 256 x 256 with a partial last column, twice, and with non-temporal stores
+# (test_gpu_gemm_plans.py holds which kernel each of them runs)
 SHAPES = [(1000, 11008, 64), (1000, 11000, 128), (4000, 4088, 64), (2040, 4088, 6208), (2040, 4088, 128), (2000, 2040, 64), (300, 64, 192),
           (129, 136, 1088), (128, 136, 1088), (200, 1032, 2624), (64, 4104, 4160), (1000, 8192, 8256), (33, 1000, 2112),
-          (1, 136, 2560), (32, 248, 2624), (32, 1000, 4160), (32, 4104, 1536), (7, 11000, 1600), (17, 50264, 128), (5, 8200, 8192)]
+          (1, 136, 2560), (32, 248, 2624), (32, 1000, 4160), (32, 4104, 1536), (7, 11000, 1600), (17, 50264, 128), (5, 8200, 8192),
+          (1000, 8192, 10560), (1000, 12296, 768), (2000, 6152, 768), (8192, 13000, 1024)]
 
 
 def operands(M, N, K, dt):

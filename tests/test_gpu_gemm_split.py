@@ -1,5 +1,5 @@
-"""fp32 products on the bf16 matrix pipe (three bf16 values to an operand, two to an fp16 weight): tiles of 64 and 128 rows by 128
-columns, 128 x 192 on whole tiles, K ranges, K remainders, columns past the end, operands at any element.
+"""fp32 products on the bf16 matrix pipe (three bf16 values to an operand, two to an fp16 weight): mostly tiles of 64 rows by 128 columns in
+K ranges, with K remainders, columns past the end, operands at any element (every instance by name: test_gpu_gemm_split_tiles.py).
 
 Bound: every 32 of K add one fp32 rounding of the running sum, the sums inside them and what the split leaves out stay below ten more:
 |error| <= (K / 32 + 10) 2^-24 sum |a| |b|."""
