@@ -1139,10 +1139,7 @@ __global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
 #pragma unroll
         for (int j = 0; j < TJ; j++) {
             bias4[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            // (two statements: one min that is only formed for CUT still changed the addresses of the whole-tile instances, 0.15 us a launch of
-            // 4096 x 768 x 768, and an attention layer of 8 x 512 x 768 took 52.9 instead of 52.6 us)
-            if constexpr (CUT) { if (g.bias) bias4[j] = *(const f32x4*)(g.bias + min(n0 + wn * WTN + 16 * j + 4 * g4, g.N - 4)); }
-            else if (g.bias) bias4[j] = *(const f32x4*)(g.bias + n0 + wn * WTN + 16 * j + 4 * g4);
+            if (g.bias) bias4[j] = *(const f32x4*)(g.bias + (CUT ? min(n0 + wn * WTN + 16 * j + 4 * g4, g.N - 4) : n0 + wn * WTN + 16 * j + 4 * g4));
         }
         unsigned char* Cw = (unsigned char*)g.C + (bz * g.sC + (long long)(m0 + wm * WTM) * g.ldc + n0 + wn * WTN) * OB;
         const bool whole_tile = __builtin_amdgcn_readfirstlane(m0 + BM <= g.M && (!CUT || n0 + BN <= g.N) && g.c_cols == 0);
