@@ -900,8 +900,11 @@ template <> struct Mma16<bf16_t> {
 // and the hint is lost).
 // CUT: N is not a multiple of the tile width (an instance of its own: with the clamps and tests in all of them whole tiles took longer,
 // 8192 x 768 x 768 17.2 -> 17.5 us).
+// On a page of its own: a launch of one or two rounds begins by fetching up to 70 KB of code, and where that lay within its pages moved an
+// attention layer of 8 x 512 x 768, three such launches in a row, by 1.7 % (us, the QKV and output projections at 0x100 and 0xc00 of a page 53.1,
+// at 0x400 and 0x800 53.3, at 0x900 and 0xd00 53.6, both at 0 52.7) with every instance added to this file.
 template <typename T, typename OutT, int TJ = 4, bool HALF = false, bool NTS = false, int HS = DL16_HALF_STAGES, bool CUT = false>
-__global__ __launch_bounds__(512, 1) void gemm_dl16_kernel(const GemmArgs g)
+__global__ __launch_bounds__(512, 1) __attribute__((aligned(4096))) void gemm_dl16_kernel(const GemmArgs g)
 {
     static_assert(!HALF || TJ == 2, "the 128-row tile is built for 128 columns");
     constexpr int E = 8, EB = 2;
