@@ -58,11 +58,12 @@ def test_odd_values_and_their_neighbours(M, N, K, half, kernel):
 
 
 # around 2^-110, where the third part of a value ends among the bf16 subnormals, and below, beside ordinary and beside large values
-@pytest.mark.parametrize("scale_a,scale_b", [(-105, 0), (-109, 29), (-112, 0), (-112, 100), (-120, 60), (-100, -20), (29, -109), (0, -125)])
-@pytest.mark.parametrize("M,N,K,half,kernel", [i for i in INSTANCES if i[:3] in ((2816, 4416, 96), (3583, 1727, 65), (65, 255, 4097))])
+SCALES = [(-105, 0), (-109, 29), (-112, 0), (-112, 100), (-120, 60), (-100, -20), (29, -109), (0, -125)]
+SMALLEST = [i + s for i in INSTANCES if i[:3] in ((2816, 4416, 96), (3583, 1727, 65), (65, 255, 4097)) for s in SCALES if not i[3] or abs(s[1]) <= 10]
+
+
+@pytest.mark.parametrize("M,N,K,half,kernel,scale_a,scale_b", SMALLEST)
 def test_smallest_values(M, N, K, half, kernel, scale_a, scale_b):
-    if half and (scale_b > 10 or scale_b < -10):
-        pytest.skip("outside fp16")
     a, b = operands(M, N, K, half, 8)
     a *= 2.0 ** scale_a; b *= 2.0 ** scale_b
     a[:, 1] = 0.0
