@@ -20,7 +20,7 @@ namespace aidn {
 //
 // Bound by the matrix pipe (half of its cycles at two workgroups per CU) and the vector pipe beside it: 5.5 instructions split a value,
 // a third of what a wave issues; a CU's clock under this load is 1.8 GHz.  Four waves that only load and split beside four that only
-// multiply came out equal (4096^3 683 / 677 us).  Against the fp32 pipe, us: 4096^3 920 / 680, 4096 x 3072 x 768 with GELU 150 / 105,
+// multiply came out equal (4096^3 683 / 677 us).  Against the fp32 pipe, us: 4096^3 920 / 680, 4096 x 3072 x 768 with GELU 149.5 / 105.9,
 // 2048 x 12288 x 1024 416 / 260, 2368 x 64 x 16181 998 / 70; fp16 weights (five products) 1991 x 2849 x 4800 1149 / 307, 50 x 192 x 5888
 // 246 / 16.  Error against float64, |error| / |result| over 140 shapes: 0.21 - 0.45 of the fp32 pipe's (4096 x 3072 x 768 5.0e-7 / 1.05e-7).
 //

@@ -80,16 +80,19 @@ AIDN_API int aidn_mi355_release_stream_workspace(void* ctx, void* stream);
  * C[M,N] = alpha * A[M,K] * op(B) + beta * C.  transB == 0: B is [K,N]; transB != 0: B is stored
  * [N,K] (C = A * B^T).  Replaces IDirectGpuBackend.Gemm (IDirectGpuBackend.cs:160-172; host
  * HipBackend.cs:1370-1447, hipblasSgemm :1502-1545) and MatMulTransposed (:184-203; host
- * HipBackend.cs:1450-1490).  Argument order (M, N, K) as at that layer.  True fp32 MFMA, fp32
- * accumulation (no TF32-style truncation).  M <= 8 with B [K,N] takes the bandwidth-bound small-M path (B streamed once,
+ * HipBackend.cs:1450-1490).  Argument order (M, N, K) as at that layer.  fp32 operands in all
+ * their 24 bits and fp32 accumulation, no TF32-style truncation: on the fp32 MFMA, or, where that is estimated to be faster (B [K,N],
+ * K >= 4), on the bf16 MFMA from three bf16 values to an operand and six products to a product (what that leaves out is at most 2^-24
+ * of a product; a sum's error against float64 is below the fp32 MFMA's, but for a sum that a single term rules, whose product is then
+ * rounded twice).  M <= 8 with B [K,N] takes the bandwidth-bound small-M path (B streamed once,
  * split-K partials in the context workspace, summed in a fixed order): the GPU form of SimdGemm.SgemmNParallelSmallM /
  * SgemmConcatenatedProjections (Engines/Simd/SimdGemm.NParallelSmallM.cs:31-109); the same holds for the bias/activation
  * and fp16-weight entry points below.  With 9 <= M <= 32 (B [K,N], N a multiple of 128, K a multiple of 32) the weight matrix is
  * likewise streamed once, through a 32-row MFMA kernel, and larger products whose tiles would not fill the chip over a long K
  * (K >= 1024, K a multiple of 32, either layout of B) run their K ranges side by side; both keep fp32 partials in the context
  * workspace and sum them in range order, so results are repeatable run to run (this entry point and the bias/activation one).
- * Rows that are not whole 16-byte chunks (K, or N with B [K,N], not a multiple of 4): a product of some size is computed from
- * zero-padded copies of A and B in the workspace (same sums; C is written in place). */
+ * Rows that are not whole 16-byte chunks (B [N,K], K not a multiple of 4): a product of some size is computed from zero-padded copies
+ * of A and B in the workspace (same sums; C is written in place). */
 AIDN_API int aidn_mi355_sgemm(void* ctx, void* stream, const float* A, const float* B, float* C,
                      int M, int N, int K, float alpha, float beta, int transB);
 
@@ -129,7 +132,8 @@ AIDN_API int aidn_mi355_sgemm_f16weight(void* ctx, void* stream, const float* A,
  * The GPU form of the reference's cached packed B (SimdGemm.SgemmWithCachedB and its PrePackedB cache, Engines/Simd/SimdGemm.cs:327-684,
  * 1030-1159: a weight matrix is packed once into the layout the kernel wants and re-used by every later product; results are those of
  * the plain call).  Here the packed layout is the weight zero-padded to whole tiles with 16-byte aligned rows, which is what a product
- * whose N or K is odd (a vocabulary of 50257 columns) otherwise copies on every call.  kind: 0 fp32 (B [K,N], or [N,K] when transB != 0),
+ * whose N or K is odd otherwise copies on every call where it takes copies (16-bit, many rows over a long K; fp32, B [N,K]); elsewhere
+ * such a weight is read in place and packing it gains nothing.  kind: 0 fp32 (B [K,N], or [N,K] when transB != 0),
  * 1 fp16, 2 bf16 (B [K,N], transB must be 0).  The caller owns `packed` (aidn_mi355_packed_b_bytes bytes, 16-byte aligned) and repacks
  * when the weight changes -- no identity or content check is made here; the reference's cache keys (array identity, version,
  * FNV-1a of the contents) are host-side bookkeeping that stays with the caller.
@@ -149,9 +153,9 @@ AIDN_API int aidn_mi355_gemm_packed_b(void* ctx, void* stream, int kind, const v
  * The bf16 pair has no member in the reference's backend interface today (its planner widens
  * bf16 tensors to fp32, Engines/Gpu/GpuPrecisionPolicy.cs:497-532); it follows the CPU kernel
  * Engines/Simd/BFloat16Kernels.cs:144-211 and NumericOperations/BFloat16.cs:64-90.
- * Any M, N and K are accepted.  When N or K is not a multiple of 8 (rows that are not whole 16-byte chunks) a product of some size
- * is computed from zero-padded copies of A and B held in the stream's workspace -- same sums, three more passes over the
- * operands; a weight of such a width that is used many times is better stored padded by the caller. */
+ * Any M, N and K are accepted.  When N or K is not a multiple of 8 (rows that are not whole 16-byte chunks) the operands are read
+ * in place, or, with many rows over a long K, computed from zero-padded copies of A and B held in the stream's workspace -- same sums,
+ * three more passes over the operands; a weight of such a width that is used many times is better stored padded by the caller. */
 AIDN_API int aidn_mi355_hgemm_f32out(void* ctx, void* stream, const uint16_t* A, const uint16_t* B, float* C, int M, int N, int K);
 AIDN_API int aidn_mi355_hgemm_f16out(void* ctx, void* stream, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K);
 AIDN_API int aidn_mi355_bf16gemm_f32out(void* ctx, void* stream, const uint16_t* A, const uint16_t* B, float* C, int M, int N, int K);
@@ -164,8 +168,8 @@ AIDN_API int aidn_mi355_bf16gemm_bf16out(void* ctx, void* stream, const uint16_t
  * pair (2i, 2i+1) of a head in row m turns by the angle of position start_position + m % seq_len (rows are [leading, seq_len]:
  * M = batch and seq_len = 1 in a decode step).  The result is what the product followed by the rotation kernel gives, rounding
  * included.  Where the product has a summing pass of its own (few rows: the weight is streamed once in K ranges side by side,
- * the decode-step shapes) the rotation rides on that pass and no separate launch is made; other shapes run the rotation as a
- * second launch over C.  The decode step the reference composes from SimdGemm.SgemmConcatenatedProjections
+ * the decode-step shapes) the rotation rides on that pass, for as few rows over a shorter K on the stores of the product's one launch;
+ * other shapes run the rotation as a second launch over C.  The decode step the reference composes from SimdGemm.SgemmConcatenatedProjections
  * (Engines/Simd/SimdGemm.NParallelSmallM.cs:95-109) and RopeInterleaved (IDirectGpuBackend.cs:1427-1446); no single member of the
  * reference does both. */
 AIDN_API int aidn_mi355_hgemm_rope(void* ctx, void* stream, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
