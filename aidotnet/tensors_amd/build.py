@@ -18,6 +18,7 @@ LIB_PATH = os.path.join(HERE, LIB_NAME)
 SOURCES = [("gemm.hip", "gemm.o", ["-DAIDN_GEMM_PART=0"]), ("gemm.hip", "gemm_f16.o", ["-DAIDN_GEMM_PART=1"]),
            ("gemm.hip", "gemm_bf16.o", ["-DAIDN_GEMM_PART=2"]), ("gemm_split.hip", "gemm_split.o", []),
            ("attention.hip", "attention.o", []), ("attention_prefill.hip", "attention_prefill.o", []),
+           ("attention_split.hip", "attention_split.o", []),
            ("decode.hip", "decode.o", []),
            ("convert.hip", "convert.o", []), ("api.hip", "api.o", [])]
 # -packed-fp32-ops off: packed fp32 VALU forms are kept out of all device code.

@@ -64,44 +64,8 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int l32 = lane & 31, h = lane >> 5;
 
-    // workgroup -> (batch*head, query tile): XCD-contiguous so the q-tiles of one head share an L2;
-    // late (heavy, under a causal mask) query tiles first.
     int bh, qt;
-    {
-        int nblk = gridDim.x, pid = blockIdx.x;
-        int per = nblk >> 3, rem = nblk & 7;
-        int xcd = pid & 7, idx = pid >> 3;
-        int logical = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + idx;
-        bh = logical / a.qtiles;
-        qt = a.qtiles - 1 - (logical - bh * a.qtiles);
-        if (a.causal && a.hgroup < 0) {
-            // A grid that is resident all at once (at most three workgroups per CU) is not balanced by the order of
-            // dispatch: hand the query tiles out heaviest first across ALL heads, so the workgroups that end up sharing a
-            // CU are a heavy one and, later in the id order, a light one.
-            // (the first 256 ids, one per CU, in ascending weight, so that the ids after them -- which land on the same
-            // CUs in the same order -- pair the lightest of the first round with the heaviest of the second; reversed by eights, so that
-            // where 8 divides the number of heads all query tiles of a head stay on one XCD, 1-4 % against reversing one by one)
-            const int nbh = nblk / a.qtiles;
-            const int rank = (nblk > 256 && pid < 256) ? 255 - (pid | 7) + (pid & 7) : pid;
-            qt = a.qtiles - 1 - rank / nbh;
-            bh = rank - (rank / nbh) * nbh;
-        } else if (a.causal && a.hgroup > 0) {
-            // A grid of several rounds: head by head (heavy tile first) leaves heavy tiles for the very end of the dispatch order
-            // and a long tail (measured: a causal launch as slow as the unmasked one).  Take the heads in groups of a.hgroup and
-            // hand out the query tiles of a group heaviest first across its heads, so that every group -- the last one included --
-            // ends on its light tiles.  When every XCD owns whole heads the groups are formed inside the XCD's own heads.
-            const bool whole = rem == 0 && per % a.qtiles == 0;
-            const int heads = whole ? per / a.qtiles : nblk / a.qtiles;      // heads the groups are cut from
-            const int at = whole ? idx : logical;                            // position among their workgroups
-            const int gsz = heads < a.hgroup ? heads : a.hgroup;
-            const int per_group = gsz * a.qtiles;
-            const int grp = at / per_group, in = at - grp * per_group;
-            const int first = grp * gsz;
-            const int cur = heads - first < gsz ? heads - first : gsz;       // the last group may be short
-            qt = a.qtiles - 1 - in / cur;
-            bh = (whole ? xcd * heads : 0) + first + in % cur;
-        }
-    }
+    attn_block(a, bh, qt);
     const int b = bh / a.H, hd = bh - b * a.H;
     const int kvh = hd / (a.H / a.Hkv);
     const int q0 = qt * BR;
@@ -1548,6 +1512,7 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     // the fast kernel addresses K/V rows of a 4-key load group with unsigned 32-bit byte offsets
     const bool rows32 = p.ks[2] > 0 && p.ks[2] < (1LL << 28) && p.vs[2] > 0 && p.vs[2] < (1LL << 28);
     const bool dl = attn_dl_applies(kind, p);
+    const bool split = kind == 0 && attn_split_applies(a);      // fp32 on the fp16 matrix pipe (attention_split.hip)
     if (dl && p.workspace) {
         int chunk;
         const int ns = attn_dl_splits(p, &chunk);
@@ -1575,12 +1540,12 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
         if (kind == 1) err = p.out16 ? launch_attn_dl<f16_t, f16_t>(a, stream) : launch_attn_dl<f16_t, float>(a, stream);
         else err = p.out16 ? launch_attn_dl<bf16_t, bf16_t>(a, stream) : launch_attn_dl<bf16_t, float>(a, stream);
     } else
+    if (split) err = launch_attn_split(a, full, stream);
+    else
     if (kind == 0) {
         // fp32: 64-key tiles while two workgroups still fit the LDS of a CU (head dimension up to 64), else 32-key tiles
         if (p.D == 64 && dma && km) err = launch_attn<float, float, 64, 64, false, 2, true, true>(a, stream);
-        else if (p.D == 128 && dma && km) err = launch_attn<float, float, 128, 32, false, 2, true, true>(a, stream);
         else if (p.D == 64 && dma) err = launch_attn<float, float, 64, 64, false, 2, true>(a, stream);
-        else if (p.D == 128 && dma) err = launch_attn<float, float, 128, 32, false, 2, true>(a, stream);
         else if (p.D <= 64) err = full ? (p.D <= 32 ? launch_attn<float, float, 32, 64, true, 2>(a, stream) : launch_attn<float, float, 64, 64, true, 2>(a, stream))
                                   : (p.D <= 32 ? launch_attn<float, float, 32, 64, false, 2>(a, stream) : launch_attn<float, float, 64, 64, false, 2>(a, stream));
         else err = dispatch_attn_d<float, float, 32>(a, full, stream);
@@ -1610,7 +1575,8 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     if (err != hipSuccess) return err;
     if (p.weights) {
         a.lse = p.lse;
-        err = kind == 0 ? launch_weights<float>(a, p.weights, stream) : kind == 1 ? launch_weights<f16_t>(a, p.weights, stream)
+        err = split ? launch_attn_weights_split(a, p.weights, stream)
+              : kind == 0 ? launch_weights<float>(a, p.weights, stream) : kind == 1 ? launch_weights<f16_t>(a, p.weights, stream)
                                                                                   : launch_weights<bf16_t>(a, p.weights, stream);
     }
     return err;

@@ -42,6 +42,45 @@ struct AttnArgs {
     FastDiv dbsz;  // direct-to-LDS kernels on a paged cache: the block size as a divisor
 };
 
+// Workgroup -> (batch*head, query tile): XCD-contiguous so the q-tiles of one head share an L2;
+// late (heavy, under a causal mask) query tiles first.
+__device__ __forceinline__ void attn_block(const AttnArgs& a, int& bh, int& qt)
+{
+    int nblk = gridDim.x, pid = blockIdx.x;
+    int per = nblk >> 3, rem = nblk & 7;
+    int xcd = pid & 7, idx = pid >> 3;
+    int logical = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + idx;
+    bh = logical / a.qtiles;
+    qt = a.qtiles - 1 - (logical - bh * a.qtiles);
+    if (a.causal && a.hgroup < 0) {
+        // A grid that is resident all at once (at most three workgroups per CU) is not balanced by the order of
+        // dispatch: hand the query tiles out heaviest first across ALL heads, so the workgroups that end up sharing a
+        // CU are a heavy one and, later in the id order, a light one.
+        // (the first 256 ids, one per CU, in ascending weight, so that the ids after them -- which land on the same
+        // CUs in the same order -- pair the lightest of the first round with the heaviest of the second; reversed by eights, so that
+        // where 8 divides the number of heads all query tiles of a head stay on one XCD, 1-4 % against reversing one by one)
+        const int nbh = nblk / a.qtiles;
+        const int rank = (nblk > 256 && pid < 256) ? 255 - (pid | 7) + (pid & 7) : pid;
+        qt = a.qtiles - 1 - rank / nbh;
+        bh = rank - (rank / nbh) * nbh;
+    } else if (a.causal && a.hgroup > 0) {
+        // A grid of several rounds: head by head (heavy tile first) leaves heavy tiles for the very end of the dispatch order
+        // and a long tail (measured: a causal launch as slow as the unmasked one).  Take the heads in groups of a.hgroup and
+        // hand out the query tiles of a group heaviest first across its heads, so that every group -- the last one included --
+        // ends on its light tiles.  When every XCD owns whole heads the groups are formed inside the XCD's own heads.
+        const bool whole = rem == 0 && per % a.qtiles == 0;
+        const int heads = whole ? per / a.qtiles : nblk / a.qtiles;      // heads the groups are cut from
+        const int at = whole ? idx : logical;                            // position among their workgroups
+        const int gsz = heads < a.hgroup ? heads : a.hgroup;
+        const int per_group = gsz * a.qtiles;
+        const int grp = at / per_group, in = at - grp * per_group;
+        const int first = grp * gsz;
+        const int cur = heads - first < gsz ? heads - first : gsz;       // the last group may be short
+        qt = a.qtiles - 1 - in / cur;
+        bh = (whole ? xcd * heads : 0) + first + in % cur;
+    }
+}
+
 // Pool rows of a paged cache for the direct-to-LDS kernels.  A wave loads NK consecutive keys of every key tile (NK = 16 or 8), which
 // lie in one block when the block size is a multiple of 16, so one row number serves the wave and its loads keep the form of the
 // contiguous case (uniform base, fixed lane offsets).  Lane i of `rows` holds the row of the wave's first key in tile (tile0 + i), 64
@@ -218,6 +257,10 @@ __device__ __forceinline__ float merge_partials(const float* __restrict__ P, int
 // waves per row of the merge passes: one (four rows to a workgroup) while a row's ranges fit one round of loads
 inline int merge_waves_per_row(int ranges) { return ranges <= 8 ? 1 : 4; }
 
+// fp32 attention on the bf16 matrix pipe (attention_split.hip); options: bias, masks, soft-cap
+bool attn_split_applies(const AttnArgs& a);
+hipError_t launch_attn_split(const AttnArgs& a, bool options, hipStream_t stream);
+hipError_t launch_attn_weights_split(const AttnArgs& a, float* w, hipStream_t stream);
 // 16-bit, head dimension 128, plain / causal attention in the software-pipelined form (attention_prefill.hip); kind: 1 fp16, 2 bf16
 bool attn_prefill_applies(const AttnArgs& a);
 hipError_t launch_attn_prefill(int kind, int out16, AttnArgs a, hipStream_t stream);

@@ -1,0 +1,995 @@
+// fp32 attention on the fp16 matrix pipe.  Q, K, V and the probabilities are scaled by powers of two and held as two fp16 values each,
+// x = h + m (h = fp16(x), m = fp16(x - h): 22 to 23 of the 24 bits, no value further off than 2^-25 of a unit), and three of the four products
+// are formed, m h, h m, h h; what is left out, m m, is 2^-24 of a product at most.  Sums are fp32.
+//
+// Why fp16 and not bf16: three bf16 values hold every fp32 value whatever its size, but cost six products and 5.5 vector instructions a value where
+// two fp16 values cost three and 3 (2 for a probability, which needs no scale: one v_fma_mix_f32 takes the half of the packed word as it is), and
+// the vector pipe is what bounds the kernel (B8 H12 S512 d64 causal 37.8 us, 24 this way; the fp32 pipe 44).
+//
+// Scales.  Each row of Q has its own (its largest magnitude becomes 2^12 .. 2^13), K and V one per workgroup from its first tile (2^10 and 2^11:
+// later tiles may be 32 and 16 times larger).  Probabilities are formed against the next whole number above the row maximum, times 2^4, so that
+// their exponents are near zero where fp32 is fine (times 2^14 they were off by up to 3e-7).  What the split does not hold is computed again on
+// the fp32 pipe, by workgroup: results that are not finite (infinities, NaN, values beyond the first tile's scale), and those whose scale was set
+// by values far larger than what they are formed from (below).
+//
+// Error against float64, fp32 pipe / here, 2-norm: O of B8 H12 S512 d64 causal 2.82e-7 / 2.04e-7, plain 4.09e-7 / 3.23e-7, d128 5.66e-7 / 3.61e-7,
+// d32 4.64e-7 / 3.04e-7, S64 2.38e-7 / 1.93e-7; probabilities 3.21e-7 / 3.05e-7; log-sum-exp alike.
+#include "attention_common.hpp"
+#include <algorithm>
+
+namespace aidn {
+
+constexpr float P_EXP = 4.0f;        // probabilities are held times 2^4
+
+// Power of two (its exponent) that brings a magnitude into [2^to, 2^(to + 1)); 0 for zero
+__device__ __forceinline__ int exponent_to(float magnitude, int to)
+{
+    const int e = (int)(as_u32(magnitude) >> 23);
+    return magnitude == 0.0f ? 0 : min(max(to + 127 - e, -126), 126);
+}
+__device__ __forceinline__ float power2(int e) { return as_f32((uint32_t)(e + 127) << 23); }
+
+__device__ __forceinline__ uint32_t f16_pair(float a, float b)
+{
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), f16x2));
+    asm("" : "+v"(u));               // (opaque: the compiler otherwise converts the low half a second time by itself)
+    return u;
+}
+// a s, b s as h + m: one multiply-add per value takes the half of the packed word as it is.  UNIFORM: s is the same in every lane
+template <bool UNIFORM>
+__device__ __forceinline__ void split2(float a, float b, float s, uint32_t (&p)[2])
+{
+    p[0] = f16_pair(a * s, b * s);
+    float x, y;
+    if constexpr (UNIFORM) {
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(x) : "v"(a), "s"(s), "v"(p[0]));
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(b), "s"(s), "v"(p[0]));
+    } else {
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(x) : "v"(a), "v"(s), "v"(p[0]));
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(b), "v"(s), "v"(p[0]));
+    }
+    p[1] = f16_pair(x, y);
+}
+__device__ __forceinline__ void split2(float a, float b, uint32_t (&p)[2])
+{
+    p[0] = f16_pair(a, b);
+    float x, y;
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(x) : "v"(a), "v"(p[0]));
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(b), "v"(p[0]));
+    p[1] = f16_pair(x, y);
+}
+__device__ __forceinline__ float wave_max(float v)
+{
+    auto step = [&](auto ctrl) { v = fmaxf(v, as_f32((uint32_t)__builtin_amdgcn_mov_dpp((int)as_u32(v), decltype(ctrl)::value, 0xF, 0xF, true))); };
+    step(std::integral_constant<int, 0xB1>{});          // lanes 1 and 2 apart, then the mirrors of 8 and 16 lanes
+    step(std::integral_constant<int, 0x4E>{});
+    step(std::integral_constant<int, 0x141>{});
+    step(std::integral_constant<int, 0x140>{});
+    return max_with_partner32(max_with_partner16(v));
+}
+
+// eight values to a chunk of either plane
+template <bool UNIFORM>
+__device__ __forceinline__ void split8(const u32x4 (&r)[2], float s, u32x4 (&w)[2])
+{
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        uint32_t p[2];
+        split2<UNIFORM>(as_f32(r[e >> 1][2 * (e & 1)]), as_f32(r[e >> 1][2 * (e & 1) + 1]), s, p);
+        w[0][e] = p[0];
+        w[1][e] = p[1];
+    }
+}
+__device__ __forceinline__ float largest(const u32x4 (&r)[2])
+{
+    float m = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) m = fmaxf(m, fabsf(as_f32(r[e >> 2][e & 3])));
+    return m;
+}
+// Q operand: lane (l32, h) holds values 16 s + 8 h .. + 7 of row l32, the row scaled to its own largest magnitude; returns that exponent
+template <int DS>
+__device__ __forceinline__ int split_q(const float* __restrict__ row, bool exists, int D, int h, u32x4 (&qf)[DS][2])
+{
+    u32x4 r[DS][2];
+    float most = 0.0f;
+#pragma unroll
+    for (int s = 0; s < DS; s++) {
+        const int d0 = 16 * s + 8 * h;
+        r[s][0] = r[s][1] = u32x4{0u, 0u, 0u, 0u};
+        if (exists && d0 < D) {
+            r[s][0] = *(const u32x4*)(row + d0);
+            r[s][1] = *(const u32x4*)(row + d0 + 4);
+        }
+        most = fmaxf(most, largest(r[s]));
+    }
+    most = max_with_partner32(most);
+    const int e = most == 0.0f ? 126 : exponent_to(most, 12);      // (logits of a row of zeros are not coarse)
+#pragma unroll
+    for (int s = 0; s < DS; s++) split8<false>(r[s], power2(e), qf[s]);
+    return e;
+}
+// Byte offset of 16-byte chunk `ch` (eight values) of row `key` of a plane with rows of RB bytes.  K is read as 16 rows of one chunk at a time,
+// V as four chunks of 4 rows; PER rows until the bank repeats
+template <int RB> constexpr int PER = RB == 256 ? 1 : RB == 128 ? 2 : 4;
+template <int RB> __device__ __forceinline__ int k_at(int key, int ch) { return key * RB + ((ch ^ ((key / PER<RB>) & (16 / PER<RB> - 1))) << 4); }
+template <int RB> __device__ __forceinline__ int v_at(int key, int ch) { return key * RB + ((ch ^ (((key / PER<RB>) & (4 / PER<RB> - 1)) << 2)) << 4); }
+
+// LDS: the planes of a tile of K and of V, or behind the last tile the results of all key groups but the first, then 16 rows of each wave
+constexpr int split_lds(int DP, int BC, int NW, int KG)
+{
+    const int tiles = 8 * BC * DP, merge = (KG - 1) * (NW / KG) * (DP * 32 + 128) * 4, rows = NW / KG * 16 * DP * 4;
+    return tiles > merge ? (tiles > rows ? tiles : rows) : (merge > rows ? merge : rows);
+}
+
+// One workgroup: NW waves of 32 query rows each, KG of them on the same rows and different keys of a tile.
+//
+// S^T = K Q^T and O^T += V^T P^T as in attn_fwd_kernel, on v_mfma_f32_32x32x16_f16: a lane holds one query, its row maximum is an in-lane reduction and
+// one exchange, and P is the second product's operand as it stands.  K and V are loaded to registers a tile ahead, split there and kept in LDS as
+// planes of [key][d] rows, single: V of a tile is written beside the first product and K of the next one beside the second, a barrier behind
+// either.  (Both twice in LDS with one barrier a tile: 24.4 -> 27.8 us, the loads then land a phase later.)
+//
+// Bound by issue: per 64 keys (d64) a wave issues about 400 vector instructions, 48 MFMAs and 70 LDS operations, and matrix and vector work of the
+// two waves of a SIMD overlap only in part (counted: vector pipe 63 % of a full CU's cycles, matrix pipe 44 %; no LDS bank conflicts).  Against the
+// fp32 pipe, us: B8 H12 S512 d64 causal 44 / 24, plain 69 / 32; B2 H16 S2048 causal d64 165 / 71, d128 310 / 131; B8 H16 S512 d32 48 / 23; bias, masks
+// and soft-cap alike (B4 H12 S512 d64 padded 40 / 24, soft-cap 62 / 36).
+template <int DP, int BC, int NW, int KG, bool OPT, bool PAGED>
+__global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a)
+{
+    constexpr int NT = 64 * NW, WQ = NW / KG, BR = 32 * WQ;
+    constexpr int RB = 2 * DP, PL = BC * RB;      // bytes of a row of a plane, of a plane
+    constexpr int KT = BC / 32 / KG;              // 32-key sub-tiles of a wave in a tile
+    constexpr int DS = DP / 16, DT = DP / 32;     // 16-wide steps and 32-wide blocks of the head dimension
+    constexpr int CPR = DP / 8;                   // chunks of eight values of a row
+    constexpr int U = BC * CPR / NT;              // chunks of K (and of V) that a thread stages per tile
+    constexpr int RPU = NT / CPR;                 // rows between a thread's chunks
+    constexpr int AHEAD = !OPT;       // fragments are read a step ahead where the registers hold two sets
+    static_assert(BC * CPR % NT == 0 && KT > 0 && (RPU % 16 == 0 || U == 1), "whole chunks to a thread, at one place of rows that share a swizzle");
+
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    unsigned char* Ks = smem;                     // [2][BC][DP] fp16
+    unsigned char* Vs = smem + 2 * PL;            // [2][BC][DP] fp16
+
+    int t = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    int lane = t & 63, l32 = lane & 31, h = lane >> 5;
+    int bh, qt;
+    attn_block(a, bh, qt);
+    const int b = bh / a.H, hd = bh - b * a.H;
+    const int kvh = hd / (a.H / a.Hkv);
+    const int wq = wave % WQ, kg = wave / WQ;
+    const int q0 = qt * BR + wq * 32;             // first query row of this wave
+    const float* __restrict__ Q = (const float*)a.q + b * a.qs[0] + hd * a.qs[1];
+    const float* __restrict__ K = (const float*)a.k + b * a.ks[0] + kvh * a.ks[1];
+    const float* __restrict__ V = (const float*)a.v + b * a.vs[0] + kvh * a.vs[1];
+    const int* __restrict__ bt = PAGED ? a.bt + b * a.bt_bs : nullptr;
+
+    int ntiles = (a.Sk + BC - 1) / BC;
+    if (a.causal) {
+        const long long lastkey = (long long)qt * BR + BR - 1 + a.qoff;
+        if (lastkey < 0) ntiles = 0;
+        else { const long long nt = lastkey / BC + 1; if (nt < ntiles) ntiles = (int)nt; }
+    }
+
+    // ---- staging: thread t takes chunk t % CPR of keys t / CPR + i RPU
+    u32x4 rk[U][2], rv[U][2];
+    const int col = min(8 * (t % CPR), a.D - 8);   // (chunks past the head dimension repeat the last one: they meet zeros of Q, or are not stored)
+    // what is asked for next: byte offsets of the rows, which follow the tiles and stop at the last row; paged, rows of the pool, looked up a
+    // tile ahead
+    uint32_t kat[U], vat[U], klast = 0, vlast = 0;
+    auto rows_of = [&](int tile) {
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            const int key = min(tile * BC + t / CPR + i * RPU, a.Sk - 1), blk = (int)fastdiv((uint32_t)key, a.dbsz);
+            kat[i] = bt[blk] * a.bsz + (key - blk * a.bsz);
+        }
+    };
+    auto load = [&](const float* __restrict__ src, uint32_t rs, uint32_t (&at)[U], uint32_t last, u32x4 (&v)[U][2]) {
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            const unsigned char* p;
+            if constexpr (PAGED) p = (const unsigned char*)(src + (uint64_t)at[i] * rs + col);
+            else p = (const unsigned char*)src + at[i];
+            v[i][0] = *(const u32x4*)p;
+            v[i][1] = *(const u32x4*)(p + 16);
+            if constexpr (!PAGED) at[i] = min(at[i] + 4u * BC * rs, last);
+        }
+    };
+    float ksc = 1.0f, vsc = 1.0f;
+    auto store_k = [&](int i) {
+        u32x4 w[2];
+        split8<true>(rk[i], ksc, w);
+#pragma unroll
+        for (int s = 0; s < 2; s++) *(u32x4*)(Ks + s * PL + i * RPU * RB + k_at<RB>(t / CPR, t % CPR)) = w[s];
+    };
+    auto store_v = [&](int i) {
+        u32x4 w[2];
+        split8<true>(rv[i], vsc, w);
+#pragma unroll
+        for (int s = 0; s < 2; s++) *(u32x4*)(Vs + s * PL + i * RPU * RB + v_at<RB>(t / CPR, t % CPR)) = w[s];
+    };
+    const uint32_t krs = (uint32_t)a.ks[2], vrs = (uint32_t)a.vs[2];
+    if (ntiles > 0) {
+        if constexpr (PAGED) rows_of(0);
+        else {
+            klast = 4u * ((uint32_t)(a.Sk - 1) * krs + col);
+            vlast = 4u * ((uint32_t)(a.Sk - 1) * vrs + col);
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                kat[i] = min(4u * ((uint32_t)(t / CPR + i * RPU) * krs + col), klast);
+                vat[i] = min(4u * ((uint32_t)(t / CPR + i * RPU) * vrs + col), vlast);
+            }
+        }
+        load(K, krs, kat, klast, rk);
+        load(V, vrs, PAGED ? kat : vat, vlast, rv);
+        if constexpr (PAGED) rows_of(1);
+    }
+
+    u32x4 qf[DS][2];
+    int logit_exp = -split_q(Q + (long long)min(q0 + l32, a.Sq - 1) * a.qs[2], q0 + l32 < a.Sq, a.D, h, qf);      // logits are 2^logit_exp Q' K'
+    // ---- K and V: one power of two each, from the first tile
+    int vexp = 0;
+    if (ntiles > 0) {
+        float km = 0.0f, vm = 0.0f;
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            km = fmaxf(km, largest(rk[i]));
+            vm = fmaxf(vm, largest(rv[i]));
+        }
+        km = wave_max(km);
+        vm = wave_max(vm);
+        float* red = (float*)Vs;
+        if (lane == 0) { red[wave] = km; red[NW + wave] = vm; }
+        __syncthreads();
+        km = vm = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) { km = fmaxf(km, red[w]); vm = fmaxf(vm, red[NW + w]); }
+        const int kexp = __builtin_amdgcn_readfirstlane(exponent_to(km, 10));
+        vexp = __builtin_amdgcn_readfirstlane(exponent_to(vm, 11));
+        ksc = power2(kexp);
+        vsc = power2(vexp);
+        logit_exp -= kexp;
+#pragma unroll
+        for (int i = 0; i < U; i++) store_k(i);
+        __syncthreads();                           // (the maxima have been read before V is written over them)
+    }
+
+    f32x16 oacc[DT];
+    float m_run, l_run;
+    auto clear = [&]() {
+        m_run = -INFINITY;
+        l_run = 0.0f;
+#pragma unroll
+        for (int i = 0; i < DT; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) oacc[i][r] = 0.0f;
+    };
+    clear();
+
+    float to_log2 = __builtin_ldexpf(a.scale * LOG2E, logit_exp);       // OPT: the logit itself
+    if constexpr (OPT) to_log2 = __builtin_ldexpf(a.scale, logit_exp);
+    // What the split cuts of Q' and K' (2^-25 of a value) shows in a logit as about 2^-12 of a unit of Q' K'.  Where that is more than 2^-25 of an
+    // exponent the row's logits have to be large themselves (2^13 units), or it is computed again: large values that meet zeros, or keys out of
+    // the row's sight, can have set the scale
+    const bool coarse = to_log2 > 0x1p-13f, any_coarse = __builtin_amdgcn_ballot_w64(coarse) != 0;
+    float largest_logit = 0.0f;
+    // logits of NB 32-key sub-tiles from key k0 on (st[kt][r]: key k0 + 32 kt + acc_row(r, h), query q0 + l32) to probabilities times 2^P_EXP against
+    // the new running maximum; returns what the sums so far are to be multiplied with.  Bit i of `kept`: key k0 + i is visible (OPT)
+    auto softmax = [&](auto& st, int k0, uint64_t kept) -> float {
+        constexpr int NB = sizeof(st) / sizeof(st[0]);
+        float factor = to_log2;
+        if constexpr (OPT) {
+            const int key0 = k0 + 4 * h;
+            int qr = __lane_id();
+            asm volatile("" : "+v"(qr));
+            qr = min(q0 + (qr & 31), a.Sq - 1);
+            factor = LOG2E;
+#pragma unroll
+            for (int kt = 0; kt < NB; kt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) st[kt][r] *= to_log2;
+            if (a.softcap > 0.0f) {
+#pragma unroll
+                for (int kt = 0; kt < NB; kt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        st[kt][r] = a.softcap * tanhf(st[kt][r] / a.softcap);
+                        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+            if (a.bias) {
+                const float* __restrict__ row = a.bias + b * a.bias_bs + ((long long)hd * a.Sq + qr) * a.Sk;
+#pragma unroll
+                for (int kt = 0; kt < NB; kt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        st[kt][r] += row[min(key0 + 32 * kt + acc_row(r, 0), a.Sk - 1)];
+                        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+            if (a.mask_mode == 1 || a.mask_mode == 2) {
+                const float* __restrict__ row = a.mask + ((a.mask_mode == 2 ? (long long)bh * a.Sq : 0LL) + qr) * a.Sk;
+#pragma unroll
+                for (int kt = 0; kt < NB; kt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        if (row[min(key0 + 32 * kt + acc_row(r, 0), a.Sk - 1)] == 0.0f) st[kt][r] = -INFINITY;
+                        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+        }
+        if (k0 + 32 * NB > a.Sk || (a.causal && (long long)k0 + 32 * NB - 1 > (long long)q0 + a.qoff)) {
+            // (formed here, not kept through the loop)
+            int at = __lane_id();
+            asm volatile("" : "+v"(at));
+            const int first = -4 * (at >> 5);
+            at &= 31;
+            // the query's last visible key, relative to the lane's first
+            int seen = a.Sk - 1 - k0 + first;
+            if (a.causal) seen = min(seen, (int)max(min((long long)q0 + a.qoff - k0, 1LL << 20), -(1LL << 20)) + at + first);
+#pragma unroll
+            for (int kt = 0; kt < NB; kt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) if (32 * kt + acc_row(r, 0) > seen) st[kt][r] = -INFINITY;
+        }
+        if constexpr (OPT) {
+            if (kept != ~0ull) {
+                int half = __lane_id();
+                asm volatile("" : "+v"(half));
+                half >>= 5;
+#pragma unroll
+                for (int kt = 0; kt < NB; kt++) {
+                    const uint32_t bits = (uint32_t)(kept >> (32 * kt)) >> (4 * half);
+#pragma unroll
+                    for (int r = 0; r < 16; r++) if (!(bits >> acc_row(r, 0) & 1u)) st[kt][r] = -INFINITY;
+                }
+            }
+        }
+        if constexpr (!OPT) {
+            if (any_coarse) {
+#pragma unroll
+                for (int kt = 0; kt < NB; kt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) largest_logit = fmaxf(largest_logit, st[kt][r] == -INFINITY ? 0.0f : fabsf(st[kt][r]));
+            }
+        }
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < NB; kt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, st[kt][r]);
+        // (the reference is the next whole number: what is subtracted and what the sums are rescaled with are then exact)
+        const float m_new = fmaxf(m_run, ceilf(max_with_partner32(mloc) * factor));
+        const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        const float down = P_EXP - m_use;
+        m_run = m_new;
+        float psum = 0.0f;
+#pragma unroll
+        for (int kt = 0; kt < NB; kt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float p = __builtin_amdgcn_exp2f(fmaf(st[kt][r], factor, down));
+                st[kt][r] = p;
+                psum += p;
+            }
+        l_run = l_run * alpha + psum;
+        return alpha;
+    };
+
+    auto visible = [&](int k0, int n) -> uint64_t {        // keep-mask of the keys: bit i of the result is key k0 + i
+        int ln = __lane_id();
+        asm volatile("" : "+v"(ln));
+        return __builtin_amdgcn_ballot_w64(ln < n && k0 + ln < a.Sk && ((const unsigned char*)a.mask)[(long long)b * a.Sk + min(k0 + ln, a.Sk - 1)] != 0);
+    };
+
+    const int q_last = q0 + 31;
+    const unsigned char* kbase = Ks + (kg * KT * 32) * RB;
+    const unsigned char* vbase = Vs + (kg * KT * 32) * RB;
+    const int jl = lane & 15, vkey = 4 * h + (jl >> 2), vch = 2 * ((lane >> 4) & 1) + ((jl & 3) >> 1), vcol = 8 * (jl & 1);      // transposing reads
+    for (int j = 0; j < ntiles; j++) {
+        const int kw0 = j * BC + kg * KT * 32;                      // this wave's first key
+        load(K, krs, kat, klast, rk);                                 // (past the last tile rows are repeated)
+        uint64_t kept = ~0ull;
+        if constexpr (OPT) { if (a.mask_mode == 3) kept = visible(kw0, KT * 32) | (KT == 1 ? ~0ull << 32 : 0ull); }
+        const bool none = OPT && (KT == 1 ? (uint32_t)kept == 0 : kept == 0);
+        const bool active = q0 < a.Sq && kw0 < a.Sk && !(a.causal && (long long)kw0 > (long long)q_last + a.qoff) && !none;
+        f32x16 st[KT];
+        // ---- S^T = K Q^T, beside it V to LDS
+        if (active) {
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) st[kt][r] = 0.0f;
+            f16x8 k[AHEAD + 1][KT][2];
+            auto read_k = [&](int s) {
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                    for (int p = 0; p < 2; p++) k[s & AHEAD][kt][p] = *(const f16x8*)(kbase + p * PL + kt * 32 * RB + k_at<RB>(l32, 2 * s + h));
+            };
+            if (AHEAD) read_k(0);
+#pragma unroll
+            for (int s = 0; s < DS; s++) {
+                if (s + AHEAD < DS) read_k(s + AHEAD);
+                auto add = [&](int x, int y) {
+#pragma unroll
+                    for (int kt = 0; kt < KT; kt++) st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k[s & AHEAD][kt][x], __builtin_bit_cast(f16x8, qf[s][y]), st[kt], 0, 0, 0);
+                };
+                add(1, 0); add(0, 1); add(0, 0);
+                if (s < U) store_v(s);
+                if (OPT && DP > 64) __builtin_amdgcn_sched_barrier(0);
+            }
+            static_assert(U <= DS && U <= 2 * KT, "a chunk beside every step");
+        } else {
+#pragma unroll
+            for (int i = 0; i < U; i++) store_v(i);
+        }
+        load(V, vrs, PAGED ? kat : vat, vlast, rv);
+        if constexpr (PAGED) rows_of(j + 2);
+        __syncthreads();
+        // ---- O^T += V^T P^T, beside it the next K to LDS
+        if (active) {
+            const float alpha = softmax(st, kw0, kept);
+            if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+                for (int i = 0; i < DT; i++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
+            }
+            constexpr int G = DT < 2 || DP > 64 || !AHEAD ? 1 : 2, STEPS = 2 * KT * (DT / G);      // blocks of the head dimension side by side; 16 keys to a step
+            u32x4 pf[2 * KT][2];
+            f16x8 v[AHEAD + 1][G][2];
+            auto split_p = [&](int ps) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    uint32_t p[2];
+                    split2(st[ps >> 1][8 * (ps & 1) + 2 * e], st[ps >> 1][8 * (ps & 1) + 2 * e + 1], p);
+                    pf[ps][0][e] = p[0];
+                    pf[ps][1][e] = p[1];
+                }
+            };
+            auto read_v = [&](int u) {
+                const int i0 = u / (2 * KT) * G, ps = u % (2 * KT);
+#pragma unroll
+                for (int i = 0; i < G; i++)
+#pragma unroll
+                    for (int p = 0; p < 2; p++) {
+                        u32x4 w;
+#pragma unroll
+                        for (int q = 0; q < 2; q++) {
+                            const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                (__attribute__((address_space(3))) s16x4a*)(vbase + p * PL + (16 * ps + 8 * q) * RB + v_at<RB>(vkey, 4 * (i0 + i) + vch) + vcol)));
+                            w[2 * q] = x[0];
+                            w[2 * q + 1] = x[1];
+                        }
+                        v[u & AHEAD][i][p] = __builtin_bit_cast(f16x8, w);
+                    }
+            };
+            if (AHEAD) read_v(0);
+            split_p(0);
+#pragma unroll
+            for (int u = 0; u < STEPS; u++) {
+                const int i0 = u / (2 * KT) * G, ps = u % (2 * KT);
+                if (u + AHEAD < STEPS) read_v(u + AHEAD);
+                if (u + 1 < 2 * KT) split_p(u + 1);
+                auto add = [&](int x, int y) {
+#pragma unroll
+                    for (int i = 0; i < G; i++)
+                        oacc[i0 + i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[u & AHEAD][i][x], __builtin_bit_cast(f16x8, pf[ps][y]), oacc[i0 + i], 0, 0, 0);
+                };
+                add(1, 0); add(0, 1); add(0, 0);
+                if (u < U) store_k(u);
+                if (OPT && DP > 64) __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < U; i++) store_k(i);
+        }
+        __syncthreads();
+    }
+
+    // ---- does the split hold these results?  (What follows is addressed from here: nothing of it is kept through the loop.)
+    lane = __lane_id();
+    asm volatile("" : "+v"(lane));
+    t = 64 * wave + lane;
+    l32 = lane & 31;
+    h = lane >> 5;
+    {
+        float poison = l_run * 0.0f;
+#pragma unroll
+        for (int i = 0; i < DT; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) poison = fmaf(oacc[i][r], 0.0f, poison);
+        bool bad = poison != poison;               // infinities, NaN, values beyond the scale of the first tile
+        if (any_coarse) bad |= coarse && l_run > 0.0f && (OPT || fmaxf(largest_logit, shfl_xor_f(largest_logit, 32)) < 0x1p13f);
+        // a column of O without a value of 2^-5 units of V' (whose largest in the first tile is 2^11 or more) may come from a column of V that the
+        // scale has left too few bits of
+        const float witness = l_run > 0.0f ? l_run * 0x1p-4f : INFINITY;          // (either half's share of the row sum is at most all of it)
+        uint32_t unseen = 0;
+#pragma unroll
+        for (int i = 0; i < DT; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const uint64_t w = __builtin_amdgcn_ballot_w64(fabsf(oacc[i][r]) >= witness);
+                unseen |= (uint32_t)w == 0 || (uint32_t)(w >> 32) == 0;
+            }
+        const bool look = unseen && __builtin_amdgcn_ballot_w64(l_run > 0.0f) != 0;
+        __shared__ int flags[NW];
+        auto any_thread = [&](bool x) {            // (with less to keep in registers than __syncthreads_or, which wants the thread's y and z)
+            const bool mine = __builtin_amdgcn_ballot_w64(x) != 0;
+            if (lane == 0) flags[wave] = mine;
+            __syncthreads();
+            int any = 0;
+#pragma unroll
+            for (int w = 0; w < NW; w++) any |= flags[w];
+            __syncthreads();
+            return __builtin_amdgcn_readfirstlane(any) != 0;
+        };
+        bool again = any_thread(bad | look);
+        if (again && !any_thread(bad)) {
+            // the columns' largest magnitudes
+            uint32_t* top = (uint32_t*)smem;
+            for (int d = t; d < DP; d += NT) top[d] = 0;
+            __syncthreads();
+            const int keys = min(ntiles * BC, a.Sk), d0 = 4 * (t % (DP / 4));
+            if (d0 < a.D) {
+                f32x4 m = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+                for (int key = t / (DP / 4); key < keys; key += NT / (DP / 4)) {
+                    const f32x4 x = *(const f32x4*)(V + paged_row(bt, a.bsz, key) * a.vs[2] + d0);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) m[e] = fmaxf(m[e], fabsf(x[e]));
+                }
+#pragma unroll
+                for (int e = 0; e < 4; e++) atomicMax(top + d0 + e, as_u32(m[e]));      // (not negative: ordered like their bits)
+            }
+            __syncthreads();
+            bool small = false;
+            for (int d = t; d < DP; d += NT) small |= top[d] != 0 && as_f32(top[d]) * vsc < 0.5f;
+            again = any_thread(small);
+        }
+        if (again) {
+            // again on the fp32 pipe, rows straight from memory
+            clear();
+            vexp = 0;
+            to_log2 = OPT ? a.scale : a.scale * LOG2E;
+#pragma unroll 1
+            for (int k0 = kg * KT * 32; k0 < ntiles * BC; k0 += k0 % (KT * 32) + 32 < KT * 32 ? 32 : BC - (KT - 1) * 32) {
+                if (q0 >= a.Sq || k0 >= a.Sk || (a.causal && (long long)k0 > (long long)q_last + a.qoff)) continue;
+                uint64_t kept = ~0ull;
+                if constexpr (OPT) { if (a.mask_mode == 3) kept = visible(k0, 32) | ~0ull << 32; }
+                if (OPT && (uint32_t)kept == 0) continue;
+                f32x16 s2[1];
+#pragma unroll
+                for (int r = 0; r < 16; r++) s2[0][r] = 0.0f;
+                const float* kp = K + paged_row(bt, a.bsz, min(k0 + l32, a.Sk - 1)) * a.ks[2] + 4 * h;
+                const float* qp = Q + (long long)min(q0 + l32, a.Sq - 1) * a.qs[2] + 4 * h;
+#pragma unroll 1
+                for (int d = 0; d < a.D; d += 8) Mma32<float>::run(s2[0], *(const u32x4*)(kp + d), *(const u32x4*)(qp + d));
+                const float alpha = softmax(s2, k0, kept);
+                const float* vp[16];
+#pragma unroll
+                for (int r = 0; r < 16; r++) vp[r] = V + paged_row(bt, a.bsz, min(k0 + acc_row(r, h), a.Sk - 1)) * a.vs[2];
+#pragma unroll
+                for (int i = 0; i < DT; i++) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        float x = vp[r][min(32 * i + l32, a.D - 1)];
+                        if (k0 + acc_row(r, h) >= a.Sk) x = 0.0f;              // (an infinite last row is not repeated)
+                        oacc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, s2[0][r], oacc[i], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+    }
+
+    // ---- the waves of key groups 1 .. KG - 1 leave (O, m, l) in LDS, group 0 merges them
+    if constexpr (KG > 1) {
+        constexpr int AREA = DT * 16 * 64;                          // floats of one wave's O
+        float* O1 = (float*)smem + wq * (KG - 1) * AREA;
+        float* ML = (float*)smem + (KG - 1) * WQ * AREA + wq * (KG - 1) * 128;
+        __syncthreads();
+        if (kg > 0) {
+            f32x4* dst = (f32x4*)(O1 + (kg - 1) * AREA);
+#pragma unroll
+            for (int i = 0; i < DT; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    dst[(i * 4 + g) * 64 + lane] = f32x4{oacc[i][4 * g], oacc[i][4 * g + 1], oacc[i][4 * g + 2], oacc[i][4 * g + 3]};
+            ML[(kg - 1) * 128 + lane] = m_run;
+            ML[(kg - 1) * 128 + 64 + lane] = l_run;
+        }
+        __syncthreads();
+        if (kg == 0) {
+#pragma unroll
+            for (int u = 0; u < KG - 1; u++) {
+                const float m1 = ML[u * 128 + lane], l1 = ML[u * 128 + 64 + lane];
+                const float m_new = fmaxf(m_run, m1), m_use = m_new == -INFINITY ? 0.0f : m_new;
+                const float w0 = __builtin_amdgcn_exp2f(m_run - m_use), w1 = __builtin_amdgcn_exp2f(m1 - m_use);
+                m_run = m_new;
+                l_run = l_run * w0 + l1 * w1;
+                const f32x4* src = (const f32x4*)(O1 + u * AREA);
+#pragma unroll
+                for (int i = 0; i < DT; i++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const f32x4 v = src[(i * 4 + g) * 64 + lane];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) oacc[i][4 * g + e] = oacc[i][4 * g + e] * w0 + v[e] * w1;
+                    }
+            }
+        }
+        __syncthreads();
+        if (kg > 0) return;
+    }
+
+    // ---- normalise and store: lane holds query q0 + l32, head-dim elements 32 i + 8 g + 4 h + (0..3)
+    const int qi = q0 + l32;
+    const float l = sum_with_partner32(l_run);
+    const float inv = l > 0.0f ? power2(-vexp) / l : 0.0f;
+    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? (m_run + (__builtin_amdgcn_logf(l) - P_EXP)) * LN2 : -INFINITY;
+    float* __restrict__ O = (float*)a.o + b * a.os[0] + hd * a.os[1];
+    if (a.vec_out && a.D == DP) {
+        // through LDS (16 rows at a time for each wave: chunk c of row r at position c ^ r) and written as whole rows past the caches
+        constexpr int CH = DP / 4, RPI = 64 / CH;
+        unsigned char* stg = smem + wq * (16 * DP * 4);
+        const int c = lane % CH;
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            if ((l32 >> 4) == half) {
+#pragma unroll
+                for (int i = 0; i < DT; i++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++)
+                        *(f32x4*)(stg + (l32 & 15) * (DP * 4) + (((8 * i + 2 * g + h) ^ (l32 & (CH - 1) & 15)) << 4)) =
+                            f32x4{oacc[i][4 * g] * inv, oacc[i][4 * g + 1] * inv, oacc[i][4 * g + 2] * inv, oacc[i][4 * g + 3] * inv};
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int q = 0; q < 16 / RPI; q++) {
+                const int r = RPI * q + lane / CH, row = q0 + 16 * half + r;
+                const f32x4 v = *(const f32x4*)(stg + r * (DP * 4) + ((c ^ (r & (CH - 1) & 15)) << 4));
+                if (row < a.Sq) __builtin_nontemporal_store(v, (f32x4*)(O + (long long)row * a.os[2] + 4 * c));
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    } else if (qi < a.Sq) {
+        float* __restrict__ p = O + (long long)qi * a.os[2];
+#pragma unroll
+        for (int i = 0; i < DT; i++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int d0 = 32 * i + 8 * g + 4 * h;
+                if (a.vec_out) { if (d0 < a.D) *(f32x4*)(p + d0) = f32x4{oacc[i][4 * g] * inv, oacc[i][4 * g + 1] * inv, oacc[i][4 * g + 2] * inv, oacc[i][4 * g + 3] * inv}; }
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) if (d0 + e < a.D) p[d0 + e] = oacc[i][4 * g + e] * inv;
+                }
+            }
+    }
+}
+
+template <int DP, int BC, int NW, int KG, bool OPT, bool PAGED>
+static hipError_t launch_split_as(AttnArgs a, hipStream_t stream)
+{
+    constexpr int BR = 32 * NW / KG, smem = split_lds(DP, BC, NW, KG);
+    auto kern = attn_split_kernel<DP, BC, NW, KG, OPT, PAGED>;
+    static unsigned long long attr_done = 0;
+    if (hipError_t e = ensure_dynamic_smem((const void*)kern, smem, &attr_done)) return e;
+    a.qtiles = (a.Sq + BR - 1) / BR;
+    const long long nblk = (long long)a.qtiles * a.B * a.H;
+    if (nblk > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+    a.hgroup = !a.causal ? 0 : nblk <= 768 ? -1 : (a.qtiles >= 8 ? 16 : (128 + a.qtiles - 1) / a.qtiles);
+    hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(64 * NW), smem, stream, a);
+    return hipGetLastError();
+}
+
+// keys that some query sees
+static long long seen_keys(const AttnArgs& a) { return a.causal ? std::min((long long)a.Sk, (long long)a.Sq + a.qoff) : a.Sk; }
+
+// fp32, rows on the 16-byte grid, head dimension up to 128 in whole chunks of eight, a head's K and V within 4 GB (contiguous).  At head
+// dimensions 33 .. 64 up to 64 keys stay on the fp32 pipe: one tile of them costs less than the splitting beside it (us: B1 H8 S52 7.9 / 8.6, B15 H32
+// S27 8.5 / 9.8; 71 keys 10.0 / 9.0; d32 S53 6.9 / 7.0, d128 S62 12.1 / 12.2)
+bool attn_split_applies(const AttnArgs& a)
+{
+    auto fits = [&](long long row) { return row > 0 && row < (1LL << 30) && (a.bt || row * a.Sk < (1LL << 30)); };
+    if (a.bt && (a.bias || a.mask_mode != 0 || a.softcap > 0.0f)) return false;
+    if (a.D > 32 && a.D <= 64 && seen_keys(a) <= 64) return false;
+    return a.vec_in && a.D % 8 == 0 && a.D <= 128 && a.scale > 0.0f && a.scale < 0x1p20f && fits(a.ks[2]) && fits(a.vs[2]);
+}
+
+// Waves and key groups.  A wave alone on its SIMD issues half as fast as two do together, so grids that do not fill the chip take workgroups of
+// fewer rows whose waves share the keys; full grids lose by it (every workgroup splits the K and V that it reads).  From 128 drawn shapes, us with
+// 128 rows / 64 rows in two key groups / 64 rows of eight waves in four:
+//   d64: four groups up to 256 workgroups from 448 keys on (S1024 H12 36 / 28 / 25; S300 H16 16.2 / 13.9 / 14.5)
+//        two groups up to 64 queries, causal up to 640 workgroups (B4 H12 S512 21.5 / 18.7; 576: 28.8 / 26.5; 768: 24.8 / 29.7), plain up to 256
+//        (264: 44.4 / 46.0) and where the coarser grid just needs a second workgroup per CU (280 of 128 rows 31.4 / 25.8)
+//   d32: two groups up to 768 (648: 16.4 / 14.6; 2520: 97 / 109), four as above (S1525 H12 33 / 27 / 21)
+//   d65 .. 128: 64-key tiles of eight waves in two groups up to 256 from 224 keys on (S1024 H8 65 / 54; B2 H16 S512 37.7 / 33.5; 288: 27 / 36; S152 19.0 / 20.3),
+//        else 32-key tiles
+template <bool OPT, bool PAGED>
+static hipError_t launch_split_opt(const AttnArgs& a, hipStream_t stream)
+{
+    auto grid = [&](int rows) { return (long long)((a.Sq + rows - 1) / rows) * a.B * a.H; };
+    if (a.D <= 32) {
+        if (grid(64) <= 256 && seen_keys(a) >= 448) return launch_split_as<32, 128, 8, 4, OPT, PAGED>(a, stream);
+        return a.Sq <= 64 || grid(64) <= 768 ? launch_split_as<32, 64, 4, 2, OPT, PAGED>(a, stream) : launch_split_as<32, 64, 4, 1, OPT, PAGED>(a, stream);
+    }
+    if (a.D <= 64) {
+        if (grid(64) <= 256 && seen_keys(a) >= 448) return launch_split_as<64, 128, 8, 4, OPT, PAGED>(a, stream);
+        const bool fine = a.Sq <= 64 || (a.causal ? grid(64) <= 640 : grid(64) <= 256 || (grid(128) > 256 && grid(64) <= 512));
+        return fine ? launch_split_as<64, 64, 4, 2, OPT, PAGED>(a, stream) : launch_split_as<64, 64, 4, 1, OPT, PAGED>(a, stream);
+    }
+    return grid(128) <= 256 && seen_keys(a) >= 224 ? launch_split_as<128, 64, 8, 2, OPT, PAGED>(a, stream) : launch_split_as<128, 32, 4, 1, OPT, PAGED>(a, stream);
+}
+hipError_t launch_attn_split(const AttnArgs& a, bool options, hipStream_t stream)
+{
+    if (a.bt) return launch_split_opt<false, true>(a, stream);
+    return options ? launch_split_opt<true, false>(a, stream) : launch_split_opt<false, false>(a, stream);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The probabilities that ScaledDotProductAttention returns, from the log-sum-exp of the pass above.  One workgroup: 128 query rows (four waves of
+// 32) and `tiles` tiles of 64 keys.  S = Q K^T with the queries as rows, so that a lane holds one key of 16 rows and a store covers whole lines.
+template <int DP, bool OPT>
+__global__ __launch_bounds__(256, 2) void attn_weights_split_kernel(const AttnArgs a, float* __restrict__ w, int ktiles, int chunks, int tiles)
+{
+    constexpr int BK = 64, RB = 2 * DP, PL = BK * RB, DS = DP / 16, CPR = DP / 8, U = BK * CPR / 256, RPU = 256 / CPR;
+    __shared__ __attribute__((aligned(1024))) unsigned char Ks[4 * PL];      // two stages of [2][64][DP] fp16
+    __shared__ __attribute__((aligned(16))) float rows[2][128], red[4];                                   // of each query: factor of its logits, its log-sum-exp
+    constexpr int SROW = BK + 4;                                             // (16 bytes on: the rows of a store's four pieces on other banks)
+    constexpr bool STAGE = !OPT && DP <= 64;                                 // (elsewhere it would cost a workgroup per CU)
+    __shared__ __attribute__((aligned(16))) float stage[STAGE ? 4 : 1][STAGE ? 16 * SROW : 4];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l32 = lane & 31, h = lane >> 5;
+    // XCD-contiguous order: the tiles of one head share an L2
+    int bh, qt, chunk;
+    {
+        const int nblk = gridDim.x, pid = blockIdx.x, per = nblk >> 3, rem = nblk & 7, xcd = pid & 7, idx = pid >> 3;
+        const int logical = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + idx;
+        chunk = logical % chunks;
+        qt = logical / chunks % a.qtiles;
+        bh = logical / chunks / a.qtiles;
+    }
+    const int b = bh / a.H, hd = bh - b * a.H, q0 = qt * 128 + wave * 32;
+    const float* __restrict__ Q = (const float*)a.q + b * a.qs[0] + hd * a.qs[1];
+    const float* __restrict__ K = (const float*)a.k + b * a.ks[0] + (hd / (a.H / a.Hkv)) * a.ks[1];
+    float* __restrict__ W = w + (long long)bh * a.Sq * a.Sk;
+    const int first = chunk * tiles, end = min(first + tiles, ktiles);
+    // tiles from `seen` on lie above the causal diagonal of all 128 rows
+    int seen = end;
+    if (a.causal) {
+        const long long last = (long long)qt * 128 + 127 + a.qoff;
+        seen = last < 0 ? first : (int)min((long long)end, max((long long)first, last / BK + 1));
+    }
+    auto zeros = [&](int k0, int k1) {             // columns k0 .. k1 - 1 of this wave's rows
+        for (int r = lane >> 4; r < 32 && q0 + r < a.Sq; r += 4)
+            for (int c = k0 + 4 * (lane & 15); c < k1; c += 64) {
+                float* __restrict__ out = W + (long long)(q0 + r) * a.Sk + c;
+                if (c + 4 <= k1) __builtin_nontemporal_store((u32x4_a4){0u, 0u, 0u, 0u}, (u32x4_a4*)out);
+                else for (int e = 0; c + e < k1; e++) out[e] = 0.0f;
+            }
+    };
+    if (seen < end) zeros(seen * BK, min(end * BK, a.Sk));
+    if (seen == first) return;
+
+    const uint32_t krs = (uint32_t)a.ks[2];
+    const int col = min(8 * (t % CPR), a.D - 8);
+    const uint32_t klast = 4u * ((uint32_t)(a.Sk - 1) * krs + col);
+    uint32_t kat[U];
+    u32x4 rk[U][2];
+    auto load = [&]() {
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            const unsigned char* p = (const unsigned char*)K + kat[i];
+            rk[i][0] = *(const u32x4*)p;
+            rk[i][1] = *(const u32x4*)(p + 16);
+            kat[i] = min(kat[i] + 4u * BK * krs, klast);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < U; i++) kat[i] = min(4u * ((uint32_t)(first * BK + t / CPR + i * RPU) * krs + col), klast);
+    load();
+    const float lse = a.lse[(long long)bh * a.Sq + min(q0 + l32, a.Sq - 1)];
+    u32x4 qf[DS][2];
+    int logit_exp = -split_q(Q + (long long)min(q0 + l32, a.Sq - 1) * a.qs[2], q0 + l32 < a.Sq, a.D, h, qf);
+    float km = 0.0f;
+#pragma unroll
+    for (int i = 0; i < U; i++) km = fmaxf(km, largest(rk[i]));
+    km = wave_max(km);
+    if (lane == 0) red[wave] = km;
+    __syncthreads();
+    km = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const int kexp = __builtin_amdgcn_readfirstlane(exponent_to(km, 10));
+    const float ksc = power2(kexp);
+    logit_exp -= kexp;
+    const float to_logit = __builtin_ldexpf(a.scale, logit_exp);
+    // (such rows are formed on the fp32 pipe, as above)
+    const bool coarse = __builtin_amdgcn_ballot_w64(to_logit * LOG2E > 0x1p-13f) != 0;
+    if (h == 0) { rows[0][32 * wave + l32] = OPT ? to_logit : to_logit * LOG2E; rows[1][32 * wave + l32] = lse == -INFINITY ? INFINITY : lse * LOG2E; }
+    __builtin_amdgcn_wave_barrier();
+    for (int j = first; j < seen; j++) {
+        unsigned char* ks = Ks + (j & 1) * 2 * PL;
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            u32x4 p[2];
+            split8<true>(rk[i], ksc, p);
+            *(u32x4*)(ks + i * RPU * RB + k_at<RB>(t / CPR, t % CPR)) = p[0];
+            *(u32x4*)(ks + PL + i * RPU * RB + k_at<RB>(t / CPR, t % CPR)) = p[1];
+        }
+        __syncthreads();
+        load();                                    // (past the last tile rows are repeated)
+        const int k0 = j * BK;
+        if (q0 >= a.Sq) continue;
+        if (a.causal && (long long)k0 > (long long)q0 + 31 + a.qoff) { zeros(k0, min(k0 + BK, a.Sk)); continue; }
+        f32x16 s[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[i][r] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < DS; d++) {
+            f16x8 k[2][2];
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int p = 0; p < 2; p++) k[i][p] = *(const f16x8*)(ks + p * PL + i * 32 * RB + k_at<RB>(l32, 2 * d + h));
+            auto add = [&](int x, int y) {
+#pragma unroll
+                for (int i = 0; i < 2; i++) s[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, qf[d][y]), k[i][x], s[i], 0, 0, 0);
+            };
+            add(1, 0); add(0, 1); add(0, 0);
+        }
+        float poison = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) poison = fmaf(s[i][r], 0.0f, poison);
+        bool exact = coarse;
+        if (__builtin_amdgcn_ballot_w64(poison != poison) != 0) exact = true;
+        if (exact) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) s[i][r] = 0.0f;
+                const float* kp = K + (long long)min(k0 + 32 * i + l32, a.Sk - 1) * a.ks[2] + 4 * h;
+                const float* qp = Q + (long long)min(q0 + l32, a.Sq - 1) * a.qs[2] + 4 * h;
+#pragma unroll 1
+                for (int d = 0; d < a.D; d += 8) Mma32<float>::run(s[i], *(const u32x4*)(qp + d), *(const u32x4*)(kp + d));
+            }
+        }
+        int keys[2] = {k0 + l32, k0 + 32 + l32}, h = lane >> 5;
+        asm volatile("" : "+v"(h));                // (rows are formed anew for every tile, not kept beside the fragments)
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 factors[4], sums[4];                 // of rows 8 g + 4 h .. + 3
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            factors[g] = *(const u32x4*)&rows[0][32 * wave + 8 * g + 4 * h];
+            sums[g] = *(const u32x4*)&rows[1][32 * wave + 8 * g + 4 * h];
+        }
+        // logits in place, one pass over the tile per option, out-of-range elements on clamped addresses
+        if constexpr (OPT) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float f = exact ? a.scale : as_f32(factors[r >> 2][r & 3]);
+#pragma unroll
+                for (int i = 0; i < 2; i++) s[i][r] *= f;
+            }
+            if (a.softcap > 0.0f) {
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        s[i][r] = a.softcap * tanhf(s[i][r] / a.softcap);
+                        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+            if (a.bias) {
+                const float* __restrict__ Bi = a.bias + b * a.bias_bs + (long long)hd * a.Sq * a.Sk;
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        s[i][r] += Bi[(long long)min(q0 + acc_row(r, h), a.Sq - 1) * a.Sk + min(keys[i], a.Sk - 1)];
+                        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+            if (a.mask_mode == 3) {
+                const unsigned char* __restrict__ Mk = (const unsigned char*)a.mask + (long long)b * a.Sk;
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const bool hidden = Mk[min(keys[i], a.Sk - 1)] == 0;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) s[i][r] = hidden ? -INFINITY : s[i][r];
+                }
+            } else if (a.mask_mode != 0) {
+                const float* __restrict__ Mk = a.mask + (a.mask_mode == 2 ? (long long)bh * a.Sq * a.Sk : 0LL);
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        if (Mk[(long long)min(q0 + acc_row(r, h), a.Sq - 1) * a.Sk + min(keys[i], a.Sk - 1)] == 0.0f) s[i][r] = -INFINITY;
+                        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+        }
+        if (a.causal && (long long)k0 + 63 > (long long)q0 + a.qoff) {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) if ((long long)keys[i] > (long long)q0 + acc_row(r, h) + a.qoff) s[i][r] = -INFINITY;
+        }
+        // (a row without any visible key has no probabilities: its log-sum-exp counts as infinite)
+        auto probability = [&](int i, int r) {
+            const float f = OPT ? LOG2E : exact ? a.scale * LOG2E : as_f32(factors[r >> 2][r & 3]);
+            return __builtin_amdgcn_exp2f(fmaf(s[i][r], f, -as_f32(sums[r >> 2][r & 3])));
+        };
+        if constexpr (STAGE) {
+            // 16 rows at a time through LDS, so that a store is four whole pieces of a row, past the caches
+            float* mine = stage[wave];
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+#pragma unroll
+                for (int r = 8 * half; r < 8 * half + 8; r++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) mine[(acc_row(r, h) - 16 * half) * SROW + 32 * i + l32] = probability(i, r);
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int r = 4 * u + (lane >> 4), c = 4 * (lane & 15), row = q0 + 16 * half + r;
+                    const u32x4 v = *(const u32x4*)(mine + r * SROW + c);
+                    float* __restrict__ out = W + (long long)row * a.Sk + k0 + c;
+                    if (row < a.Sq) {
+                        if (k0 + c + 4 <= a.Sk) __builtin_nontemporal_store((u32x4_a4)v, (u32x4_a4*)out);
+                        else {
+#pragma unroll
+                            for (int e = 0; e < 4; e++) if (k0 + c + e < a.Sk) out[e] = as_f32(v[e]);
+                        }
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+        } else {
+            const bool whole = q0 + 32 <= a.Sq && k0 + BK <= a.Sk;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                float* __restrict__ out = W + (long long)(q0 + acc_row(r, h)) * a.Sk;
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const float p = probability(i, r);
+                    if (whole || (q0 + acc_row(r, h) < a.Sq && keys[i] < a.Sk)) __builtin_nontemporal_store(p, out + keys[i]);
+                }
+            }
+        }
+    }
+}
+
+template <int DP>
+static hipError_t launch_weights_split_as(AttnArgs a, float* w, hipStream_t stream)
+{
+    a.qtiles = (a.Sq + 127) / 128;
+    const int ktiles = (a.Sk + 63) / 64;
+    const long long rows = (long long)a.qtiles * a.B * a.H;
+    // Key tiles to a workgroup: two where that makes a grid of several rounds (fp32 B8 H16 S1000 d64 with attention 319 us, 296 this way;
+    // B2 H16/4 700 x 900 d128 causal 98, 91), else as many as leave two workgroups per CU (B4 H12 S512 d64 causal, of which two tiles each make
+    // 768: 40, 36)
+    const int split = (int)std::max(1LL, std::min((long long)ktiles, 512 / rows));
+    const int tiles = rows * ktiles >= 2048 ? 2 : (ktiles + split - 1) / split;
+    const int chunks = (ktiles + tiles - 1) / tiles;
+    if (rows * chunks > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)(rows * chunks)), dim3(256), 0, stream, a, w, ktiles, chunks, tiles); };
+    if (a.bias || a.mask_mode != 0 || a.softcap > 0.0f) go(attn_weights_split_kernel<DP, true>);
+    else go(attn_weights_split_kernel<DP, false>);
+    return hipGetLastError();
+}
+hipError_t launch_attn_weights_split(const AttnArgs& a, float* w, hipStream_t stream)
+{
+    return a.D <= 32 ? launch_weights_split_as<32>(a, w, stream) : a.D <= 64 ? launch_weights_split_as<64>(a, w, stream) : launch_weights_split_as<128>(a, w, stream);
+}
+
+}  // namespace aidn
