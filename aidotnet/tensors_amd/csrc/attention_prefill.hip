@@ -371,7 +371,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a)
         const u32x4 klo = {k_lane_off, k_lane_off ^ 64u, k_lane_off ^ 128u, k_lane_off ^ 192u};
         const uint32_t vlo = v_lane_off, vlo_odd = v_lane_off ^ 32u;
         const float negm0 = (m_ref[0] == -INFINITY) ? -0.0f : -m_ref[0], negm1 = (m_ref[1] == -INFINITY) ? -0.0f : -m_ref[1];
-        float ps0 = 0.0f, ps1 = 0.0f;
+        f32x4 ps0, ps1;                                    // (a query's sum in every element of its four lanes)
         const int tl = u >> 1;
         unsigned long long kptr = (unsigned long long)(uintptr_t)((const unsigned char*)K + (long long)((tl + 2) * BC + 16 * wave_s) * k_row_bytes);
         unsigned long long vptr = (unsigned long long)(uintptr_t)((const unsigned char*)V + (long long)((tl + 1) * BC + 16 * wave_s) * v_row_bytes);
@@ -393,19 +393,19 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a)
         u32x4 p0 = pf[0], p1 = pf[1];
 #define PREFILL_LOOP_OPERANDS \
             : "+{v[0:15]}"(oacc[0]), "+{v[16:31]}"(oacc[1]), "+{v[32:47]}"(oacc[2]), "+{v[48:63]}"(oacc[3]), "+{v[64:79]}"(sacc), \
-              "+{v[80:83]}"(p0), "+{v[84:87]}"(p1), "+{v167}"(ps0), "+{v168}"(ps1), "+{s[40:41]}"(kptr), "+{s[42:43]}"(vptr), "+{s53}"(count), "+{s57}"(kleft), "+{s58}"(vleft), "+{s59}"(mask_follows) \
+              "+{v[80:83]}"(p0), "+{v[84:87]}"(p1), "=&{v[200:203]}"(ps0), "=&{v[204:207]}"(ps1), "+{s[40:41]}"(kptr), "+{s[42:43]}"(vptr), "+{s53}"(count), "+{s57}"(kleft), "+{s58}"(vleft), "+{s59}"(mask_follows) \
             : "{v[88:103]}"(qlo), "{v[104:119]}"(qhi), "{v[152:155]}"(kad), "{v[192:195]}"(vad0), "{v[196:199]}"(vad1), \
               "{v[160:163]}"(klo), "{v164}"(vlo), "{v174}"(vlo_odd), "{v165}"(negm0), "{v166}"(negm1), "{s[44:51]}"(sc), "{s52}"(sl2s), "{s56}"(phase), "{s60}"(flavour), \
               "{v171}"(mask_rel0), "{v172}"(mask_rel1), "{v173}"(ninf) \
             : "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127", "v128", "v129", "v130", "v131", "v132", "v133", "v134", \
               "v135", "v136", "v137", "v138", "v139", "v140", "v141", "v142", "v143", "v144", "v145", "v146", "v147", "v148", "v149", \
-              "v150", "v151", "v169", "v170", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", \
+              "v150", "v151", "v156", "v157", "v158", "v159", "v169", "v170", "v176", "v177", "v178", "v179", "v180", "v181", "v182", "v183", "v184", "v185", "v186", \
               "v187", "v188", "v189", "v190", "v191", "s54", "s55", "scc", "vcc", "memory"
         if constexpr (std::is_same<T, f16_t>::value) asm volatile(PREFILL_LOOP_F16 PREFILL_LOOP_OPERANDS);
         else asm volatile(PREFILL_LOOP_BF16 PREFILL_LOOP_OPERANDS);
 #undef PREFILL_LOOP_OPERANDS
         pf[0] = p0; pf[1] = p1;
-        l_run[0] += ps0; l_run[1] += ps1;
+        l_run[0] += 0.25f * ps0[0]; l_run[1] += 0.25f * ps1[0];
         for (int i = 0; i < (n & 3); i++) { next_k_unit(); next_v_unit(); }
         k_unit += n & ~3; v_unit += n & ~3;
     };

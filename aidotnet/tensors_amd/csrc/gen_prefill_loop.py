@@ -24,8 +24,11 @@ def gen(kind, ablate=(), flip=0, period=1):
     consuming fragment i:
       slots 0..7   the V^T fragment of d-block i: P(u-1) V into the accumulators of both query blocks; beside them FMA + exp2 of the
                    logits of unit u (two per slot)
+      slots 3, 6   the row sums of P(u-1), query block 0 / 1, as one more product, with ones in the place of V^T: every accumulator of a
+                   query holds its sum.  (v_dot2 row sums hold up the MFMAs behind them: two MFMAs with two of them to each take 16.0 ns on a
+                   full SIMD, with two multiply-adds 7.5.)
       slots 8..15  the K fragment (kb, ks) = ((i - 8) % 2, (i - 8) / 2): the S(u+1) chains of both query blocks; beside them packed
-                   convert + row sum (one pair per slot)
+                   convert (one pair per slot)
       every slot   the LDS read of the fragment seven slots ahead (ring of eight), one wait per two slots, counted from the reads in flight
       odd units    the direct-to-LDS loads of K(t+2), V(t+1), one per slot 0..7, while s57 / s58 say a K / V tile is left to load
                    (K and V rows are 256 bytes apart: the four loads of a wave's share differ by an immediate offset)
@@ -33,7 +36,7 @@ def gen(kind, ablate=(), flip=0, period=1):
 
     Registers (fixed; the kernel binds its variables to them at the asm statement): v[0:63] O (block (db, qb) at 4 (2 db + qb)),
     v[64:79] logits (block (kb, qb) at 64 + 4 (2 kb + qb)), v[80:87] P (qb 0, qb 1), v[88:119] Q (block (qb, ks) at
-    88 + 4 (4 qb + ks)), v[120:151] fragment ring, v[152:155] K read addresses per ks (kb by an offset), v[192:199] V read
+    88 + 4 (4 qb + ks)), v[120:151] fragment ring, v[152:155] K read addresses per ks (kb by an offset), v[156:159] ones, v[192:199] V read
     addresses per d-block, v[160:163] lane offsets of the four K wave-loads, v164 / v174 of the even / odd V wave-loads, v165 v166 minus the
     exponent reference of query block 0 / 1, v167 v168 their running row sums, v169 v170 scratch, v171 v172 the lane's key limit
     inside a masked unit per query block, v173 minus infinity, v[176:191] exponentials.
@@ -51,7 +54,6 @@ def gen(kind, ablate=(), flip=0, period=1):
     to 4 us and gains nothing more: the board's power management pays a lone workgroup back in clock)."""
     mfma = "v_mfma_f32_16x16x32_" + kind
     cvt = "v_cvt_pk_%s_f32" % kind
-    dot = "v_dot2c_f32_%s_e32" % kind
     ones = "0x3c003c00" if kind == "f16" else "0x3f803f80"
     out = []
     emit = out.append
@@ -87,7 +89,19 @@ def gen(kind, ablate=(), flip=0, period=1):
         emit("s_waitcnt lgkmcnt(%d)" % left)
         del queue[:last + 1]
 
+    def row_sum(qb, a="v[156:159]", c=None):
+        n = 200 + 4 * qb
+        emit("%s v[%d:%d], %s, v[%d:%d], %s" % (mfma, n, n + 3, a, 80 + 4 * qb, 83 + 4 * qb, c or "v[%d:%d]" % (n, n + 3)))
+
     label = "L_prefill_%s%s_" % (kind, "_alt" if flip else "")
+    # (the P that the run starts with is in the caller's row sum already: taken off here, added again beside its product)
+    minus = "0xbc00bc00" if kind == "f16" else "0xbf80bf80"
+    for r in range(4):
+        emit("v_mov_b32_e32 v%d, %s" % (156 + r, ones))
+        emit("v_mov_b32_e32 v%d, %s" % (176 + r, minus))
+    emit("s_nop 1")
+    for qb in (0, 1):
+        row_sum(qb, "v[176:179]", "0")
     first7 = lambda blk: [(blk, f) for f in range(7) for _ in (0, 1)]
     for j in (1, 2, 3):
         emit("s_cmp_eq_u32 s56, %d" % j)
@@ -114,6 +128,8 @@ def gen(kind, ablate=(), flip=0, period=1):
             for qb in (0, 1):
                 o = 4 * (2 * i + qb)
                 emit("%s v[%d:%d], %s, v[%d:%d], v[%d:%d]" % (mfma, o, o + 3, f4, 80 + 4 * qb, 83 + 4 * qb, o, o + 3))
+            if i in (3, 6):
+                row_sum(i // 4)
         else:
             j = i - 8
             ks, kb = j >> 1, j & 1
@@ -145,7 +161,6 @@ def gen(kind, ablate=(), flip=0, period=1):
             qb, e2 = p >> 2, p & 3
             t0 = 8 * (e2 >> 1) + 4 * qb + 2 * (e2 & 1)
             emit("%s v%d, v%d, v%d" % (cvt, 80 + 4 * qb + e2, 176 + t0, 177 + t0))
-            emit("%s v%d, %s, v%d" % (dot, 167 + qb, ones, 80 + 4 * qb + e2))
 
     for blk in range(4):
         is_b = (blk & 1) == 0
@@ -202,9 +217,13 @@ def gen(kind, ablate=(), flip=0, period=1):
             emit("v_cndmask_b32_e32 v%d, v%d, v173, vcc" % (64 + t, 64 + t))
         emit("s_branch %sblk%d_%%=" % (label, (blk + 1) & 3))
     emit("%sexit_%%=:" % label)
+    for qb in (0, 1):
+        row_sum(qb)
     if "prio" not in ablate:
         emit("s_setprio 0")
     emit("s_waitcnt lgkmcnt(0)")
+    emit("s_nop 7")
+    emit("s_nop 7")
     return out
 
 
