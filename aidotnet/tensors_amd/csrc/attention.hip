@@ -22,6 +22,10 @@
 
 namespace aidn {
 
+// Per tile and wave the general form of 16-bit head dimension 64 is bound by what it issues (64 keys: 16 MFMAs of 32 cycles beside some 300 other
+// instructions, a lone wave one in 5 cycles): loads of a whole tile by a uniform base and fixed lane offsets, one multiply-add per logit, masks
+// against one bound a lane.  Against 64-bit addresses a load, a multiplication and a subtraction a logit, two tests an element, bf16 us: B8 H32
+// S2048 causal 218 -> 195, B16 H12 S512 29.8 -> 23.7, B8 H12 S512 causal 14.3 -> 12.9.  (A third stage of LDS gained nothing: 19.9 / 20.3.)
 // DMA (fp32, plain / causal, aligned contiguous K/V): the K and V tiles go global -> LDS directly, unpadded [key][d] rows with
 // XOR-swizzled 16-byte chunks (K: c ^ (key & 15) for the b128 fragment reads; V: c ^ (((key >> 2) & 1) << 3), read as the
 // A operand of O^T += V^T P^T with 32-bit LDS reads, the two lane halves -- keys 4 apart -- in different bank halves).  This
@@ -193,13 +197,24 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     auto k_swz = [](int key) -> int { return (EB == 4 || WIDE16) ? (key & 15) : ((key >> 1) & 7); };
     auto v_swz = [](int key) -> int { return EB == 4 ? (((key >> 2) & 1) << 3) : WIDE16 ? ((key & 3) << 2) : (((key >> 1) & 1) << 2); };
     int rows = 0;                  // paged cache: pool rows of this wave's keys, one tile per lane
+    constexpr int ROWB = DP * EB;                          // 256 / 128 bytes per key row
+    constexpr int KPL = 1024 / ROWB;                       // keys per 1 KiB wave-load
+    constexpr int LPW = DMA ? BC / KPL / 4 : 1;            // wave-loads per wave and tile (K and V each)
+    constexpr int CPRW = ROWB / 16;                        // chunks per row
+    constexpr int NK = KPL * LPW;                          // keys per wave and tile
+    constexpr int NO = LPW < 16 / KPL ? LPW : 16 / KPL;    // loads until the swizzle repeats
+    const int ld_key = lane / CPRW, ld_pos = lane % CPRW;
+    constexpr bool FIXED = DMA && DP <= 128;               // (at 256 the offsets do not fit the registers)
+    uint32_t koff[NO], voff[NO];
+    if constexpr (FIXED) {
+#pragma unroll
+        for (int i = 0; i < NO; i++) {
+            const int key = NK * wave + KPL * i + ld_key;
+            koff[i] = (uint32_t)(ld_key * (int)a.ks[2] + (ld_pos ^ k_swz(key)) * E) * EB;
+            voff[i] = (uint32_t)(ld_key * (int)a.vs[2] + (ld_pos ^ v_swz(key)) * E) * EB;
+        }
+    }
     auto issue_tile = [&](int tile, int stage) {
-        constexpr int ROWB = DP * EB;                      // 256 / 128 bytes per key row
-        constexpr int KPL = 1024 / ROWB;                   // keys per 1 KiB wave-load
-        constexpr int LPW = BC / KPL / 4;                  // wave-loads per wave and tile (K and V each)
-        constexpr int CPRW = ROWB / 16;                    // chunks per row
-        constexpr int NK = KPL * LPW;                      // keys per wave and tile
-        const int ld_key = lane / CPRW, ld_pos = lane % CPRW;
         // first row of the wave's keys and the last one to load, relative to it
         int row0 = tile * BC + NK * wave_s, left = a.Sk - 1 - row0;
         if (bt) {
@@ -207,6 +222,17 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
             if ((tile & 63) == 0) rows = paged_tile_rows(bt, a.bsz, a.dbsz, NK * wave_s, BC, tile, lane, last_group);
             left = a.Sk - 1 - min(row0, last_group);
             row0 = __builtin_amdgcn_readlane(rows, tile & 63);
+        }
+        if (FIXED && left >= NK - 1) {
+            // whole: a uniform base and lane offsets that stay (the swizzle repeats with 16 keys)
+            const unsigned char* kb = (const unsigned char*)(K + (long long)row0 * a.ks[2]);
+            const unsigned char* vb = (const unsigned char*)(V + (long long)row0 * a.vs[2]);
+#pragma unroll
+            for (int i = 0; i < LPW; i++) {
+                attn_dma16_base(kb + (long long)(KPL * i) * a.ks[2] * EB, koff[i % NO], lds0 + stage * KBYTES + (LPW * wave_s + i) * 1024);
+                attn_dma16_base(vb + (long long)(KPL * i) * a.vs[2] * EB, voff[i % NO], lds0 + 2 * KBYTES + stage * VBYTES + (LPW * wave_s + i) * 1024);
+            }
+            return;
         }
 #pragma unroll
         for (int i = 0; i < LPW; i++) {
@@ -336,26 +362,44 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                     groups([&](int kt, int r, int key) { if (row[key] == 0.0f) st[kt][r] = -INFINITY; });
                 }
             }
-            float mloc = -INFINITY;
+            const float factor = FULL ? LOG2E : fabsf(sl2);
+            if constexpr (!FULL) {
+                if (sl2 < 0.0f) {
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++) {
-                const uint32_t kept = (uint32_t)(kbits >> (kr0 + 32 * kt)) >> (4 * h);       // bit acc_row(r, 0): the key of element r
+                    for (int kt = 0; kt < KT; kt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    float x;
-                    const int key = kw0 + kt * 32 + acc_row(r, h);
-                    if constexpr (FULL) x = st[kt][r] * LOG2E;
-                    else x = st[kt][r] * sl2;
-                    if (need_mask) {
-                        if (key >= a.Sk || (a.causal && (long long)key > (long long)qi + a.qoff)) x = -INFINITY;
-                    }
-                    if constexpr (KM || FULL)
-                        if (mixed && !(kept >> acc_row(r, 0) & 1u)) x = -INFINITY;
-                    st[kt][r] = x;
-                    mloc = fmaxf(mloc, x);
+                        for (int r = 0; r < 16; r++) st[kt][r] = -st[kt][r];
                 }
             }
-            mloc = fmaxf(mloc, shfl_xor_f(mloc, 32));
+            if (need_mask) {
+                // the query's last visible key, relative to the lane's first (formed here, not kept through the loop)
+                int first = __lane_id();
+                asm volatile("" : "+v"(first));
+                const int row = first & 31;
+                first = -4 * (first >> 5);
+                int seen = a.Sk - 1 - kw0 + first;
+                if (a.causal) seen = min(seen, (int)max(min((long long)wq_min + a.qoff - kw0, 1LL << 20), -(1LL << 20)) + row + first);
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) if (kt * 32 + acc_row(r, 0) > seen) st[kt][r] = -INFINITY;
+            }
+            if constexpr (KM || FULL) {
+                if (mixed) {
+#pragma unroll
+                    for (int kt = 0; kt < KT; kt++) {
+                        const uint32_t kept = (uint32_t)(kbits >> (kr0 + 32 * kt)) >> (4 * h);       // bit acc_row(r, 0): the key of element r
+#pragma unroll
+                        for (int r = 0; r < 16; r++) if (!(kept >> acc_row(r, 0) & 1u)) st[kt][r] = -INFINITY;
+                    }
+                }
+            }
+            float mloc = -INFINITY;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, st[kt][r]);
+            mloc = max_with_partner32(mloc) * factor;
             const float m_new = fmaxf(m_run, mloc);
             const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
             const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
@@ -366,7 +410,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
             for (int kt = 0; kt < KT; kt++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    float p = __builtin_amdgcn_exp2f(st[kt][r] - m_use);
+                    float p = __builtin_amdgcn_exp2f(fmaf(st[kt][r], factor, -m_use));
                     st[kt][r] = p;
                     psum += p;
                 }
@@ -1376,12 +1420,23 @@ static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
 //   fp32 above 64: up to 32 keys the second group has none (Sk 12 10.6 / 12.8); causal 384 only where the row tiles differ in length
 //     (Sq 204 n 288 44 / 35; but Sq 62, Sk 12 n 352 16 / 26)
 // The lines do not depend on how the tiles are loaded, so the direct-to-LDS and the register-staged forms add up the same way.
+// 16-bit head dimension 64 (direct loads; measured with what a tile costs there): two groups plain
+// up to 256 (84 keys n 384 7.5 / 6.6, S1249 n 640 31.6 / 30.0), causal up to 640 (S1960 n 620 28.2, 24.4 on 128-key tiles / 33.9; S432 n 896
+// 13.9 / 12.0), none up to 64 keys (S43 5.5 / 5.3); from 96 keys on 128-key tiles, a barrier for twice the work (S1489 n 192 21.6 / 18.0, S239
+// n 192 7.9 / 7.5; 69 keys 5.8 / 6.1); four groups gain no more there (S379 n 96 8.6 / 8.3).
 template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
 static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
 {
     constexpr bool WIDE32 = Elem<T>::BYTES == 4 && BC == 32 && DP == 128;
     if constexpr ((BC == 64 && MINB == 2) || WIDE32) {
         auto grid = [&](int rows) { return (long long)((a.Sq + rows - 1) / rows) * a.B * a.H; };
+        if constexpr (!FULL && Elem<T>::BYTES == 2 && DP == 64) {
+            if (a.Sk > 64 && grid(64) <= (a.causal ? 640 : 256)) {
+                if constexpr (!KM) { if (a.Sk >= 96) return launch_attn_kg<T, OutT, DP, 128, FULL, DMA ? 2 : 1, DMA, KM, 2>(a, stream); }
+                return launch_attn_kg<T, OutT, DP, 64, FULL, 2, DMA, KM, 2>(a, stream);
+            }
+            return launch_attn_kg<T, OutT, DP, BC, FULL, MINB, DMA, KM>(a, stream);
+        }
         if constexpr (!FULL && !KM && DP == 64) {
             if (!a.bt && a.Sk >= 192 && grid(32) <= (a.causal ? 384 : 256)) return launch_attn_kg<T, OutT, DP, 128, FULL, 1, DMA, KM, 4>(a, stream);
         }
@@ -1505,12 +1560,12 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     const bool full = p.bias != nullptr || a.mask_mode != 0 || p.softcap > 0.0f;
     // a mask of the keys alone is followed by the direct-to-LDS instances at head dimensions 64 and 128 as well
     const bool km = a.mask_mode == 3 && !p.block_table && (p.D == 64 || p.D == 128);
+    // the direct-to-LDS kernels address K/V rows of a load group with unsigned 32-bit byte offsets
+    const bool rows32 = p.ks[2] > 0 && p.ks[2] < (1LL << 28) && p.vs[2] > 0 && p.vs[2] < (1LL << 28);
     // the direct-to-LDS instances: plain / causal, 16-byte aligned rows, contiguous or in blocks of a multiple of 16 keys
-    const bool dma = p.bias == nullptr && !(p.softcap > 0.0f) && (a.mask_mode == 0 || km) && a.vec_in && paged_block_fits(p.block_table, p.block_size) && g_attn_allow_dl;
+    const bool dma = p.bias == nullptr && !(p.softcap > 0.0f) && (a.mask_mode == 0 || km) && a.vec_in && paged_block_fits(p.block_table, p.block_size) && g_attn_allow_dl && rows32;
     hipError_t err;
     // fast path: 16-bit, head dim 128, aligned rows, plain (optionally causal) attention
-    // the fast kernel addresses K/V rows of a 4-key load group with unsigned 32-bit byte offsets
-    const bool rows32 = p.ks[2] > 0 && p.ks[2] < (1LL << 28) && p.vs[2] > 0 && p.vs[2] < (1LL << 28);
     const bool dl = attn_dl_applies(kind, p);
     const bool split = kind == 0 && attn_split_applies(a);      // fp32 on the fp16 matrix pipe (attention_split.hip)
     if (dl && p.workspace) {
