@@ -605,7 +605,8 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 // PAGED: K and V are pools behind a block table (block size a multiple of 16); a wave's 16 keys of a tile then lie in one block, and all
 // that changes is where the uniform base of its loads comes from (paged_tile_rows).  A 512-query chunk after 3584 keys (bf16, 32 / 8
 // heads) took 347 us on the general kernel, whose loads go through registers and which cannot split the keys of its 128 query tiles; here
-// 65 us with the merge of its four key ranges.
+// 54 us with the merge of its four key ranges (the kernel alone 49; bound by what the vector unit issues beside the MFMAs: which heads share
+// K and V, and the order of the blocks, make no difference).
 // KM: a keep-mask of the keys shared by the heads and queries of a batch (mask_mode 3), one ballot per tile as in the kernel above.
 template <typename T, typename OutT, int D = 128, bool PAGED = false, bool KM = false>
 __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(const AttnArgs a)
@@ -623,7 +624,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
     // under a key mask not at all, as in the general kernel that served those calls before: the largest probability of a row is then 1,
     // which the 16-bit operand of the P V product holds exactly, where one that lags rounds it like any other (relative error against
     // float64, 512 queries after 3584 keys bf16: 1.45e-3 against 1.62e-3, general kernel 1.53e-3; f16 154 + 130: 1.68e-4, 1.97e-4, 1.74e-4).
-    // The rescales cost 5-18 %: that call 65 us (347 on the general kernel, 56 with a lag of 8).
+    // The rescales cost 8 %: that call 54 us, contiguous keys with a lag of 8 50.
     constexpr float SLACK = PAGED || KM ? 0.0f : 8.0f;
 
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -825,22 +826,25 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
     __syncthreads();
 
     // raise the exponent reference only when a row max has moved by more than SLACK (or on first use)
+    auto rescale = [&](float m_old) {
+        const float alpha = (m_ref == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m_old - m_ref);
+        l_run *= alpha;
+#pragma unroll
+        for (int i = 0; i < DT; i++) {
+            // (head dimension 256: the accumulators live in accumulation registers, which the multiply cannot read.  The two
+            // opaque statements pin them there on both sides of it, so that the copies to and from vector registers are made
+            // here, on this rare path, and not once per tile on the common one.)
+            if constexpr (D == 256) asm volatile("" : "+a"(oacc[i]));
+#pragma unroll
+            for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
+            if constexpr (D == 256) asm volatile("" : "+a"(oacc[i]));
+        }
+    };
     auto lazy_rescale = [&](float mloc) {
         if (__builtin_amdgcn_ballot_w64(mloc > m_ref + SLACK) != 0ull) {
-            const float m_new = (mloc > m_ref + SLACK) ? mloc : m_ref;
-            const float alpha = (m_new == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m_ref - m_new);
-            m_ref = m_new;
-            l_run *= alpha;
-#pragma unroll
-            for (int i = 0; i < DT; i++) {
-                // (head dimension 256: the accumulators live in accumulation registers, which the multiply cannot read.  The two
-                // opaque statements pin them there on both sides of it, so that the copies to and from vector registers are made
-                // here, on this rare path, and not once per tile on the common one.)
-                if constexpr (D == 256) asm volatile("" : "+a"(oacc[i]));
-#pragma unroll
-                for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
-                if constexpr (D == 256) asm volatile("" : "+a"(oacc[i]));
-            }
+            const float m_old = m_ref;
+            if (mloc > m_ref + SLACK) m_ref = mloc;
+            rescale(m_old);
         }
     };
     // p = exp2(s * c - m) of two scores, rounded and packed; the row sum accumulates the rounded values (the
@@ -965,8 +969,14 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (need_mask) mask_sub(1, s1);
+            // ---- O^T += V[0:32]^T P0^T interleaved with P1 = exp(S1).  P1 is formed against the reference that S1 asks for at once; what is
+            // accumulated against the older one, P0 V among it, is rescaled behind this phase.  (Formed against the old reference and a
+            // second time when S1 raised it, 512 queries after 3584 keys took 56 us in this kernel; so, and with the partials through LDS, 49.)
             const float mloc1 = sub_max(s1);
-            // ---- O^T += V[0:32]^T P0^T interleaved with P1 = exp(S1) against the standing reference
+            const bool raised = __builtin_amdgcn_ballot_w64(mloc1 > m_ref + SLACK) != 0ull;
+            const float m_old = m_ref;
+            if (mloc1 > m_ref + SLACK) m_ref = mloc1;
+            m_use = (m_ref == -INFINITY) ? 0.0f : m_ref;
             float psum1 = 0.0f;
 #pragma unroll
             for (int s = 0; s < 2 * DT; s++) {
@@ -982,20 +992,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
                 __builtin_amdgcn_sched_barrier(0);
             }
             l_run += psum;
-            if (__builtin_amdgcn_ballot_w64(mloc1 > m_ref + SLACK) != 0ull) {
-                // rare: the second sub-tile raises the reference.  P0 (formed against the old one) is already
-                // accumulated; O and l are rescaled and P1 is formed again against the new reference (the
-                // values computed above may have overflowed and are dropped).
-                lazy_rescale(mloc1);
-                m_use = (m_ref == -INFINITY) ? 0.0f : m_ref;
-                psum1 = 0.0f;
-#pragma unroll
-                for (int s = 0; s < 8; s++) {
-                    uint32_t pk;
-                    exp_pair(s1[2 * s], s1[2 * s + 1], m_use, pk, psum1);
-                    p1f[s >> 2][s & 3] = pk;
-                }
-            }
+            if (raised) rescale(m_old);
             l_run += psum1;
 
             // ---- O^T += V[32:64]^T P1^T
@@ -1019,19 +1016,31 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
     const float l_tot = sum_with_partner32(l_run);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
     if (a.part) {
-        // grouped decode over several splits: query row qi is head hd * Sq + qi of the caller; unnormalised partial for the merge
-        if (qi < a.Sq) {
-            float* __restrict__ P = a.part + (((long long)bh * a.Sq + qi) * a.nsplit + split) * (D + 2);
-            if (h == 0) { P[0] = m_ref; P[1] = l_tot; }
+        // partial of a key range, unnormalised, for the merge: [2 + D] floats a row, whole rows at a time through LDS as below (the tile
+        // memory is idle).  From the registers a store instruction touched 8 bytes in each of 64 places: contiguous 512 queries after 3584
+        // keys, four ranges, 53.5 us with the merge, so 50.
+        constexpr int OROWB = 4 * D;
+        const int nrow = min(32, a.Sq - q0 - wave * 32);
+        if (nrow <= 0) return;                                             // (one pass: a key range is never paired)
+        unsigned char* stg = smem + wave * (32 * OROWB);
 #pragma unroll
-            for (int i = 0; i < DT; i++)
+        for (int i = 0; i < DT; i++)
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int d0 = i * 32 + 8 * g + 4 * h;
-                    *(u32x2*)(P + 2 + d0) = u32x2{as_u32(oacc[i][4 * g + 0]), as_u32(oacc[i][4 * g + 1])};      // 8-byte aligned
-                    *(u32x2*)(P + 4 + d0) = u32x2{as_u32(oacc[i][4 * g + 2]), as_u32(oacc[i][4 * g + 3])};
-                }
-        }
+            for (int g = 0; g < 4; g++)
+                *(f32x4*)(stg + l32 * OROWB + (((8 * i + 2 * g + h) ^ l32) << 4)) =
+                    f32x4{oacc[i][4 * g + 0], oacc[i][4 * g + 1], oacc[i][4 * g + 2], oacc[i][4 * g + 3]};
+        float* __restrict__ P = a.part + (((long long)bh * a.Sq + q0 + wave * 32) * a.nsplit + split) * (D + 2);
+        const long long pitch = (long long)a.nsplit * (D + 2);
+        if (h == 0 && qi < a.Sq) *(f32x2p*)(P + l32 * pitch) = f32x2p{m_ref, l_tot};
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+#pragma unroll 4
+        for (int r = 0; r < nrow; r++)
+#pragma unroll
+            for (int u = 0; u < D / 128; u++) {
+                const int d2 = ln + 64 * u;                                // this lane's pair of elements
+                *(f32x2p*)(P + r * pitch + 2 + 2 * d2) = *(const f32x2p*)(stg + r * OROWB + (((d2 >> 1) ^ r) << 4) + 8 * (d2 & 1));
+            }
     } else
     if (Elem<OutT>::BYTES == 4 && a.vec_out && a.stage_out) {
         // fp32 O through LDS: the lane holds 16-byte pieces of ONE row (64 rows per store instruction, each a partial line);
