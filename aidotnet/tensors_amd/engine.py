@@ -176,7 +176,7 @@ class Mi355Engine:
         be = self.backend
         a = input.contiguous(); w = weights.contiguous()
         M = a.numel() // K
-        bb = be.WrapTensor(bias.to(torch.float32).contiguous()) if bias is not None else None
+        bb = be.WrapTensor((bias if bias.dtype == torch.float32 else bias.to(torch.float32)).contiguous()) if bias is not None else None
         if a.dtype == torch.float32:
             out = torch.empty(*a.shape[:-1], N, dtype=torch.float32, device=a.device)
             be.GemmBiasActivationInto(be.WrapTensor(a), be.WrapTensor(w), bb, be.WrapTensor(out), M, N, K, act, alpha)
@@ -211,7 +211,7 @@ class Mi355Engine:
         a = input.contiguous(); w = weightsFp16.contiguous()
         M = a.numel() // K
         out = torch.empty(*a.shape[:-1], N, dtype=torch.float32, device=a.device)
-        bb = be.WrapTensor(bias.to(torch.float32).contiguous()) if bias is not None else None
+        bb = be.WrapTensor((bias if bias.dtype == torch.float32 else bias.to(torch.float32)).contiguous()) if bias is not None else None
         be.GemmFp16WeightB(be.WrapTensor(a), be.WrapTensor(w), bb, be.WrapTensor(out), M, N, K, act, alpha)
         return out
 
