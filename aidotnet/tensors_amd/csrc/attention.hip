@@ -328,12 +328,15 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                     for (int r = 0; r < 16; r++) st[kt][r] *= a.scale;
                 if (a.softcap > 0.0f) {
 #pragma unroll
-                    for (int kt = 0; kt < KT; kt++)
+                    for (int kt = 0; kt < KT; kt++) {
+                        if constexpr (DP == 256 && Elem<T>::BYTES == 2) {      // (out of registers: 11 of them would go to scratch memory)
 #pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            st[kt][r] = a.softcap * tanhf(st[kt][r] / a.softcap);
-                            if (DP == 256) __builtin_amdgcn_sched_barrier(0);
-                        }
+                            for (int r = 0; r < 16; r++) {
+                                st[kt][r] = a.softcap * tanhf(st[kt][r] / a.softcap);
+                                __builtin_amdgcn_sched_barrier(0);
+                            }
+                        } else soft_cap<16>(st[kt], a.softcap);
+                    }
                 }
                 // (rows and keys are formed anew, the keys for each pass, and few loads are asked for at a time where registers are short)
                 int qr = min(qi, a.Sq - 1), key0 = kw0 + 4 * h;
@@ -1325,9 +1328,7 @@ __global__ __launch_bounds__(256) void attn_weights_kernel(const AttnArgs a, flo
     if constexpr (FULL) {
         if (a.softcap > 0.0f) {
 #pragma unroll
-            for (int j = 0; j < 2; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) s[j][r] = a.softcap * tanhf(s[j][r] / a.softcap);
+            for (int j = 0; j < 2; j++) soft_cap<16>(s[j], a.softcap);
         }
         if (a.bias) {
             const float* __restrict__ Bi = a.bias + b * a.bias_bs + (long long)hd * a.Sq * a.Sk;

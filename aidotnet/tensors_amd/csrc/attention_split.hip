@@ -292,12 +292,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
                 for (int r = 0; r < 16; r++) st[kt][r] *= to_log2;
             if (a.softcap > 0.0f) {
 #pragma unroll
-                for (int kt = 0; kt < NB; kt++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        st[kt][r] = a.softcap * tanhf(st[kt][r] / a.softcap);
-                        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-                    }
+                for (int kt = 0; kt < NB; kt++) soft_cap<16>(st[kt], a.softcap);
             }
             if (a.bias) {
                 const float* __restrict__ row = a.bias + b * a.bias_bs + ((long long)hd * a.Sq + qr) * a.Sk;
@@ -882,12 +877,7 @@ __global__ __launch_bounds__(256, 2) void attn_weights_split_kernel(const AttnAr
             }
             if (a.softcap > 0.0f) {
 #pragma unroll
-                for (int i = 0; i < 2; i++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        s[i][r] = a.softcap * tanhf(s[i][r] / a.softcap);
-                        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-                    }
+                for (int i = 0; i < 2; i++) soft_cap<16>(s[i], a.softcap);
             }
             if (a.bias) {
                 const float* __restrict__ Bi = a.bias + b * a.bias_bs + (long long)hd * a.Sq * a.Sk;
