@@ -1709,7 +1709,7 @@ static int splitk16_ranges(int M, int N, int K, int* kper, int* big_tile = nullp
 {
     if (big_tile) *big_tile = 0;
     *kper = K;
-    if (N % 8 != 0 || N < 128 || K % 64 != 0) return 0;
+    if (N % 8 != 0 || K % 64 != 0) return 0;
     const int kt = K / 64;
     // (the last range may be shorter by up to a K-tile per range)
     auto ranges = [&](long long t, int min_k) {
@@ -1725,12 +1725,14 @@ static int splitk16_ranges(int M, int N, int K, int* kper, int* big_tile = nullp
     if (t <= 128) {                           // up to half a chip of 128 x 128 tiles
         // (below, the second launch costs what the ranges save: 1000 x 1024 x 1024 8 -> 15 us, 512 x 1024 x 1344 8.9 -> 14.0, 64 x 512 x 1536 9.4 -> 9.8;
         // 128 x 136 x 2112, whose one launch is shorter than what two cost the caller)
-        if (K < (N % 128 == 0 ? 1792 : 2560)) return 0;
+        if (K < (N % 128 == 0 || N < 128 ? 1792 : 2560)) return 0;
         // estimates in us: in one launch 0.5 a K-tile and 3; in ranges 0.425 a K-tile, 6.9 for both launches and the sums, and the partials
         // written and read at 3.55 TB/s (fitted on 310 timings of 60 shapes to 5 %; one / two / three / four: 2048 x 512 x 2048 19.3 / 18.5 / 17.8 /
         // 18.0, 1000 x 1024 x 2048 20.0 / 17.8 / 17.5 / 18.2, 512 x 1024 x 1792 16.5 / 15.6 / 15.3 / 15.2; 2048 x 1024 x 2112 19.9 in one, 23.1 in two)
         int best = 1;
-        double best_us = 0.5 * kt + 3.0;
+        // (fewer than 128 columns: one launch is of 64 x 64 tiles, 0.3 a K-tile; us, one launch / ranges and
+        // their sums: 496 x 64 x 8064 39.9 / 13.2, 1433 x 64 x 5120 27.0 / 14.6, 4 x 64 x 3008 25.8 / 9.7, 200 x 96 x 1856 11.6 / 11.0)
+        double best_us = (N < 128 ? 0.3 : 0.5) * kt + 3.0;
         for (int ks = 2; ks <= 16 && ks * t <= 256 && K / ks >= 512; ks++) {
             const int per = (kt + ks - 1) / ks, n = (kt + per - 1) / per;
             const double us = 0.425 * per + 6.9 + (double)n * M * N * 8.0 / 3.55e6;
@@ -3068,6 +3070,20 @@ hipError_t gemm_f32_f16weight(hipStream_t stream, const float* A, const uint16_t
 
 #endif
 
+// The products of the K ranges of splitk16_ranges, as batches into the workspace; *ks = 0: not taken (no ranges, or too little workspace)
+template <typename T>
+static hipError_t launch_k_ranges16(const GemmArgs& g, hipStream_t stream, void* workspace, size_t workspace_bytes, int* ks)
+{
+    int big = 0, kper;
+    *ks = splitk16_ranges(g.M, g.N, g.K, &kper, &big);
+    GemmArgs gp = g;
+    gp.C = workspace; gp.K = kper; gp.k_total = g.K; gp.ldc = g.N;
+    gp.sA = kper; gp.sB = (long long)kper * g.N; gp.sC = (long long)g.M * g.N;
+    gp.bias = nullptr; gp.act = 0;
+    if (*ks == 0 || (size_t)*ks * g.M * g.N * sizeof(float) > workspace_bytes || !dl16_applies<float>(gp)) { *ks = 0; return hipSuccess; }
+    return big ? launch_gemm_dl16<T, float, 4>(gp, *ks, stream) : launch_gemm_dl16<T, float, 2, true>(gp, *ks, stream);
+}
+
 // one 16-bit type per part: T = f16_t in part 1, bf16_t in part 2; out32: C is fp32 (else the same 16-bit type as the inputs)
 template <typename T>
 static hipError_t gemm_16_typed(hipStream_t stream, const uint16_t* A, const uint16_t* B, void* C, int out32,
@@ -3147,21 +3163,13 @@ static hipError_t gemm_16_typed(hipStream_t stream, const uint16_t* A, const uin
         }
     }
     if (force_tile == 0 && workspace) {
-        int big = 0, kper;
-        const int ks = splitk16_ranges(M, N, K, &kper, &big);
-        if (ks && (size_t)ks * M * N * sizeof(float) <= workspace_bytes) {
-            GemmArgs gp = g;
-            gp.C = workspace; gp.K = kper; gp.k_total = K; gp.ldc = N;
-            gp.sA = kper; gp.sB = (long long)kper * N; gp.sC = (long long)M * N;
-            gp.bias = nullptr; gp.act = 0;
-            if (dl16_applies<float>(gp)) {
-                if (hipError_t e = big ? launch_gemm_dl16<T, float, 4>(gp, ks, stream) : launch_gemm_dl16<T, float, 2, true>(gp, ks, stream)) return e;
-                const long long total = (long long)M * N;
-                const unsigned grid = (unsigned)((total + 255) / 256);
-                if (out32) hipLaunchKernelGGL((skinny_reduce_kernel<float>), dim3(grid), dim3(256), 0, stream, (const float*)workspace, C, M, N, ks, bias, act, act_param, 1.0f, 0.0f);
-                else hipLaunchKernelGGL((skinny_reduce_kernel<T>), dim3(grid), dim3(256), 0, stream, (const float*)workspace, C, M, N, ks, bias, act, act_param, 1.0f, 0.0f);
-                return hipGetLastError();
-            }
+        int ks;
+        if (hipError_t e = launch_k_ranges16<T>(g, stream, workspace, workspace_bytes, &ks)) return e;
+        if (ks) {
+            const unsigned grid = (unsigned)(((long long)M * N + 255) / 256);
+            if (out32) hipLaunchKernelGGL((skinny_reduce_kernel<float>), dim3(grid), dim3(256), 0, stream, (const float*)workspace, C, M, N, ks, bias, act, act_param, 1.0f, 0.0f);
+            else hipLaunchKernelGGL((skinny_reduce_kernel<T>), dim3(grid), dim3(256), 0, stream, (const float*)workspace, C, M, N, ks, bias, act, act_param, 1.0f, 0.0f);
+            return hipGetLastError();
         }
     }
     if (out32) return dispatch_gemm<T, float, false>(g, 1, stream, force_tile);
@@ -3183,9 +3191,13 @@ hipError_t gemm_16_rope_bf16(hipStream_t stream, const uint16_t* A, const uint16
 // chip better), and the rotation rides on its stores: same sums, one launch (us, product and rotation in two launches / here / on the stream's
 // summing pass: 1 x 4096 x 512 7.5 / 6.6 / 6.8, 32 x 512 x 384 7.2 / 6.1 / 7.2, 32 x 12288 x 768 12.6 / 11.0 / 11.7; only towards the
 // upper end of that K the stream would be ahead: 1 x 2048 x 704 8.4 / 7.4 / 6.9, 32 x 1024 x 960 9.8 / 8.6 / 7.7, where the plain product is not).
+// 33 - 64 rows fill that tile better still and take it over any K that has no ranges, where no wider tile is chosen (49 x 512 x 512, product and
+// rotation 6.4 + 2.6 us in two launches / 6.5).
 static bool rope_on_tile(const GemmArgs& g)
 {
-    return g.M <= 32 && g.N % 128 == 0 && g.N <= 16384 && g.K % 64 == 0 && !skinny_applies(g.M, g.N, g.K) && aligned16(g.A) && aligned16(g.B);
+    if (!(g.M <= 64 && g.N % 128 == 0 && g.N <= 16384 && g.K % 64 == 0 && !skinny_applies(g.M, g.N, g.K) && aligned16(g.A) && aligned16(g.B))) return false;
+    int kper;
+    return g.M <= 32 || (splitk16_ranges(g.M, g.N, g.K, &kper) == 0 && dl16_width(g.M, g.N, g.K, 1) == 0);
 }
 // C = A B, then interleaved RoPE over the leading columns of C (launch.hpp)
 template <typename T>
@@ -3194,10 +3206,20 @@ static hipError_t gemm_16_rope_typed(hipStream_t stream, const uint16_t* A, cons
 {
     if (!workspace) workspace_bytes = 0;
     GemmArgs g{A, B, C, M, N, K, K, N, N, 0, 0, 0, 1.0f, 0.0f, 0, 0, nullptr, 0, 0.0f};
-    // the plan of gemm_16_typed that sums K ranges in a pass of its own takes the rotation into that pass
+    // the plans of gemm_16_typed that sum K ranges in a pass of their own take the rotation into that pass (the second from 33 rows on;
+    // 34 x 2048 x 2048, us of the second and third launch before / the one that does both: 2.7 + 2.6 / 3.1)
     if (force_tile == 0 && workspace && skinny_applies(M, N, K) && aligned16(A) && aligned16(B) &&
         (size_t)skinny_ksplit(N, K) * M * N * sizeof(float) <= workspace_bytes) {
         return launch_skinny<T, T>(g, stream, (float*)workspace, &rope);
+    }
+    if (force_tile == 0 && workspace && aligned16(A) && aligned16(B) && ((uintptr_t)C & 3u) == 0 && !skinny_applies(M, N, K) && msplit16_rows(M, N, K) == 0) {
+        int ks;
+        if (hipError_t e = launch_k_ranges16<T>(g, stream, workspace, workspace_bytes, &ks)) return e;
+        if (ks) {
+            const long long pairs = (long long)M * N / 2;
+            hipLaunchKernelGGL((skinny_reduce_rope_kernel<T>), dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream, (const float*)workspace, C, M, N, ks, rope);
+            return hipGetLastError();
+        }
     }
     if (force_tile == 0 && rope.cols > 0 && rope_on_tile(g)) return launch_gemm_dl<T, T, true, 64, false, 1, GemmRopeArgs>(GemmRopeArgs{g, rope}, 1, stream);
     if (hipError_t e = gemm_16_typed<T>(stream, A, B, C, 0, M, N, K, force_tile, workspace, workspace_bytes, nullptr, 0, 0.0f)) return e;
