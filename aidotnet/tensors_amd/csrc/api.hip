@@ -285,9 +285,20 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
     const bool x3 = c->force_tile == 0 && (at & 15u) == 0 && aidn::gemm_x3_suits(kind, (int)rows, dModel, dModel);
     const size_t wf_bytes = wqkv || x3 ? 0 : up((size_t)dModel * 3 * dModel * es), qkv_bytes = up((size_t)rows * 3 * dModel * es);
     const size_t cc_bytes = up((size_t)rows * dModel * es);
+    // scratch of the products behind it: K ranges where few rows leave the chip idle (us of the output projection without / with:
+    // fp32 B11 S31 dModel 2048 53.9 / 36.6, B6 S161 dModel 1536 57 / 51, bf16 B2 S128 dModel 2048 17.9 / 13.2).
+    // A stream under capture whose workspace was reserved without it goes without.
+    auto product_bytes = [&](int n) -> size_t {
+        if (c->force_tile != 0) return 0;
+        return kind == 0 ? aidn::gemm_f32_workspace_bytes((int)rows, n, dModel, 0) : aidn::gemm_16_workspace_bytes((int)rows, n, dModel, ((uintptr_t)wo & 15u) != 0);
+    };
+    const size_t base_bytes = wf_bytes + qkv_bytes + cc_bytes;
+    size_t gemm_bytes = std::max(product_bytes(dModel), x3 ? 0 : product_bytes(3 * dModel));
     void* ws = nullptr;
-    int st = acquire_ws(c, stream, wf_bytes + qkv_bytes + cc_bytes, &ws);
+    int st = acquire_ws(c, stream, base_bytes + gemm_bytes, &ws);
+    if (st && gemm_bytes) { gemm_bytes = 0; st = acquire_ws(c, stream, base_bytes, &ws); }
     if (st) return st;
+    void* const gws = gemm_bytes ? (unsigned char*)ws + base_bytes : nullptr;
     unsigned char* wf = (unsigned char*)ws;
     unsigned char* qkv = wf + wf_bytes;
     unsigned char* cc = qkv + qkv_bytes;
@@ -312,8 +323,8 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
             e = aidn::gemm_16_x3(sm, kind - 1, (const uint16_t*)input, b16, (uint16_t*)qkv, M, dModel, dModel, ldb, 0);
         }
     }
-    else if (kind == 0) e = aidn::gemm_f32(sm, (const float*)input, (const float*)w3, (float*)qkv, M, N3, dModel, 1.0f, 0.0f, 0, 1, 0, 0, 0, tile32);
-    else e = aidn::gemm_16(sm, kind - 1, (const uint16_t*)input, (const uint16_t*)w3, qkv, 0, M, N3, dModel, c->force_tile, nullptr, 0);
+    else if (kind == 0) e = aidn::gemm_f32(sm, (const float*)input, (const float*)w3, (float*)qkv, M, N3, dModel, 1.0f, 0.0f, 0, 1, 0, 0, 0, tile32, nullptr, 0, 0.0f, gws, nullptr, gemm_bytes);
+    else e = aidn::gemm_16(sm, kind - 1, (const uint16_t*)input, (const uint16_t*)w3, qkv, 0, M, N3, dModel, c->force_tile, gws, gemm_bytes);
     if (e != hipSuccess) return hip_status(c, e, "mha: QKV projection");
 
     aidn::AttnParams p{};
@@ -328,8 +339,8 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
     e = aidn::attn_fwd(sm, kind, p);
     if (e != hipSuccess) return hip_status(c, e, "mha: attention");
 
-    if (kind == 0) e = aidn::gemm_f32(sm, (const float*)cc, (const float*)wo, (float*)output, M, dModel, dModel, 1.0f, 0.0f, 0, 1, 0, 0, 0, tile32);
-    else e = aidn::gemm_16(sm, kind - 1, (const uint16_t*)cc, (const uint16_t*)wo, output, 0, M, dModel, dModel, c->force_tile, nullptr, 0);
+    if (kind == 0) e = aidn::gemm_f32(sm, (const float*)cc, (const float*)wo, (float*)output, M, dModel, dModel, 1.0f, 0.0f, 0, 1, 0, 0, 0, tile32, nullptr, 0, 0.0f, gws, nullptr, gemm_bytes);
+    else e = aidn::gemm_16(sm, kind - 1, (const uint16_t*)cc, (const uint16_t*)wo, output, 0, M, dModel, dModel, c->force_tile, gws, gemm_bytes);
     return hip_status(c, e, "mha: output projection");
 }
 
