@@ -139,22 +139,19 @@ int attn_common(void* ctx, void* stream, int kind, const aidn_attn_desc* d, cons
     if (kind == 0 && p.out16) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "attention: fp32 kernel has no 16-bit output");
     if (p.mask_mode != 0 && !mask) return fail(c, AIDN_ERR_INVALID_ARGUMENT, "attention: mask_mode set but mask is null");
     p.q = q; p.k = k; p.v = v; p.o = o; p.lse = lse; p.bias = bias; p.mask = p.mask_mode ? mask : nullptr; p.weights = weights;
-    if (weights && !lse) {
-        // the probabilities are rebuilt from the saved log-sum-exp: borrow the workspace for it
-        size_t need = (size_t)p.B * p.H * p.Sq * sizeof(float);
-        void* ws = nullptr;
-        st = acquire_ws(c, stream, need, &ws);
-        if (st) return st;
-        p.lse = (float*)ws;
-    }
     p.allow_fast_path = c->attn_fast_path;
-    if (!(weights && !lse)) {
-        // key-range partials of a call whose query tiles alone would leave most of the chip idle; a stream under capture whose
-        // workspace would have to grow simply runs unsplit
-        const size_t need = aidn::attn_fwd_workspace_bytes(kind, p);
-        void* ws = nullptr;
-        if (need && acquire_ws(c, stream, need, &ws) == AIDN_OK) { p.workspace = ws; p.workspace_bytes = need; }
+    // key-range partials of a call whose query tiles alone would leave most of the chip idle; a stream under capture whose
+    // workspace would have to grow simply runs unsplit
+    const size_t part = aidn::attn_fwd_workspace_bytes(kind, p);
+    // the probabilities are rebuilt from the saved log-sum-exp: borrow the workspace for it
+    const size_t stats = weights && !lse ? ((size_t)p.B * p.H * p.Sq * sizeof(float) + 255) & ~(size_t)255 : 0;
+    void* ws = nullptr;
+    if (part && acquire_ws(c, stream, stats + part, &ws) == AIDN_OK) { p.workspace = (unsigned char*)ws + stats; p.workspace_bytes = part; }
+    else if (stats) {
+        st = acquire_ws(c, stream, stats, &ws);
+        if (st) return st;
     }
+    if (stats) p.lse = (float*)ws;
     return hip_status(c, aidn::attn_fwd((hipStream_t)stream, kind, p), "attn_fwd");
 }
 
@@ -294,6 +291,20 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
     };
     const size_t base_bytes = wf_bytes + qkv_bytes + cc_bytes;
     size_t gemm_bytes = std::max(product_bytes(dModel), x3 ? 0 : product_bytes(3 * dModel));
+    // the attention reads the packed activation and writes the rows behind it, both 256-byte aligned (the addresses follow below); its key
+    // ranges share the scratch of the products
+    const int M = (int)rows, N3 = 3 * dModel;
+    aidn::AttnParams p{};
+    p.k = (const void*)((size_t)dModel * es); p.v = (const void*)((size_t)2 * dModel * es);
+    p.lse = nullptr; p.bias = nullptr; p.mask = mask_mode ? mask : nullptr; p.weights = nullptr;
+    p.B = B; p.H = heads; p.Hkv = heads; p.Sq = S; p.Sk = S; p.D = dHead;
+    p.scale = 1.0f / sqrtf((float)dHead); p.causal = 0; p.qoff = 0; p.softcap = 0.0f; p.mask_mode = mask_mode; p.out16 = kind != 0;
+    p.bias_bs = 0;
+    p.allow_fast_path = c->attn_fast_path;
+    for (int i = 0; i < 3; i++) { long long v = i == 0 ? (long long)S * N3 : (i == 1 ? dHead : N3); p.qs[i] = v; p.ks[i] = v; p.vs[i] = v; }
+    p.os[0] = (long long)S * dModel; p.os[1] = dHead; p.os[2] = dModel;
+    const size_t attn_bytes = aidn::attn_fwd_workspace_bytes(kind, p);
+    gemm_bytes = std::max(gemm_bytes, attn_bytes);
     void* ws = nullptr;
     int st = acquire_ws(c, stream, base_bytes + gemm_bytes, &ws);
     if (st && gemm_bytes) { gemm_bytes = 0; st = acquire_ws(c, stream, base_bytes, &ws); }
@@ -309,7 +320,6 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
         if (e != hipSuccess) return hip_status(c, e, "mha: weight gather");
     }
     const void* w3 = wqkv ? wqkv : (const void*)wf;
-    const int M = (int)rows, N3 = 3 * dModel;
     const int tile32 = c->force_tile;
     if (x3) {
         const void* b[3] = {wq, wk, wv};
@@ -327,15 +337,8 @@ int mha_common(void* ctx, void* stream, int kind, const void* input, const void*
     else e = aidn::gemm_16(sm, kind - 1, (const uint16_t*)input, (const uint16_t*)w3, qkv, 0, M, N3, dModel, c->force_tile, gws, gemm_bytes);
     if (e != hipSuccess) return hip_status(c, e, "mha: QKV projection");
 
-    aidn::AttnParams p{};
     p.q = qkv; p.k = qkv + (size_t)dModel * es; p.v = qkv + (size_t)2 * dModel * es; p.o = cc;
-    p.lse = nullptr; p.bias = nullptr; p.mask = mask_mode ? mask : nullptr; p.weights = nullptr;
-    p.B = B; p.H = heads; p.Hkv = heads; p.Sq = S; p.Sk = S; p.D = dHead;
-    p.scale = 1.0f / sqrtf((float)dHead); p.causal = 0; p.qoff = 0; p.softcap = 0.0f; p.mask_mode = mask_mode; p.out16 = kind != 0;
-    p.bias_bs = 0;
-    p.allow_fast_path = c->attn_fast_path;
-    for (int i = 0; i < 3; i++) { long long v = i == 0 ? (long long)S * N3 : (i == 1 ? dHead : N3); p.qs[i] = v; p.ks[i] = v; p.vs[i] = v; }
-    p.os[0] = (long long)S * dModel; p.os[1] = dHead; p.os[2] = dModel;
+    if (gemm_bytes >= attn_bytes) { p.workspace = gws; p.workspace_bytes = attn_bytes; }
     e = aidn::attn_fwd(sm, kind, p);
     if (e != hipSuccess) return hip_status(c, e, "mha: attention");
 

@@ -1106,9 +1106,9 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void attn_fwd_dl_kernel(cons
     }   // pass
 }
 
-// Merge of the key-range partials of the fast kernel (head dimension 128; part: [row][nsplit][130]), WPR waves per query row.  With a
+// Merge of the key-range partials of the fast kernel and of the split one (part: [row][nsplit][2 + D], D up to 128), WPR waves per query row.  With a
 // workgroup of 128 threads per row (weights through LDS, then the rows) 16384 rows of four ranges took 16.2 us, this way 8.8 (34 MB).
-template <typename OutT, int WPR>
+template <typename OutT, int WPR, bool KEEP_NAN>
 __global__ __launch_bounds__(256) void attn_split_merge_kernel(const AttnArgs a, int rows)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -1117,8 +1117,10 @@ __global__ __launch_bounds__(256) void attn_split_merge_kernel(const AttnArgs a,
     const int bh = row / a.Sq, qi = row - bh * a.Sq;
     const int b = bh / a.H, hd = bh - b * a.H;
     f32x2p o[1];
-    const float lse = merge_partials<1, WPR>(a.part + (long long)row * a.nsplit * 130, a.nsplit, 128, 128, wave % WPR, lane, o);
+    const float lse = merge_partials<1, WPR, KEEP_NAN>(a.part + (long long)row * a.nsplit * (2 + a.D), a.nsplit, a.D, a.D, wave % WPR, lane, o);
     if (wave % WPR != 0) return;
+    if (lane == 0 && a.lse) a.lse[row] = lse;
+    if (2 * lane >= a.D) return;
     typedef typename Raw2<OutT>::type out_t;
     out_t* O = (out_t*)a.o + b * a.os[0] + hd * a.os[1] + (long long)qi * a.os[2] + 2 * lane;
     if constexpr (Elem<OutT>::BYTES == 4) {
@@ -1129,7 +1131,15 @@ __global__ __launch_bounds__(256) void attn_split_merge_kernel(const AttnArgs a,
         if (a.vec_out) *(uint32_t*)O = w;
         else { O[0] = (out_t)(w & 0xFFFFu); O[1] = (out_t)(w >> 16); }
     }
-    if (lane == 0 && a.lse) a.lse[row] = lse;
+}
+template <typename OutT, bool KEEP_NAN>
+static hipError_t launch_merge(const AttnArgs& a, hipStream_t stream)
+{
+    const long long rows = (long long)a.B * a.H * a.Sq;
+    if (rows > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+    if (merge_waves_per_row(a.nsplit) == 1) hipLaunchKernelGGL((attn_split_merge_kernel<OutT, 1, KEEP_NAN>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, a, (int)rows);
+    else hipLaunchKernelGGL((attn_split_merge_kernel<OutT, 4, KEEP_NAN>), dim3((unsigned)rows), dim3(256), 0, stream, a, (int)rows);
+    return hipGetLastError();
 }
 
 template <typename T, typename OutT, int D = 128, bool PAGED = false, bool KM = false>
@@ -1146,13 +1156,10 @@ static hipError_t launch_attn_dl(AttnArgs a, hipStream_t stream)
         // few query tiles over a long key sequence: every tile's keys are cut into ranges that run side by side; a merge pass follows
         a.paired = 0;
         const long long nblk = (long long)a.qtiles * a.B * a.H * a.nsplit;
-        const long long rows = (long long)a.B * a.H * a.Sq;
-        if (nblk > 0x7FFFFFFFLL || rows > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+        if (nblk > 0x7FFFFFFFLL || (long long)a.B * a.H * a.Sq > 0x7FFFFFFFLL) return hipErrorInvalidValue;
         hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(256), smem, stream, a);
         if (hipError_t e = hipGetLastError()) return e;
-        if (merge_waves_per_row(a.nsplit) == 1) hipLaunchKernelGGL((attn_split_merge_kernel<OutT, 1>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, a, (int)rows);
-        else hipLaunchKernelGGL((attn_split_merge_kernel<OutT, 4>), dim3((unsigned)rows), dim3(256), 0, stream, a, (int)rows);
-        return hipGetLastError();
+        return launch_merge<OutT, false>(a, stream);
     }
     // causal self-attention with an even number of query tiles: pair tile i with tile qtiles-1-i, so every workgroup has the same work
     a.paired = (a.causal && a.qoff == 0 && a.Sq == a.Sk && a.qtiles >= 2 && a.qtiles % 2 == 0) ? 1 : 0;
@@ -1535,18 +1542,8 @@ static int attn_dl_splits(const AttnParams& p, int* chunk)
     return ns >= 2 ? ns : 1;
 }
 
-size_t attn_fwd_workspace_bytes(int kind, const AttnParams& p)
+static AttnArgs attn_args(int kind, const AttnParams& p)
 {
-    if (!attn_dl_applies(kind, p)) return 0;
-    int chunk;
-    const int ns = attn_dl_splits(p, &chunk);
-    return ns > 1 ? (size_t)p.B * p.H * p.Sq * ns * 130 * sizeof(float) : 0;
-}
-
-// kind: 0 fp32, 1 fp16, 2 bf16
-hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
-{
-    const bool g_attn_allow_dl = p.allow_fast_path != 0;      // 0 (test hook of the context): every shape takes the general kernel
     AttnArgs a;
     a.paired = 0;
     a.hgroup = 0;
@@ -1559,7 +1556,6 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     a.qtiles = 0;
     a.bt = p.block_table; a.bsz = p.block_size; a.bt_bs = p.block_table_stride;
     a.dbsz = make_fastdiv((uint32_t)(p.block_table ? p.block_size : 1));
-    if (p.block_table && p.weights) return hipErrorInvalidValue;      // the weights output does not follow a block table
     const int eb = kind == 0 ? 4 : 2, e = 16 / eb;
     const int oeb = (kind == 0 || !p.out16) ? 4 : 2;
     auto al = [](const void* ptr, const long long* s, int bytes) {
@@ -1567,6 +1563,25 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     };
     a.vec_in = (p.D % e == 0) && al(p.q, p.qs, eb) && al(p.k, p.ks, eb) && al(p.v, p.vs, eb);
     a.vec_out = (p.D % 4 == 0) && al(p.o, p.os, oeb);
+    return a;
+}
+
+size_t attn_fwd_workspace_bytes(int kind, const AttnParams& p)
+{
+    int chunk, ns = 1;
+    if (kind == 0) {
+        const AttnArgs a = attn_args(kind, p);
+        if (attn_split_applies(a)) ns = attn_split_ranges(a);
+    } else if (attn_dl_applies(kind, p)) ns = attn_dl_splits(p, &chunk);
+    return ns > 1 ? (size_t)p.B * p.H * p.Sq * ns * (2 + p.D) * sizeof(float) : 0;
+}
+
+// kind: 0 fp32, 1 fp16, 2 bf16
+hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
+{
+    const bool g_attn_allow_dl = p.allow_fast_path != 0;      // 0 (test hook of the context): every shape takes the general kernel
+    if (p.block_table && p.weights) return hipErrorInvalidValue;      // the weights output does not follow a block table
+    AttnArgs a = attn_args(kind, p);
     const bool full = p.bias != nullptr || a.mask_mode != 0 || p.softcap > 0.0f;
     // a mask of the keys alone is followed by the direct-to-LDS instances at head dimensions 64 and 128 as well
     const bool km = a.mask_mode == 3 && !p.block_table && (p.D == 64 || p.D == 128);
@@ -1584,6 +1599,10 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
         if (ns > 1 && p.workspace_bytes >= (size_t)p.B * p.H * p.Sq * ns * 130 * sizeof(float)) {
             a.nsplit = ns; a.chunk = chunk; a.part = (float*)p.workspace;
         }
+    }
+    if (split && p.workspace) {
+        const int ns = attn_split_ranges(a);
+        if (ns > 1 && p.workspace_bytes >= (size_t)p.B * p.H * p.Sq * ns * (2 + p.D) * sizeof(float)) { a.nsplit = ns; a.part = (float*)p.workspace; }
     }
     // Unsplit prefill has two kernels.  The software-pipelined one is the faster (894 against 840 TFLOP/s on causal B4 H32 S2048 fp16,
     // 1035 against 983 without the mask, 312 against 292 at S 128) except where a sequence ends inside a 64-key tile and the passes
@@ -1605,7 +1624,10 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
         if (kind == 1) err = p.out16 ? launch_attn_dl<f16_t, f16_t>(a, stream) : launch_attn_dl<f16_t, float>(a, stream);
         else err = p.out16 ? launch_attn_dl<bf16_t, bf16_t>(a, stream) : launch_attn_dl<bf16_t, float>(a, stream);
     } else
-    if (split) err = launch_attn_split(a, full, stream);
+    if (split) {
+        err = launch_attn_split(a, full, stream);
+        if (err == hipSuccess && a.nsplit > 1) err = launch_merge<float, true>(a, stream);
+    }
     else
     if (kind == 0) {
         // fp32: 64-key tiles while two workgroups still fit the LDS of a CU (head dimension up to 64), else 32-key tiles

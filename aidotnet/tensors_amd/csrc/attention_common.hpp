@@ -30,6 +30,7 @@ struct AttnArgs {
     int alt_from;  // pipelined prefill kernel: first workgroup of the second half of a resident grid (shares its CU with an earlier one)
     FastDiv dgroup, dunits, dqtiles;      // pipelined prefill kernel: H / Hkv, qtiles / 2, qtiles as divisors
     int hgroup;    // general kernel, causal: > 0 heads per group of the workgroup order of a large grid; < 0 the placement of a small one
+    // fp32 on the fp16 pipe: workgroup (x, y) of the grid takes the y-th of nsplit equal shares of its query tile's keys, part as below with D in the place of 128
     // fast kernel, grouped decode: the workgroup's key range is split `split` of nsplit (chunk keys each) and, when part is not
     // null, it stores its unnormalised partial (m, l, O[128]) at part + ((b H_q + head) nsplit + split) * 130 for the merge pass
     int nsplit, chunk; float* part;
@@ -237,7 +238,8 @@ template <> __device__ __forceinline__ uint32_t pack2_p<bf16_t>(float a, float b
 // Bound by memory latency: eight partial rows per wave are asked for together with the (m, l) pairs, so up to 8 WPR ranges cost one
 // round trip; up to eight ranges need no barrier and no LDS.  A range that saw no key weighs zero and adds nothing.
 typedef float f32x2p __attribute__((ext_vector_type(2)));
-template <int NV, int WPR>
+// KEEP_NAN: a sum that is no number gives NaN instead of zeros, as a single range of the fp32 split kernel does.
+template <int NV, int WPR, bool KEEP_NAN = false>
 __device__ __forceinline__ float merge_partials(const float* __restrict__ P, int n, int dpad, int D, int part, int lane, f32x2p (&out)[NV])
 {
     const long long stride = 2 + dpad;
@@ -295,7 +297,7 @@ __device__ __forceinline__ float merge_partials(const float* __restrict__ P, int
 #pragma unroll
     for (int j = 0; j < NV; j++)
 #pragma unroll
-        for (int e = 0; e < 2; e++) out[j][e] = L > 0.0f ? out[j][e] / L : 0.0f;
+        for (int e = 0; e < 2; e++) out[j][e] = (KEEP_NAN ? L != 0.0f : L > 0.0f) ? out[j][e] / L : 0.0f;
     return L > 0.0f ? (M + __builtin_amdgcn_logf(L)) * LN2 : -INFINITY;
 }
 // waves per row of the merge passes: one (four rows to a workgroup) while a row's ranges fit one round of loads
@@ -303,6 +305,7 @@ inline int merge_waves_per_row(int ranges) { return ranges <= 8 ? 1 : 4; }
 
 // fp32 attention on the bf16 matrix pipe (attention_split.hip); options: bias, masks, soft-cap
 bool attn_split_applies(const AttnArgs& a);
+int attn_split_ranges(const AttnArgs& a);
 hipError_t launch_attn_split(const AttnArgs& a, bool options, hipStream_t stream);
 hipError_t launch_attn_weights_split(const AttnArgs& a, float* w, hipStream_t stream);
 // 16-bit, head dimension 128, plain / causal attention in the software-pipelined form (attention_prefill.hip); kind: 1 fp16, 2 bf16

@@ -172,6 +172,14 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         if (lastkey < 0) ntiles = 0;
         else { const long long nt = lastkey / BC + 1; if (nt < ntiles) ntiles = (int)nt; }
     }
+    // this workgroup's share of them (from here on ntiles is where it ends)
+    constexpr bool RANGES = !OPT || DP <= 64;     // (the others are out of registers: 12 of them would go to scratch memory)
+    int first = 0;
+    if (RANGES && a.nsplit > 1) {
+        const int per = (ntiles + a.nsplit - 1) / a.nsplit;
+        first = min((int)blockIdx.y * per, ntiles);
+        ntiles = min(ntiles, first + per);
+    }
 
     // ---- staging: thread t takes chunk t % CPR of keys t / CPR + i RPU
     u32x4 rk[U][2], rv[U][2];
@@ -211,27 +219,27 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         for (int s = 0; s < 2; s++) *(u32x4*)(Vs + s * PL + i * RPU * RB + v_at<RB>(t / CPR, t % CPR)) = w[s];
     };
     const uint32_t krs = (uint32_t)a.ks[2], vrs = (uint32_t)a.vs[2];
-    if (ntiles > 0) {
-        if constexpr (PAGED) rows_of(0);
+    if (first < ntiles) {
+        if constexpr (PAGED) rows_of(first);
         else {
             klast = 4u * ((uint32_t)(a.Sk - 1) * krs + col);
             vlast = 4u * ((uint32_t)(a.Sk - 1) * vrs + col);
 #pragma unroll
             for (int i = 0; i < U; i++) {
-                kat[i] = min(4u * ((uint32_t)(t / CPR + i * RPU) * krs + col), klast);
-                vat[i] = min(4u * ((uint32_t)(t / CPR + i * RPU) * vrs + col), vlast);
+                kat[i] = min(4u * ((uint32_t)(first * BC + t / CPR + i * RPU) * krs + col), klast);
+                vat[i] = min(4u * ((uint32_t)(first * BC + t / CPR + i * RPU) * vrs + col), vlast);
             }
         }
         load(K, krs, kat, klast, rk);
         load(V, vrs, PAGED ? kat : vat, vlast, rv);
-        if constexpr (PAGED) rows_of(1);
+        if constexpr (PAGED) rows_of(first + 1);
     }
 
     u32x4 qf[DS][2];
     int logit_exp = -split_q(Q + (long long)min(q0 + l32, a.Sq - 1) * a.qs[2], q0 + l32 < a.Sq, a.D, h, qf);      // logits are 2^logit_exp Q' K'
     // ---- K and V: one power of two each, from the first tile
     int vexp = 0;
-    if (ntiles > 0) {
+    if (first < ntiles) {
         float km = 0.0f, vm = 0.0f;
 #pragma unroll
         for (int i = 0; i < U; i++) {
@@ -384,7 +392,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     const unsigned char* kbase = Ks + (kg * KT * 32) * RB;
     const unsigned char* vbase = Vs + (kg * KT * 32) * RB;
     const int jl = lane & 15, vkey = 4 * h + (jl >> 2), vch = 2 * ((lane >> 4) & 1) + ((jl & 3) >> 1), vcol = 8 * (jl & 1);      // transposing reads
-    for (int j = 0; j < ntiles; j++) {
+    for (int j = first; j < ntiles; j++) {
         const int kw0 = j * BC + kg * KT * 32;                      // this wave's first key
         load(K, krs, kat, klast, rk);                                 // (past the last tile rows are repeated)
         uint64_t kept = ~0ull;
@@ -533,7 +541,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
             if (d0 < a.D) {
                 f32x4 m = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 8
-                for (int key = t / (DP / 4); key < keys; key += NT / (DP / 4)) {
+                for (int key = first * BC + t / (DP / 4); key < keys; key += NT / (DP / 4)) {
                     const f32x4 x = *(const f32x4*)(V + paged_row(bt, a.bsz, key) * a.vs[2] + d0);
 #pragma unroll
                     for (int e = 0; e < 4; e++) m[e] = fmaxf(m[e], fabsf(x[e]));
@@ -552,7 +560,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
             vexp = 0;
             to_log2 = OPT ? a.scale : a.scale * LOG2E;
 #pragma unroll 1
-            for (int k0 = kg * KT * 32; k0 < ntiles * BC; k0 += k0 % (KT * 32) + 32 < KT * 32 ? 32 : BC - (KT - 1) * 32) {
+            for (int k0 = first * BC + kg * KT * 32; k0 < ntiles * BC; k0 += k0 % (KT * 32) + 32 < KT * 32 ? 32 : BC - (KT - 1) * 32) {
                 if (q0 >= a.Sq || k0 >= a.Sk || (a.causal && (long long)k0 > (long long)q_last + a.qoff)) continue;
                 uint64_t kept = ~0ull;
                 if constexpr (OPT) { if (a.mask_mode == 3) kept = visible(k0, 32) | ~0ull << 32; }
@@ -627,11 +635,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     // ---- normalise and store: lane holds query q0 + l32, head-dim elements 32 i + 8 g + 4 h + (0..3)
     const int qi = q0 + l32;
     const float l = sum_with_partner32(l_run);
-    const float inv = l > 0.0f ? power2(-vexp) / l : 0.0f;
-    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? (m_run + (__builtin_amdgcn_logf(l) - P_EXP)) * LN2 : -INFINITY;
-    float* __restrict__ O = (float*)a.o + b * a.os[0] + hd * a.os[1];
-    if (a.vec_out && a.D == DP) {
-        // through LDS (16 rows at a time for each wave: chunk c of row r at position c ^ r) and written as whole rows past the caches
+    // through LDS (16 rows at a time for each wave: chunk c of row r at position c ^ r) and written as whole rows
+    auto by_rows = [&](auto value, auto store) {
         constexpr int CH = DP / 4, RPI = 64 / CH;
         unsigned char* stg = smem + wq * (16 * DP * 4);
         const int c = lane % CH;
@@ -643,17 +648,40 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
 #pragma unroll
                     for (int g = 0; g < 4; g++)
                         *(f32x4*)(stg + (l32 & 15) * (DP * 4) + (((8 * i + 2 * g + h) ^ (l32 & (CH - 1) & 15)) << 4)) =
-                            f32x4{oacc[i][4 * g] * inv, oacc[i][4 * g + 1] * inv, oacc[i][4 * g + 2] * inv, oacc[i][4 * g + 3] * inv};
+                            f32x4{value(oacc[i][4 * g]), value(oacc[i][4 * g + 1]), value(oacc[i][4 * g + 2]), value(oacc[i][4 * g + 3])};
             }
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int q = 0; q < 16 / RPI; q++) {
                 const int r = RPI * q + lane / CH, row = q0 + 16 * half + r;
                 const f32x4 v = *(const f32x4*)(stg + r * (DP * 4) + ((c ^ (r & (CH - 1) & 15)) << 4));
-                if (row < a.Sq) __builtin_nontemporal_store(v, (f32x4*)(O + (long long)row * a.os[2] + 4 * c));
+                if (row < a.Sq) store(row, 4 * c, v);
             }
             __builtin_amdgcn_wave_barrier();
         }
+    };
+    if (RANGES && a.part) {
+        // a key range: (m, l, O) for the merge.  Everything is scaled by a power of two that brings l below 2^-5 (2^0 where V is small), so that
+        // the sum over up to 32 ranges does not leave the range of fp32 where the result does not; m takes that power and stays exact, being whole
+        float* __restrict__ P = a.part + ((long long)bh * a.Sq * a.nsplit + blockIdx.y) * (2 + a.D);
+        const long long pitch = (long long)a.nsplit * (2 + a.D);
+        const int e = __builtin_amdgcn_frexp_expf(l) + (vexp > 0 ? 0 : 5);
+        if (h == 0 && qi < a.Sq) *(f32x2p*)(P + qi * pitch) = f32x2p{m_run + ((float)e - P_EXP), __builtin_amdgcn_ldexpf(l, -e)};
+        by_rows([&](float x) { return __builtin_amdgcn_ldexpf(x, -vexp - e); },
+                [&](int row, int d0, f32x4 v) {
+                    if (d0 >= a.D) return;
+                    float* __restrict__ p = P + row * pitch + 2 + d0;                  // (8-byte aligned)
+                    *(f32x2p*)p = f32x2p{v[0], v[1]};
+                    *(f32x2p*)(p + 2) = f32x2p{v[2], v[3]};
+                });
+        return;
+    }
+    const float inv = l > 0.0f ? power2(-vexp) / l : 0.0f;
+    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? (m_run + (__builtin_amdgcn_logf(l) - P_EXP)) * LN2 : -INFINITY;
+    float* __restrict__ O = (float*)a.o + b * a.os[0] + hd * a.os[1];
+    if (a.vec_out && a.D == DP) {
+        by_rows([&](float x) { return x * inv; },
+                [&](int row, int d0, f32x4 v) { __builtin_nontemporal_store(v, (f32x4*)(O + (long long)row * a.os[2] + d0)); });
     } else if (qi < a.Sq) {
         float* __restrict__ p = O + (long long)qi * a.os[2];
 #pragma unroll
@@ -680,8 +708,8 @@ static hipError_t launch_split_as(AttnArgs a, hipStream_t stream)
     a.qtiles = (a.Sq + BR - 1) / BR;
     const long long nblk = (long long)a.qtiles * a.B * a.H;
     if (nblk > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-    a.hgroup = !a.causal ? 0 : nblk <= 768 ? -1 : (a.qtiles >= 8 ? 16 : (128 + a.qtiles - 1) / a.qtiles);
-    hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(64 * NW), smem, stream, a);
+    a.hgroup = !a.causal || a.nsplit > 1 ? 0 : nblk <= 768 ? -1 : (a.qtiles >= 8 ? 16 : (128 + a.qtiles - 1) / a.qtiles);
+    hipLaunchKernelGGL(kern, dim3((unsigned)nblk, (unsigned)a.nsplit), dim3(64 * NW), smem, stream, a);
     return hipGetLastError();
 }
 
@@ -722,6 +750,27 @@ static hipError_t launch_split_opt(const AttnArgs& a, hipStream_t stream)
         return fine ? launch_split_as<64, 64, 4, 2, OPT, PAGED>(a, stream) : launch_split_as<64, 64, 4, 1, OPT, PAGED>(a, stream);
     }
     return grid(128) <= 256 && seen_keys(a) >= 224 ? launch_split_as<128, 64, 8, 2, OPT, PAGED>(a, stream) : launch_split_as<128, 32, 4, 1, OPT, PAGED>(a, stream);
+}
+// Ranges of the keys that run as workgroups of their own and are merged by a pass behind (1 = none), where the query tiles leave at least half of
+// the CUs without one.  A workgroup on a CU of its own takes 2.4 us a tile of 64 keys beyond head dimension 64, 1.7 and 1.0 a tile of 128 up to 64
+// and 32; the second launch is 4, the partials are written and read at 4 TB/s (us a call, in one / cut: 8 heads of 40 queries d128
+// 256 keys 20.2 / 16.4, 1024 47.9 / 17.6, 2048 84.4 / 19.4; d64 1024 22.7 / 14.7, 2048 36.2 / 15.1; plain self-attention d128 H8 S1000 52.8 / 36.3, H16 S1000
+// 53.0 / 48.2, H16 S500 33.0 / 30.7, d64 H4 S2000 37.1 / 30.8, H8 S1000 23.2 / 23.2; in two ranges d128 H32 S390 29.9 / 34.5, d64 H8 S800 20.9 / 22.3, d32 14.3 / 16.1).
+int attn_split_ranges(const AttnArgs& a)
+{
+    const bool wide = a.D > 64;
+    const int rows = wide ? 128 : 64, tile = wide ? 64 : 128;
+    const long long grid = (long long)((a.Sq + rows - 1) / rows) * a.B * a.H, keys = seen_keys(a);
+    if (grid > 128 || keys < (wide ? 224 : 448) || (wide && (a.bias || a.mask_mode != 0 || a.softcap > 0.0f))) return 1;
+    const long long tiles = (keys + tile - 1) / tile, most = std::min(std::min(256 / grid, tiles), 32LL);
+    const double tile_us = wide ? 2.4 : a.D > 32 ? 1.7 : 1.0, part_us = (double)a.B * a.H * a.Sq * (2 + a.D) * 8.0 / 4e6;
+    int best = 1;
+    double gain = 0.5;
+    for (int ns = 2; ns <= most; ns++) {
+        const double g = tile_us * (double)(tiles - (tiles + ns - 1) / ns) - 4.0 - part_us * ns;
+        if (g > gain) { gain = g; best = ns; }
+    }
+    return best;
 }
 hipError_t launch_attn_split(const AttnArgs& a, bool options, hipStream_t stream)
 {

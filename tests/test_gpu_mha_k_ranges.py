@@ -58,3 +58,26 @@ def test_output_projection_in_ranges(kind, B, S, dM, heads, packed):
             graph.replay()
             torch.cuda.synchronize()
             assert err() <= limit
+
+
+@pytest.mark.parametrize("kind,B,S,dM,heads", [("f32", 1, 1100, 256, 4), ("f32", 2, 800, 384, 3), ("bf16", 1, 1100, 512, 4), ("f16", 2, 1500, 256, 2)])
+def test_attention_of_the_layer_in_key_ranges(kind, B, S, dM, heads):
+    """Few heads over a long sequence: the layer's attention cuts its keys too, with a padding mask that hides whole ranges."""
+    from aidotnet.tensors_amd import Mi355Backend, Mi355Engine
+    eng = Mi355Engine(Mi355Backend())
+    dt = TORCH16.get(kind, torch.float32)
+    gen = torch.Generator(device="cuda").manual_seed(dM + S)
+    x = torch.randn(B, S, dM, device="cuda", generator=gen).to(dt)
+    ws = [(torch.randn(dM, dM, device="cuda", generator=gen) / math.sqrt(dM)).to(dt) for _ in range(4)]
+    for keep in (None, torch.arange(S, device="cuda")[None, :] < torch.tensor([S // 3, S - 1][:B], device="cuda")[:, None]):
+        mask = None if keep is None else keep[:, None, None, :]
+        call = lambda: eng.MultiHeadAttentionForward(x, *ws, heads, mask)
+        if kind != "f32" or keep is None or dM // heads <= 64:
+            assert any(n.startswith("attn_split_merge_kernel") for n in kernels_of(call))
+        out = call()
+        q, k, v = ((x.double() @ w.double()).view(B, S, heads, dM // heads).transpose(1, 2) for w in ws[:3])
+        s = (q @ k.transpose(-1, -2).contiguous()) / math.sqrt(dM // heads)
+        if keep is not None:
+            s = s.masked_fill(~mask, -math.inf)
+        want = (torch.softmax(s, -1) @ v).transpose(1, 2).reshape(B, S, dM) @ ws[3].double()
+        assert float(((out.double() - want).abs() / want.abs().clamp(min=1.0)).max()) <= (1e-4 if kind == "f32" else 2e-2)
