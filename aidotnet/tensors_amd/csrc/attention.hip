@@ -1449,7 +1449,8 @@ static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
         auto grid = [&](int rows) { return (long long)((a.Sq + rows - 1) / rows) * a.B * a.H; };
         if constexpr (!FULL && Elem<T>::BYTES == 2 && DP == 64) {
             if (a.Sk > 64 && grid(64) <= (a.causal ? 640 : 256)) {
-                if constexpr (!KM) { if (a.Sk >= 96) return launch_attn_kg<T, OutT, DP, 128, FULL, DMA ? 2 : 1, DMA, KM, 2>(a, stream); }
+                // (direct loads of a 128-key tile: a wave's 32 keys lie in one block)
+                if constexpr (!KM) { if (a.Sk >= 96 && (!DMA || !a.bt || a.bsz % 32 == 0)) return launch_attn_kg<T, OutT, DP, 128, FULL, DMA ? 2 : 1, DMA, KM, 2>(a, stream); }
                 return launch_attn_kg<T, OutT, DP, 64, FULL, 2, DMA, KM, 2>(a, stream);
             }
             return launch_attn_kg<T, OutT, DP, BC, FULL, MINB, DMA, KM>(a, stream);
