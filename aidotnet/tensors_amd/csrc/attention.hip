@@ -104,6 +104,14 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
         if (lastkey < 0) ntiles = 0;
         else { long long nt = lastkey / BC + 1; if (nt < ntiles) ntiles = (int)nt; }
     }
+    // a share of them (ranges of the keys; from here on ntiles is where it ends)
+    constexpr bool RANGES = EB == 2 && DP == 64 && !FULL;
+    int first = 0;
+    if (RANGES && a.nsplit > 1) {
+        const int per = (ntiles + a.nsplit - 1) / a.nsplit;
+        first = min((int)blockIdx.y * per, ntiles);
+        ntiles = min(ntiles, first + per);
+    }
 
     u32x4 rk[UK];
     u32x4 rv[UV * 4];
@@ -219,9 +227,9 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
         int row0 = tile * BC + NK * wave_s, left = a.Sk - 1 - row0;
         if (bt) {
             const int last_group = (a.Sk - 1) / NK * NK;
-            if ((tile & 63) == 0) rows = paged_tile_rows(bt, a.bsz, a.dbsz, NK * wave_s, BC, tile, lane, last_group);
+            if (((tile - first) & 63) == 0) rows = paged_tile_rows(bt, a.bsz, a.dbsz, NK * wave_s, BC, tile, lane, last_group);
             left = a.Sk - 1 - min(row0, last_group);
-            row0 = __builtin_amdgcn_readlane(rows, tile & 63);
+            row0 = __builtin_amdgcn_readlane(rows, (tile - first) & 63);
         }
         if (FIXED && left >= NK - 1) {
             // whole: a uniform base and lane offsets that stay (the swizzle repeats with 16 keys)
@@ -250,18 +258,18 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     };
     uint64_t kbits = ~0ull;
     if constexpr (DMA) {
-        if (ntiles > 0) issue_tile(0, 0);
-        if constexpr (KM) kbits = tile_keys(0, kmask[min(lane, a.Sk - 1)]);
+        if (first < ntiles) issue_tile(first, first & 1);
+        if constexpr (KM) kbits = tile_keys(first * BC, kmask[min(first * BC + lane, a.Sk - 1)]);
         __builtin_amdgcn_s_waitcnt(0);
     } else {
-        if (ntiles > 0) {
-            load_tile(0);
-            store_tile(0);
+        if (first < ntiles) {
+            load_tile(first * BC);
+            store_tile(first & 1);
         }
     }
     __syncthreads();
 
-    for (int j = 0; j < ntiles; j++) {
+    for (int j = first; j < ntiles; j++) {
         const int stage = j & 1;
         const int kv0 = j * BC;
         const int kw0 = kv0 + kg * KT * 32;      // first key of this wave's sub-tiles
@@ -520,6 +528,26 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 
     // ---- normalise and store: lane holds query qi, head-dim elements i*32 + 8 g + 4 h + (0..3)
     const float l_tot = l_run + shfl_xor_f(l_run, 32);
+    if constexpr (RANGES) {
+        if (a.part) {
+            // a key range: (m, l, O) for the merge, whole rows at a time through the (idle) tile memory
+            unsigned char* stg = smem + wq * (32 * DP * 4);
+            const int row0 = q0 + wq * 32, nrow = min(32, a.Sq - row0);
+            if (nrow <= 0) return;
+#pragma unroll
+            for (int i = 0; i < DT; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *(f32x4*)(stg + l32 * (DP * 4) + (((8 * i + 2 * g + h) ^ (l32 & 15)) << 4)) =
+                        f32x4{oacc[i][4 * g + 0], oacc[i][4 * g + 1], oacc[i][4 * g + 2], oacc[i][4 * g + 3]};
+            float* __restrict__ P = a.part + (((long long)bh * a.Sq + row0) * a.nsplit + blockIdx.y) * (2 + DP);
+            const long long pitch = (long long)a.nsplit * (2 + DP);
+            if (h == 0 && l32 < nrow) *(f32x2p*)(P + l32 * pitch) = f32x2p{m_run, l_tot};
+            for (int r = h; r < nrow; r += 2)                           // a row to each half of the wave, a pair of elements to a lane
+                *(f32x2p*)(P + r * pitch + 2 + 2 * l32) = *(const f32x2p*)(stg + r * (DP * 4) + (((l32 >> 1) ^ (r & 15)) << 4) + 8 * (l32 & 1));
+            return;
+        }
+    }
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
     if constexpr (DMA && Elem<OutT>::BYTES == 4 && DP <= 128) {
         if (a.vec_out && a.D == DP) {
@@ -1408,8 +1436,8 @@ static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
     if (nblk > 0x7FFFFFFFLL) return hipErrorInvalidValue;
     // causal order: up to 768 workgroups the balanced placement of a grid that is (nearly) resident at once (measured equal or
     // better than the grouped order up to that size); beyond, groups of at least 16 heads and at least 128 workgroups
-    a.hgroup = !a.causal ? 0 : nblk <= 768 ? -1 : (a.qtiles >= 8 ? 16 : (128 + a.qtiles - 1) / a.qtiles);
-    hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(256), smem, stream, a);
+    a.hgroup = !a.causal || a.nsplit > 1 ? 0 : nblk <= 768 ? -1 : (a.qtiles >= 8 ? 16 : (128 + a.qtiles - 1) / a.qtiles);
+    hipLaunchKernelGGL(kern, dim3((unsigned)nblk, (unsigned)a.nsplit), dim3(256), smem, stream, a);
     return hipGetLastError();
 }
 
@@ -1543,6 +1571,26 @@ static int attn_dl_splits(const AttnParams& p, int* chunk)
     return ns >= 2 ? ns : 1;
 }
 
+// 16-bit, head dimension 64, at most half of the CUs with a workgroup of 64 queries: shares of each query tile's keys run as workgroups of their
+// own (1 = none).  A workgroup takes 4.5 us and 1.15 for 128 keys there, the second launch 4 and the partials as in attn_split_ranges; a call costs its
+// caller 11.7 us, with two launches 14 (us in one / cut: 189 queries on 3984 keys, 16 heads 40 / 18.1, 614 on 3138, 12 heads 33 / 25.4; self-attention
+// H4 S2000 23.1 / 20.8, H2 S4000 41 / 29.4; left whole: 40 queries on 1024 keys 13.4 / 14.7, H32 100 on 900 14.1 / 14.7).
+static int attn_half64_ranges(int kind, const AttnParams& p)
+{
+    if (kind == 0 || p.D != 64 || p.bias || p.softcap > 0.0f || (p.mask && p.mask_mode != 0)) return 1;
+    const long long keys = p.causal ? std::min((long long)p.Sk, std::max(0LL, (long long)p.Sq + p.qoff)) : p.Sk;
+    const long long grid = (long long)((p.Sq + 63) / 64) * p.B * p.H, tiles = (keys + 127) / 128;
+    if (grid > 128) return 1;
+    const double part_us = (double)p.B * p.H * p.Sq * (2 + p.D) * 8.0 / 4e6;
+    int best = 1;
+    double least = std::max(11.7, 4.5 + 1.15 * tiles) - 0.3;
+    for (int ns = 2; ns <= std::min(std::min(256 / grid, tiles), 32LL); ns++) {
+        const double us = std::max(14.0, 8.5 + 1.15 * (double)((tiles + ns - 1) / ns) + part_us * ns);
+        if (us < least) { least = us; best = ns; }
+    }
+    return best;
+}
+
 static AttnArgs attn_args(int kind, const AttnParams& p)
 {
     AttnArgs a;
@@ -1574,6 +1622,7 @@ size_t attn_fwd_workspace_bytes(int kind, const AttnParams& p)
         const AttnArgs a = attn_args(kind, p);
         if (attn_split_applies(a)) ns = attn_split_ranges(a);
     } else if (attn_dl_applies(kind, p)) ns = attn_dl_splits(p, &chunk);
+    else ns = attn_half64_ranges(kind, p);
     return ns > 1 ? (size_t)p.B * p.H * p.Sq * ns * (2 + p.D) * sizeof(float) : 0;
 }
 
@@ -1601,8 +1650,9 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
             a.nsplit = ns; a.chunk = chunk; a.part = (float*)p.workspace;
         }
     }
-    if (split && p.workspace) {
-        const int ns = attn_split_ranges(a);
+    const int ns64 = attn_half64_ranges(kind, p);
+    if ((split || ns64 > 1) && p.workspace) {
+        const int ns = split ? attn_split_ranges(a) : ns64;
         if (ns > 1 && p.workspace_bytes >= (size_t)p.B * p.H * p.Sq * ns * (2 + p.D) * sizeof(float)) { a.nsplit = ns; a.part = (float*)p.workspace; }
     }
     // Unsplit prefill has two kernels.  The software-pipelined one is the faster (894 against 840 TFLOP/s on causal B4 H32 S2048 fp16,
@@ -1661,6 +1711,10 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     else if (kind == 1) err = p.out16 ? dispatch_attn_d<f16_t, f16_t, 64>(a, full, stream) : dispatch_attn_d<f16_t, float, 64>(a, full, stream);
     else err = p.out16 ? dispatch_attn_d<bf16_t, bf16_t, 64>(a, full, stream) : dispatch_attn_d<bf16_t, float, 64>(a, full, stream);
     if (err != hipSuccess) return err;
+    if (ns64 > 1 && a.nsplit > 1) {
+        err = !p.out16 ? launch_merge<float, true>(a, stream) : kind == 1 ? launch_merge<f16_t, true>(a, stream) : launch_merge<bf16_t, true>(a, stream);
+        if (err != hipSuccess) return err;
+    }
     if (p.weights) {
         a.lse = p.lse;
         err = split ? launch_attn_weights_split(a, p.weights, stream)
