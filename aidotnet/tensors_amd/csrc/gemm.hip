@@ -2547,8 +2547,8 @@ static SplitPlan split_choice(int M, int N, int K, int batch, bool b16, size_t p
     const SplitPlan p = split_plan(M, N, K, batch, b16, partial_bytes);
     bool two;
     const double other = fp32_pipe_us(M, N, K, batch, b16, &two);
-    // a call costs its caller about 12 us, one of two launches 15.5, whatever its kernels take (10 x 320 x 640: one launch of 14.5, two of 11)
-    auto call = [](double us, bool two_launches) { return std::max(us, two_launches ? 15.5 : 12.0) + 0.05 * us; };
+    // a call costs its caller about 9.5 us, one of two launches 12, whatever its kernels take (10 x 320 x 640: one launch of 14.5, two of 11)
+    auto call = [](double us, bool two_launches) { return std::max(us, two_launches ? 12.0 : 9.5) + 0.05 * us; };
     return 1.08 * call(p.us, p.ks > 1) < call(other, two) ? p : SplitPlan{};
 }
 static hipError_t run_split(const GemmArgs& g, const SplitPlan& p, int batch, hipStream_t stream, void* workspace, bool b16)
