@@ -1642,7 +1642,12 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     hipError_t err;
     // fast path: 16-bit, head dim 128, aligned rows, plain (optionally causal) attention
     const bool dl = attn_dl_applies(kind, p);
-    const bool split = kind == 0 && attn_split_applies(a);      // fp32 on the fp16 matrix pipe (attention_split.hip)
+    // fp32 on the fp16 matrix pipe (attention_split.hip), but for two 128-key tiles of head dimension 64 on a grid that leaves CUs idle: four waves to
+    // a row's keys on the fp32 pipe take less there (us a launch, split / so: H4 S256 12.5 / 12.0, H16 S200 12.9 / 12.3, B2 H16 S256 13.1 / 12.2;
+    // S150 11.1 / 13.2 and S300 13.9 / 15.3 the other way; the probabilities' pass is faster split)
+    const long long grid32 = (long long)((a.Sq + 31) / 32) * a.B * a.H;
+    const bool groups32 = !full && a.vec_in && p.D == 64 && !p.block_table && !p.weights && p.Sk >= 192 && p.Sk <= 256 && p.Sq > 64 && grid32 <= (p.causal ? 384 : 256);
+    const bool split = kind == 0 && !groups32 && attn_split_applies(a);
     if (dl && p.workspace) {
         int chunk;
         const int ns = attn_dl_splits(p, &chunk);
