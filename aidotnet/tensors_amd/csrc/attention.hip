@@ -373,13 +373,15 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                     groups([&](int kt, int r, int key) { if (row[key] == 0.0f) st[kt][r] = -INFINITY; });
                 }
             }
-            const float factor = FULL ? LOG2E : fabsf(sl2);
+            // (the factor is positive: the -inf of a masked key stays one)
+            const float factor = FULL ? LOG2E : sl2 != 0.0f ? fabsf(sl2) : 1.0f;
             if constexpr (!FULL) {
-                if (sl2 < 0.0f) {
+                if (sl2 <= 0.0f) {
+                    const float sign = sl2 < 0.0f ? -1.0f : 0.0f;
 #pragma unroll
                     for (int kt = 0; kt < KT; kt++)
 #pragma unroll
-                        for (int r = 0; r < 16; r++) st[kt][r] = -st[kt][r];
+                        for (int r = 0; r < 16; r++) st[kt][r] *= sign;
                 }
             }
             if (need_mask) {
