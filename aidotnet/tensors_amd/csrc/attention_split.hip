@@ -28,6 +28,9 @@ __device__ __forceinline__ int exponent_to(float magnitude, int to)
     return magnitude == 0.0f ? 0 : min(max(to + 127 - e, -126), 126);
 }
 __device__ __forceinline__ float power2(int e) { return as_f32((uint32_t)(e + 127) << 23); }
+// Factor 2^e of the logits of a row.  Below 2^-100 they are zero in any case (2^36 units at most); the factor itself stays above zero, so that the
+// -inf of a masked key does
+__device__ __forceinline__ float logit_factor(float scale, int e) { return fmaxf(__builtin_ldexpf(scale, e), 0x1p-100f); }
 
 __device__ __forceinline__ uint32_t f16_pair(float a, float b)
 {
@@ -276,8 +279,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     };
     clear();
 
-    float to_log2 = __builtin_ldexpf(a.scale * LOG2E, logit_exp);       // OPT: the logit itself
-    if constexpr (OPT) to_log2 = __builtin_ldexpf(a.scale, logit_exp);
+    float to_log2 = logit_factor(OPT ? a.scale : a.scale * LOG2E, logit_exp);       // OPT: the logit itself
     // What the split cuts of Q' and K' (2^-25 of a value) shows in a logit as about 2^-12 of a unit of Q' K'.  Where that is more than 2^-25 of an
     // exponent the row's logits have to be large themselves (2^13 units), or it is computed again: large values that meet zeros, or keys out of
     // the row's sight, can have set the scale
@@ -852,10 +854,10 @@ __global__ __launch_bounds__(256, 2) void attn_weights_split_kernel(const AttnAr
     const int kexp = __builtin_amdgcn_readfirstlane(exponent_to(km, 10));
     const float ksc = power2(kexp);
     logit_exp -= kexp;
-    const float to_logit = __builtin_ldexpf(a.scale, logit_exp);
+    const float to_logit = logit_factor(OPT ? a.scale : a.scale * LOG2E, logit_exp);
     // (such rows are formed on the fp32 pipe, as above)
-    const bool coarse = __builtin_amdgcn_ballot_w64(to_logit * LOG2E > 0x1p-13f) != 0;
-    if (h == 0) { rows[0][32 * wave + l32] = OPT ? to_logit : to_logit * LOG2E; rows[1][32 * wave + l32] = lse == -INFINITY ? INFINITY : lse * LOG2E; }
+    const bool coarse = __builtin_amdgcn_ballot_w64((OPT ? to_logit * LOG2E : to_logit) > 0x1p-13f) != 0;
+    if (h == 0) { rows[0][32 * wave + l32] = to_logit; rows[1][32 * wave + l32] = lse == -INFINITY ? INFINITY : lse * LOG2E; }
     __builtin_amdgcn_wave_barrier();
     for (int j = first; j < seen; j++) {
         unsigned char* ks = Ks + (j & 1) * 2 * PL;

@@ -1,0 +1,58 @@
+"""fp32 attention on the fp16 matrix pipe: results that a scale taken from other values has left too few bits, each row and each column for itself.
+
+Bounds: 4e-6 of a row's 2-norm (fp32 logits, probabilities and sums of up to 1100 terms; such rows show up to 1e-6), times an eighth of the largest
+visible logit where that is above eight, since 2^-24 of a logit is a relative error of its probability."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng():
+    from aidotnet.tensors_amd import Mi355Engine
+    return Mi355Engine()
+
+
+def randn(seed, *shapes):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return [torch.randn(*s, device="cuda", generator=gen) for s in shapes]
+
+
+def reference(q, k, v, hidden=None):
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) / math.sqrt(q.shape[-1])
+    if hidden is not None:
+        s = s.masked_fill(hidden, -math.inf)
+    p = torch.softmax(s, -1)
+    return torch.matmul(p, v.double()), p, s.masked_fill(s == -math.inf, 0.0).abs().amax()
+
+
+def worst_row(got, want):
+    return float(((got.double() - want).norm(dim=-1) / want.norm(dim=-1)).nan_to_num(math.inf).max())
+
+
+def later(Sq, Sk, offset=0):
+    return torch.arange(Sk, device="cuda")[None, :] > torch.arange(Sq, device="cuda")[:, None] + offset
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("case", ["zero rows", "small", "zero rows, padded"])
+def test_probabilities_of_vanishing_logits(eng, case, D):
+    """Rows of zeros, and products below the range of fp32: equal probabilities, zeros above the diagonal."""
+    q, k, v = randn(D, (1, 2, 100, D), (1, 2, 100, D), (1, 2, 100, D))
+    if case == "small":
+        q, k = q * 1e-20, k * 1e-20
+    else:
+        q[:, :, ::3] = 0.0
+        k *= 1e-5
+    hidden, mask = later(100, 100), None
+    if case == "zero rows, padded":
+        hidden = torch.zeros(1, 1, 1, 100, dtype=torch.bool, device="cuda")
+        hidden[..., 40:50] = True
+        mask = ~hidden
+    want, p, _ = reference(q, k, v, hidden)
+    o, w = eng.ScaledDotProductAttention(q, k, v, mask, isCausal=mask is None)
+    assert worst_row(o, want) <= 4e-6 and worst_row(w, p) <= 4e-6
+    assert bool((w[hidden.expand_as(w)] == 0).all())
