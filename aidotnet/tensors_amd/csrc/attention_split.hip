@@ -284,8 +284,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     // exponent the row's logits have to be large themselves (2^13 units), or it is computed again: large values that meet zeros, or keys out of
     // the row's sight, can have set the scale
     const bool coarse = to_log2 > 0x1p-13f, any_coarse = __builtin_amdgcn_ballot_w64(coarse) != 0;
-    float largest_logit = 0.0f;
-    // logits of NB 32-key sub-tiles from key k0 on (st[kt][r]: key k0 + 32 kt + acc_row(r, h), query q0 + l32) to probabilities times 2^P_EXP against
+    float largest_logit = 0.0f, pexp = P_EXP;
+    // logits of NB 32-key sub-tiles from key k0 on (st[kt][r]: key k0 + 32 kt + acc_row(r, h), query q0 + l32) to probabilities times 2^pexp against
     // the new running maximum; returns what the sums so far are to be multiplied with.  Bit i of `kept`: key k0 + i is visible (OPT)
     auto softmax = [&](auto& st, int k0, uint64_t kept) -> float {
         constexpr int NB = sizeof(st) / sizeof(st[0]);
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         const float m_new = fmaxf(m_run, ceilf(max_with_partner32(mloc) * factor));
         const float m_use = m_new == -INFINITY ? 0.0f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
-        const float down = P_EXP - m_use;
+        const float down = pexp - m_use;
         m_run = m_new;
         float psum = 0.0f;
 #pragma unroll
@@ -560,6 +560,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
             // again on the fp32 pipe, rows straight from memory
             clear();
             vexp = 0;
+            pexp = 0.0f;                           // (V at the end of the range: nothing above one is to meet it)
             to_log2 = OPT ? a.scale : a.scale * LOG2E;
 #pragma unroll 1
             for (int k0 = first * BC + kg * KT * 32; k0 < ntiles * BC; k0 += k0 % (KT * 32) + 32 < KT * 32 ? 32 : BC - (KT - 1) * 32) {
@@ -668,7 +669,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         float* __restrict__ P = a.part + ((long long)bh * a.Sq * a.nsplit + blockIdx.y) * (2 + a.D);
         const long long pitch = (long long)a.nsplit * (2 + a.D);
         const int e = __builtin_amdgcn_frexp_expf(l) + (vexp > 0 ? 0 : 5);
-        if (h == 0 && qi < a.Sq) *(f32x2p*)(P + qi * pitch) = f32x2p{m_run + ((float)e - P_EXP), __builtin_amdgcn_ldexpf(l, -e)};
+        if (h == 0 && qi < a.Sq) *(f32x2p*)(P + qi * pitch) = f32x2p{m_run + ((float)e - pexp), __builtin_amdgcn_ldexpf(l, -e)};
         by_rows([&](float x) { return __builtin_amdgcn_ldexpf(x, -vexp - e); },
                 [&](int row, int d0, f32x4 v) {
                     if (d0 >= a.D) return;
@@ -679,7 +680,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         return;
     }
     const float inv = l > 0.0f ? power2(-vexp) / l : 0.0f;
-    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? (m_run + (__builtin_amdgcn_logf(l) - P_EXP)) * LN2 : -INFINITY;
+    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? (m_run + (__builtin_amdgcn_logf(l) - pexp)) * LN2 : -INFINITY;
     float* __restrict__ O = (float*)a.o + b * a.os[0] + hd * a.os[1];
     if (a.vec_out && a.D == DP) {
         by_rows([&](float x) { return x * inv; },

@@ -38,6 +38,20 @@ def later(Sq, Sk, offset=0):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Sk", [300, 1600])
+@pytest.mark.parametrize("size", [1e38, 3.3e38])
+def test_values_at_the_upper_end_of_a_later_tile(eng, size, Sk, D):
+    q, k, v = randn(Sk + D, (1, 2, 40, D), (1, 2, Sk, D), (1, 2, Sk, D))
+    q[..., 0] = 30.0
+    k[..., 0] = 0.0
+    k[:, :, 250, 0] = 30.0
+    v[:, :, 250] = size * torch.sign(v[:, :, 250])
+    want, _, big = reference(q, k, v)
+    o, _ = eng.FlashAttention(q, k, v)
+    assert bool(o.isfinite().all()) and worst_row(o, want) <= 4e-6 * max(1.0, float(big) / 8)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("case", ["zero rows", "small", "zero rows, padded"])
 def test_probabilities_of_vanishing_logits(eng, case, D):
     """Rows of zeros, and products below the range of fp32: equal probabilities, zeros above the diagonal."""
