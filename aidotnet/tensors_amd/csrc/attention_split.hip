@@ -679,11 +679,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
                 });
         return;
     }
-    const float inv = l > 0.0f ? power2(-vexp) / l : 0.0f;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    auto result = [&](float x) { return __builtin_amdgcn_ldexpf(x * inv, -vexp); };       // (in this order: 2^-vexp / l may lie below the normal numbers)
     if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? (m_run + (__builtin_amdgcn_logf(l) - pexp)) * LN2 : -INFINITY;
     float* __restrict__ O = (float*)a.o + b * a.os[0] + hd * a.os[1];
     if (a.vec_out && a.D == DP) {
-        by_rows([&](float x) { return x * inv; },
+        by_rows(result,
                 [&](int row, int d0, f32x4 v) { __builtin_nontemporal_store(v, (f32x4*)(O + (long long)row * a.os[2] + d0)); });
     } else if (qi < a.Sq) {
         float* __restrict__ p = O + (long long)qi * a.os[2];
@@ -692,10 +693,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 const int d0 = 32 * i + 8 * g + 4 * h;
-                if (a.vec_out) { if (d0 < a.D) *(f32x4*)(p + d0) = f32x4{oacc[i][4 * g] * inv, oacc[i][4 * g + 1] * inv, oacc[i][4 * g + 2] * inv, oacc[i][4 * g + 3] * inv}; }
+                if (a.vec_out) { if (d0 < a.D) *(f32x4*)(p + d0) = f32x4{result(oacc[i][4 * g]), result(oacc[i][4 * g + 1]), result(oacc[i][4 * g + 2]), result(oacc[i][4 * g + 3])}; }
                 else {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) if (d0 + e < a.D) p[d0 + e] = oacc[i][4 * g + e] * inv;
+                    for (int e = 0; e < 4; e++) if (d0 + e < a.D) p[d0 + e] = result(oacc[i][4 * g + e]);
                 }
             }
     }

@@ -39,6 +39,18 @@ def later(Sq, Sk, offset=0):
 
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Sk", [300, 1600])
+@pytest.mark.parametrize("size", [1e-33, 1e-35])
+def test_values_at_the_lower_end(eng, size, Sk, D):
+    """(numbers below 1.2e-38 have fewer bits: half a unit of 2^-149 of each result is granted)"""
+    q, k, v = randn(Sk + D, (1, 2, 40, D), (1, 2, Sk, D), (1, 2, Sk, D))
+    v *= size
+    want, _, _ = reference(q, k, v)
+    o, _ = eng.FlashAttention(q, k, v)
+    assert worst_row(o, want) <= 4e-6 + math.sqrt(D) * 2.0 ** -149 / float(want.norm(dim=-1).min())
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Sk", [300, 1600])
 @pytest.mark.parametrize("size", [1e38, 3.3e38])
 def test_values_at_the_upper_end_of_a_later_tile(eng, size, Sk, D):
     q, k, v = randn(Sk + D, (1, 2, 40, D), (1, 2, Sk, D), (1, 2, Sk, D))
