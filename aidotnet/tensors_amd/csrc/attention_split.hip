@@ -3,14 +3,16 @@
 // are formed, m h, h m, h h; what is left out, m m, is 2^-24 of a product at most.  Sums are fp32.
 //
 // Why fp16 and not bf16: three bf16 values hold every fp32 value whatever its size, but cost six products and 5.5 vector instructions a value where
-// two fp16 values cost three and 3 (2 for a probability, which needs no scale: one v_fma_mix_f32 takes the half of the packed word as it is), and
-// the vector pipe is what bounds the kernel (B8 H12 S512 d64 causal 37.8 us, 24 this way; the fp32 pipe 44).
+// two fp16 values cost three and 3 (one v_fma_mix_f32 takes the scale and the half of the packed word as they are), and the vector pipe is what
+// bounds the kernel (B8 H12 S512 d64 causal 37.8 us, 24 this way; the fp32 pipe 44).
 //
 // Scales.  Each row of Q has its own (its largest magnitude becomes 2^12 .. 2^13), K and V one per workgroup from its first tile (2^10 and 2^11:
 // later tiles may be 32 and 16 times larger).  Probabilities are formed against the next whole number above the row maximum, times 2^4, so that
-// their exponents are near zero where fp32 is fine (times 2^14 they were off by up to 3e-7).  What the split does not hold is computed again on
-// the fp32 pipe, by workgroup: results that are not finite (infinities, NaN, values beyond the first tile's scale), and those whose scale was set
-// by values far larger than what they are formed from (below).
+// their exponents are near zero where fp32 is fine (times 2^14 they were off by up to 3e-7), and split times 2^14: a row whose weight lies on a key
+// with next to nothing in V is the sum of its smallest probabilities, and what the split cuts of those, 2^-39 of the largest, does not show in it
+// (2^-29 did: V of 2e-3 at the key of the weight, 2^-14 at the others, 1e-5 of O).  What the split does not hold is computed again on the fp32
+// pipe, by workgroup: results that are not finite (infinities, NaN, values beyond the first tile's scale), and those whose scale was set by values
+// far larger than what they are formed from (below).
 //
 // Error against float64, fp32 pipe / here, 2-norm: O of B8 H12 S512 d64 causal 2.82e-7 / 2.04e-7, plain 4.09e-7 / 3.23e-7, d128 5.66e-7 / 3.61e-7,
 // d32 4.64e-7 / 3.04e-7, S64 2.38e-7 / 1.93e-7; probabilities 3.21e-7 / 3.05e-7; log-sum-exp alike.
@@ -19,7 +21,8 @@
 
 namespace aidn {
 
-constexpr float P_EXP = 4.0f;        // probabilities are held times 2^4
+constexpr float P_EXP = 4.0f;        // probabilities are formed and summed times 2^4
+constexpr int P_SPLIT = 10;          // and split times 2^10 more
 
 // Power of two (its exponent) that brings a magnitude into [2^to, 2^(to + 1)); 0 for zero
 __device__ __forceinline__ int exponent_to(float magnitude, int to)
@@ -53,14 +56,6 @@ __device__ __forceinline__ void split2(float a, float b, float s, uint32_t (&p)[
         asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(x) : "v"(a), "v"(s), "v"(p[0]));
         asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(b), "v"(s), "v"(p[0]));
     }
-    p[1] = f16_pair(x, y);
-}
-__device__ __forceinline__ void split2(float a, float b, uint32_t (&p)[2])
-{
-    p[0] = f16_pair(a, b);
-    float x, y;
-    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(x) : "v"(a), "v"(p[0]));
-    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(y) : "v"(b), "v"(p[0]));
     p[1] = f16_pair(x, y);
 }
 __device__ __forceinline__ float wave_max(float v)
@@ -241,7 +236,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     u32x4 qf[DS][2];
     int logit_exp = -split_q(Q + (long long)min(q0 + l32, a.Sq - 1) * a.qs[2], q0 + l32 < a.Sq, a.D, h, qf);      // logits are 2^logit_exp Q' K'
     // ---- K and V: one power of two each, from the first tile
-    int vexp = 0;
+    int vexp = 0, oexp = 0;                        // O is formed times 2^oexp
     if (first < ntiles) {
         float km = 0.0f, vm = 0.0f;
 #pragma unroll
@@ -261,6 +256,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         vexp = __builtin_amdgcn_readfirstlane(exponent_to(vm, 11));
         ksc = power2(kexp);
         vsc = power2(vexp);
+        oexp = vexp + P_SPLIT;
         logit_exp -= kexp;
 #pragma unroll
         for (int i = 0; i < U; i++) store_k(i);
@@ -451,7 +447,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     uint32_t p[2];
-                    split2(st[ps >> 1][8 * (ps & 1) + 2 * e], st[ps >> 1][8 * (ps & 1) + 2 * e + 1], p);
+                    split2<true>(st[ps >> 1][8 * (ps & 1) + 2 * e], st[ps >> 1][8 * (ps & 1) + 2 * e + 1], power2(P_SPLIT), p);
                     pf[ps][0][e] = p[0];
                     pf[ps][1][e] = p[1];
                 }
@@ -512,7 +508,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         if (any_coarse) bad |= coarse && l_run > 0.0f && (OPT || fmaxf(largest_logit, shfl_xor_f(largest_logit, 32)) < 0x1p13f);
         // a column of O without a value of 2^-5 units of V' (whose largest in the first tile is 2^11 or more) may come from a column of V that the
         // scale has left too few bits of
-        const float witness = l_run > 0.0f ? l_run * 0x1p-4f : INFINITY;          // (either half's share of the row sum is at most all of it)
+        const float witness = l_run > 0.0f ? l_run * (0x1p-4f * (1 << P_SPLIT)) : INFINITY;          // (either half's share of the row sum is at most all of it)
         uint32_t unseen = 0;
 #pragma unroll
         for (int i = 0; i < DT; i++)
@@ -559,7 +555,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         if (again) {
             // again on the fp32 pipe, rows straight from memory
             clear();
-            vexp = 0;
+            oexp = 0;
             pexp = 0.0f;                           // (V at the end of the range: nothing above one is to meet it)
             to_log2 = OPT ? a.scale : a.scale * LOG2E;
 #pragma unroll 1
@@ -668,9 +664,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         // the sum over up to 32 ranges does not leave the range of fp32 where the result does not; m takes that power and stays exact, being whole
         float* __restrict__ P = a.part + ((long long)bh * a.Sq * a.nsplit + blockIdx.y) * (2 + a.D);
         const long long pitch = (long long)a.nsplit * (2 + a.D);
-        const int e = __builtin_amdgcn_frexp_expf(l) + (vexp > 0 ? 0 : 5);
+        const int e = __builtin_amdgcn_frexp_expf(l) + (oexp > P_SPLIT ? 0 : 5);
         if (h == 0 && qi < a.Sq) *(f32x2p*)(P + qi * pitch) = f32x2p{m_run + ((float)e - pexp), __builtin_amdgcn_ldexpf(l, -e)};
-        by_rows([&](float x) { return __builtin_amdgcn_ldexpf(x, -vexp - e); },
+        by_rows([&](float x) { return __builtin_amdgcn_ldexpf(x, -oexp - e); },
                 [&](int row, int d0, f32x4 v) {
                     if (d0 >= a.D) return;
                     float* __restrict__ p = P + row * pitch + 2 + d0;                  // (8-byte aligned)
@@ -680,7 +676,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         return;
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    auto result = [&](float x) { return __builtin_amdgcn_ldexpf(x * inv, -vexp); };       // (in this order: 2^-vexp / l may lie below the normal numbers)
+    auto result = [&](float x) { return __builtin_amdgcn_ldexpf(x * inv, -oexp); };       // (in this order: 2^-oexp / l may lie below the normal numbers)
     if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? (m_run + (__builtin_amdgcn_logf(l) - pexp)) * LN2 : -INFINITY;
     float* __restrict__ O = (float*)a.o + b * a.os[0] + hd * a.os[1];
     if (a.vec_out && a.D == DP) {

@@ -38,6 +38,21 @@ def later(Sq, Sk, offset=0):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Sk", [200, 1000])
+def test_weight_far_below_the_largest(eng, Sk, D):
+    """One key takes nearly all of the weight and carries almost nothing: the rows are sums of probabilities of 2^-14."""
+    q, k, v = randn(Sk + D, (1, 2, 40, D), (1, 2, Sk, D), (1, 2, Sk, D))
+    q[..., 0] = 8.0
+    k[..., 0] = 0.0
+    k[:, :, 3, 1:] = 0.0
+    k[:, :, 3, 0] = 14 * math.log(2) * math.sqrt(D) / 8
+    v[:, :, 3] *= 2e-3
+    want, _, big = reference(q, k, v)
+    o, _ = eng.FlashAttention(q, k, v)
+    assert worst_row(o, want) <= 4e-6 * max(1.0, float(big) / 8)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Sk", [300, 1600])
 @pytest.mark.parametrize("size", [1e-33, 1e-35])
 def test_values_at_the_lower_end(eng, size, Sk, D):
