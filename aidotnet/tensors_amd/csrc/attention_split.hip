@@ -508,7 +508,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         if (any_coarse) bad |= coarse && l_run > 0.0f && (OPT || fmaxf(largest_logit, shfl_xor_f(largest_logit, 32)) < 0x1p13f);
         // a column of O without a value of 2^-5 units of V' (whose largest in the first tile is 2^11 or more) may come from a column of V that the
         // scale has left too few bits of
-        const float witness = l_run > 0.0f ? l_run * (0x1p-4f * (1 << P_SPLIT)) : INFINITY;          // (either half's share of the row sum is at most all of it)
+        const float l = sum_with_partner32(l_run);                                // (the products run over the keys of both halves)
+        const float witness = l > 0.0f ? l * (0x1p-5f * (1 << P_SPLIT)) : INFINITY;
         uint32_t unseen = 0;
 #pragma unroll
         for (int i = 0; i < DT; i++)

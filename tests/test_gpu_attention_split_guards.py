@@ -38,6 +38,26 @@ def later(Sq, Sk, offset=0):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Sq,Sk", [(200, 200), (40, 1000)])
+@pytest.mark.parametrize("small", [1.0, 1e-3])
+def test_sharp_probabilities_over_a_first_tile_of_zeros(eng, small, Sq, Sk, D):
+    """A left-padded cache: the first tiles of V give no scale; each row's weight lies on a few of the keys behind them."""
+    q, k, v = randn(Sk + D, (1, 4, Sq, D), (1, 4, Sk, D), (1, 4, Sk, D))
+    q *= 8
+    v *= small
+    v[:, :, :130] = 0.0
+    hidden = torch.zeros(1, 1, 1, Sk, dtype=torch.bool, device="cuda")
+    hidden[..., :130] = True
+    want, _, big = reference(q, k, v)
+    o, _ = eng.FlashAttention(q, k, v)
+    seen = want.norm(dim=-1) > 1e-3 * small                   # (rows whose weight lies on the zeros have nothing left but their tails)
+    assert float(((o.double() - want).norm(dim=-1) / want.norm(dim=-1))[seen].max()) <= 4e-6 * max(1.0, float(big) / 8)
+    want, _, big = reference(q, k, v, hidden)
+    o, _ = eng.ScaledDotProductAttention(q, k, v, ~hidden, returnWeights=False)
+    assert worst_row(o, want) <= 4e-6 * max(1.0, float(big) / 8)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Sk", [200, 1000])
 def test_weight_far_below_the_largest(eng, Sk, D):
     """One key takes nearly all of the weight and carries almost nothing: the rows are sums of probabilities of 2^-14."""
@@ -54,18 +74,6 @@ def test_weight_far_below_the_largest(eng, Sk, D):
 
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Sk", [300, 1600])
-@pytest.mark.parametrize("size", [1e-33, 1e-35])
-def test_values_at_the_lower_end(eng, size, Sk, D):
-    """(numbers below 1.2e-38 have fewer bits: half a unit of 2^-149 of each result is granted)"""
-    q, k, v = randn(Sk + D, (1, 2, 40, D), (1, 2, Sk, D), (1, 2, Sk, D))
-    v *= size
-    want, _, _ = reference(q, k, v)
-    o, _ = eng.FlashAttention(q, k, v)
-    assert worst_row(o, want) <= 4e-6 + math.sqrt(D) * 2.0 ** -149 / float(want.norm(dim=-1).min())
-
-
-@pytest.mark.parametrize("D", [32, 64, 128])
-@pytest.mark.parametrize("Sk", [300, 1600])
 @pytest.mark.parametrize("size", [1e38, 3.3e38])
 def test_values_at_the_upper_end_of_a_later_tile(eng, size, Sk, D):
     q, k, v = randn(Sk + D, (1, 2, 40, D), (1, 2, Sk, D), (1, 2, Sk, D))
@@ -76,6 +84,18 @@ def test_values_at_the_upper_end_of_a_later_tile(eng, size, Sk, D):
     want, _, big = reference(q, k, v)
     o, _ = eng.FlashAttention(q, k, v)
     assert bool(o.isfinite().all()) and worst_row(o, want) <= 4e-6 * max(1.0, float(big) / 8)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Sk", [300, 1600])
+@pytest.mark.parametrize("size", [1e-33, 1e-35])
+def test_values_at_the_lower_end(eng, size, Sk, D):
+    """(numbers below 1.2e-38 have fewer bits: half a unit of 2^-149 of each result is granted)"""
+    q, k, v = randn(Sk + D, (1, 2, 40, D), (1, 2, Sk, D), (1, 2, Sk, D))
+    v *= size
+    want, _, _ = reference(q, k, v)
+    o, _ = eng.FlashAttention(q, k, v)
+    assert worst_row(o, want) <= 4e-6 + math.sqrt(D) * 2.0 ** -149 / float(want.norm(dim=-1).min())
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
