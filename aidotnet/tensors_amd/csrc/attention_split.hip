@@ -277,10 +277,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
 
     float to_log2 = logit_factor(OPT ? a.scale : a.scale * LOG2E, logit_exp);       // OPT: the logit itself
     // What the split cuts of Q' and K' (2^-25 of a value) shows in a logit as about 2^-12 of a unit of Q' K'.  Where that is more than 2^-25 of an
-    // exponent the row's logits have to be large themselves (2^13 units), or it is computed again: large values that meet zeros, or keys out of
-    // the row's sight, can have set the scale
-    const bool coarse = to_log2 > 0x1p-13f, any_coarse = __builtin_amdgcn_ballot_w64(coarse) != 0;
-    float largest_logit = 0.0f, pexp = P_EXP;
+    // exponent the row's largest logit, near which all of its weight lies, has to be that far from zero itself (2^13 units), or it is computed
+    // again: large values that meet zeros, keys out of the row's sight, or far lower logits can have set the scale
+    const bool coarse = to_log2 > 0x1p-13f;
+    float pexp = P_EXP;
     // logits of NB 32-key sub-tiles from key k0 on (st[kt][r]: key k0 + 32 kt + acc_row(r, h), query q0 + l32) to probabilities times 2^pexp against
     // the new running maximum; returns what the sums so far are to be multiplied with.  Bit i of `kept`: key k0 + i is visible (OPT)
     auto softmax = [&](auto& st, int k0, uint64_t kept) -> float {
@@ -346,14 +346,6 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
 #pragma unroll
                     for (int r = 0; r < 16; r++) if (!(bits >> acc_row(r, 0) & 1u)) st[kt][r] = -INFINITY;
                 }
-            }
-        }
-        if constexpr (!OPT) {
-            if (any_coarse) {
-#pragma unroll
-                for (int kt = 0; kt < NB; kt++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) largest_logit = fmaxf(largest_logit, st[kt][r] == -INFINITY ? 0.0f : fabsf(st[kt][r]));
             }
         }
         float mloc = -INFINITY;
@@ -505,10 +497,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
 #pragma unroll
             for (int r = 0; r < 16; r++) poison = fmaf(oacc[i][r], 0.0f, poison);
         bool bad = poison != poison;               // infinities, NaN, values beyond the scale of the first tile
-        if (any_coarse) bad |= coarse && l_run > 0.0f && (OPT || fmaxf(largest_logit, shfl_xor_f(largest_logit, 32)) < 0x1p13f);
         // a column of O without a value of 2^-5 units of V' (whose largest in the first tile is 2^11 or more) may come from a column of V that the
         // scale has left too few bits of
         const float l = sum_with_partner32(l_run);                                // (the products run over the keys of both halves)
+        bad |= coarse && l > 0.0f && (OPT || fabsf(m_run) - 1.0f < 0x1p13f * to_log2);        // (m_run is rounded up to a whole number)
         const float witness = l > 0.0f ? l * (0x1p-5f * (1 << P_SPLIT)) : INFINITY;
         uint32_t unseen = 0;
 #pragma unroll

@@ -73,6 +73,19 @@ def test_weight_far_below_the_largest(eng, Sk, D):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+def test_one_far_lower_logit(eng, D):
+    """Visible keys whose logits are far below all others set the scales of Q and K, and do not vouch for the others' logits."""
+    q, k, v = randn(D, (1, 2, 40, D), (1, 2, 200, D), (1, 2, 200, D))
+    q[..., 0] = 1e7
+    k[..., 0] = 0.0
+    k[:, :, 7::16, 0] = -1e7
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) / math.sqrt(D)
+    want = torch.matmul(torch.softmax(s, -1), v.double())
+    o, _ = eng.FlashAttention(q, k, v)
+    assert worst_row(o, want) <= 4e-6
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Sk", [300, 1600])
 @pytest.mark.parametrize("size", [1e38, 3.3e38])
 def test_values_at_the_upper_end_of_a_later_tile(eng, size, Sk, D):
