@@ -24,11 +24,12 @@ namespace aidn {
 constexpr float P_EXP = 4.0f;        // probabilities are formed and summed times 2^4
 constexpr int P_SPLIT = 10;          // and split times 2^10 more
 
-// Power of two (its exponent) that brings a magnitude into [2^to, 2^(to + 1)); 0 for zero
+// Power of two (its exponent) that brings a magnitude into [2^to, 2^(to + 1)); 2^8 for zero: behind a first tile of zeros values from 2^-10 to 2^7
+// have their bits
 __device__ __forceinline__ int exponent_to(float magnitude, int to)
 {
     const int e = (int)(as_u32(magnitude) >> 23);
-    return magnitude == 0.0f ? 0 : min(max(to + 127 - e, -126), 126);
+    return magnitude == 0.0f ? 8 : min(max(to + 127 - e, -126), 126);
 }
 __device__ __forceinline__ float power2(int e) { return as_f32((uint32_t)(e + 127) << 23); }
 // Factor 2^e of the logits of a row.  Below 2^-100 they are zero in any case (2^36 units at most); the factor itself stays above zero, so that the
@@ -491,59 +492,77 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     l32 = lane & 31;
     h = lane >> 5;
     {
-        float poison = l_run * 0.0f;
+        const float l = sum_with_partner32(l_run);                                // (the products run over the keys of both halves)
+        const bool row = l > 0.0f;
+        float poison = l_run * 0.0f, top = 0.0f;
 #pragma unroll
         for (int i = 0; i < DT; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) poison = fmaf(oacc[i][r], 0.0f, poison);
+            for (int r = 0; r < 16; r++) {
+                poison = fmaf(oacc[i][r], 0.0f, poison);
+                top = fmaxf(top, fabsf(oacc[i][r]));
+            }
         bool bad = poison != poison;               // infinities, NaN, values beyond the scale of the first tile
-        // a column of O without a value of 2^-5 units of V' (whose largest in the first tile is 2^11 or more) may come from a column of V that the
-        // scale has left too few bits of
-        const float l = sum_with_partner32(l_run);                                // (the products run over the keys of both halves)
-        bad |= coarse && l > 0.0f && (OPT || fabsf(m_run) - 1.0f < 0x1p13f * to_log2);        // (m_run is rounded up to a whole number)
-        const float witness = l > 0.0f ? l * (0x1p-5f * (1 << P_SPLIT)) : INFINITY;
-        uint32_t unseen = 0;
+        bad |= coarse && row && (OPT || fabsf(m_run) - 1.0f < 0x1p13f * to_log2);        // (m_run is rounded up to a whole number)
+        // V' is cut at 2^-25 units, and its largest value in the first tile is 2^11 or more.  A row of O that nowhere reaches one unit may be made of
+        // values that the scale has left too few bits of: those that set it can be hidden from the row, or weigh nothing in it
+        const bool dim = row && q0 + l32 < a.Sq && max_with_partner32(top) < l * (1 << P_SPLIT);
+        // ... and so may a column without a value of 2^-5 units in any row
+        const float witness = row ? l * (0x1p-5f * (1 << P_SPLIT)) : INFINITY;
+        uint32_t fewest = ~0u;                     // (rows that reach it, a bit each: zero where some column has none)
 #pragma unroll
         for (int i = 0; i < DT; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const uint64_t w = __builtin_amdgcn_ballot_w64(fabsf(oacc[i][r]) >= witness);
-                unseen |= (uint32_t)w == 0 || (uint32_t)(w >> 32) == 0;
+                fewest = min(fewest, min((uint32_t)w, (uint32_t)(w >> 32)));
             }
-        const bool look = unseen && __builtin_amdgcn_ballot_w64(l_run > 0.0f) != 0;
+        const bool blank = fewest == 0 && __builtin_amdgcn_ballot_w64(row) != 0;
         __shared__ int flags[NW];
-        auto any_thread = [&](bool x) {            // (with less to keep in registers than __syncthreads_or, which wants the thread's y and z)
-            const bool mine = __builtin_amdgcn_ballot_w64(x) != 0;
-            if (lane == 0) flags[wave] = mine;
+        auto any_wave = [&](int x) {               // (with less to keep in registers than __syncthreads_or, which wants the thread's y and z)
+            if (lane == 0) flags[wave] = x;
             __syncthreads();
             int any = 0;
 #pragma unroll
             for (int w = 0; w < NW; w++) any |= flags[w];
             __syncthreads();
-            return __builtin_amdgcn_readfirstlane(any) != 0;
+            return __builtin_amdgcn_readfirstlane(any);
         };
-        bool again = any_thread(bad | look);
-        if (again && !any_thread(bad)) {
-            // the columns' largest magnitudes
-            uint32_t* top = (uint32_t*)smem;
-            for (int d = t; d < DP; d += NT) top[d] = 0;
+        constexpr int BAD = 1, DIM = 2, BLANK = 4;
+        const int found = any_wave((__builtin_amdgcn_ballot_w64(bad) != 0 ? BAD : 0) | (__builtin_amdgcn_ballot_w64(dim) != 0 ? DIM : 0) | (blank ? BLANK : 0));
+        bool again = (found & BAD) != 0;
+        if (found != 0 && !again) {
+            // The split holds them all the same where every value of such a column is zero or has its bits (half a unit), and for such rows where
+            // V is zero.  Which rows see which values is not asked: a hidden one may cost a needless second computation
+            uint32_t* cols = (uint32_t*)smem;
+            if (t < DT) cols[t] = (found & DIM) != 0 ? ~0u : 0u;
+            __syncthreads();
+            if (blank) {
+#pragma unroll
+                for (int i = 0; i < DT; i++) {
+                    uint32_t none = 0;             // bit d: no row reaches it in column 32 i + d
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const uint64_t w = __builtin_amdgcn_ballot_w64(fabsf(oacc[i][r]) >= witness);
+                        none |= ((uint32_t)w == 0 ? 1u << acc_row(r, 0) : 0u) | ((uint32_t)(w >> 32) == 0 ? 1u << acc_row(r, 1) : 0u);
+                    }
+                    if (lane == 0) atomicOr(cols + i, none);
+                }
+            }
             __syncthreads();
             const int keys = min(ntiles * BC, a.Sk), d0 = 4 * (t % (DP / 4));
-            if (d0 < a.D) {
-                f32x4 m = {0.0f, 0.0f, 0.0f, 0.0f};
+            const uint32_t mine = cols[d0 / 32] >> (d0 % 32) & 15u;
+            const float least = (found & DIM) != 0 ? INFINITY : 0.5f;
+            bool small = false;
+            if (d0 < a.D && mine != 0) {
 #pragma unroll 8
                 for (int key = first * BC + t / (DP / 4); key < keys; key += NT / (DP / 4)) {
                     const f32x4 x = *(const f32x4*)(V + paged_row(bt, a.bsz, key) * a.vs[2] + d0);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) m[e] = fmaxf(m[e], fabsf(x[e]));
+                    for (int e = 0; e < 4; e++) small |= (mine >> e & 1u) != 0 && x[e] != 0.0f && fabsf(x[e]) * vsc < least;
                 }
-#pragma unroll
-                for (int e = 0; e < 4; e++) atomicMax(top + d0 + e, as_u32(m[e]));      // (not negative: ordered like their bits)
             }
-            __syncthreads();
-            bool small = false;
-            for (int d = t; d < DP; d += NT) small |= top[d] != 0 && as_f32(top[d]) * vsc < 0.5f;
-            again = any_thread(small);
+            again = any_wave(__builtin_amdgcn_ballot_w64(small) != 0 ? 1 : 0) != 0;
         }
         if (again) {
             // again on the fp32 pipe, rows straight from memory

@@ -37,6 +37,33 @@ def later(Sq, Sk, offset=0):
     return torch.arange(Sk, device="cuda")[None, :] > torch.arange(Sq, device="cuda")[:, None] + offset
 
 
+# one range of the keys, several of them; workgroups of one, two and four key groups
+SHAPES = [(70, 70, 32), (200, 200, 64), (40, 200, 64), (130, 300, 128), (40, 1000, 32), (40, 1000, 64), (40, 1000, 128)]
+
+
+@pytest.mark.parametrize("size", [1e6, 1e10, 1e30])
+@pytest.mark.parametrize("option", ["padding", "plane", "causal", "range"])
+@pytest.mark.parametrize("Sq,Sk,D", SHAPES)
+def test_large_values_out_of_sight(eng, Sq, Sk, D, option, size):
+    """V far larger at keys that a row does not see, in its first tile among others."""
+    q, k, v = randn(Sk + D, (1, 2, Sq, D), (1, 2, Sk, D), (1, 2, Sk, D))
+    if option in ("padding", "plane"):
+        hidden = torch.zeros(1, 1, 1 if option == "padding" else Sq, Sk, dtype=torch.bool, device="cuda")
+        hidden[..., 20:29] = True
+        hidden[..., Sk - 9:] = True
+        v[:, :, 20:29] *= size
+        v[:, :, Sk - 9:] *= size
+        want, _, _ = reference(q, k, v, hidden)
+        o, _ = eng.ScaledDotProductAttention(q, k, v, ~hidden, returnWeights=False)
+        assert worst_row(o, want) <= 4e-6
+        return
+    offset = Sk - Sq if option == "range" else 0
+    v[:, :, offset + min(Sq, Sk) // 2:] *= size              # from the middle query's diagonal on
+    want, _, _ = reference(q, k, v, later(Sq, Sk, offset))
+    o, _ = eng.FlashAttention(q, k, v, isCausal=True, queryOffset=offset)
+    assert worst_row(o, want) <= 4e-6
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Sq,Sk", [(200, 200), (40, 1000)])
 @pytest.mark.parametrize("small", [1.0, 1e-3])
@@ -130,3 +157,22 @@ def test_probabilities_of_vanishing_logits(eng, case, D):
     o, w = eng.ScaledDotProductAttention(q, k, v, mask, isCausal=mask is None)
     assert worst_row(o, want) <= 4e-6 and worst_row(w, p) <= 4e-6
     assert bool((w[hidden.expand_as(w)] == 0).all())
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("hidden_key", [False, True])
+def test_columns(eng, hidden_key, D):
+    """A column of zeros and one far below the others, or far below them but at keys that no row sees."""
+    q, k, v = randn(D, (1, 2, 200, D), (1, 2, 200, D), (1, 2, 200, D))
+    v[..., 1] = 0.0
+    v[..., 5] *= 1e-9
+    hidden, mask = None, None
+    if hidden_key:
+        hidden = torch.zeros(1, 1, 1, 200, dtype=torch.bool, device="cuda")
+        hidden[..., 30:34] = True
+        mask = ~hidden
+        v[:, :, 30:34, 5] = 1.0
+    want, _, _ = reference(q, k, v, hidden)
+    o, _ = eng.ScaledDotProductAttention(q, k, v, mask, returnWeights=False)
+    assert float((o[..., 5].double() - want[..., 5]).norm() / want[..., 5].norm()) <= 4e-6
+    assert bool((o[..., 1] == 0).all())
