@@ -1622,7 +1622,7 @@ size_t attn_fwd_workspace_bytes(int kind, const AttnParams& p)
     int chunk, ns = 1;
     if (kind == 0) {
         const AttnArgs a = attn_args(kind, p);
-        if (attn_split_applies(a)) ns = attn_split_ranges(a);
+        if (p.allow_fast_path && attn_split_applies(a)) ns = attn_split_ranges(a);
     } else if (attn_dl_applies(kind, p)) ns = attn_dl_splits(p, &chunk);
     else ns = attn_half64_ranges(kind, p);
     return ns > 1 ? (size_t)p.B * p.H * p.Sq * ns * (2 + p.D) * sizeof(float) : 0;
@@ -1649,7 +1649,7 @@ hipError_t attn_fwd(hipStream_t stream, int kind, const AttnParams& p)
     // S150 11.1 / 13.2 and S300 13.9 / 15.3 the other way; the probabilities' pass is faster split)
     const long long grid32 = (long long)((a.Sq + 31) / 32) * a.B * a.H;
     const bool groups32 = !full && a.vec_in && p.D == 64 && !p.block_table && !p.weights && p.Sk >= 192 && p.Sk <= 256 && p.Sq > 64 && grid32 <= (p.causal ? 384 : 256);
-    const bool split = kind == 0 && !groups32 && attn_split_applies(a);
+    const bool split = kind == 0 && p.allow_fast_path && !groups32 && attn_split_applies(a);
     if (dl && p.workspace) {
         int chunk;
         const int ns = attn_dl_splits(p, &chunk);

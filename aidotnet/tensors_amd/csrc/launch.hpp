@@ -73,7 +73,7 @@ struct AttnParams {
     const int* block_table = nullptr;
     int block_size = 0;
     long long block_table_stride = 0;
-    // 0: every shape takes the general kernel (the direct-to-LDS instances are not used); set per call from the context
+    // 0: every shape takes the general kernel (not its direct-to-LDS instances, nor fp32 on the fp16 pipe); set per call from the context
     int allow_fast_path = 1;
     // optional scratch of attn_fwd_workspace_bytes() bytes: lets attn_fwd cut the key sequence into ranges when the query tiles
     // alone would leave most of the chip idle

@@ -354,7 +354,7 @@ AIDN_API int aidn_mi355_mha_fwd_packed_bf16(void* ctx, void* stream, const uint1
  * reference. */
 AIDN_API int aidn_mi355_set_gemm_tile(void* ctx, int tile);
 /* enabled == 0 routes every attention shape through the general kernel (the head-dim-128 16-bit fast
- * paths are then not taken), so the parity suite can hold the kernels against each other; unsplit
+ * paths and the fp32 kernel on the fp16 matrix pipe are then not taken), so the parity suite can hold the kernels against each other; unsplit
  * head-dim-128 prefill on dense 16-bit arrays has two kernels (the software-pipelined one is the default, the
  * phase-structured one takes the other layouts): enabled == 2 pins the phase-structured one, enabled == 3 the
  * software-pipelined one wherever it applies (each of the three is checked against the others); at head dimension 256

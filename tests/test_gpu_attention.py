@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle
-from _util import TORCH16, dev, from_bits16, mixed_err, round_to
+from _util import TORCH16, dev, from_bits16, kernels_of, mixed_err, rel_frobenius, round_to
 
 pytestmark = pytest.mark.gpu
 
@@ -477,27 +477,34 @@ def test_pipelined_prefill_long_passes(be, kind, B, H, Hkv, Sq, Sk, causal, offs
         be.SetAttentionFastPath(True)
 
 
-# --------------------------------------------------------------- fp32 head-dim-64 direct-to-LDS form of the general kernel
+# --------------------------------------------------------------- fp32: the kernel that is chosen against the general one, staged through registers
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,causal,offset", FAST_CASES + [(2, 4, 2, 17, 40, True, 23), (1, 4, 4, 70, 70, True, 0),
                                                                    (1, 2, 2, 512, 512, True, 0), (1, 3, 3, 200, 50, True, 0),
-                                                                   (8, 49, 7, 200, 200, True, 0)])
+                                                                   (8, 49, 7, 200, 200, True, 0), (1, 4, 4, 256, 256, False, 0)])
 @pytest.mark.parametrize("D", [64, 128])
-def test_fp32_d64_direct_load_form_matches_oracle_and_general_form(be, eng, D, B, H, Hkv, Sq, Sk, causal, offset):
+def test_fp32_chosen_kernel_matches_oracle_and_general_kernel(be, eng, D, B, H, Hkv, Sq, Sk, causal, offset):
     rng = np.random.default_rng(B + 3 * H + 7 * Sq + 11 * Sk + 64)
     q, k, v = _rand(rng, B, H, Sq, D), _rand(rng, B, Hkv, Sk, D), _rand(rng, B, Hkv, Sk, D)
     scale = 1.0 / math.sqrt(D)
     o64, lse64 = oracle.attention_f64(q, k, v, scale, causal, offset)
-    outs = {}
+    outs, names = {}, {}
+    call = lambda: eng.FlashAttention(dev(q), dev(k), dev(v), scale, causal, queryOffset=offset)
     try:
-        for direct in (True, False):
-            be.SetAttentionFastPath(direct)
-            o, lse = eng.FlashAttention(dev(q), dev(k), dev(v), scale, causal, queryOffset=offset)
-            outs[direct] = (o.cpu().numpy(), lse.cpu().numpy())
-            assert mixed_err(outs[direct][0], o64) <= FP32_TOL and mixed_err(outs[direct][1], lse64) <= FP32_TOL
+        for fast in (True, False):
+            be.SetAttentionFastPath(fast)
+            names[fast] = kernels_of(call)[0].split("<")[0]
+            o, lse = call()
+            outs[fast] = (o.cpu().numpy(), lse.cpu().numpy())
+            assert mixed_err(outs[fast][0], o64) <= FP32_TOL and mixed_err(outs[fast][1], lse64) <= FP32_TOL
     finally:
         be.SetAttentionFastPath(True)
-    # the two forms multiply and sum the same values in the same order: identical results
-    assert np.array_equal(outs[True][0], outs[False][0]) and np.array_equal(outs[True][1], outs[False][1])
+    assert names[False] == "attn_fwd_kernel"
+    if names[True] == "attn_fwd_kernel":
+        # the direct-to-LDS form (head dimension 64): the same values multiplied and summed in the same order, identical results
+        assert D == 64 and np.array_equal(outs[True][0], outs[False][0]) and np.array_equal(outs[True][1], outs[False][1])
+    else:
+        assert names[True] == "attn_split_kernel"
+        assert rel_frobenius(outs[True][0], outs[False][0]) <= 4e-6 and rel_frobenius(outs[True][1], outs[False][1]) <= 1e-6
 
 
 # --------------------------------------------------------------- head dimension 256, 16-bit: the phase-structured kernel at that width

@@ -7,6 +7,8 @@ import math
 import pytest
 import torch
 
+from _util import kernels_of
+
 pytestmark = pytest.mark.gpu
 
 
@@ -176,3 +178,20 @@ def test_columns(eng, hidden_key, D):
     o, _ = eng.ScaledDotProductAttention(q, k, v, mask, returnWeights=False)
     assert float((o[..., 5].double() - want[..., 5]).norm() / want[..., 5].norm()) <= 4e-6
     assert bool((o[..., 1] == 0).all())
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_general_kernel_on_request(D):
+    """The switch that routes every attention shape through the general kernel reaches fp32, its key ranges and its probabilities."""
+    from aidotnet.tensors_amd import Mi355Backend, Mi355Engine
+    be = Mi355Backend()
+    eng = Mi355Engine(be)
+    q, k, v = randn(D, (1, 2, 40, D), (1, 2, 1000, D), (1, 2, 1000, D))
+    call = lambda: eng.ScaledDotProductAttention(q, k, v)
+    o, w = call()
+    assert [n.split("<")[0] for n in kernels_of(call)] == ["attn_split_kernel", "attn_split_merge_kernel", "attn_weights_split_kernel"]
+    be.SetAttentionFastPath(False)
+    names = kernels_of(call)
+    assert [n.split("<")[0] for n in names] == ["attn_fwd_kernel", "attn_weights_kernel"], names
+    o2, w2 = call()
+    assert float((o - o2).norm() / o2.norm()) <= 4e-6 and float((w - w2).norm() / w2.norm()) <= 4e-6
