@@ -238,6 +238,8 @@ template <> __device__ __forceinline__ uint32_t pack2_p<bf16_t>(float a, float b
 // Bound by memory latency: eight partial rows per wave are asked for together with the (m, l) pairs, so up to 8 WPR ranges cost one
 // round trip; up to eight ranges need no barrier and no LDS.  A range that saw no key weighs zero and adds nothing.
 typedef float f32x2p __attribute__((ext_vector_type(2)));
+// log(2^m l); rounded once beyond the logarithm and its product (the sum m + log2(l) in units of 2 was a rounding more at nearly twice the size)
+__device__ __forceinline__ float log_sum(float m, float l) { return fmaf(m, LN2, __builtin_amdgcn_logf(l) * LN2); }
 // KEEP_NAN: a sum that is no number gives NaN instead of zeros, as a single range of the fp32 split kernel does.
 template <int NV, int WPR, bool KEEP_NAN = false>
 __device__ __forceinline__ float merge_partials(const float* __restrict__ P, int n, int dpad, int D, int part, int lane, f32x2p (&out)[NV])
@@ -298,7 +300,7 @@ __device__ __forceinline__ float merge_partials(const float* __restrict__ P, int
     for (int j = 0; j < NV; j++)
 #pragma unroll
         for (int e = 0; e < 2; e++) out[j][e] = (KEEP_NAN ? L != 0.0f : L > 0.0f) ? out[j][e] / L : 0.0f;
-    return L > 0.0f ? (M + __builtin_amdgcn_logf(L)) * LN2 : -INFINITY;
+    return L > 0.0f ? log_sum(M, L) : -INFINITY;
 }
 // waves per row of the merge passes: one (four rows to a workgroup) while a row's ranges fit one round of loads
 inline int merge_waves_per_row(int ranges) { return ranges <= 8 ? 1 : 4; }

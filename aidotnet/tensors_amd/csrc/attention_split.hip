@@ -689,7 +689,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     auto result = [&](float x) { return __builtin_amdgcn_ldexpf(x * inv, -oexp); };       // (in this order: 2^-oexp / l may lie below the normal numbers)
-    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? (m_run + (__builtin_amdgcn_logf(l) - pexp)) * LN2 : -INFINITY;
+    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? log_sum(m_run, l * __builtin_amdgcn_exp2f(-pexp)) : -INFINITY;
     float* __restrict__ O = (float*)a.o + b * a.os[0] + hd * a.os[1];
     if (a.vec_out && a.D == DP) {
         by_rows(result,

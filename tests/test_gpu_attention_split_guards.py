@@ -195,3 +195,26 @@ def test_general_kernel_on_request(D):
     assert [n.split("<")[0] for n in names] == ["attn_fwd_kernel", "attn_weights_kernel"], names
     o2, w2 = call()
     assert float((o - o2).norm() / o2.norm()) <= 4e-6 and float((w - w2).norm() / w2.norm()) <= 4e-6
+
+
+def versus_general_kernel(call, exact):
+    """Error of each output of `call` against float64 in the 2-norm, as chosen and on the general kernel (fp32 pipe)."""
+    from aidotnet.tensors_amd import Mi355Backend, Mi355Engine
+    be = Mi355Backend()
+    eng = Mi355Engine(be)
+    found = []
+    for fast in (True, False):
+        be.SetAttentionFastPath(fast)
+        found.append([float((got.double() - want).norm() / want.norm()) for got, want in zip(call(eng), exact)])
+    return list(zip(*found))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("B,H,Sq,Sk,D", [(8, 12, 512, 512, 64), (2, 16, 200, 200, 32), (4, 16, 300, 300, 128), (1, 8, 1024, 1024, 128), (1, 8, 200, 1000, 64)])
+def test_log_sum_is_as_exact_as_on_the_fp32_pipe(B, H, Sq, Sk, D, causal):
+    """(4.1e-8 where the fp32 pipe has 5.0e-8; the margin is for what two sums of some ten thousand errors differ by)"""
+    q, k, v = randn(Sk + D, (B, H, Sq, D), (B, H, Sk, D), (B, H, Sk, D))
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) / math.sqrt(D)
+    lse = torch.logsumexp(s.masked_fill(later(Sq, Sk), -math.inf) if causal else s, -1)
+    (chosen, general), = versus_general_kernel(lambda eng: [eng.FlashAttention(q, k, v, isCausal=causal)[1]], [lse])
+    assert chosen <= 1.03 * general
