@@ -730,12 +730,16 @@ static long long seen_keys(const AttnArgs& a) { return a.causal ? std::min((long
 
 // fp32, rows on the 16-byte grid, head dimension up to 128 in whole chunks of eight, a head's K and V within 4 GB (contiguous).  At head
 // dimensions 33 .. 64 up to 64 keys stay on the fp32 pipe: one tile of them costs less than the splitting beside it (us: B1 H8 S52 7.9 / 8.6, B15 H32
-// S27 8.5 / 9.8; 71 keys 10.0 / 9.0; d32 S53 6.9 / 7.0, d128 S62 12.1 / 12.2)
+// S27 8.5 / 9.8; 71 keys 10.0 / 9.0; d128 S62 12.1 / 12.2).  Below that width few keys stay there for the sake of the results: what the split cuts,
+// 1.2e-7 of a row of one key, shows where neither the products nor the sums are long enough to round as much (error of O against float64 in units
+// of 1e-7, split / fp32 pipe, causal: d8 S256 1.56 / 1.47, 400 1.63 / 1.63; d16 S128 1.43 / 1.37, 200 1.49 / 1.50; d24 S80 1.46 / 1.42, 128 1.52 / 1.56;
+// d32 S32 1.31 / 1.23, 56 1.37 / 1.39; plain: d8 S64 1.71 / 1.61, 81 1.77 / 1.71; d16 S20 1.48 / 1.45, 32 1.56 / 1.67).  It costs up to a half there:
+// B64 H16 S64 d16 plain 9.5 / 14.3 us, S27 B15 H32 d32 causal 7.5 / 7.0
 bool attn_split_applies(const AttnArgs& a)
 {
     auto fits = [&](long long row) { return row > 0 && row < (1LL << 30) && (a.bt || row * a.Sk < (1LL << 30)); };
     if (a.bt && (a.bias || a.mask_mode != 0 || a.softcap > 0.0f)) return false;
-    if (a.D > 32 && a.D <= 64 && seen_keys(a) <= 64) return false;
+    if (a.D <= 64 && seen_keys(a) <= (a.D > 32 ? 64 : a.causal ? 4096 / a.D - 80 : 1024 / a.D)) return false;
     return a.vec_in && a.D % 8 == 0 && a.D <= 128 && a.scale > 0.0f && a.scale < 0x1p20f && fits(a.ks[2]) && fits(a.vs[2]);
 }
 
