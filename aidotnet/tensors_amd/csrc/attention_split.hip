@@ -552,17 +552,19 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
             __syncthreads();
             const int keys = min(ntiles * BC, a.Sk), d0 = 4 * (t % (DP / 4));
             const uint32_t mine = cols[d0 / 32] >> (d0 % 32) & 15u;
-            const float least = (found & DIM) != 0 ? INFINITY : 0.5f;
-            bool small = false;
+            int small = 0;
             if (d0 < a.D && mine != 0) {
+                f32x4 least = {INFINITY, INFINITY, INFINITY, INFINITY};           // magnitude that is not zero
 #pragma unroll 8
                 for (int key = first * BC + t / (DP / 4); key < keys; key += NT / (DP / 4)) {
                     const f32x4 x = *(const f32x4*)(V + paged_row(bt, a.bsz, key) * a.vs[2] + d0);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) small |= (mine >> e & 1u) != 0 && x[e] != 0.0f && fabsf(x[e]) * vsc < least;
+                    for (int e = 0; e < 4; e++) least[e] = fminf(least[e], x[e] == 0.0f ? INFINITY : fabsf(x[e]));
                 }
+#pragma unroll
+                for (int e = 0; e < 4; e++) small |= (int)((mine >> e & 1u) != 0 && least[e] < ((found & DIM) != 0 ? INFINITY : 0.5f / vsc));
             }
-            again = any_wave(__builtin_amdgcn_ballot_w64(small) != 0 ? 1 : 0) != 0;
+            again = any_wave(__builtin_amdgcn_ballot_w64(small != 0) != 0 ? 1 : 0) != 0;
         }
         if (again) {
             // again on the fp32 pipe, rows straight from memory
