@@ -503,7 +503,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
                 top = fmaxf(top, fabsf(oacc[i][r]));
             }
         bool bad = poison != poison;               // infinities, NaN, values beyond the scale of the first tile
-        bad |= coarse && row && (OPT || fabsf(m_run) - 1.0f < 0x1p13f * to_log2);        // (m_run is rounded up to a whole number)
+        // (m_run is rounded up to a whole number; with a bias or a cap it is not the logit's)
+        bad |= coarse && row && ((OPT && (a.bias || a.softcap > 0.0f)) || fabsf(m_run) - 1.0f < 0x1p13f * (OPT ? LOG2E : 1.0f) * to_log2);
         // V' is cut at 2^-25 units, and its largest value in the first tile is 2^11 or more.  A row of O that nowhere reaches one unit may be made of
         // values that the scale has left too few bits of: those that set it can be hidden from the row, or weigh nothing in it
         const bool dim = row && q0 + l32 < a.Sq && max_with_partner32(top) < l * (1 << P_SPLIT);

@@ -240,3 +240,19 @@ def test_few_keys_are_as_exact_as_on_the_fp32_pipe(D, Sk, causal):
     want, _, _ = reference(q, k, v, later(Sk, Sk) if causal else None)
     (chosen, general), = versus_general_kernel(lambda eng: [eng.FlashAttention(q, k, v, isCausal=causal)[0]], [want])
     assert chosen <= 1.03 * general
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("option", ["padding", "plane"])
+def test_large_logits_under_a_mask(eng, option, D):
+    """Logits of thousands: rows whose largest one is far from zero are held, those that see one key of little weight are not."""
+    q, k, v = randn(D, (1, 2, 100, D), (1, 2, 200, D), (1, 2, 200, D))
+    q, k = q * 60, k * 60
+    q[:, :, 7] *= 1e-4
+    hidden = torch.zeros(1, 1, 1 if option == "padding" else 100, 200, dtype=torch.bool, device="cuda")
+    hidden[..., :50] = True
+    want, _, big = reference(q, k, v, hidden)
+    o, _ = eng.ScaledDotProductAttention(q, k, v, ~hidden, returnWeights=False)
+    # (2^-24 of a logit is a relative error of its probability)
+    assert float((o.double() - want).norm() / want.norm()) <= 1.5e-6 * max(1.0, float(big) / 4)
+    assert worst_row(o[:, :, 7], want[:, :, 7]) <= 4e-6
