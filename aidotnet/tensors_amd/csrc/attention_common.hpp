@@ -305,7 +305,7 @@ __device__ __forceinline__ float merge_partials(const float* __restrict__ P, int
 // waves per row of the merge passes: one (four rows to a workgroup) while a row's ranges fit one round of loads
 inline int merge_waves_per_row(int ranges) { return ranges <= 8 ? 1 : 4; }
 
-// fp32 attention on the bf16 matrix pipe (attention_split.hip); options: bias, masks, soft-cap
+// fp32 attention on the fp16 matrix pipe (attention_split.hip); options: bias, masks, soft-cap
 bool attn_split_applies(const AttnArgs& a);
 int attn_split_ranges(const AttnArgs& a);
 hipError_t launch_attn_split(const AttnArgs& a, bool options, hipStream_t stream);

@@ -38,8 +38,9 @@ def gen(kind, ablate=(), flip=0, period=1):
     v[64:79] logits (block (kb, qb) at 64 + 4 (2 kb + qb)), v[80:87] P (qb 0, qb 1), v[88:119] Q (block (qb, ks) at
     88 + 4 (4 qb + ks)), v[120:151] fragment ring, v[152:155] K read addresses per ks (kb by an offset), v[156:159] ones, v[192:199] V read
     addresses per d-block, v[160:163] lane offsets of the four K wave-loads, v164 / v174 of the even / odd V wave-loads, v165 v166 minus the
-    exponent reference of query block 0 / 1, v167 v168 their running row sums, v169 v170 scratch, v171 v172 the lane's key limit
-    inside a masked unit per query block, v173 minus infinity, v[176:191] exponentials.
+    exponent reference of query block 0 / 1, v169 v170 scratch, v171 v172 the lane's key limit inside a masked unit per query block, v173
+    minus infinity, v[176:191] exponentials (v[176:179] minus ones ahead of the run), v[200:203] v[204:207] the running row sums of query
+    block 0 / 1.
     s[40:41] / s[42:43] source of this wave's next K / V tile load, s[46:47] s[48:49] one K / V tile in bytes, s50 s51 LDS
     destination of this wave's K / V loads in stage 0, s52 scale * log2(e), s53 units left, s56 block of the first unit, s57 s58
     odd units that still load a K / V tile, s59 whether a masked unit follows the run, s60 the priority flavour (below).
