@@ -9,15 +9,14 @@ immediate; a run enters at the block of its first unit (through that block's col
 fragments) and leaves behind any block; with s59 set one more unit follows the run whose logits are masked first (the unit on the
 causal diagonal).
 
-No arguments: the routine into attention_prefill_loop.inc beside this script.  FILE PARTS: the routine into FILE with the comma-
-separated PARTS left out (dma, barrier, valu, lds: timing experiments only, the results are wrong).
+Writes the routine into attention_prefill_loop.inc beside this script.
 """
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def gen(kind, ablate=(), flip=0, period=1):
+def gen(kind, flip=0):
     """One routine on v_mfma_f32_16x16x32.  A wave's 32 queries are two blocks of 16 (qb), a unit's 32 keys two blocks of 16 (kb),
     the head dimension eight blocks of 16 (db); every fragment read from LDS feeds two MFMAs (one per query block).  Lane (c, g) =
     (lane % 16, lane / 16) holds query c of a block and keys / dims 4 g + r of a block.  Per unit u a block has 16 slots, slot i
@@ -47,7 +46,7 @@ def gen(kind, ablate=(), flip=0, period=1):
 
     Wave priority: the two workgroups of a CU run this routine side by side, and a SIMD serves the older of two waves of equal
     priority first -- left alone the older workgroup gets about 63 % of the issue slots, finishes early, and the younger one runs the
-    last fifth of the launch on its own.  Each unit therefore starts with s_setprio ((unit / period) % 2) ^ flip: the workgroups of
+    last fifth of the launch on its own.  Each unit therefore starts with s_setprio (unit % 2) ^ flip: the workgroups of
     the first and of the second half of the grid (which share the CUs) take the flavours flip = 0 and flip = 1, so that at any time
     one of the two leads and they take turns; the routine leaves at priority 0.  Measured on causal and unmasked B4 H32 S2048 and
     causal S8192: the gap between the two workgroups' finish times halves (30 -> 16 us of 148) and the launch is 0.5-2.5 % shorter
@@ -65,8 +64,6 @@ def gen(kind, ablate=(), flip=0, period=1):
 
     def read_frag(blk, f):
         b = fr(f)
-        if "lds" in ablate:
-            return
         if f < 8:
             voff = blk * 8192
             emit("ds_read_b64_tr_b16 v[%d:%d], v%d offset:%d" % (b, b + 1, 192 + f, voff))
@@ -118,8 +115,7 @@ def gen(kind, ablate=(), flip=0, period=1):
         if not is_b and i == 9:
             emit("s_waitcnt vmcnt(0) lgkmcnt(0)")
             del queue[:]
-            if "barrier" not in ablate:
-                emit("s_barrier")
+            emit("s_barrier")
         if (i & 1) == 0:
             wait_frag(blk, i + 1)
         else:
@@ -143,13 +139,11 @@ def gen(kind, ablate=(), flip=0, period=1):
             read_frag(blk, f)
         else:
             read_frag((blk + 1) & 3, f - 16)
-        if dma and "dma" not in ablate:
+        if dma:
             n = i & 3
             ptr, lane = (40, 160 + n) if i < 4 else (42, 174 if n & 1 else 164)
             emit("global_load_lds_dwordx4 v%d, s[%d:%d] offset:%d" % (lane, ptr, ptr + 1, 1024 * n))
-        if "valu" in ablate:
-            pass
-        elif i < 8:
+        if i < 8:
             if i == 0:
                 emit("s_nop 1")
             for t in (2 * i, 2 * i + 1):
@@ -167,8 +161,7 @@ def gen(kind, ablate=(), flip=0, period=1):
         is_b = (blk & 1) == 0
         kstage = (blk >> 1) & 1
         emit("%sblk%d_%%=:" % (label, blk))
-        if "prio" not in ablate:
-            emit("s_setprio %d" % ((((blk // period) & 1) ^ flip)))
+        emit("s_setprio %d" % ((blk & 1) ^ flip))
         del queue[:]
         queue.extend(first7(blk))
         if is_b:
@@ -198,7 +191,7 @@ def gen(kind, ablate=(), flip=0, period=1):
         else:
             for i in range(16):
                 slot(blk, i, False, False)
-        assert "lds" in ablate or queue == first7((blk + 1) & 3), queue
+        assert queue == first7((blk + 1) & 3), queue
         emit("s_sub_u32 s53, s53, 1")
         emit("s_cmp_eq_u32 s53, 0")
         emit("s_cbranch_scc1 %sfin%d_%%=" % (label, blk))
@@ -220,36 +213,26 @@ def gen(kind, ablate=(), flip=0, period=1):
     emit("%sexit_%%=:" % label)
     for qb in (0, 1):
         row_sum(qb)
-    if "prio" not in ablate:
-        emit("s_setprio 0")
+    emit("s_setprio 0")
     emit("s_waitcnt lgkmcnt(0)")
     emit("s_nop 7")
     emit("s_nop 7")
     return out
 
 
-def write(name, ablate=()):
-    with open(name, "w") as fh:
+def main():
+    with open(os.path.join(HERE, "attention_prefill_loop.inc"), "w") as fh:
         fh.write("// Generated by gen_prefill_loop.py (the run of whole units of attn_prefill_kernel as gfx950 assembly); do not edit.\n")
-        period = 2 if "period2" in ablate else 1
         for kind in ("f16", "bf16"):
             # both priority flavours in one statement (s60 != 0 selects the second): one set of register bindings in the kernel
             lines = ["s_cmp_eq_u32 s60, 0", "s_cbranch_scc0 L_prefill_%s_second_%%=" % kind]
-            lines += gen(kind, ablate, 0, period) + ["s_branch L_prefill_%s_end_%%=" % kind, "L_prefill_%s_second_%%=:" % kind]
-            lines += gen(kind, ablate, 1, period) + ["L_prefill_%s_end_%%=:" % kind]
+            lines += gen(kind, 0) + ["s_branch L_prefill_%s_end_%%=" % kind, "L_prefill_%s_second_%%=:" % kind]
+            lines += gen(kind, 1) + ["L_prefill_%s_end_%%=:" % kind]
             fh.write("#define PREFILL_LOOP_%s \\\n" % kind.upper())
             for n, line in enumerate(lines):
                 sep = "\\n" if line.endswith(":") else "\\n\\t"
                 fh.write('    "%s%s"%s\n' % (line, sep, " \\" if n + 1 < len(lines) else ""))
             fh.write("// %d instructions\n" % sum(1 for x in lines if not x.endswith(":")))
-
-
-def main():
-    import sys
-    if len(sys.argv) > 1:
-        write(sys.argv[1], tuple(sys.argv[2].split(",")) if len(sys.argv) > 2 else ())
-    else:
-        write(os.path.join(HERE, "attention_prefill_loop.inc"))
 
 
 if __name__ == "__main__":
