@@ -1470,17 +1470,19 @@ static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
 // 16-bit head dimension 64 (direct loads; measured with what a tile costs there): two groups plain
 // up to 256 (84 keys n 384 7.5 / 6.6, S1249 n 640 31.6 / 30.0), causal up to 640 (S1960 n 620 28.2, 24.4 on 128-key tiles / 33.9; S432 n 896
 // 13.9 / 12.0), none up to 64 keys (S43 5.5 / 5.3); from 96 keys on 128-key tiles, a barrier for twice the work (S1489 n 192 21.6 / 18.0, S239
-// n 192 7.9 / 7.5; 69 keys 5.8 / 6.1); four groups gain no more there (S379 n 96 8.6 / 8.3).
+// n 192 7.9 / 7.5; 69 keys 5.8 / 6.1); four groups gain no more there (S379 n 96 8.6 / 8.3).  Under a key mask the lines of the other kinds hold:
+// either group's largest probability is one, which 16 bits hold exactly, and padded layers come out closer for 1 - 2 % of their time (error against
+// float64, two groups / one: bf16 B8 S512 H12 3.88e-3 / 3.90e-3, 49.9 / 49.1 us; B13 S198 H12 3.89e-3 / 3.92e-3, 37.5 / 36.8; f16 B5 S277 H12 4.85e-4 / 4.89e-4).
 template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
 static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
 {
     constexpr bool WIDE32 = Elem<T>::BYTES == 4 && BC == 32 && DP == 128;
     if constexpr ((BC == 64 && MINB == 2) || WIDE32) {
         auto grid = [&](int rows) { return (long long)((a.Sq + rows - 1) / rows) * a.B * a.H; };
-        if constexpr (!FULL && Elem<T>::BYTES == 2 && DP == 64) {
+        if constexpr (!FULL && !KM && Elem<T>::BYTES == 2 && DP == 64) {
             if (a.Sk > 64 && grid(64) <= (a.causal ? 640 : 256)) {
                 // (direct loads of a 128-key tile: a wave's 32 keys lie in one block)
-                if constexpr (!KM) { if (a.Sk >= 96 && (!DMA || !a.bt || a.bsz % 32 == 0)) return launch_attn_kg<T, OutT, DP, 128, FULL, DMA ? 2 : 1, DMA, KM, 2>(a, stream); }
+                if (a.Sk >= 96 && (!DMA || !a.bt || a.bsz % 32 == 0)) return launch_attn_kg<T, OutT, DP, 128, FULL, DMA ? 2 : 1, DMA, KM, 2>(a, stream);
                 return launch_attn_kg<T, OutT, DP, 64, FULL, 2, DMA, KM, 2>(a, stream);
             }
             return launch_attn_kg<T, OutT, DP, BC, FULL, MINB, DMA, KM>(a, stream);
