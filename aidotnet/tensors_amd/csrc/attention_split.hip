@@ -328,7 +328,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
             int at = __lane_id();
             asm volatile("" : "+v"(at));
             const int first = -4 * (at >> 5);
-            at &= 31;
+            at = min(at & 31, a.Sq - 1 - q0);          // (rows past the last one see what it sees: they stand beside it in the tests below)
             // the query's last visible key, relative to the lane's first
             int seen = a.Sk - 1 - k0 + first;
             if (a.causal) seen = min(seen, (int)max(min((long long)q0 + a.qoff - k0, 1LL << 20), -(1LL << 20)) + at + first);

@@ -256,3 +256,13 @@ def test_large_logits_under_a_mask(eng, option, D):
     # (2^-24 of a logit is a relative error of its probability)
     assert float((o.double() - want).norm() / want.norm()) <= 1.5e-6 * max(1.0, float(big) / 4)
     assert worst_row(o[:, :, 7], want[:, :, 7]) <= 4e-6
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_column_beyond_the_last_row(eng, D):
+    """Keys behind the last row's diagonal, which the idle rows of its wave would see, do not vouch for a column."""
+    q, k, v = randn(D, (1, 2, 20, D), (1, 2, 400, D), (1, 2, 400, D))
+    v[:, :, :120, 5] *= 1e-9
+    want, _, _ = reference(q, k, v, later(20, 400, 100))
+    o, _ = eng.FlashAttention(q, k, v, isCausal=True, queryOffset=100)
+    assert float((o[..., 5].double() - want[..., 5]).norm() / want[..., 5].norm()) <= 4e-6
