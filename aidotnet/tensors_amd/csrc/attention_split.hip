@@ -486,14 +486,56 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         __syncthreads();
     }
 
-    // ---- does the split hold these results?  (What follows is addressed from here: nothing of it is kept through the loop.)
+    // (what follows is addressed from here: nothing of it is kept through the loop)
     lane = __lane_id();
     asm volatile("" : "+v"(lane));
     t = 64 * wave + lane;
     l32 = lane & 31;
     h = lane >> 5;
+    // ---- the waves of key groups 1 .. KG - 1 leave (O, m, l) in LDS, group 0 merges them
+    auto merge_groups = [&]() {
+        if constexpr (KG > 1) {
+            constexpr int AREA = DT * 16 * 64;                          // floats of one wave's O
+            float* O1 = (float*)smem + wq * (KG - 1) * AREA;
+            float* ML = (float*)smem + (KG - 1) * WQ * AREA + wq * (KG - 1) * 128;
+            __syncthreads();
+            if (kg > 0) {
+                f32x4* dst = (f32x4*)(O1 + (kg - 1) * AREA);
+#pragma unroll
+                for (int i = 0; i < DT; i++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++)
+                        dst[(i * 4 + g) * 64 + lane] = f32x4{oacc[i][4 * g], oacc[i][4 * g + 1], oacc[i][4 * g + 2], oacc[i][4 * g + 3]};
+                ML[(kg - 1) * 128 + lane] = m_run;
+                ML[(kg - 1) * 128 + 64 + lane] = l_run;
+            }
+            __syncthreads();
+            if (kg == 0) {
+#pragma unroll
+                for (int u = 0; u < KG - 1; u++) {
+                    const float m1 = ML[u * 128 + lane], l1 = ML[u * 128 + 64 + lane];
+                    const float m_new = fmaxf(m_run, m1), m_use = m_new == -INFINITY ? 0.0f : m_new;
+                    const float w0 = __builtin_amdgcn_exp2f(m_run - m_use), w1 = __builtin_amdgcn_exp2f(m1 - m_use);
+                    m_run = m_new;
+                    l_run = l_run * w0 + l1 * w1;
+                    const f32x4* src = (const f32x4*)(O1 + u * AREA);
+#pragma unroll
+                    for (int i = 0; i < DT; i++)
+#pragma unroll
+                        for (int g = 0; g < 4; g++) {
+                            const f32x4 v = src[(i * 4 + g) * 64 + lane];
+#pragma unroll
+                            for (int e = 0; e < 4; e++) oacc[i][4 * g + e] = oacc[i][4 * g + e] * w0 + v[e] * w1;
+                        }
+                }
+            }
+            __syncthreads();
+        }
+    };
+    merge_groups();
+    // ---- does the split hold these results?  Group 0 has them
     {
-        const float l = sum_with_partner32(l_run);                                // (the products run over the keys of both halves)
+        const float l = kg == 0 ? sum_with_partner32(l_run) : 0.0f;               // (the products run over the keys of both halves)
         const bool row = l > 0.0f;
         float poison = l_run * 0.0f, top = 0.0f;
 #pragma unroll
@@ -503,7 +545,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
                 poison = fmaf(oacc[i][r], 0.0f, poison);
                 top = fmaxf(top, fabsf(oacc[i][r]));
             }
-        bool bad = poison != poison;               // infinities, NaN, values beyond the scale of the first tile
+        bool bad = kg == 0 && poison != poison;    // infinities, NaN, values beyond the scale of the first tile
         // (m_run is rounded up to a whole number; with a bias or a cap it is not the logit's)
         bad |= coarse && row && ((OPT && (a.bias || a.softcap > 0.0f)) || fabsf(m_run) - 1.0f < 0x1p13f * (OPT ? LOG2E : 1.0f) * to_log2);
         // V' is cut at 2^-25 units, and its largest value in the first tile is 2^11 or more.  A row of O that nowhere reaches one unit may be made of
@@ -604,48 +646,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
+            merge_groups();
         }
     }
-
-    // ---- the waves of key groups 1 .. KG - 1 leave (O, m, l) in LDS, group 0 merges them
-    if constexpr (KG > 1) {
-        constexpr int AREA = DT * 16 * 64;                          // floats of one wave's O
-        float* O1 = (float*)smem + wq * (KG - 1) * AREA;
-        float* ML = (float*)smem + (KG - 1) * WQ * AREA + wq * (KG - 1) * 128;
-        __syncthreads();
-        if (kg > 0) {
-            f32x4* dst = (f32x4*)(O1 + (kg - 1) * AREA);
-#pragma unroll
-            for (int i = 0; i < DT; i++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-                    dst[(i * 4 + g) * 64 + lane] = f32x4{oacc[i][4 * g], oacc[i][4 * g + 1], oacc[i][4 * g + 2], oacc[i][4 * g + 3]};
-            ML[(kg - 1) * 128 + lane] = m_run;
-            ML[(kg - 1) * 128 + 64 + lane] = l_run;
-        }
-        __syncthreads();
-        if (kg == 0) {
-#pragma unroll
-            for (int u = 0; u < KG - 1; u++) {
-                const float m1 = ML[u * 128 + lane], l1 = ML[u * 128 + 64 + lane];
-                const float m_new = fmaxf(m_run, m1), m_use = m_new == -INFINITY ? 0.0f : m_new;
-                const float w0 = __builtin_amdgcn_exp2f(m_run - m_use), w1 = __builtin_amdgcn_exp2f(m1 - m_use);
-                m_run = m_new;
-                l_run = l_run * w0 + l1 * w1;
-                const f32x4* src = (const f32x4*)(O1 + u * AREA);
-#pragma unroll
-                for (int i = 0; i < DT; i++)
-#pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        const f32x4 v = src[(i * 4 + g) * 64 + lane];
-#pragma unroll
-                        for (int e = 0; e < 4; e++) oacc[i][4 * g + e] = oacc[i][4 * g + e] * w0 + v[e] * w1;
-                    }
-            }
-        }
-        __syncthreads();
-        if (kg > 0) return;
-    }
+    if (kg > 0) return;
 
     // ---- normalise and store: lane holds query q0 + l32, head-dim elements 32 i + 8 g + 4 h + (0..3)
     const int qi = q0 + l32;
