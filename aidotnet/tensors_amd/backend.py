@@ -726,6 +726,10 @@ class Mi355Backend:
             raise ArgumentException("Attention tensor buffers are smaller than the requested dimensions.")
         if softmaxStats.Size < batch * numHeads * seqQ:
             raise ArgumentException("The softmax-statistics buffer is too small.")
+        if attentionBias is not None:
+            if batch > 1 and biasBatchStride < 0:
+                raise ArgumentOutOfRangeException("biasBatchStride must not be negative.")
+            self._capacity(attentionBias, ((batch - 1) * biasBatchStride + numHeads * seqQ * seqK) * 4, "attentionBias", "FlashAttentionV2")
         d = AttnDesc(B=batch, H=numHeads, Hkv=numHeads, Sq=seqQ, Sk=seqK, D=headDim, scale=scale,
                      causal=1 if isCausal else 0, causal_query_offset=0, bias_batch_stride=biasBatchStride)
         self._attn("f32", query, key, value, output, softmaxStats, attentionBias, None, None, d)

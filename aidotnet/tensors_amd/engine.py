@@ -267,7 +267,7 @@ class Mi355Engine:
             bstride = 0
             if attentionBias is not None:
                 bias = be.WrapTensor(attentionBias.contiguous().float())
-                bstride = H * Sq * Sk if attentionBias.dim() == 4 else 0
+                bstride = H * Sq * Sk if attentionBias.dim() == 4 and attentionBias.shape[0] != 1 else 0
             be.FlashAttentionV2(be.WrapTensor(q), be.WrapTensor(k), be.WrapTensor(v), be.WrapTensor(out), be.WrapTensor(lse),
                                 B, H, Sq, Sk, D, scale, isCausal, bias, bstride)
         else:
