@@ -53,6 +53,13 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     constexpr int KBYTES = DMA ? BC * DP * EB : BC * KPITCH, VBYTES = DMA ? BC * DP * EB : DP * VPITCH;
     constexpr int KT = BC / 32 / KG;           // 32-key sub-tiles per tile and wave
     static_assert(KT >= 1, "every key group has a sub-tile of its own");
+    // The two groups of a 16-bit 128-key tile take its 32-key blocks in turn and each block moves the exponent reference: the same keys to a group and
+    // the same probabilities that are exactly one as on 64-key tiles, so the same error (64 keys to a reference: 3 - 6 % more).  For half as many
+    // barriers (bf16 causal n 480 S2525 33.1 -> 28.8 us, n 528 S1355 20.7 -> 18.7, n 264 S674 13.4 -> 12.6)
+    constexpr bool TURNS = EB == 2 && DP == 64 && !FULL && BC == 128 && KG == 2;
+    constexpr int KSTEP = TURNS ? 64 : 32;     // keys from one sub-tile of a wave to the next
+    constexpr int KG0 = TURNS ? 32 : KT * 32;  // and from a group's first key to the next group's
+    constexpr int REF = TURNS ? 1 : KT;        // sub-tiles to one exponent reference
     constexpr int DT = DP / 32;                // 32-row tiles of O^T
     constexpr int PSTEPS = 32 / KS;            // PV fragment steps per key sub-tile
     constexpr int CPR = DP / E;                // 16-byte chunks per K row
@@ -272,7 +279,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
     for (int j = first; j < ntiles; j++) {
         const int stage = j & 1;
         const int kv0 = j * BC;
-        const int kw0 = kv0 + kg * KT * 32;      // first key of this wave's sub-tiles
+        const int kw0 = kv0 + kg * KG0;          // first key of this wave's sub-tiles
         unsigned next_keep = 0;        // (read with the next tile's loads, looked at when they have landed)
         if constexpr (KM) next_keep = kmask[min(kv0 + BC + lane, a.Sk - 1)];
         if constexpr (DMA) { if (j + 1 < ntiles) issue_tile(j + 1, stage ^ 1); }
@@ -281,7 +288,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
         // a wave whose 32 rows are all above the causal diagonal of its keys, or past the last row or key, only helps with the copies
         const bool active = wq_min < a.Sq && kw0 < a.Sk && !(a.causal && (long long)kw0 > (long long)wq_max + a.qoff) && (!KM || kbits != 0);
         if (active) {
-            const int kr0 = kg * KT * 32;        // this wave's first key inside the tile
+            const int kr0 = kg * KG0;            // this wave's first key inside the tile
             const unsigned char* ks = Ks + stage * KBYTES + (kr0 + l32) * KPITCH + h * 16;
             const unsigned char* vs = Vs + stage * VBYTES + l32 * VPITCH + kr0 * EB + h * 16;
 
@@ -315,15 +322,15 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 #pragma unroll
                 for (int kt = 0; kt < KT; kt++) {
                     u32x4 kf;
-                    if constexpr (DMA) kf = *(const u32x4*)(Ks + stage * KBYTES + (kr0 + kt * 32 + l32) * (DP * EB) + (((2 * s + h) ^ k_swz(l32)) << 4));
-                    else kf = *(const u32x4*)(ks + kt * 32 * KPITCH + s * 32);
+                    if constexpr (DMA) kf = *(const u32x4*)(Ks + stage * KBYTES + (kr0 + kt * KSTEP + l32) * (DP * EB) + (((2 * s + h) ^ k_swz(l32)) << 4));
+                    else kf = *(const u32x4*)(ks + kt * KSTEP * KPITCH + s * 32);
                     Mma32<T>::run(st[kt], kf, qs);
                 }
             }
             if constexpr (EB == 4) __builtin_amdgcn_s_setprio(0);
 
             // ---- logits in the log2 domain, masks
-            const bool need_mask = (kw0 + KT * 32 > a.Sk) || (a.causal && (long long)kw0 + KT * 32 - 1 > (long long)wq_min + a.qoff);
+            const bool need_mask = (kw0 + (KT - 1) * KSTEP + 32 > a.Sk) || (a.causal && (long long)kw0 + (KT - 1) * KSTEP + 31 > (long long)wq_min + a.qoff);
             if constexpr (FULL) kbits = __builtin_amdgcn_ballot_w64(keep != 0);      // (keys past the end are masked below)
             const bool mixed = (KM || FULL) && (BC == 64 ? kbits != ~0ull : (uint32_t)kbits != ~0u);
             if constexpr (FULL) {
@@ -395,7 +402,7 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
 #pragma unroll
                 for (int kt = 0; kt < KT; kt++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) if (kt * 32 + acc_row(r, 0) > seen) st[kt][r] = -INFINITY;
+                    for (int r = 0; r < 16; r++) if (kt * KSTEP + acc_row(r, 0) > seen) st[kt][r] = -INFINITY;
             }
             if constexpr (KM || FULL) {
                 if (mixed) {
@@ -407,76 +414,79 @@ __global__ __launch_bounds__(256, MINB) void attn_fwd_kernel(const AttnArgs a)
                     }
                 }
             }
-            float mloc = -INFINITY;
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++)
+            for (int k0 = 0; k0 < KT; k0 += REF) {
+                float mloc = -INFINITY;
 #pragma unroll
-                for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, st[kt][r]);
-            mloc = max_with_partner32(mloc) * factor;
-            const float m_new = fmaxf(m_run, mloc);
-            const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
-            m_run = m_new;
+                for (int kt = k0; kt < k0 + REF; kt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, st[kt][r]);
+                mloc = max_with_partner32(mloc) * factor;
+                const float m_new = fmaxf(m_run, mloc);
+                const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
+                const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+                m_run = m_new;
 
-            float psum = 0.0f;
+                float psum = 0.0f;
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++)
+                for (int kt = k0; kt < k0 + REF; kt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    float p = __builtin_amdgcn_exp2f(fmaf(st[kt][r], factor, -m_use));
-                    st[kt][r] = p;
-                    psum += p;
-                }
-            l_run = l_run * alpha + psum;
-            // alpha == 1 in every lane (no row maximum moved) is the common case once a few tiles have been seen
-            if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0ull) {
-#pragma unroll
-                for (int i = 0; i < DT; i++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
-            }
-
-            // ---- O^T += V^T * P^T
-            if constexpr (EB == 4) __builtin_amdgcn_s_setprio(2);
-#pragma unroll
-            for (int kt = 0; kt < KT; kt++) {
-#pragma unroll
-                for (int ps = 0; ps < PSTEPS; ps++) {
-                    u32x4 pf;
-                    if constexpr (E == 8) {
-#pragma unroll
-                        for (int w = 0; w < 4; w++) pf[w] = pack2_p<T>(st[kt][8 * ps + 2 * w], st[kt][8 * ps + 2 * w + 1]);
-                    } else {
-#pragma unroll
-                        for (int w = 0; w < 4; w++) pf[w] = as_u32(st[kt][4 * ps + w]);
+                    for (int r = 0; r < 16; r++) {
+                        float p = __builtin_amdgcn_exp2f(fmaf(st[kt][r], factor, -m_use));
+                        st[kt][r] = p;
+                        psum += p;
                     }
+                l_run = l_run * alpha + psum;
+                // alpha == 1 in every lane (no row maximum moved) is the common case once a few tiles have been seen
+                if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0ull) {
 #pragma unroll
-                    for (int i = 0; i < DT; i++) {
-                        u32x4 vf;
-                        if constexpr (DMA && EB == 4) {
-                            // V[key = 32 kt + 8 ps + 4 h + q][d = 32 i + l32]; (key >> 2) & 1 == h
-                            const int d = i * 32 + l32;
-                            const unsigned char* vp = Vs + stage * VBYTES + (kr0 + kt * 32 + 8 * ps + 4 * h) * (DP * 4) + ((((d >> 2) ^ (h << 3)) << 4) + (d & 3) * 4);
+                    for (int i = 0; i < DT; i++)
 #pragma unroll
-                            for (int q = 0; q < 4; q++) vf[q] = *(const uint32_t*)(vp + q * (DP * 4));
-                        } else if constexpr (DMA) {
-                            // 16-bit: the lane's eight k-slots are keys 16 ps + 4 h + (0..3) and 16 ps + 8 + 4 h + (0..3) (the order of
-                            // the accumulator rows its P values come from); one transposing read per group of four: in a
-                            // 16-lane group lane j addresses key (base + j / 4), 8 bytes at head-dim 4 (j % 4) of the 16-wide block
-                            const int jl = lane & 15;
-                            const int chunk = (i * 32 + 16 * ((lane >> 4) & 1) + 4 * (jl & 3)) >> 3;
+                        for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
+                }
+
+                // ---- O^T += V^T * P^T
+                if constexpr (EB == 4) __builtin_amdgcn_s_setprio(2);
 #pragma unroll
-                            for (int q = 0; q < 2; q++) {
-                                const int row = kr0 + kt * 32 + 16 * ps + 8 * q + 4 * h + (jl >> 2);
-                                u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                    (__attribute__((address_space(3))) s16x4a*)(Vs + stage * VBYTES + row * (DP * 2) + ((chunk ^ v_swz(row)) << 4) + (jl & 1) * 8)));
-                                vf[2 * q] = w[0];
-                                vf[2 * q + 1] = w[1];
-                            }
+                for (int kt = k0; kt < k0 + REF; kt++) {
+#pragma unroll
+                    for (int ps = 0; ps < PSTEPS; ps++) {
+                        u32x4 pf;
+                        if constexpr (E == 8) {
+#pragma unroll
+                            for (int w = 0; w < 4; w++) pf[w] = pack2_p<T>(st[kt][8 * ps + 2 * w], st[kt][8 * ps + 2 * w + 1]);
                         } else {
-                            vf = *(const u32x4*)(vs + i * 32 * VPITCH + kt * 32 * EB + ps * 32);
+#pragma unroll
+                            for (int w = 0; w < 4; w++) pf[w] = as_u32(st[kt][4 * ps + w]);
                         }
-                        Mma32<T>::run(oacc[i], vf, pf);
+#pragma unroll
+                        for (int i = 0; i < DT; i++) {
+                            u32x4 vf;
+                            if constexpr (DMA && EB == 4) {
+                                // V[key = 32 kt + 8 ps + 4 h + q][d = 32 i + l32]; (key >> 2) & 1 == h
+                                const int d = i * 32 + l32;
+                                const unsigned char* vp = Vs + stage * VBYTES + (kr0 + kt * 32 + 8 * ps + 4 * h) * (DP * 4) + ((((d >> 2) ^ (h << 3)) << 4) + (d & 3) * 4);
+#pragma unroll
+                                for (int q = 0; q < 4; q++) vf[q] = *(const uint32_t*)(vp + q * (DP * 4));
+                            } else if constexpr (DMA) {
+                                // 16-bit: the lane's eight k-slots are keys 16 ps + 4 h + (0..3) and 16 ps + 8 + 4 h + (0..3) (the order of
+                                // the accumulator rows its P values come from); one transposing read per group of four: in a
+                                // 16-lane group lane j addresses key (base + j / 4), 8 bytes at head-dim 4 (j % 4) of the 16-wide block
+                                const int jl = lane & 15;
+                                const int chunk = (i * 32 + 16 * ((lane >> 4) & 1) + 4 * (jl & 3)) >> 3;
+#pragma unroll
+                                for (int q = 0; q < 2; q++) {
+                                    const int row = kr0 + kt * KSTEP + 16 * ps + 8 * q + 4 * h + (jl >> 2);
+                                    u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                        (__attribute__((address_space(3))) s16x4a*)(Vs + stage * VBYTES + row * (DP * 2) + ((chunk ^ v_swz(row)) << 4) + (jl & 1) * 8)));
+                                    vf[2 * q] = w[0];
+                                    vf[2 * q + 1] = w[1];
+                                }
+                            } else {
+                                vf = *(const u32x4*)(vs + i * 32 * VPITCH + kt * KSTEP * EB + ps * 32);
+                            }
+                            Mma32<T>::run(oacc[i], vf, pf);
+                        }
                     }
                 }
             }
@@ -1466,29 +1476,29 @@ static hipError_t launch_attn_kg(AttnArgs a, hipStream_t stream)
 //   16-bit causal beyond 768: a 128-row grid of more than 512, or long rows (S 300 n 1000 14.0 / 11.9; but S 232 n 944 10.5 / 11.5)
 //   fp32 above 64: up to 32 keys the second group has none (Sk 12 10.6 / 12.8); causal 384 only where the row tiles differ in length
 //     (Sq 204 n 288 44 / 35; but Sq 62, Sk 12 n 352 16 / 26)
-// The lines do not depend on how the tiles are loaded, so the direct-to-LDS and the register-staged forms add up the same way.
-// 16-bit head dimension 64 (direct loads; measured with what a tile costs there): two groups plain
-// up to 256 (84 keys n 384 7.5 / 6.6, S1249 n 640 31.6 / 30.0), causal up to 640 (S1960 n 620 28.2, 24.4 on 128-key tiles / 33.9; S432 n 896
-// 13.9 / 12.0), none up to 64 keys (S43 5.5 / 5.3); from 96 keys on 128-key tiles, a barrier for twice the work (S1489 n 192 21.6 / 18.0, S239
-// n 192 7.9 / 7.5; 69 keys 5.8 / 6.1); four groups gain no more there (S379 n 96 8.6 / 8.3).  Under a key mask the lines of the other kinds hold:
-// either group's largest probability is one, which 16 bits hold exactly, and padded layers come out closer for 1 - 2 % of their time (error against
-// float64, two groups / one: bf16 B8 S512 H12 3.88e-3 / 3.90e-3, 49.9 / 49.1 us; B13 S198 H12 3.89e-3 / 3.92e-3, 37.5 / 36.8; f16 B5 S277 H12 4.85e-4 / 4.89e-4).
+// These lines do not depend on how the tiles are loaded, so the direct-to-LDS and the register-staged forms add up the same way.
+// 16-bit head dimension 64 with direct loads goes further, two workgroups of four groups to a CU (us on two groups and 64-key tiles / so):
+//   four groups over long rows up to 512 plain (from 320 keys on: S910 n 464 16.5 / 14.3, 1940 on 3042 n 488 39.5 / 29.4, S406 n 312 10.2 / 10.0; S271 n 288
+//     8.7 / 9.2) and 640 causal (from 1024 keys on: S2145 n 544 29.8 / 20.1; S471 n 720 10.7 / 13.9, S1355 n 1032 20.7 / 25.4); also behind a block table
+//     whose blocks hold a wave's 32 keys
+//   beyond, causal, two groups on 128-key tiles up to 512 (S471 n 384 10.7 / 10.0, S834 n 448 14.7 / 13.4, S1534 n 384 22.7 / 19.6) and over long rows 576
+//     (S1355 n 528 20.7 / 18.6; S530 n 544 11.5 / 13.2)
+// More groups also make more of the probabilities exactly one.  Fewer than all these lines give, as one group from n 257 plain and 641 causal on, are 3 - 9 %
+// further from float64 (S200 plain f16 1.51e-4, on two groups where four are now 1.64e-4; S251 causal bf16 1.035e-3 / 1.088e-3), padded layers 0.3 - 0.8 %,
+// and slower (S1191 plain n 304 22.2 on two, 26.7 on one; S1964 causal n 744 28.4 / 40.7).
 template <typename T, typename OutT, int DP, int BC, bool FULL, int MINB, bool DMA = false, bool KM = false>
 static hipError_t launch_attn(const AttnArgs& a, hipStream_t stream)
 {
     constexpr bool WIDE32 = Elem<T>::BYTES == 4 && BC == 32 && DP == 128;
     if constexpr ((BC == 64 && MINB == 2) || WIDE32) {
         auto grid = [&](int rows) { return (long long)((a.Sq + rows - 1) / rows) * a.B * a.H; };
-        if constexpr (!FULL && !KM && Elem<T>::BYTES == 2 && DP == 64) {
-            if (a.Sk > 64 && grid(64) <= (a.causal ? 640 : 256)) {
-                // (direct loads of a 128-key tile: a wave's 32 keys lie in one block)
-                if (a.Sk >= 96 && (!DMA || !a.bt || a.bsz % 32 == 0)) return launch_attn_kg<T, OutT, DP, 128, FULL, DMA ? 2 : 1, DMA, KM, 2>(a, stream);
-                return launch_attn_kg<T, OutT, DP, 64, FULL, 2, DMA, KM, 2>(a, stream);
-            }
-            return launch_attn_kg<T, OutT, DP, BC, FULL, MINB, DMA, KM>(a, stream);
-        }
         if constexpr (!FULL && !KM && DP == 64) {
-            if (!a.bt && a.Sk >= 192 && grid(32) <= (a.causal ? 384 : 256)) return launch_attn_kg<T, OutT, DP, 128, FULL, 1, DMA, KM, 4>(a, stream);
+            constexpr bool HALF = Elem<T>::BYTES == 2 && DMA;
+            const long long four = !a.causal ? (HALF && a.Sk >= 320 ? 512 : 256) : HALF && a.Sk >= 1024 ? 640 : 384;
+            if ((!a.bt || (HALF && a.bsz % 32 == 0)) && a.Sk >= 192 && grid(32) <= four) return launch_attn_kg<T, OutT, DP, 128, FULL, HALF ? 2 : 1, DMA, KM, 4>(a, stream);
+            if constexpr (HALF) {
+                if ((!a.bt || a.bsz % 32 == 0) && a.causal && a.Sk >= 192 && grid(64) <= (a.Sk >= 1024 ? 576 : 512)) return launch_attn_kg<T, OutT, DP, 128, FULL, 2, DMA, KM, 2>(a, stream);
+            }
         }
         long long line;
         if constexpr (WIDE32) line = a.Sk <= 32 ? 0 : a.causal && a.Sq > 64 && a.Sk > 128 ? 384 : 256;
@@ -1577,8 +1587,8 @@ static int attn_dl_splits(const AttnParams& p, int* chunk)
 
 // 16-bit, head dimension 64, at most half of the CUs with a workgroup of 64 queries: shares of each query tile's keys run as workgroups of their
 // own (1 = none).  A workgroup takes 4.5 us and 1.15 for 128 keys there, the second launch 4 and the partials as in attn_split_ranges; a call costs its
-// caller 11.7 us, with two launches 14 (us in one / cut: 189 queries on 3984 keys, 16 heads 40 / 18.1, 614 on 3138, 12 heads 33 / 25.4; self-attention
-// H4 S2000 23.1 / 20.8, H2 S4000 41 / 29.4; left whole: 40 queries on 1024 keys 13.4 / 14.7, H32 100 on 900 14.1 / 14.7).
+// caller 11.7 us, with two launches 14 (us in one / cut: 189 queries on 3984 keys, 16 heads 31.3 / 18.7, 614 on 3138, 12 heads 25.7 / 24.0; self-attention
+// H2 S4000 31.3 / 27.5, causal 30.9 / 25.4, H1 S3595 28.0 / 17.6, but H4 S2000 18.5 / 20.2; left whole: 40 queries on 1024 keys, 16 heads 12.0).
 static int attn_half64_ranges(int kind, const AttnParams& p)
 {
     if (kind == 0 || p.D != 64 || p.bias || p.softcap > 0.0f || (p.mask && p.mask_mode != 0)) return 1;
