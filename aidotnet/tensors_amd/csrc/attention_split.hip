@@ -877,8 +877,10 @@ __global__ __launch_bounds__(256, 2) void attn_weights_split_kernel(const AttnAr
     const float ksc = power2(kexp);
     logit_exp -= kexp;
     const float to_logit = logit_factor(OPT ? a.scale : a.scale * LOG2E, logit_exp);
-    // (such rows are formed on the fp32 pipe, as above)
-    const bool coarse = __builtin_amdgcn_ballot_w64((OPT ? to_logit * LOG2E : to_logit) > 0x1p-13f) != 0;
+    // (such rows are formed on the fp32 pipe, as above, and as above not where their largest logits, here the log-sum-exp, are far from zero: with the
+    // two passes on different pipes a probability of one was off by the logits' error of either, 7e-4 - 2e-3 over logits of thousands)
+    const float unit = OPT ? to_logit * LOG2E : to_logit;
+    const bool coarse = __builtin_amdgcn_ballot_w64(unit > 0x1p-13f && ((OPT && (a.bias || a.softcap > 0.0f)) || fabsf(lse) * LOG2E - 1.0f < 0x1p13f * unit)) != 0;
     if (h == 0) { rows[0][32 * wave + l32] = to_logit; rows[1][32 * wave + l32] = lse == -INFINITY ? INFINITY : lse * LOG2E; }
     __builtin_amdgcn_wave_barrier();
     for (int j = first; j < seen; j++) {
