@@ -534,10 +534,14 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     };
     merge_groups();
     // ---- does the split hold these results?  Group 0 has them
+    float m_sum, l_sum;                            // the row's reference and sum as they leave
     {
         const float l = kg == 0 ? sum_with_partner32(l_run) : 0.0f;               // (the products run over the keys of both halves)
+        m_sum = m_run;
+        l_sum = l * __builtin_amdgcn_exp2f(-P_EXP);
         const bool row = l > 0.0f;
-        float poison = l_run * 0.0f, top = 0.0f;
+        float poison = l * 0.0f, top = 0.0f;
+        bool own = poison == poison;               // the sum is held, whatever the results are
 #pragma unroll
         for (int i = 0; i < DT; i++)
 #pragma unroll
@@ -547,7 +551,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
             }
         bool bad = kg == 0 && poison != poison;    // infinities, NaN, values beyond the scale of the first tile
         // (m_run is rounded up to a whole number; with a bias or a cap it is not the logit's)
-        bad |= coarse && row && ((OPT && (a.bias || a.softcap > 0.0f)) || fabsf(m_run) - 1.0f < 0x1p13f * (OPT ? LOG2E : 1.0f) * to_log2);
+        if (coarse && row && ((OPT && (a.bias || a.softcap > 0.0f)) || fabsf(m_run) - 1.0f < 0x1p13f * (OPT ? LOG2E : 1.0f) * to_log2)) {
+            bad = true;
+            own = false;
+        }
         // V' is cut at 2^-25 units, and its largest value in the first tile is 2^11 or more.  A row of O that nowhere reaches one unit may be made of
         // values that the scale has left too few bits of: those that set it can be hidden from the row, or weigh nothing in it
         const bool dim = row && q0 + l32 < a.Sq && max_with_partner32(top) < l * (1 << P_SPLIT);
@@ -647,6 +654,13 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
                 }
             }
             merge_groups();
+            // A sum that the split holds is kept where the results are not, or another row's: the pass behind this one forms its probabilities, and
+            // on the pipe that the sum was formed on (apart, over V with a column of 1e-12 they were 2 - 5 times as far off as both passes on the
+            // fp32 pipe have them, 3.6e-5 over logits of deviation 64)
+            if (!own) {
+                m_sum = m_run;
+                l_sum = sum_with_partner32(l_run);
+            }
         }
     }
     if (kg > 0) return;
@@ -684,9 +698,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
         // the sum over up to 32 ranges does not leave the range of fp32 where the result does not; m takes that power and stays exact, being whole
         float* __restrict__ P = a.part + ((long long)bh * a.Sq * a.nsplit + blockIdx.y) * (2 + a.D);
         const long long pitch = (long long)a.nsplit * (2 + a.D);
-        const int e = __builtin_amdgcn_frexp_expf(l) + (oexp > P_SPLIT ? 0 : 5);
-        if (h == 0 && qi < a.Sq) *(f32x2p*)(P + qi * pitch) = f32x2p{m_run + ((float)e - pexp), __builtin_amdgcn_ldexpf(l, -e)};
-        by_rows([&](float x) { return __builtin_amdgcn_ldexpf(x, -oexp - e); },
+        const float inv = l > 0.0f ? l_sum / l : __builtin_amdgcn_exp2f(-pexp);       // (results to the sum that leaves: a power of two where that is theirs)
+        const int e = __builtin_amdgcn_frexp_expf(l_sum) + (oexp > P_SPLIT ? 0 : 5);
+        if (h == 0 && qi < a.Sq) *(f32x2p*)(P + qi * pitch) = f32x2p{m_sum + (float)e, __builtin_amdgcn_ldexpf(l_sum, -e)};
+        by_rows([&](float x) { return __builtin_amdgcn_ldexpf(x * inv, -oexp - e); },
                 [&](int row, int d0, f32x4 v) {
                     if (d0 >= a.D) return;
                     float* __restrict__ p = P + row * pitch + 2 + d0;                  // (8-byte aligned)
@@ -697,7 +712,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_split_kernel(const AttnArgs a
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     auto result = [&](float x) { return __builtin_amdgcn_ldexpf(x * inv, -oexp); };       // (in this order: 2^-oexp / l may lie below the normal numbers)
-    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l > 0.0f ? log_sum(m_run, l * __builtin_amdgcn_exp2f(-pexp)) : -INFINITY;
+    if (a.lse && h == 0 && qi < a.Sq) a.lse[(long long)bh * a.Sq + qi] = l_sum > 0.0f ? log_sum(m_sum, l_sum) : -INFINITY;
     float* __restrict__ O = (float*)a.o + b * a.os[0] + hd * a.os[1];
     if (a.vec_out && a.D == DP) {
         by_rows(result,
@@ -880,8 +895,9 @@ __global__ __launch_bounds__(256, 2) void attn_weights_split_kernel(const AttnAr
     // (such rows are formed on the fp32 pipe, as above, and as above not where their largest logits, here the log-sum-exp, are far from zero: with the
     // two passes on different pipes a probability of one was off by the logits' error of either, 7e-4 - 2e-3 over logits of thousands)
     const float unit = OPT ? to_logit * LOG2E : to_logit;
-    const bool coarse = __builtin_amdgcn_ballot_w64(unit > 0x1p-13f && ((OPT && (a.bias || a.softcap > 0.0f)) || fabsf(lse) * LOG2E - 1.0f < 0x1p13f * unit)) != 0;
-    if (h == 0) { rows[0][32 * wave + l32] = to_logit; rows[1][32 * wave + l32] = lse == -INFINITY ? INFINITY : lse * LOG2E; }
+    const bool coarse = unit > 0x1p-13f && ((OPT && (a.bias || a.softcap > 0.0f)) || fabsf(lse) * LOG2E - 1.0f < 0x1p13f * unit);
+    const uint32_t coarse_rows = (uint32_t)__builtin_amdgcn_ballot_w64(coarse);
+    if (h == 0) { rows[0][32 * wave + l32] = !coarse ? to_logit : OPT ? a.scale : a.scale * LOG2E; rows[1][32 * wave + l32] = lse == -INFINITY ? INFINITY : lse * LOG2E; }
     __builtin_amdgcn_wave_barrier();
     for (int j = first; j < seen; j++) {
         unsigned char* ks = Ks + (j & 1) * 2 * PL;
@@ -920,17 +936,21 @@ __global__ __launch_bounds__(256, 2) void attn_weights_split_kernel(const AttnAr
         for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++) poison = fmaf(s[i][r], 0.0f, poison);
-        bool exact = coarse;
-        if (__builtin_amdgcn_ballot_w64(poison != poison) != 0) exact = true;
-        if (exact) {
+        const bool exact = __builtin_amdgcn_ballot_w64(poison != poison) != 0;
+        const uint32_t again = exact ? ~0u : coarse_rows;
+        if (again != 0) {
+            // (the other rows stay as they are: zeros are added to them)
+            int ln = __lane_id();
+            asm volatile("" : "+v"(ln));           // (which rows is formed here, not kept)
+            const uint32_t mine = (again >> (ln & 31) & 1u) != 0 ? ~0u : 0u, those = again >> (4 * (ln >> 5));
 #pragma unroll
             for (int i = 0; i < 2; i++) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) s[i][r] = 0.0f;
-                const float* kp = K + (long long)min(k0 + 32 * i + l32, a.Sk - 1) * a.ks[2] + 4 * h;
-                const float* qp = Q + (long long)min(q0 + l32, a.Sq - 1) * a.qs[2] + 4 * h;
+                for (int r = 0; r < 16; r++) s[i][r] = (those >> acc_row(r, 0) & 1u) != 0 ? 0.0f : s[i][r];
+                const float* kp = K + (long long)min(k0 + 32 * i + (ln & 31), a.Sk - 1) * a.ks[2] + 4 * (ln >> 5);
+                const float* qp = Q + (long long)min(q0 + (ln & 31), a.Sq - 1) * a.qs[2] + 4 * (ln >> 5);
 #pragma unroll 1
-                for (int d = 0; d < a.D; d += 8) Mma32<float>::run(s[i], *(const u32x4*)(qp + d), *(const u32x4*)(kp + d));
+                for (int d = 0; d < a.D; d += 8) Mma32<float>::run(s[i], *(const u32x4*)(qp + d) & mine, *(const u32x4*)(kp + d));
             }
         }
         int keys[2] = {k0 + l32, k0 + 32 + l32}, h = lane >> 5;

@@ -292,3 +292,32 @@ def test_probabilities_of_large_logits(eng, option, D):
     want, p, _ = reference(q, k, v, hidden)
     (o, _), (chosen, general) = versus_general_kernel(lambda eng: eng.ScaledDotProductAttention(q, k, v, ~hidden if option == "plane" else None, isCausal=option == "causal"), [want, p])
     assert chosen <= 1.3 * general
+
+
+@pytest.mark.parametrize("Sq,Sk", [(200, 200), (40, 1000)])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("option", ["plain", "padding"])
+@pytest.mark.parametrize("case", ["column", "first tile", "row"])
+def test_probabilities_beside_a_second_computation(eng, case, option, D, Sq, Sk):
+    """Where V or another row has the results computed again on the fp32 pipe, a row's probabilities and its sum are still of one pipe (apart, 2 to 5 times
+    the fp32 pipe's error over logits of deviation 64, 7 over 3600; bound as above)."""
+    for size in (8, 60):
+        q, k, v = randn(D, (1, 4, Sq, D), (1, 4, Sk, D), (1, 4, Sk, D))
+        q, k = q * size, k * size
+        if case == "column":
+            v[..., 3] *= 1e-12
+        elif case == "first tile":                              # far larger values at keys of no weight
+            v[:, :, :64] *= 1e12
+            k[:, :, :64, 1] = -1000.0 * size
+            q[..., 1] = size
+        else:                                                   # one row of small logits under a coarse scale
+            k[..., 0] = 0
+            q[:, :, 5] = 0
+            q[:, :, 5, 0] = size
+        hidden = None
+        if option == "padding":
+            hidden = torch.zeros(1, 1, 1, Sk, dtype=torch.bool, device="cuda")
+            hidden[..., Sk - 20:] = True
+        _, p, _ = reference(q, k, v, hidden)
+        (chosen, general), = versus_general_kernel(lambda eng: [eng.ScaledDotProductAttention(q, k, v, None if hidden is None else ~hidden)[1]], [p])
+        assert chosen <= 1.3 * general, (size, chosen, general)
